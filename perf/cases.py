@@ -304,3 +304,48 @@ def tolerance(case):
     if case.get("out") == "q8":  # a sum next to a rounding boundary: 4e-4 of the bytes, and 6e-6
         return {"differ": 2e-3 if aligned else 3e-5}
     return {"rel": 5e-5, "max": 4e-4} if aligned else {"rel": 3e-6, "max": 2.5e-5}
+
+
+def _in_64_bits(x, kind):
+    """A stored operand as float64."""
+    if kind in ("e4m3", "e5m2"):
+        x = x.view(torch.float8_e4m3fn if kind == "e4m3" else torch.float8_e5m2).float()
+    return x.double()
+
+
+def exact(case, seed):
+    """The result in 64 bits; the 8-bit outputs, and what a conversion writes, have no other value than the one they are compared with."""
+    if case["op"] == "cvt" or case.get("out") == "q8":
+        return None
+    state = prepare(case, seed)
+    if case.get("count", 1) > 1:
+        return [_exact_gemm(case, one["keep"][0], one["keep"][1], one["out"], one["keep"][2]) for one in state["keep"]]
+    m, n, k = case["m"], case["n"], case["k"]
+    a, b = state["keep"][0], state["keep"][1]
+    if case["op"] == "f4":
+        values = torch.tensor([0, 0.5, 1, 1.5, 2, 3, 4, 6, 0, -0.5, -1, -1.5, -2, -3, -4, -6], dtype=torch.float64, device="cuda")
+        w = values[torch.stack((b & 15, b >> 4), dim=-1).long()].reshape(n, k)
+        if case["scaled"]:
+            w *= torch.exp2(state["keep"][2].double() - 127).repeat_interleave(32, dim=1)
+        return (_in_64_bits(a, "e4m3") @ w.t())
+    if case["op"] == "k4":
+        return (a.double() @ b.permute(0, 2, 1).reshape(k, n).double()).round()
+    if case["op"] == "packed":
+        return _in_64_bits(a, case["kind"]) @ _in_64_bits(b, case["kind"])
+    return _exact_gemm(case, a, b, state["out"], state["keep"][2])
+
+
+def _exact_gemm(case, a, b, c, bias):
+    a, b = _in_64_bits(a, case["kind"]), _in_64_bits(b, case["kind"])
+    v = (a.t() if case["layout"] == "tn" else a) @ (b.t() if case["layout"] == "nt" else b)
+    if case["beta"]:
+        v += case["beta"] * c.double()
+    if case["bias"]:
+        v += bias.double()
+    if case["act"] == "relu":
+        v = torch.relu(v)
+    elif case["act"] == "silu":
+        v = v * torch.sigmoid(v)
+    elif case["act"] == "gelu":
+        v = 0.5 * v * (1 + torch.erf(v / math.sqrt(2)))
+    return v
