@@ -6,18 +6,31 @@
 // Every element of C is accumulated exactly as the reference's loop does it - k ascending, a separately rounded
 // multiply and add per step (f16: the sum rounded to half per step) - so results equal the reference's bit for
 // bit for finite data, like the any-stride kernel's; what changes is where the operands come from: a workgroup
-// of 256 threads keeps a 128 x 128 (or 64 x 64) tile of C in registers, 8 x 8 (4 x 4) per thread, and walks K in
-// slabs of 16 staged through LDS (two stages, the next slab's global loads issued before the current slab's
-// arithmetic). A thread's rows and columns are two runs of TM/2, half a tile apart, so that the lanes of a wave
+// keeps a tile of C in registers and walks K in slabs of 16 or 32 staged through LDS (two stages, the next slab's
+// global loads issued before the current slab's arithmetic, four elements per load along the operand's unit stride).
+// A thread's rows and columns are runs of up to four, a share of the tile apart, so that the lanes of a wave
 // read consecutive 16-byte pieces of the LDS rows. The last slab is zero-filled past K: adding the product
 // (+0)*(+0) leaves an accumulator unchanged, and an accumulator that started at +0 is never -0.
+//
+// What bounds it: the order of the sum is fixed, so K cannot be shared out, and a wave alone on its SIMD issues one
+// vector instruction in five to six cycles where several waves together issue one in three. So a tile is split over
+// as many waves as its LDS reads allow: 8 x 4 per thread on the 128 x 128 tile (8 x 8, one wave per SIMD at
+// 2048^3: 600 us; 8 x 4: 345), and fewer elements per thread, on smaller tiles, the fewer tiles there are - which
+// also shortens the chain of K steps that every thread goes through (f32 512 x 512 x 2048: 64 x 64 tiles of 4 x 4
+// per thread 182 us, 4 x 2 121, 32 x 32 tiles of 2 x 2 78, 16 x 32 tiles of 2 x 1 70).
+// f32 2048^3: 427 us with 64 x 64 tiles, one element per load and bounds checks on each -> 345 us, 50 T
+// vector operations per second (a multiply and an add per step); 4096 x 4096 x 2048 1381 -> 1243 us, 55 T.
 #include <hip/hip_runtime.h>
+
+#include <type_traits>
 
 #include "skl_device.hpp"
 
 namespace {
 
-constexpr int kThreads = 256;
+// Whether the beta == 0 case needs the old C at all (kinds that cannot tell say yes).
+__device__ __forceinline__ bool tiled_needs_c(float acc, skl_scalar alpha, skl_scalar beta) { return skl_initialise_needs_c(acc, alpha, beta); }
+__device__ __forceinline__ bool tiled_needs_c(double, skl_scalar, skl_scalar) { return true; }
 
 template <int DT>
 struct Kind;
@@ -59,133 +72,186 @@ struct TiledArgs {
   size_t rsc0, csc0, rsc1, csc1;
   skl_scalar alpha, beta;
   unsigned tiles_n;
-  int a_along_k, b_along_k;  // lanes run along K when fetching (the operand's unit stride is along K)
 };
 
-// One operand's share of a slab: BT rows/columns x kSlab k (16, or 8 for the 128 x 128 tile of doubles, whose
-// two stages would not fit the 64 KiB of static LDS otherwise), kPer elements per thread. Element e of the thread is
-// (x, p) = (e*kThreads + tid) split along K first (`along_k`) or along x first.
-template <int DT, int BT, int kSlab>
+// N values that lie side by side, at the alignment of one of them: the memory unit takes 16-byte accesses on any
+// element boundary, so no layout needs a copy or a path of its own for its alignment.
+template <typename T, int N>
+struct Run {
+  typedef T Vec __attribute__((ext_vector_type(N)));
+  typedef Vec Type __attribute__((aligned(sizeof(T))));
+};
+
+// One operand's share of a slab: BT rows (columns) x kSlab k, in groups of four elements along the operand's unit
+// stride (K if KC, else its rows / columns); kGroups groups per thread. A thread's groups keep their place from slab to
+// slab, so the addresses are worked out once.
+template <int DT, int BT, int kSlab, int kThreads, bool KC>
 struct Fetch {
-  static constexpr int kPer = BT * kSlab / kThreads;
+  static constexpr int kTotal = BT * kSlab / 4, kGroups = (kTotal + kThreads - 1) / kThreads;
   using In = typename Kind<DT>::In;
   using Stage = typename Kind<DT>::Stage;
+  using Four = typename Run<In, 4>::Type;
+  const In *at[kGroups];  // the group's first element in the first slab (clamped into the operand)
+  int inside[kGroups];    // elements along the rows / columns in range: 4 or fewer (KC: 1 or 0)
+  size_t s0, sk;
+  bool unit;              // the stride groups run along is 1
 
-  __device__ static void coords(int e, int tid, int along_k, int &x, int &p) {
-    const int idx = e * kThreads + tid;
-    if (along_k) {
-      p = idx % kSlab;
-      x = idx / kSlab;
-    } else {
-      x = idx % BT;
-      p = idx / BT;
+  __device__ static int group(int e) { return e * kThreads + (int)threadIdx.x; }
+  __device__ static bool whole(int e) { return kTotal % kThreads == 0 || group(e) < kTotal; }
+  __device__ static int x_of(int e) { return KC ? group(e) / (kSlab / 4) : group(e) % (BT / 4) * 4; }
+  __device__ static int p_of(int e) { return KC ? group(e) % (kSlab / 4) * 4 : group(e) / (BT / 4); }
+
+  __device__ void init(const In *base, size_t s1, size_t s0_, size_t sk_, size_t x0, size_t xn) {
+    s0 = s0_, sk = sk_;
+    unit = (KC ? sk : s0) == 1;
+#pragma unroll
+    for (int e = 0; e < kGroups; ++e) {
+      const size_t x = x0 + (whole(e) ? x_of(e) : 0);
+      const size_t left = x < xn ? xn - x : 0;
+      inside[e] = KC ? left != 0 : left < 4 ? (int)left : 4;
+      const size_t y = left ? x : 0;
+      at[e] = base + (y / 64) * s1 + (y % 64) * s0 + (whole(e) ? p_of(e) : 0) * sk;
     }
   }
 
-  __device__ static void load(Stage (&r)[kPer], const In *base, size_t s1, size_t s0, size_t sk, size_t x0, size_t xn,
-                              size_t p0, size_t k, int tid, int along_k) {
+  // The slab that starts `p0` k into the operand and has `left` of them (kSlab or more: whole).
+  __device__ __forceinline__ void load(Stage (&r)[kGroups][4], size_t p0, size_t left) const {
 #pragma unroll
-    for (int e = 0; e < kPer; ++e) {
-      int x, p;
-      coords(e, tid, along_k, x, p);
-      const size_t xx = x0 + x, pp = p0 + p;
-      r[e] = (xx < xn && pp < k) ? Kind<DT>::stage(base[(xx / 64) * s1 + (xx % 64) * s0 + pp * sk]) : Stage(0);
+    for (int e = 0; e < kGroups; ++e) {
+      const In *g = at[e] + p0 * sk;
+      if (!whole(e)) continue;
+      if (left >= (size_t)kSlab && unit && inside[e] == (KC ? 1 : 4)) {
+        const Four v = *reinterpret_cast<const Four *>(g);
+#pragma unroll
+        for (int i = 0; i < 4; ++i) r[e][i] = Kind<DT>::stage(v[i]);
+      } else {
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          const bool in = KC ? inside[e] != 0 && (size_t)(p_of(e) + i) < left : i < inside[e] && (size_t)p_of(e) < left;
+          r[e][i] = in ? Kind<DT>::stage(g[i * (KC ? sk : s0)]) : Stage(0);
+        }
+      }
     }
   }
 
-  __device__ static void store(const Stage (&r)[kPer], Stage (*tile)[BT + 4], int tid, int along_k) {
+  __device__ __forceinline__ void store(const Stage (&r)[kGroups][4], Stage (*tile)[BT + 4]) const {
 #pragma unroll
-    for (int e = 0; e < kPer; ++e) {
-      int x, p;
-      coords(e, tid, along_k, x, p);
-      tile[p][x] = r[e];
+    for (int e = 0; e < kGroups; ++e) {
+      if (!whole(e)) continue;
+      const int x = x_of(e), p = p_of(e);
+      if constexpr (KC) {
+#pragma unroll
+        for (int i = 0; i < 4; ++i) tile[p + i][x] = r[e][i];
+      } else {
+        typedef Stage V4 __attribute__((ext_vector_type(4)));
+        *reinterpret_cast<V4 *>(&tile[p][x]) = V4{r[e][0], r[e][1], r[e][2], r[e][3]};
+      }
     }
   }
 };
 
-template <int DT, int TM>
-__global__ void __launch_bounds__(kThreads) gemm_tiled_kernel(TiledArgs g) {
+// A thread's rows (columns): T of them in runs of up to four, the runs a share of the tile apart.
+template <int BT, int T>
+__device__ constexpr int tiled_index(int t, int i) {
+  constexpr int W = T < 4 ? T : 4;
+  return (i / W) * (BT / (T / W)) + t * W + i % W;
+}
+template <int T, typename Stage, int BT>
+__device__ __forceinline__ void tiled_read(Stage (&v)[T], const Stage (&row)[BT], int t, int edge) {
+  constexpr int W = T < 4 ? T : 4;
+  typedef Stage V __attribute__((ext_vector_type(W)));
+#pragma unroll
+  for (int q = 0; q < T / W; ++q) {
+    const V x = *reinterpret_cast<const V *>(&row[q * (edge / (T / W)) + t * W]);
+#pragma unroll
+    for (int i = 0; i < W; ++i) v[q * W + i] = x[i];
+  }
+}
+
+template <int DT, int BM, int BN, int TR, int TC, int kSlab, bool A_KC, bool B_KC>
+__global__ void __launch_bounds__((BM / TR) * (BN / TC)) gemm_tiled_kernel(TiledArgs g) {
   using K = Kind<DT>;
   using Stage = typename K::Stage;
   using Acc = typename K::Acc;
-  constexpr int BT = 16 * TM;  // tile edge
-  constexpr int H = TM / 2;    // a thread's rows (columns): H at ty*H and H at BT/2 + ty*H
-  constexpr int kSlab = (sizeof(Stage) == 8 && TM == 8) ? 8 : 16;
-  constexpr int kUnrollK = TM == 8 ? 2 : 4;
-  using F = Fetch<DT, BT, kSlab>;
-  __shared__ Stage As[2][kSlab][BT + 4];
-  __shared__ Stage Bs[2][kSlab][BT + 4];
+  constexpr int kThreads = (BM / TR) * (BN / TC);
+  using FA = Fetch<DT, BM, kSlab, kThreads, A_KC>;
+  using FB = Fetch<DT, BN, kSlab, kThreads, B_KC>;
+  constexpr int kUnrollK = TR * TC >= 64 ? 2 : 4;
+  __shared__ __attribute__((aligned(16))) Stage As[2][kSlab][BM + 4];
+  __shared__ __attribute__((aligned(16))) Stage Bs[2][kSlab][BN + 4];
 
-  const int tid = threadIdx.x, ty = tid / 16, tx = tid % 16;
-  const size_t row0 = (size_t)(blockIdx.x / g.tiles_n) * BT, col0 = (size_t)(blockIdx.x % g.tiles_n) * BT;
-  const typename K::In *a = (const typename K::In *)g.a, *b = (const typename K::In *)g.b;
+  const int tid = threadIdx.x, ty = tid / (BN / TC), tx = tid % (BN / TC);
+  const size_t row0 = (size_t)(blockIdx.x / g.tiles_n) * BM, col0 = (size_t)(blockIdx.x % g.tiles_n) * BN;
 
-  Acc acc[TM][TM];
+  Acc acc[TR][TC];
 #pragma unroll
-  for (int r = 0; r < TM; ++r)
+  for (int r = 0; r < TR; ++r)
 #pragma unroll
-    for (int c = 0; c < TM; ++c) acc[r][c] = Acc(0);
+    for (int c = 0; c < TC; ++c) acc[r][c] = Acc(0);
 
-  Stage ra[F::kPer], rb[F::kPer];
-  const size_t slabs = (g.k + kSlab - 1) / kSlab;
-  F::load(ra, a, g.a_s1, g.a_s0, g.a_sk, row0, g.m, 0, g.k, tid, g.a_along_k);
-  F::load(rb, b, g.b_s1, g.b_s0, g.b_sk, col0, g.n, 0, g.k, tid, g.b_along_k);
-  F::store(ra, As[0], tid, g.a_along_k);
-  F::store(rb, Bs[0], tid, g.b_along_k);
+  FA fa;
+  FB fb;
+  fa.init((const typename K::In *)g.a, g.a_s1, g.a_s0, g.a_sk, row0, g.m);
+  fb.init((const typename K::In *)g.b, g.b_s1, g.b_s0, g.b_sk, col0, g.n);
+  Stage ra[FA::kGroups][4], rb[FB::kGroups][4];
+  fa.load(ra, 0, g.k);
+  fb.load(rb, 0, g.k);
+  fa.store(ra, As[0]);
+  fb.store(rb, Bs[0]);
   __syncthreads();
-  for (size_t s = 0; s < slabs; ++s) {
-    const int cur = (int)(s & 1);
-    if (s + 1 < slabs) {
-      F::load(ra, a, g.a_s1, g.a_s0, g.a_sk, row0, g.m, (s + 1) * kSlab, g.k, tid, g.a_along_k);
-      F::load(rb, b, g.b_s1, g.b_s0, g.b_sk, col0, g.n, (s + 1) * kSlab, g.k, tid, g.b_along_k);
+  int cur = 0;
+  for (size_t p0 = 0; p0 < g.k; p0 += kSlab, cur ^= 1) {
+    const size_t next = p0 + kSlab;
+    if (next < g.k) {
+      fa.load(ra, next, g.k - next);
+      fb.load(rb, next, g.k - next);
     }
 #pragma unroll kUnrollK  // a full unroll makes the compiler fetch a whole slab into registers (256 + AGPRs)
     for (int kk = 0; kk < kSlab; ++kk) {
-      Stage av[TM], bv[TM];
+      Stage av[TR], bv[TC];
+      tiled_read(av, As[cur][kk], ty, BM);
+      tiled_read(bv, Bs[cur][kk], tx, BN);
 #pragma unroll
-      for (int r = 0; r < H; ++r) {
-        av[r] = As[cur][kk][ty * H + r];
-        av[H + r] = As[cur][kk][BT / 2 + ty * H + r];
-        bv[r] = Bs[cur][kk][tx * H + r];
-        bv[H + r] = Bs[cur][kk][BT / 2 + tx * H + r];
-      }
+      for (int r = 0; r < TR; ++r)
 #pragma unroll
-      for (int r = 0; r < TM; ++r)
-#pragma unroll
-        for (int c = 0; c < TM; ++c) acc[r][c] = K::step(acc[r][c], av[r], bv[c]);
+        for (int c = 0; c < TC; ++c) acc[r][c] = K::step(acc[r][c], av[r], bv[c]);
     }
-    if (s + 1 < slabs) {
-      F::store(ra, As[cur ^ 1], tid, g.a_along_k);
-      F::store(rb, Bs[cur ^ 1], tid, g.b_along_k);
+    if (next < g.k) {
+      fa.store(ra, As[cur ^ 1]);
+      fb.store(rb, Bs[cur ^ 1]);
     }
     __syncthreads();
   }
 
-  typename K::C *cbase = (typename K::C *)g.c;
+  using Out = typename K::C;
+  using Wide = typename std::conditional<DT == SKL_DT_F16H, float, Out>::type;  // what alpha and beta are applied in
+  Out *cbase = (Out *)g.c;
+  const bool init = skl_beta_is_zero<Wide>(g.beta);
 #pragma unroll
-  for (int r = 0; r < TM; ++r) {
-    const size_t i = row0 + (r < H ? ty * H + r : BT / 2 + ty * H + (r - H));
+  for (int r = 0; r < TR; ++r) {
+    const size_t i = row0 + tiled_index<BM, TR>(ty, r);
     if (i >= g.m) continue;
+    Out *crow = cbase + (i / 64) * g.rsc1 + (i % 64) * g.rsc0;
+    // a row's old values are requested together, ahead of its first store
+    Out *cp[TC];
+    Wide old[TC];
 #pragma unroll
-    for (int c = 0; c < TM; ++c) {
-      const size_t j = col0 + (c < H ? tx * H + c : BT / 2 + tx * H + (c - H));
-      if (j >= g.n) continue;
-      typename K::C *cp = cbase + (i / 64) * g.rsc1 + (i % 64) * g.rsc0 + (j / 64) * g.csc1 + (j % 64) * g.csc0;
-      if constexpr (DT == SKL_DT_F16H) {
-        float wide = (float)*cp;
-        float *alias = &wide;
-        skl_update((float)acc[r][c], alias, g.alpha, g.beta);
-        *cp = (_Float16)wide;
-      } else {
-        skl_update(acc[r][c], cp, g.alpha, g.beta);
-      }
+    for (int c = 0; c < TC; ++c) {
+      const size_t j = col0 + tiled_index<BN, TC>(tx, c);
+      cp[c] = j < g.n ? crow + (j / 64) * g.csc1 + (j % 64) * g.csc0 : nullptr;
+      old[c] = Wide(0);
+      if (cp[c] && (!init || tiled_needs_c((Wide)acc[r][c], g.alpha, g.beta))) old[c] = (Wide)*cp[c];
+    }
+#pragma unroll
+    for (int c = 0; c < TC; ++c) {
+      if (!cp[c]) continue;
+      *cp[c] = (Out)(init ? skl_initialise((Wide)acc[r][c], &old[c], g.alpha, g.beta) : skl_combine((Wide)acc[r][c], old[c], g.alpha, g.beta));
     }
   }
 }
 
-template <int DT, int TM>
-int launch(const skl_gemm_canon *g) {
-  constexpr int BT = 16 * TM;
+template <int DT, int BM, int BN, int TR, int TC, int kSlab, bool A_KC, bool B_KC>
+int launch_layout(const skl_gemm_canon *g) {
   TiledArgs p;
   p.a = g->a, p.b = g->b, p.c = g->c;
   p.m = g->m, p.n = g->n, p.k = g->k;
@@ -193,23 +259,43 @@ int launch(const skl_gemm_canon *g) {
   p.b_s1 = g->b_s1, p.b_s0 = g->b_s0, p.b_sk = g->b_sk;
   p.rsc0 = g->rsc0, p.csc0 = g->csc0, p.rsc1 = g->rsc1, p.csc1 = g->csc1;
   p.alpha = g->alpha, p.beta = g->beta;
-  p.a_along_k = g->a_sk <= g->a_s0;
-  p.b_along_k = g->b_sk <= g->b_s0;
-  const size_t tm = (g->m + BT - 1) / BT, tn = (g->n + BT - 1) / BT;
+  const size_t tm = (g->m + BM - 1) / BM, tn = (g->n + BN - 1) / BN;
   if (tm * tn > 0x7FFFFFFFu) {
     skl_hip_record_error(-2, "gemm_tiled: too many tiles for one launch");
     return -2;
   }
   p.tiles_n = (unsigned)tn;
-  gemm_tiled_kernel<DT, TM><<<(unsigned)(tm * tn), kThreads, 0, skl_current_stream()>>>(p);
+  gemm_tiled_kernel<DT, BM, BN, TR, TC, kSlab, A_KC, B_KC><<<(unsigned)(tm * tn), (BM / TR) * (BN / TC), 0, skl_current_stream()>>>(p);
   return skl_check_launch("gemm_tiled");
 }
 
+template <int DT, int BM, int BN, int TR, int TC, int kSlab>
+int launch(const skl_gemm_canon *g) {
+  const bool a_kc = g->a_sk <= g->a_s0, b_kc = g->b_sk <= g->b_s0;
+  if (a_kc && b_kc) return launch_layout<DT, BM, BN, TR, TC, kSlab, true, true>(g);
+  if (a_kc) return launch_layout<DT, BM, BN, TR, TC, kSlab, true, false>(g);
+  if (b_kc) return launch_layout<DT, BM, BN, TR, TC, kSlab, false, true>(g);
+  return launch_layout<DT, BM, BN, TR, TC, kSlab, false, false>(g);
+}
+
+// The tile by the number of 64 x 64 and 32 x 32 tiles there are: the largest that still gives every SIMD several waves.
+// f32, us, at K = 2048 (128 x 128 / 64 x 64 of 4 x 4 / 64 x 64 of 4 x 2 / 32 x 32 / 16 x 32 tiles):
+//   4096^2: 1243 / 1275 / 1356 / 2110 / 3066    2048^2: 347 / 349 / 364 / 532 / 779
+//   1024^2: 349 / 180 / 132 / 159 / 220          512^2: 338 / 170 / 121 / 78 / 70     256^2: 337 / 169 / 121 / 76 / 61
 template <int DT>
 int launch_sized(const skl_gemm_canon *g) {
-  // 128 x 128 tiles once they fill the chip twice over, 64 x 64 below that
-  const size_t big = ((g->m + 127) / 128) * ((g->n + 127) / 128);
-  return big >= 512 ? launch<DT, 8>(g) : launch<DT, 4>(g);
+  constexpr int kSlab = sizeof(typename Kind<DT>::Stage) == 8 ? 16 : 32;  // 68 KiB of LDS for the largest tile of floats
+  const auto tiles = [&](size_t bm, size_t bn) { return ((g->m + bm - 1) / bm) * ((g->n + bn - 1) / bn); };
+  if (tiles(128, 128) >= 512) {
+    // doubles: twice the bytes of LDS per step, so 8 x 8 per thread (4096 x 4096 x 2048: 8 x 4 2517 us, 8 x 8
+    // 2203 us)
+    if constexpr (sizeof(typename Kind<DT>::Stage) == 8) return launch<DT, 128, 128, 8, 8, 8>(g);
+    else return launch<DT, 128, 128, 8, 4, kSlab>(g);
+  }
+  if (tiles(64, 64) >= 768) return launch<DT, 64, 64, 4, 4, kSlab>(g);
+  if (tiles(64, 64) >= 176) return launch<DT, 64, 64, 4, 2, 16>(g);
+  if (tiles(32, 32) > 256) return launch<DT, 32, 32, 2, 2, kSlab>(g);
+  return launch<DT, 16, 32, 2, 1, kSlab>(g);
 }
 
 }  // namespace

@@ -1105,6 +1105,26 @@ def test_register_tiled_kernel_bit_identical(gpu, ta):
         assert np.array_equal(got.view(np.uint8), want.view(np.uint8)), (ta, i, vars(case))
 
 
+@pytest.mark.parametrize("ta", ("f32", "f64", "f16h"))
+@pytest.mark.parametrize("m,n,k", ((1, 30, 33), (16, 32, 32), (17, 35, 31), (40, 47, 129), (513, 517, 33), (830, 901, 18), (1730, 1797, 35)))
+def test_register_tiled_kernel_at_the_edges_of_its_tiles(gpu, ta, m, n, k):
+    """The tiles of fewer than 64 x 64 and the two of 64 x 64 (16 x 32, 32 x 32 from 257 tiles on, 64 x 64 from 176 and
+    from 768 on), with remainders in M, N and K, rows at every alignment, operands contiguous along either dimension and
+    along none: bit for bit. C starts as -0 here and there, so that the sign of zeros with beta == 0 is seen."""
+    from support import GemmCase
+    for i, (a_strides, b_strides) in enumerate((((k, 1), (n, 1)), ((1, m), (1, k)), ((k + 1, 1), (1, k + 3)), ((1, m + 1), (n + 3, 1)),
+                                                ((2 * k + 1, 2), (3, 3 * k)))):
+        alpha, beta = ((1.0, 0.0), (1.5, -0.5))[i % 2]
+        case = GemmCase(ta, None, alpha, beta, m0=1, n0=1, k0=1, m1=m, n1=n, k1=k, rsa0=0, csa0=0, rsa1=a_strides[0], csa1=a_strides[1],
+                        rsb0=0, csb0=0, rsb1=b_strides[0], csb1=b_strides[1], rsc0=0, csc0=0, rsc1=n + i, csc1=1)
+        a, b, c = case.make_inputs(9700 + i)
+        a[: k if i in (0, 2) else 1] = 0
+        c[::7] = -0.0
+        want = run_oracle_gemm(case, a, b, c)
+        got = run_gemm(gpu, "rcprc", case, a, b, c, "device")
+        assert np.array_equal(got.view(np.uint8), want.view(np.uint8)), (ta, i, vars(case))
+
+
 @pytest.mark.parametrize("ta,tb", (("i8", "i8"), ("bf16", "bf16"), ("f16", "f16"), ("f8e4m3", "f8e4m3"), ("f8e4m3", "f8e5m2")))
 def test_ragged_problems_on_padded_copies(gpu, ta, tb):
     """Ragged M, N and K (and odd leading dimensions) on a problem large enough to fill the chip: A and B are copied
