@@ -584,6 +584,113 @@ __device__ __forceinline__ void write_wave_tile(const MfmaArgs &p, const Acc (&a
   fused.finish();
 }
 
+// ---------------------------------------------------------------------------
+// The streaming kernel's epilogue for fused calls with any activation and any 8-bit copy. Such steps - a GELU is some
+// fifty instructions - cannot be written out for each of a lane's 128 accumulators (spilled registers, code beyond the
+// instruction cache), and accumulators cannot be indexed by a loop counter. So a wave puts 32 rows of its tile at a time
+// into LDS, the operands' ring being over, and loops over them: a lane takes four neighbouring columns of a row, the
+// same columns every time, so their biases, scales and offsets are fetched once, and C and the copy go out 16 and 4
+// bytes per lane where the layout has them side by side. Every element goes through the same operations in the same
+// order as in the other epilogues. `stage`: this wave's 32 x (32 NI + 8) elements; eight elements of padding put the
+// two halves of a wave's writes, four rows apart, into different banks.
+// What it is worth: such calls ran on the bounds-checked 128 x 128 kernels; see launch_tile.
+// ---------------------------------------------------------------------------
+template <int NI>
+constexpr int staged_pitch() { return 32 * NI + 8; }
+template <int MI, int NI, bool CHECK, typename Acc>
+__device__ __forceinline__ void write_wave_tile_staged(const MfmaArgs &p, const Acc (&acc)[MI][NI], size_t row0, size_t col0, char *stage_bytes) {
+  using T = decltype(Acc{}.x);
+  typedef T V4 __attribute__((ext_vector_type(4)));
+  constexpr int P = staged_pitch<NI>(), kLanesPerRow = 8 * NI, kRowsPerPass = 64 / kLanesPerRow;
+  const int lane = (int)__builtin_amdgcn_mbcnt_hi(~0u, __builtin_amdgcn_mbcnt_lo(~0u, 0u));
+  T *const stage = reinterpret_cast<T *>(stage_bytes);
+  T *const stage_in = stage + (lane >> 5) * 4 * P + (lane & 31);
+  const int r_first = lane / kLanesPerRow, c_first = lane % kLanesPerRow * 4;
+  const T *const stage_out = stage + r_first * P + c_first;
+  const size_t col = col0 + c_first;
+  const int cols = !CHECK ? 4 : col >= p.n ? 0 : p.n - col < 4 ? (int)(p.n - col) : 4;
+  const size_t rmask = (size_t(1) << p.crs) - 1, cmask = (size_t(1) << p.ccs) - 1;
+  const bool init = skl_beta_is_zero<T>(p.beta);
+  const T *const bias = reinterpret_cast<const T *>(p.bias);
+  size_t c_off[4];
+  T bias_of[4];
+  float scale_of[4];
+#pragma unroll
+  for (int e = 0; e < 4; ++e) {
+    const size_t j = e < cols ? col + e : 0;
+    c_off[e] = (j >> p.ccs) * p.csc1 + (j & cmask) * p.csc0;
+    bias_of[e] = bias && e < cols ? bias[j] : T(0);
+    scale_of[e] = p.rq.q && e < cols ? p.rq.q_scale[p.rq.q_per_column ? j : 0] : 0.0f;
+  }
+  // C's four columns side by side on a 16-byte boundary (columns come in blocks of 2^ccs, col is a multiple of four), and
+  // the copy's four bytes on a dword
+  const bool c_run = cols == 4 && p.csc0 == 1 && p.ccs >= 2 && (((uintptr_t)p.c | (p.csc1 * 4) | (p.rsc0 * 4) | (p.rsc1 * 4)) & 15) == 0;
+  const bool q_run = cols == 4 && p.rq.csq == 1 && (p.rq.rsq & 3) == 0 && ((uintptr_t)p.rq.q & 3) == 0;
+  T running = skl_lowest<T>();
+#pragma unroll
+  for (int i = 0; i < MI; ++i) {
+#pragma unroll
+    for (int j = 0; j < NI; ++j)
+#pragma unroll
+      for (int r = 0; r < 16; ++r) stage_in[((r >> 2) * 8 + (r & 3)) * P + j * 32] = acc[i][j][r];
+    // the wave's own LDS accesses complete in order; the compiler must not move them across each other
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+#pragma unroll 1
+    for (int pass = 0; pass < 32 / kRowsPerPass; ++pass) {
+      const V4 sum = *reinterpret_cast<const V4 *>(stage_out + pass * kRowsPerPass * P);
+      const size_t row = row0 + (size_t)(i * 32 + pass * kRowsPerPass + r_first);
+      if (CHECK && (row >= p.m || cols == 0)) continue;
+      T *const c_row = reinterpret_cast<T *>(p.c) + (row >> p.crs) * p.rsc1 + (row & rmask) * p.rsc0;
+      V4 old = {T(0), T(0), T(0), T(0)};
+      bool need = !init;
+#pragma unroll
+      for (int e = 0; e < 4; ++e) need |= init && skl_initialise_needs_c(sum[e], p.alpha, p.beta);
+      if (need) {
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
+          if (e < cols) old[e] = c_row[c_off[e]];
+      }
+      V4 v;
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        T x = init ? skl_initialise_with(sum[e], old[e], p.alpha, p.beta) : skl_combine(sum[e], old[e], p.alpha, p.beta);
+        if (bias) x = skl_add_bias(x, bias_of[e]);
+        v[e] = skl_activate(x, p.rq.act);
+        if (p.max && e < cols && v[e] > running) running = v[e];
+      }
+      if (!p.rq.q_only) {
+        if (c_run) {
+          __builtin_nontemporal_store(v, reinterpret_cast<V4 *>(c_row + c_off[0]));
+        } else {
+#pragma unroll
+          for (int e = 0; e < 4; ++e)
+            if (e < cols) c_row[c_off[e]] = v[e];
+        }
+      }
+      if (p.rq.q) {
+        unsigned packed = 0;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) packed |= ((unsigned)skl_quantise((float)v[e], scale_of[e], p.rq.q_zero, p.rq.q_fmt) & 0xFFu) << (8 * e);
+        int8_t *const q = reinterpret_cast<int8_t *>(p.rq.q) + row * p.rq.rsq + col * p.rq.csq;
+        if (q_run) {
+          *reinterpret_cast<unsigned *>(q) = packed;
+        } else {
+#pragma unroll
+          for (int e = 0; e < 4; ++e)
+            if (e < cols) q[e * p.rq.csq] = (int8_t)(packed >> (8 * e));
+        }
+      }
+    }
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+  }
+  if (p.max) {
+    const T best = skl_wave_max(running);
+    if (lane == 0 && best > skl_lowest<T>()) skl_atomic_max(reinterpret_cast<T *>(p.max), best);
+  }
+}
+
 // Tile index of a workgroup. Consecutive workgroup ids go to different XCDs
 // (eight of them, each with its own L2), so ids are first regrouped per XCD into
 // contiguous ranges, then walked in column-major groups of kGroupM tile rows so
@@ -747,6 +854,7 @@ __global__ void __launch_bounds__(WAVES_M *WAVES_N * 64, (BM == 128 ? 4 : 6)) ge
 // halves of such a load next to each other: one KiB, as the load writes it.
 // ===========================================================================
 constexpr int kRingSlice = 64;   // bytes of K per stage
+constexpr int kStagedSteps = 4;  // EXTRA: any fused steps, by write_wave_tile_staged
 constexpr int kRingStages = 4;
 // Stages of the ring for tiles of BN columns. The kernel's load schedule is written for any even number of stages;
 // four it is for both tile widths: six stages for the 256 x 128 tile (144 KiB; its slices take half the time, so
@@ -1366,6 +1474,11 @@ __global__ void __launch_bounds__(512) gemm_mfma_ring_kernel(MfmaArgs p) {
     MfmaArgs q = p;
     if (any == 0) q.beta.fz.skip_c_read = 1;  // 0 * c is a zero everywhere in this tile
     write_wave_tile<MI, NI, EDGE, EXTRA>(q, acc, m0 + wm, n0 + wn);
+  } else if constexpr (EXTRA == kStagedSteps) {
+    constexpr int kStageBytes = 32 * staged_pitch<NI>() * 4;
+    static_assert(WAVES * kStageBytes <= TileA::kRegion + TileB::kRegion, "the waves' rows take the place of the operand stages");
+    __syncthreads();  // every wave's reads of the stages and loads into them are over
+    write_wave_tile_staged<MI, NI, EDGE>(p, acc, m0 + wm, n0 + wn, smem + wave * kStageBytes);
   } else {
     write_wave_tile<MI, NI, EDGE, EXTRA>(p, acc, m0 + wm, n0 + wn);
   }
@@ -1414,9 +1527,10 @@ struct SequenceGuard {
 
 constexpr size_t kRingMinSlicesPerSplit = 64;  // below 8 KiB of K per row the pass over the planes costs what the split saves
 
-// The streaming kernels for whole tiles also exist with the activation (none or ReLU) and requantisation steps, for a
-// copy that can be written as dwords (a quantised layer's 8-bit output at a quarter of C's bytes: int8 behind an
-// int32 C, fp8 behind an fp32 C); every other call with those steps goes to the bounds-checked kernels.
+// The streaming kernels for whole tiles also exist with the activation (none or ReLU) and requantisation steps written
+// out per accumulator, for a copy that can be written as dwords (a quantised layer's 8-bit output at a quarter of C's
+// bytes: int8 behind an int32 C, fp8 behind an fp32 C); every other call with those steps takes the epilogue that loops
+// over rows in LDS (kStagedSteps).
 template <int TA, int TB>
 constexpr bool kRingCarriesExtraSteps = TA == TB;   // every kind but the mixed fp8 pairings
 
@@ -1429,6 +1543,11 @@ inline bool c_in_row_quads(const MfmaArgs &p) {
 
 template <int TA, int TB, bool A_KC, bool B_KC, int BN, bool EDGE = false, int EXTRA = 0, bool CQUADS = false, bool SCAN = false>
 int launch_ring(const MfmaArgs &args) {
+  if constexpr (EXTRA == 0 && !CQUADS && !SCAN) {
+    using Steps = FusedSteps<decltype(typename Kind<TA>::Acc{}.x), 2>;
+    if ((args.rq.act || args.rq.q) && !(kRingCarriesExtraSteps<TA, TB> && !EDGE && Steps::dword_copy(args.rq)))
+      return launch_ring<TA, TB, A_KC, B_KC, BN, EDGE, kStagedSteps>(args);
+  }
   if constexpr (EXTRA == 0 && kRingCarriesExtraSteps<TA, TB> && !EDGE) {
     if (args.rq.q) return args.rq.q_only ? launch_ring<TA, TB, A_KC, B_KC, BN, EDGE, 2>(args) : launch_ring<TA, TB, A_KC, B_KC, BN, EDGE, 3>(args);
   }
@@ -1575,10 +1694,7 @@ int launch_tile(const MfmaArgs &p) {
   // The streaming kernel takes problems that its tiles divide evenly: 256 x 256 tiles when those
   // can fill the 256 compute units, 256 x 128 tiles for the sizes below that; everything else runs
   // on the small, bounds-checked kernel.
-  // activation / requantised copy: on the streaming kernel only int8 with a copy that goes out as dwords
-  using AccElem = decltype(typename Kind<TA>::Acc{}.x);
-  const bool extra_steps = (p.rq.act || p.rq.q) && !(kRingCarriesExtraSteps<TA, TB> && FusedSteps<AccElem, 2>::dword_copy(p.rq));
-  if (!extra_steps && p.m % 256 == 0 && (p.k * ES) % 128 == 0) {
+  if (p.m % 256 == 0 && (p.k * ES) % 128 == 0) {
     const size_t tiles_m = p.m / 256;
     if (p.n % 256 == 0 && tiles_m * (p.n / 256) >= 200) {
       // A last round that would fill at most half of the 256 compute units is run as 256 x 128 tiles

@@ -1125,6 +1125,39 @@ def test_register_tiled_kernel_at_the_edges_of_its_tiles(gpu, ta, m, n, k):
         assert np.array_equal(got.view(np.uint8), want.view(np.uint8)), (ta, i, vars(case))
 
 
+@pytest.mark.parametrize("ta", ("i8", "bf16", "f8e4m3"))
+@pytest.mark.parametrize("m,n,k,a_pad,c_by_columns", ((2304, 2048, 2432, 0, False), (2304, 2048, 2432, 0, True), (1537, 2051, 2500, 1, False), (1537, 2051, 2500, 1, True)))
+def test_fused_steps_looped_over_rows(gpu, ta, m, n, k, a_pad, c_by_columns):
+    """The streaming kernel's epilogue for any activation and any 8-bit copy, on whole tiles and on padded copies of
+    operands off the 16-byte rule (C and the copy end inside a tile): C row-major and by columns, the copy in dwords, in
+    bytes and by columns. The same call without those steps runs on the same kernel and is the anchor: what they make of
+    its C must come out bit for bit (SiLU: within the reference's bounds)."""
+    from support import GemmCase
+    rng = np.random.default_rng(m + n + k + a_pad)
+    rsc, csc = (1, m + 2) if c_by_columns else (n + (4 - n) % 4, 1)
+    beta = 1 if c_by_columns else 0
+    case = GemmCase(ta, None if ta == "i8" else ta, 1, beta, m0=1, n0=1, k0=1, m1=m, n1=n, k1=k, rsa0=0, csa0=0, rsa1=k + (3 * a_pad) + (-k) % 16 * (1 - a_pad), csa1=1,
+                    rsb0=0, csb0=0, rsb1=n + (1 - n % 2) * a_pad, csb1=1, rsc0=0, csc0=0, rsc1=rsc, csc1=csc)
+    a, b, c = case.make_inputs(int(rng.integers(1 << 30)))
+    bias = rng.integers(-1 << 12, 1 << 12, n).astype(np.int32) if case.is_int else rng.uniform(-4, 4, n).astype(np.float32)
+    start = np.array([-(1 << 31)], np.int32) if case.is_int else np.array([-np.inf], np.float32)
+    anchor, _ = run_fused_gemm(gpu, "rc", case, a, b, c, bias, None, "device")
+    scales = (rng.uniform(0.5, 2.0, n) * 100.0 / float(np.abs(anchor.astype(np.float64)).max())).astype(np.float32)
+    for rsq, csq, only in ((n + (-n) % 4, 1, False), (n + 5, 1, True), (1, m + 5, False)):
+        rq = dict(q=np.full((m - 1) * rsq + (n - 1) * csq + 1, 0x55, np.int8), rsq=rsq, csq=csq, scale=scales, per_column=True, zero=3, only=only)
+        got, top, q = run_fused_gemm(gpu, "rc", case, a, b, c, bias, start, "device", activation=1, requant=rq)
+        want_c, want_top, want_q = fused_expectation(case, anchor, None, start, activation=1, requant=rq)
+        assert np.array_equal(q, want_q) and top[0] == want_top[0], (ta, rsq, csq)
+        assert np.array_equal(got.view(np.uint8), (c if only else want_c).view(np.uint8)), (ta, rsq, csq)
+    if not case.is_int:
+        got, _ = run_fused_gemm(gpu, "rc", case, a, b, c, bias, None, "device", activation=2)
+        inside = np.zeros(c.shape, bool)
+        np.lib.stride_tricks.as_strided(inside, (m, n), (rsc, csc))[:] = True
+        assert np.array_equal(got[~inside].view(np.uint32), c[~inside].view(np.uint32))
+        err = support.ulp_error_f32(got[inside], support.activation_reference(anchor[inside], 2))
+        assert np.all(err <= support.activation_ulp_bound(anchor[inside], 2)), float(err.max())
+
+
 @pytest.mark.parametrize("ta,tb", (("i8", "i8"), ("bf16", "bf16"), ("f16", "f16"), ("f8e4m3", "f8e4m3"), ("f8e4m3", "f8e5m2")))
 def test_ragged_problems_on_padded_copies(gpu, ta, tb):
     """Ragged M, N and K (and odd leading dimensions) on a problem large enough to fill the chip: A and B are copied
