@@ -63,12 +63,12 @@ extern "C" int skl_hip_gemm_mfma_padded_plan(const skl_gemm_canon *g, size_t *mp
   // place, is the faster one for merely ragged sizes (bf16 2000 x 5000 x 3000 with SiLU 127 against 139 us, E4M3
   // 1027 x 8190 x 4096 into E4M3 87 against 114), the padded copies behind its own copies (int8 3001 x 4099 x 5003
   // with ReLU into int8 172 against 124 us).
-  if ((g->rq.act || g->rq.q) && skl_hip_gemm_mfma_supported(g)) return 0;
+  if ((g->rq.act || g->rq.q) && (skl_hip_gemm_mfma_supported(g) || (g->rq.act >= 2 && g->k * es < 2048))) return 0;
   if (fp8a && g->k <= kF8ExactMaxK) return 0;  // short K: the exact fp8 product, which the streaming kernel does not have
   const size_t tiles_m = (g->m + 255) / 256;
   int tile_cols = 0;
   if (tiles_m * ((g->n + 255) / 256) >= 200) tile_cols = 256;
-  else if (tiles_m * ((g->n + 127) / 128) >= 96) tile_cols = 128;
+  else if (tiles_m * ((g->n + 127) / 128) >= (g->rq.act || g->rq.q ? 200 : 96)) tile_cols = 128;  // the rules of launch_whole_tiles
   if (!tile_cols) return 0;
   *mp = tiles_m * 256;
   *np = (g->n + tile_cols - 1) / tile_cols * tile_cols;

@@ -593,7 +593,10 @@ __device__ __forceinline__ void write_wave_tile(const MfmaArgs &p, const Acc (&a
 // bytes per lane where the layout has them side by side. Every element goes through the same operations in the same
 // order as in the other epilogues. `stage`: this wave's 32 x (32 NI + 8) elements; eight elements of padding put the
 // two halves of a wave's writes, four rows apart, into different banks.
-// What it is worth: such calls ran on the bounds-checked 128 x 128 kernels; see launch_tile.
+// Such calls ran on the bounds-checked 128 x 128 kernels: bf16 2048 x 8192 x 4096 with SiLU 188 -> 137 us, int8 4096^3
+// with ReLU 105 -> 72, E4M3 2048 x 8192 x 4096 with GELU into E4M3 125 -> 99 (110 while every lane multiplied out the
+// addresses of its rows); what is left of the last over the same call with ReLU, 37 us, is mostly the erfc of 16.8 million
+// elements. launch_whole_tiles says where the line lies.
 // ---------------------------------------------------------------------------
 template <int NI>
 constexpr int staged_pitch() { return 32 * NI + 8; }
@@ -626,6 +629,12 @@ __device__ __forceinline__ void write_wave_tile_staged(const MfmaArgs &p, const 
   // the copy's four bytes on a dword
   const bool c_run = cols == 4 && p.csc0 == 1 && p.ccs >= 2 && (((uintptr_t)p.c | (p.csc1 * 4) | (p.rsc0 * 4) | (p.rsc1 * 4)) & 15) == 0;
   const bool q_run = cols == 4 && p.rq.csq == 1 && (p.rq.rsq & 3) == 0 && ((uintptr_t)p.rq.q & 3) == 0;
+  // A pass covers four rows from a multiple of four on, which lie in one block of C: where they start is the same for the
+  // whole wave (scalar arithmetic), the lane's row among them a constant.
+  static_assert(kRowsPerPass == 4, "four rows per pass");
+  T *const c_lane = reinterpret_cast<T *>(p.c) + (size_t)r_first * p.rsc0;
+  int8_t *const q_lane = reinterpret_cast<int8_t *>(p.rq.q) + (size_t)r_first * p.rq.rsq + col * p.rq.csq;
+  const skl_fp8::Ofp8Format f8(p.rq.q_fmt);
   T running = skl_lowest<T>();
 #pragma unroll
   for (int i = 0; i < MI; ++i) {
@@ -636,12 +645,12 @@ __device__ __forceinline__ void write_wave_tile_staged(const MfmaArgs &p, const 
     // the wave's own LDS accesses complete in order; the compiler must not move them across each other
     __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
     __builtin_amdgcn_wave_barrier();
-#pragma unroll 1
+#pragma unroll 2
     for (int pass = 0; pass < 32 / kRowsPerPass; ++pass) {
       const V4 sum = *reinterpret_cast<const V4 *>(stage_out + pass * kRowsPerPass * P);
-      const size_t row = row0 + (size_t)(i * 32 + pass * kRowsPerPass + r_first);
-      if (CHECK && (row >= p.m || cols == 0)) continue;
-      T *const c_row = reinterpret_cast<T *>(p.c) + (row >> p.crs) * p.rsc1 + (row & rmask) * p.rsc0;
+      const size_t four = row0 + (size_t)(i * 32 + pass * kRowsPerPass);  // a scalar
+      if (CHECK && (four + r_first >= p.m || cols == 0)) continue;
+      T *const c_row = c_lane + ((four >> p.crs) * p.rsc1 + (four & rmask) * p.rsc0);
       V4 old = {T(0), T(0), T(0), T(0)};
       bool need = !init;
 #pragma unroll
@@ -671,8 +680,12 @@ __device__ __forceinline__ void write_wave_tile_staged(const MfmaArgs &p, const 
       if (p.rq.q) {
         unsigned packed = 0;
 #pragma unroll
-        for (int e = 0; e < 4; ++e) packed |= ((unsigned)skl_quantise((float)v[e], scale_of[e], p.rq.q_zero, p.rq.q_fmt) & 0xFFu) << (8 * e);
-        int8_t *const q = reinterpret_cast<int8_t *>(p.rq.q) + row * p.rq.rsq + col * p.rq.csq;
+        for (int e = 0; e < 4; ++e) {
+          const unsigned byte = p.rq.q_fmt == 0 ? (unsigned)skl_requantise_int((float)v[e], scale_of[e], p.rq.q_zero) & 0xFFu
+                                                : skl_fp8::encode_ofp8_hw(__fmul_rn((float)v[e], scale_of[e]), f8) & 0xFFu;
+          packed |= byte << (8 * e);
+        }
+        int8_t *const q = q_lane + four * p.rq.rsq;
         if (q_run) {
           *reinterpret_cast<unsigned *>(q) = packed;
         } else {
@@ -1060,16 +1073,21 @@ constexpr int ceil_div(int a, int b) { return (a + b - 1) / b; }
 // layout of C, 64-bit block arithmetic per load - cost 62-70 us of 415 whether it loaded 4 bytes per lane every slice
 // or 16 every other one, 25-43 us of that with the rows already in cache: the instructions between two MFMAs, not the
 // loads. Hence contiguous rows, whose address is a scalar product and a shift of the lane index.)
-template <int TA, int TB, bool A_KC, bool B_KC, int BN, bool EDGE = false, int EXTRA = 0, bool CQUADS = false, bool SCAN = false>
+// EXACT: OCP fp8 operands multiplied exactly (MmaF8Exact). The bytes travel and are read like int8's; a fragment is
+// widened behind the MFMAs in front of its first use, B's NI and A's first at the top of the k-step. A wave widens
+// MI + NI fragments for MI x NI products - on the 128 x 128 kernels, with 64 x 32 per wave, three for two, which is
+// more vector work than the matrix cores take for the products; here six for eight. E4M3 2048 x 8192 x 2048: 77 us there,
+// 62 here (1.1 PFLOP/s, what the f16 kernel reaches).
+template <int TA, int TB, bool A_KC, bool B_KC, int BN, bool EDGE = false, int EXTRA = 0, bool CQUADS = false, bool SCAN = false, bool EXACT = false>
 __global__ void __launch_bounds__(512) gemm_mfma_ring_kernel(MfmaArgs p) {
   using KA = Kind<TA>;
-  using M = Mma<TA, TB>;
+  using M = typename std::conditional<EXACT, MmaF8Exact<TA, TB>, Mma<TA, TB>>::type;
   using Frag = typename M::Frag;
   using Acc = typename KA::Acc;
   using AccElem = decltype(Acc{}.x);
   constexpr int SB = kRingSlice, STAGES = ring_stages(BN);
   static_assert(STAGES % 2 == 0, "pair loads fill two neighbouring stages");
-  constexpr int ES = KA::ES, KB = KA::KB, FRB = KB / 2;
+  constexpr int ES = KA::ES, KB = EXACT ? 32 : KA::KB, FRB = KB / 2;
   // Eight waves: 2 x 4 blocks of 128 x 64 on a 256 x 256 tile, 4 x 2 blocks of 64 x 64 on a 256 x 128 one.
   constexpr int BM = 256, WAVES = 8, WAVES_N = BN == 256 ? 4 : 2, WAVES_M = WAVES / WAVES_N;
   constexpr int WM = BM / WAVES_M, WN = BN / WAVES_N, MI = WM / 32, NI = WN / 32;
@@ -1311,6 +1329,18 @@ __global__ void __launch_bounds__(512) gemm_mfma_ring_kernel(MfmaArgs p) {
                     for (int i = 0; i < MI; ++i) fa[i] = join_pieces<Frag>(pa[cur][i]);
 #pragma unroll
                     for (int j = 0; j < NI; ++j) fb[j] = join_pieces<Frag>(pb[cur][j]);
+                    decltype(prep_a<M>(fa[0])) wa[MI];  // as the multiply wants them
+                    decltype(prep_b<M>(fb[0])) wb[NI];
+                    if constexpr (EXACT) {
+                      wa[0] = prep_a<M>(fa[0]);
+#pragma unroll
+                      for (int j = 0; j < NI; ++j) wb[j] = prep_b<M>(fb[j]);
+                    } else {
+#pragma unroll
+                      for (int i = 0; i < MI; ++i) wa[i] = fa[i];
+#pragma unroll
+                      for (int j = 0; j < NI; ++j) wb[j] = fb[j];
+                    }
                     const unsigned sa = addr_a + (kLast ? nxt_a : cur_a) * TileA::kStageStep;
                     const unsigned sb = addr_b + (kLast ? nxt_b : cur_b) * TileB::kStageStep;
                     __builtin_amdgcn_sched_barrier(0);
@@ -1319,13 +1349,14 @@ __global__ void __launch_bounds__(512) gemm_mfma_ring_kernel(MfmaArgs p) {
                           [&](auto qc) {
                             constexpr int Q = decltype(qc)::value, kSlot = KS * kMfmas + Q;
                             constexpr int i = Q / NI, j = Q % NI;
-                            acc[i][j] = M::run(fa[i], fb[j], acc[i][j]);
+                            acc[i][j] = M::run(wa[i], wb[j], acc[i][j]);
                             // The MFMA first, what belongs to its slot in its shadow. Left to itself the compiler moves a slot's address
                             // arithmetic, reads and loads in front of the MFMA - and behind a barrier, which the waves leave together,
                             // instructions in front of the first MFMA are a gap in every SIMD's matrix core at once (measured, same job,
                             // alternating libraries: int8 8192^3 -1.5 %, fp8 with column-major A -3 %, bf16 config 3 -2.3 %; for the
                             // extra instructions of SCAN the difference between +43 and +14 us).
                             __builtin_amdgcn_sched_barrier(0);
+                            if constexpr (EXACT && j == 0 && i + 1 < MI) wa[i + 1] = prep_a<M>(fa[i + 1]);
                             if constexpr (SCAN && U == 0 && kSlot == 0) scan_issue(s);
                             if constexpr (SCAN && kSlot == 1) scan_check();  // what the last slot of the k-step before has read, behind this k-step's lgkmcnt(0)
                             // Behind the barrier of slice 2q + 3 the rows requested in slice 2q have landed: half of them is
@@ -1541,14 +1572,14 @@ inline bool c_in_row_quads(const MfmaArgs &p) {
          (((uintptr_t)p.c | (p.rsc0 * 4) | (p.rsc1 * 4) | (p.csc1 * 4)) & 15) == 0;
 }
 
-template <int TA, int TB, bool A_KC, bool B_KC, int BN, bool EDGE = false, int EXTRA = 0, bool CQUADS = false, bool SCAN = false>
+template <int TA, int TB, bool A_KC, bool B_KC, int BN, bool EDGE = false, int EXTRA = 0, bool CQUADS = false, bool SCAN = false, bool EXACT = false>
 int launch_ring(const MfmaArgs &args) {
   if constexpr (EXTRA == 0 && !CQUADS && !SCAN) {
     using Steps = FusedSteps<decltype(typename Kind<TA>::Acc{}.x), 2>;
-    if ((args.rq.act || args.rq.q) && !(kRingCarriesExtraSteps<TA, TB> && !EDGE && Steps::dword_copy(args.rq)))
-      return launch_ring<TA, TB, A_KC, B_KC, BN, EDGE, kStagedSteps>(args);
+    if ((args.rq.act || args.rq.q) && !(kRingCarriesExtraSteps<TA, TB> && !EDGE && !EXACT && Steps::dword_copy(args.rq)))
+      return launch_ring<TA, TB, A_KC, B_KC, BN, EDGE, kStagedSteps, false, false, EXACT>(args);
   }
-  if constexpr (EXTRA == 0 && kRingCarriesExtraSteps<TA, TB> && !EDGE) {
+  if constexpr (EXTRA == 0 && kRingCarriesExtraSteps<TA, TB> && !EDGE && !EXACT) {
     if (args.rq.q) return args.rq.q_only ? launch_ring<TA, TB, A_KC, B_KC, BN, EDGE, 2>(args) : launch_ring<TA, TB, A_KC, B_KC, BN, EDGE, 3>(args);
   }
   if constexpr (TA == SKL_DT_I8 && TB == SKL_DT_I8 && A_KC && B_KC && !EDGE && EXTRA == 0 && !CQUADS) {  // what copies of blocked operands look like
@@ -1556,7 +1587,7 @@ int launch_ring(const MfmaArgs &args) {
   }
   constexpr int ES = Kind<TA>::ES;
   using AccElem = decltype(typename Kind<TA>::Acc{}.x);
-  if constexpr (std::is_same<AccElem, float>::value && !EDGE && EXTRA == 0 && !CQUADS && !SCAN) {
+  if constexpr (std::is_same<AccElem, float>::value && !EDGE && EXTRA == 0 && !CQUADS && !SCAN && !EXACT) {
     // beta == 0 evaluated as the reference's loops do (0 * c: a NaN or an infinity in C stays a NaN): the old C is
     // looked through while the tile is multiplied, 8 KiB of it per two slices - needs 64 slices on the wide tile, 32
     // on the narrow one, a tile to itself (no shared K) and a row-major C.
@@ -1573,7 +1604,7 @@ int launch_ring(const MfmaArgs &args) {
       return launch_ring<TA, TB, A_KC, B_KC, BN, EDGE, EXTRA, CQUADS, true>(args);
   }
   constexpr int lds = ring_stages(BN) * (256 + BN) * kRingSlice + (SCAN ? 4 * 8 * 1024 : 0);
-  auto kernel = gemm_mfma_ring_kernel<TA, TB, A_KC, B_KC, BN, EDGE, EXTRA, CQUADS, SCAN>;
+  auto kernel = gemm_mfma_ring_kernel<TA, TB, A_KC, B_KC, BN, EDGE, EXTRA, CQUADS, SCAN, EXACT>;
   static std::atomic<bool> configured{false};  // per instantiation; racing threads set the same value
   if (!configured.load(std::memory_order_acquire)) {
     int rc = skl_check_hip(hipFuncSetAttribute(reinterpret_cast<const void *>(kernel),
@@ -1678,48 +1709,68 @@ int launch_one(const MfmaArgs &args) {
   return skl_check_launch("gemm_split_reduce");
 }
 
+// The streaming kernel takes problems that its tiles divide evenly: 256 x 256 tiles when those can fill the 256 compute
+// units, 256 x 128 tiles for the sizes below that. Returns kNotWholeTiles for the others.
+constexpr int kNotWholeTiles = 0x7FFFFFFF;
+template <int TA, int TB, bool A_KC, bool B_KC, bool EXACT>
+int launch_whole_tiles(const MfmaArgs &p) {
+  constexpr int ES = Kind<TA>::ES;
+  constexpr size_t kRing128FromTiles = 96;
+  const auto wide = [](const MfmaArgs &q) { return launch_ring<TA, TB, A_KC, B_KC, 256, false, 0, false, false, EXACT>(q); };
+  const auto narrow = [](const MfmaArgs &q) { return launch_ring<TA, TB, A_KC, B_KC, 128, false, 0, false, false, EXACT>(q); };
+  if (p.m % 256 != 0 || (p.k * ES) % 128 != 0) return kNotWholeTiles;
+  const size_t tiles_m = p.m / 256;
+  // Steps that the epilogue over LDS rows applies: nothing overlaps it, where the bounds-checked kernels have several
+  // workgroups on a compute unit. So not for tiles that leave half of the chip idle (f16 1024 x 3072 x 1024 with ReLU 22.1
+  // against 23.3 us, E4M3 1024 x 4096 x 3072 with SiLU 36.6 / 42.9; 2048 x 4096 x 512 with SiLU, 256 narrow tiles: bf16
+  // 37.3 / 31.8, E4M3 36.1 / 33.6), nor for SiLU or GELU over several rounds of a K too short to outweigh them
+  // (4096 x 8192 x 512: bf16 with GELU 106.7 / 109.8 us, E4M3 with SiLU 94.8 / 103.5; int8 with ReLU 52.0 / 49.4).
+  using AccElem = decltype(typename Kind<TA>::Acc{}.x);
+  const bool staged = (p.rq.act || p.rq.q) && !(kRingCarriesExtraSteps<TA, TB> && !EXACT && FusedSteps<AccElem, 2>::dword_copy(p.rq));
+  if (staged && p.rq.act >= 2 && p.k * ES < 2048 && tiles_m * (p.n / 256) > 256) return kNotWholeTiles;
+  if (p.n % 256 == 0 && tiles_m * (p.n / 256) >= 200) {
+    // A last round that would fill at most half of the 256 compute units is run as 256 x 128 tiles
+    // instead (a second launch on the trailing columns): twice the workgroups at half the length.
+    const size_t tiles = tiles_m * (p.n / 256), rest = tiles % 256;
+    if (rest != 0 && rest <= 128 && rest % tiles_m == 0) {
+      const size_t tail_cols = rest / tiles_m * 256, head_cols = p.n - tail_cols;
+      MfmaArgs head = p, tail = p;
+      head.n = head_cols;
+      tail.n = tail_cols;
+      tail.b = p.b + (head_cols / 64) * p.b_s1 * ES;
+      tail.c = p.c + (head_cols >> p.ccs) * p.csc1 * sizeof(float);  // whole blocks; C elements are 4 bytes for every kind
+      if (p.bias) tail.bias = p.bias + head_cols * sizeof(float);
+      if (p.rq.q) tail.rq.q = p.rq.q + head_cols * p.rq.csq;
+      if (p.rq.q && p.rq.q_per_column) tail.rq.q_scale = p.rq.q_scale + head_cols;
+      const int rc = wide(head);
+      return rc != 0 ? rc : narrow(tail);
+    }
+    return wide(p);
+  }
+  // ... from 96 tiles on, or from 64 when K is long enough to be shared between two workgroups per tile
+  const size_t tiles128 = p.n % 128 == 0 ? tiles_m * (p.n / 128) : 0, slices = p.k * ES / kRingSlice;
+  if (tiles128 >= (EXACT || staged ? 200 : kRing128FromTiles) || (tiles128 >= 64 && slices % 4 == 0 && slices / 2 >= kRingMinSlicesPerSplit)) return narrow(p);
+  return kNotWholeTiles;
+}
+
 template <int TA, int TB, bool A_KC, bool B_KC>
 int launch_tile(const MfmaArgs &p) {
   constexpr int ES = Kind<TA>::ES;
-  constexpr size_t kRing128FromTiles = 96;
   constexpr bool kFp8 = TA == SKL_DT_F8E4M3 || TA == SKL_DT_F8E5M2;
   if constexpr (kFp8) {
-    // short K: exact products (see MmaF8Exact), on the bounds-checked kernel whatever the shape
+    // short K: exact products (see MmaF8Exact), on the streaming kernel when its tiles fill the chip (us, bounds-checked
+    // 128 x 128 / streaming: 2048 x 8192 x 2048 77 / 62, with GELU into E4M3 111 / 98; 2048 x 4096 x 2048 42 / 34, x 1024
+    // with GELU into E4M3 43 / 40; on 128 tiles, 512 x 8192 x 2048, 25.4 / 26.2)
     if (p.k <= kF8ExactMaxK) {
+      const int rc = launch_whole_tiles<TA, TB, A_KC, B_KC, true>(p);
+      if (rc != kNotWholeTiles) return rc;
       if (skl_div_up(p.m, 128) * (size_t)skl_div_up(p.n, 128) < 64)
         return launch_one<TA, TB, A_KC, B_KC, 64, 64, 2, 2, true, true>(p);
       return launch_one<TA, TB, A_KC, B_KC, 128, 128, 2, 4, true, true>(p);
     }
   }
-  // The streaming kernel takes problems that its tiles divide evenly: 256 x 256 tiles when those
-  // can fill the 256 compute units, 256 x 128 tiles for the sizes below that; everything else runs
-  // on the small, bounds-checked kernel.
-  if (p.m % 256 == 0 && (p.k * ES) % 128 == 0) {
-    const size_t tiles_m = p.m / 256;
-    if (p.n % 256 == 0 && tiles_m * (p.n / 256) >= 200) {
-      // A last round that would fill at most half of the 256 compute units is run as 256 x 128 tiles
-      // instead (a second launch on the trailing columns): twice the workgroups at half the length.
-      const size_t tiles = tiles_m * (p.n / 256), rest = tiles % 256;
-      if (rest != 0 && rest <= 128 && rest % tiles_m == 0) {
-        const size_t tail_cols = rest / tiles_m * 256, head_cols = p.n - tail_cols;
-        MfmaArgs head = p, tail = p;
-        head.n = head_cols;
-        tail.n = tail_cols;
-        tail.b = p.b + (head_cols / 64) * p.b_s1 * ES;
-        tail.c = p.c + (head_cols >> p.ccs) * p.csc1 * sizeof(float);  // whole blocks; C elements are 4 bytes for every kind
-        if (p.bias) tail.bias = p.bias + head_cols * sizeof(float);
-        if (p.rq.q) tail.rq.q = p.rq.q + head_cols * p.rq.csq;
-        if (p.rq.q && p.rq.q_per_column) tail.rq.q_scale = p.rq.q_scale + head_cols;
-        const int rc = launch_ring<TA, TB, A_KC, B_KC, 256>(head);
-        return rc != 0 ? rc : launch_ring<TA, TB, A_KC, B_KC, 128>(tail);
-      }
-      return launch_ring<TA, TB, A_KC, B_KC, 256>(p);
-    }
-    // ... from 96 tiles on, or from 64 when K is long enough to be shared between two workgroups per tile
-    const size_t tiles128 = p.n % 128 == 0 ? tiles_m * (p.n / 128) : 0, slices = p.k * ES / kRingSlice;
-    if (tiles128 >= kRing128FromTiles || (tiles128 >= 64 && slices % 4 == 0 && slices / 2 >= kRingMinSlicesPerSplit))
-      return launch_ring<TA, TB, A_KC, B_KC, 128>(p);
-  }
+  const int rc = launch_whole_tiles<TA, TB, A_KC, B_KC, false>(p);
+  if (rc != kNotWholeTiles) return rc;
   // Small problems: 64 x 64 tiles put four times as many workgroups on the chip.
   // ... and for the 16-bit kinds up to 64 rows of A: a 128-row tile would fetch and multiply rows that do not exist
   // (bf16 64 x 11008 x 4096: 36 -> 28 us; the 8-bit kinds are faster on the larger tile, 23 against 25 us).

@@ -1126,7 +1126,7 @@ def test_register_tiled_kernel_at_the_edges_of_its_tiles(gpu, ta, m, n, k):
 
 
 @pytest.mark.parametrize("ta", ("i8", "bf16", "f8e4m3"))
-@pytest.mark.parametrize("m,n,k,a_pad,c_by_columns", ((2304, 2048, 2432, 0, False), (2304, 2048, 2432, 0, True), (1537, 2051, 2500, 1, False), (1537, 2051, 2500, 1, True)))
+@pytest.mark.parametrize("m,n,k,a_pad,c_by_columns", ((2304, 2944, 2432, 0, False), (2304, 2944, 2432, 0, True), (2305, 2563, 2500, 1, False), (2305, 2563, 2500, 1, True)))
 def test_fused_steps_looped_over_rows(gpu, ta, m, n, k, a_pad, c_by_columns):
     """The streaming kernel's epilogue for any activation and any 8-bit copy, on whole tiles and on padded copies of
     operands off the 16-byte rule (C and the copy end inside a tile): C row-major and by columns, the copy in dwords, in
