@@ -9,8 +9,9 @@
 // keeps a tile of C in registers and walks K in slabs of 16 or 32 staged through LDS (two stages, the next slab's
 // global loads issued before the current slab's arithmetic, four elements per load along the operand's unit stride).
 // A thread's rows and columns are runs of up to four, a share of the tile apart, so that the lanes of a wave
-// read consecutive 16-byte pieces of the LDS rows. The last slab is zero-filled past K: adding the product
-// (+0)*(+0) leaves an accumulator unchanged, and an accumulator that started at +0 is never -0.
+// read consecutive 16-byte pieces of the LDS rows. The last slab is filled past K with +0 in A and -0 in B: their
+// product is -0, and adding -0 leaves every accumulator as it is. (Adding +0 would not: a negative sum that underflows
+// when it is rounded to half is a -0, and so is C then if beta*C is one.)
 //
 // What bounds it: the order of the sum is fixed, so K cannot be shared out, and a wave alone on its SIMD issues one
 // vector instruction in five to six cycles where several waves together issue one in three. So a tile is split over
@@ -114,8 +115,9 @@ struct Fetch {
     }
   }
 
-  // The slab that starts `p0` k into the operand and has `left` of them (kSlab or more: whole).
-  __device__ __forceinline__ void load(Stage (&r)[kGroups][4], size_t p0, size_t left) const {
+  // The slab that starts `p0` k into the operand and has `left` of them (kSlab or more: whole); `past`: what stands
+  // for elements outside the operand.
+  __device__ __forceinline__ void load(Stage (&r)[kGroups][4], size_t p0, size_t left, Stage past) const {
 #pragma unroll
     for (int e = 0; e < kGroups; ++e) {
       const In *g = at[e] + p0 * sk;
@@ -128,7 +130,7 @@ struct Fetch {
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
           const bool in = KC ? inside[e] != 0 && (size_t)(p_of(e) + i) < left : i < inside[e] && (size_t)p_of(e) < left;
-          r[e][i] = in ? Kind<DT>::stage(g[i * (KC ? sk : s0)]) : Stage(0);
+          r[e][i] = in ? Kind<DT>::stage(g[i * (KC ? sk : s0)]) : past;
         }
       }
     }
@@ -194,8 +196,8 @@ __global__ void __launch_bounds__((BM / TR) * (BN / TC)) gemm_tiled_kernel(Tiled
   fa.init((const typename K::In *)g.a, g.a_s1, g.a_s0, g.a_sk, row0, g.m);
   fb.init((const typename K::In *)g.b, g.b_s1, g.b_s0, g.b_sk, col0, g.n);
   Stage ra[FA::kGroups][4], rb[FB::kGroups][4];
-  fa.load(ra, 0, g.k);
-  fb.load(rb, 0, g.k);
+  fa.load(ra, 0, g.k, Stage(0.0));
+  fb.load(rb, 0, g.k, Stage(-0.0));
   fa.store(ra, As[0]);
   fb.store(rb, Bs[0]);
   __syncthreads();
@@ -203,8 +205,8 @@ __global__ void __launch_bounds__((BM / TR) * (BN / TC)) gemm_tiled_kernel(Tiled
   for (size_t p0 = 0; p0 < g.k; p0 += kSlab, cur ^= 1) {
     const size_t next = p0 + kSlab;
     if (next < g.k) {
-      fa.load(ra, next, g.k - next);
-      fb.load(rb, next, g.k - next);
+      fa.load(ra, next, g.k - next, Stage(0.0));
+      fb.load(rb, next, g.k - next, Stage(-0.0));
     }
 #pragma unroll kUnrollK  // a full unroll makes the compiler fetch a whole slab into registers (256 + AGPRs)
     for (int kk = 0; kk < kSlab; ++kk) {

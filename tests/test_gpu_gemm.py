@@ -1125,6 +1125,27 @@ def test_register_tiled_kernel_at_the_edges_of_its_tiles(gpu, ta, m, n, k):
         assert np.array_equal(got.view(np.uint8), want.view(np.uint8)), (ta, i, vars(case))
 
 
+@pytest.mark.parametrize("ta", ("f32", "f64", "f16h"))
+@pytest.mark.parametrize("m,n,k", ((40, 47, 48), (513, 517, 5), (830, 901, 16), (1730, 1797, 35), (2890, 2950, 18)))
+def test_register_tiled_kernel_keeps_the_sign_of_sums_that_underflow(gpu, ta, m, n, k):
+    """Operands of the smallest subnormal and zero, either sign: no sum gets beyond a zero, and in f16, rounded at every
+    step, it is +0 or -0 as its last product decides. C is negative and beta zero, so that sign is C's. K ends inside a
+    slab on tiles of every size: the fill past K must not touch it."""
+    from support import GemmCase
+    case = GemmCase(ta, None, 1.0, 0.0, m0=1, n0=1, k0=1, m1=m, n1=n, k1=k, rsa0=0, csa0=0, rsa1=k, csa1=1,
+                    rsb0=0, csb0=0, rsb1=n, csb1=1, rsc0=0, csc0=0, rsc1=n, csc1=1)
+    a, b, c = case.make_inputs(1)
+    rng = np.random.default_rng(m + k)
+    for x in (a, b):  # the sign bit and the lowest bit
+        bits = x.view({2: np.uint16, 4: np.uint32, 8: np.uint64}[x.itemsize])
+        bits[:] = rng.integers(0, 2, bits.size).astype(bits.dtype) << bits.dtype.type(8 * x.itemsize - 1) | rng.integers(0, 2, bits.size).astype(bits.dtype)
+    c[:] = -1
+    want = run_oracle_gemm(case, a, b, c)
+    got = run_gemm(gpu, "rcprc", case, a, b, c, "device")
+    assert np.array_equal(got.view(np.uint8), want.view(np.uint8)), (ta, np.count_nonzero(np.signbit(got) != np.signbit(want)))
+    assert not want.any() and (ta != "f16h" or 0 < np.count_nonzero(np.signbit(want)) < want.size)
+
+
 @pytest.mark.parametrize("ta", ("i8", "bf16", "f8e4m3"))
 @pytest.mark.parametrize("m,n,k,a_pad,c_by_columns", ((2304, 2944, 2432, 0, False), (2304, 2944, 2432, 0, True), (2305, 2563, 2500, 1, False), (2305, 2563, 2500, 1, True)))
 def test_fused_steps_looped_over_rows(gpu, ta, m, n, k, a_pad, c_by_columns):
