@@ -597,6 +597,10 @@ __device__ __forceinline__ void write_wave_tile(const MfmaArgs &p, const Acc (&a
 // with ReLU 105 -> 72, E4M3 2048 x 8192 x 4096 with GELU into E4M3 125 -> 99 (110 while every lane multiplied out the
 // addresses of its rows); what is left of the last over the same call with ReLU, 37 us, is mostly the erfc of 16.8 million
 // elements. launch_whole_tiles says where the line lies.
+// alpha, beta and the old C are applied as a strip of 32 rows goes into LDS, and the old values of the next strip are
+// requested ahead of this one's stores: a load inside the loop waits for the stores of the pass before, every pass
+// (see write_wave_tile; C read, us, loads in the loop / ahead: E5M2 1024 x 14080 x 6272 with ReLU into int8 102 / 91, E4M3
+// 7424 x 8576 x 2048 with GELU into int8 433 / 389, bf16 2816^2 x 3584 with SiLU 85 / 81).
 // ---------------------------------------------------------------------------
 template <int NI>
 constexpr int staged_pitch() { return 32 * NI + 8; }
@@ -613,7 +617,6 @@ __device__ __forceinline__ void write_wave_tile_staged(const MfmaArgs &p, const 
   const size_t col = col0 + c_first;
   const int cols = !CHECK ? 4 : col >= p.n ? 0 : p.n - col < 4 ? (int)(p.n - col) : 4;
   const size_t rmask = (size_t(1) << p.crs) - 1, cmask = (size_t(1) << p.ccs) - 1;
-  const bool init = skl_beta_is_zero<T>(p.beta);
   const T *const bias = reinterpret_cast<const T *>(p.bias);
   size_t c_off[4];
   T bias_of[4];
@@ -636,12 +639,46 @@ __device__ __forceinline__ void write_wave_tile_staged(const MfmaArgs &p, const 
   int8_t *const q_lane = reinterpret_cast<int8_t *>(p.rq.q) + (size_t)r_first * p.rq.rsq + col * p.rq.csq;
   const skl_fp8::Ofp8Format f8(p.rq.q_fmt);
   T running = skl_lowest<T>();
+  const bool init = skl_beta_is_zero<T>(p.beta);
+  T old[NI][16];
+  auto request = [&](int i) {
+    bool need = !init;
+    skl_scalar alpha = p.alpha;  // a copy the compiler cannot identify with it: the products below are not kept
+    unsigned opaque = 0;         // and addresses are worked out here, not all of them ahead of the first strip
+    asm volatile("" : "+s"(alpha.i), "+s"(opaque));
+#pragma unroll
+    for (int j = 0; j < NI; ++j)
+#pragma unroll
+      for (int r = 0; r < 16; ++r) {
+        old[j][r] = T(0);
+        need |= init && skl_initialise_needs_c(acc[i][j][r], alpha, p.beta);
+      }
+    if (__builtin_amdgcn_ballot_w64(need) == 0) return;
+#pragma unroll
+    for (int j = 0; j < NI; ++j) {
+      const size_t jc = col0 + (size_t)j * 32 + (lane & 31) + opaque;
+      const T *const c = reinterpret_cast<const T *>(p.c) + ((jc >> p.ccs) * p.csc1 + (jc & cmask) * p.csc0);
+#pragma unroll
+      for (int g = 0; g < 4; ++g) {
+        const size_t row = row0 + (size_t)i * 32 + g * 8 + (lane >> 5) * 4;  // four rows, in one block of C
+        const T *const from = c + ((row >> p.crs) * p.rsc1 + (row & rmask) * p.rsc0);
+#pragma unroll
+        for (int q = 0; q < 4; ++q)
+          if (!CHECK || (jc < p.n && row + q < p.m)) old[j][4 * g + q] = from[q * p.rsc0];
+        __builtin_amdgcn_sched_barrier(0);
+      }
+    }
+  };
+  request(0);
 #pragma unroll
   for (int i = 0; i < MI; ++i) {
 #pragma unroll
     for (int j = 0; j < NI; ++j)
 #pragma unroll
-      for (int r = 0; r < 16; ++r) stage_in[((r >> 2) * 8 + (r & 3)) * P + j * 32] = acc[i][j][r];
+      for (int r = 0; r < 16; ++r)
+        stage_in[((r >> 2) * 8 + (r & 3)) * P + j * 32] =
+            init ? skl_initialise_with(acc[i][j][r], old[j][r], p.alpha, p.beta) : skl_combine(acc[i][j][r], old[j][r], p.alpha, p.beta);
+    if (i + 1 < MI) request(i + 1);
     // the wave's own LDS accesses complete in order; the compiler must not move them across each other
     __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
     __builtin_amdgcn_wave_barrier();
@@ -651,19 +688,10 @@ __device__ __forceinline__ void write_wave_tile_staged(const MfmaArgs &p, const 
       const size_t four = row0 + (size_t)(i * 32 + pass * kRowsPerPass);  // a scalar
       if (CHECK && (four + r_first >= p.m || cols == 0)) continue;
       T *const c_row = c_lane + ((four >> p.crs) * p.rsc1 + (four & rmask) * p.rsc0);
-      V4 old = {T(0), T(0), T(0), T(0)};
-      bool need = !init;
-#pragma unroll
-      for (int e = 0; e < 4; ++e) need |= init && skl_initialise_needs_c(sum[e], p.alpha, p.beta);
-      if (need) {
-#pragma unroll
-        for (int e = 0; e < 4; ++e)
-          if (e < cols) old[e] = c_row[c_off[e]];
-      }
       V4 v;
 #pragma unroll
       for (int e = 0; e < 4; ++e) {
-        T x = init ? skl_initialise_with(sum[e], old[e], p.alpha, p.beta) : skl_combine(sum[e], old[e], p.alpha, p.beta);
+        T x = sum[e];
         if (bias) x = skl_add_bias(x, bias_of[e]);
         v[e] = skl_activate(x, p.rq.act);
         if (p.max && e < cols && v[e] > running) running = v[e];

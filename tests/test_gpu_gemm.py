@@ -1179,6 +1179,39 @@ def test_fused_steps_looped_over_rows(gpu, ta, m, n, k, a_pad, c_by_columns):
         assert np.all(err <= support.activation_ulp_bound(anchor[inside], 2)), float(err.max())
 
 
+@pytest.mark.parametrize("ta,m,n,k", (("i8", 2048, 3200, 128), ("bf16", 2048, 3200, 64), ("f16", 2048, 6400, 64), ("f8e4m3", 2048, 6400, 128),
+                                       ("f8e5m2", 2048, 3200, 2432)))
+def test_fused_steps_looped_over_rows_take_the_old_c(gpu, ta, m, n, k):
+    """The row-looping epilogue where C is read: beta != 0, beta == 0 with the sign of exact zeros (zeroed rows of A) to
+    take from C, and beta == 0 as the reference evaluates it, with NaN and infinities in C. 200 tiles of 256 x 128 and of
+    256 x 256. The call without a copy is the anchor: C comes out bit for bit, the copy is what the rules make of it."""
+    rng = np.random.default_rng(n + k)
+    start = np.array([-(1 << 31)], np.int32) if ta == "i8" else np.array([-np.inf], np.float32)
+    for alpha, beta, as_reference in ((2, -3, False), (-1, 0, False), (-1, 0, True)):
+        case = rowmajor_case(ta, m, n, k, alpha, beta)
+        a, b, c = case.make_inputs(int(rng.integers(1 << 30)))
+        a.reshape(m, k)[::37] = 0
+        if as_reference and ta != "i8":
+            c = _spoil(c, m, n, np.arange(3, m, 97))
+        gpu.skl_hip_set_beta_zero_mode(int(as_reference))
+        try:
+            anchor, _ = run_fused_gemm(gpu, "rc", case, a, b, c, None, start, "device")
+            scale = np.array([100.0 / np.nanmax(np.abs(np.where(np.isfinite(anchor), anchor, 0).astype(np.float64)))], np.float32)
+            rq = dict(q=np.zeros(m * n, np.int8), rsq=n, csq=1, scale=scale, format=2 if ta == "i8" else 0)
+            got, top, q = run_fused_gemm(gpu, "rc", case, a, b, c, None, start, "device", requant=rq)
+        finally:
+            gpu.skl_hip_set_beta_zero_mode(0)
+        _, want_top, want_q = fused_expectation(case, anchor, None, start, requant=rq)
+        same = got.view(np.uint32) == anchor.view(np.uint32)
+        if ta != "i8":
+            assert np.array_equal(np.isnan(got), np.isnan(anchor)) and np.isnan(anchor).any() == as_reference
+            same |= np.isnan(got)
+        assert same.all() and np.array_equal(q, want_q) and top[0] == want_top[0], (ta, alpha, beta, as_reference)
+        if ta != "i8" and beta == 0:
+            zeros = anchor.reshape(m, n)[::37]
+            assert np.any(np.signbit(zeros)) and not np.all(np.signbit(zeros))
+
+
 @pytest.mark.parametrize("ta,tb", (("i8", "i8"), ("bf16", "bf16"), ("f16", "f16"), ("f8e4m3", "f8e4m3"), ("f8e4m3", "f8e5m2")))
 def test_ragged_problems_on_padded_copies(gpu, ta, tb):
     """Ragged M, N and K (and odd leading dimensions) on a problem large enough to fill the chip: A and B are copied
