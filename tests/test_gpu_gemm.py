@@ -1125,6 +1125,22 @@ def test_register_tiled_kernel_at_the_edges_of_its_tiles(gpu, ta, m, n, k):
         assert np.array_equal(got.view(np.uint8), want.view(np.uint8)), (ta, i, vars(case))
 
 
+@pytest.mark.parametrize("ta", ("f32", "f16h"))
+@pytest.mark.parametrize("m,n,k,a_rows,b_rows", ((2890, 2950, 67, True, True), (2944, 2944, 64, False, False), (2890, 2950, 97, False, True)))
+def test_register_tiled_kernel_walks_several_slabs_on_its_largest_tile(gpu, ta, m, n, k, a_rows, b_rows):
+    """The 128 x 128 tile (from 512 tiles on) beyond its first slab of 32: four elements per load, both LDS stages and a last
+    slab that K ends in, operands contiguous along either dimension: bit for bit."""
+    from support import GemmCase
+    rsa, csa = (k, 1) if a_rows else (1, m)
+    rsb, csb = (n, 1) if b_rows else (1, k)
+    case = GemmCase(ta, None, 1.5, -0.5, m0=1, n0=1, k0=1, m1=m, n1=n, k1=k, rsa0=0, csa0=0, rsa1=rsa, csa1=csa,
+                    rsb0=0, csb0=0, rsb1=rsb, csb1=csb, rsc0=0, csc0=0, rsc1=n, csc1=1)
+    a, b, c = case.make_inputs(9900 + k)
+    want = run_oracle_gemm(case, a, b, c)
+    got = run_gemm(gpu, "rcprc", case, a, b, c, "device")
+    assert np.array_equal(got.view(np.uint8), want.view(np.uint8)), ta
+
+
 @pytest.mark.parametrize("ta", ("f32", "f64", "f16h"))
 @pytest.mark.parametrize("m,n,k", ((40, 47, 48), (513, 517, 5), (830, 901, 16), (1730, 1797, 35), (2890, 2950, 18)))
 def test_register_tiled_kernel_keeps_the_sign_of_sums_that_underflow(gpu, ta, m, n, k):
@@ -1210,6 +1226,54 @@ def test_fused_steps_looped_over_rows_take_the_old_c(gpu, ta, m, n, k):
         if ta != "i8" and beta == 0:
             zeros = anchor.reshape(m, n)[::37]
             assert np.any(np.signbit(zeros)) and not np.all(np.signbit(zeros))
+
+
+@pytest.mark.parametrize("ta", ("i8", "bf16"))
+@pytest.mark.parametrize("cols,gap", ((2, 0), (4, 0), (4, 2), (8, 0)))
+def test_fused_steps_looped_over_rows_of_a_blocked_c(gpu, ta, cols, gap):
+    """The row-looping epilogue on a C in blocks of 4 x 2, 4 x 4 and 4 x 8, accumulating, block rows on 16-byte boundaries
+    and off them."""
+    m1, n1, k = 2048 // 4, 3200 // cols, 128
+    m, n = 4 * m1, cols * n1
+    case = support.GemmCase(ta, None, 2, -1, m0=4, n0=cols, k0=1, m1=m1, n1=n1, k1=k, rsa0=k, csa0=0, rsa1=4 * k, csa1=1,
+                            rsb0=0, csb0=1, rsb1=n, csb1=cols, rsc0=cols, csc0=1, rsc1=4 * cols * n1 + gap, csc1=4 * cols)
+    a, b, c = case.make_inputs(cols + gap)
+    rng = np.random.default_rng(cols)
+    bias = rng.integers(-999, 999, n).astype(np.int32) if ta == "i8" else rng.uniform(-4, 4, n).astype(np.float32)
+    start = np.array([-(1 << 31)], np.int32) if ta == "i8" else np.array([-np.inf], np.float32)
+    anchor, _ = run_fused_gemm(gpu, "rcprc", case, a, b, c, bias, None, "device")
+    scale = np.array([100.0 / np.abs(anchor.astype(np.float64)).max()], np.float32)
+    rq = dict(q=np.zeros(m * (n + 1), np.int8), rsq=n + 1, csq=1, scale=scale, zero=5)
+    got, top, q = run_fused_gemm(gpu, "rcprc", case, a, b, c, bias, start, "device", activation=1, requant=rq)
+    want, want_top, want_q = fused_expectation(case, anchor, None, start, activation=1, requant=rq)
+    assert np.array_equal(got.view(np.uint32), want.view(np.uint32)) and np.array_equal(q, want_q) and top[0] == want_top[0]
+
+
+@pytest.mark.parametrize("act", (2, 3))
+@pytest.mark.parametrize("ta,m,n,k", (("f8e4m3", 2048, 3200, 2048), ("f8e4m3", 2048, 6400, 256), ("f8e4m3", 2048, 3200, 2432), ("f8e5m2", 2048, 6400, 2432),
+                                       ("f16", 2048, 3200, 64), ("bf16", 2048, 6400, 64)))
+def test_silu_and_gelu_looped_over_rows(gpu, ta, m, n, k, act):
+    """SiLU and GELU in the row-looping epilogue, with an fp8 and an int8 copy: products of exact and of native fp8 and of
+    16-bit operands on 256 x 128 and 256 x 256 tiles. C is the reference routine's value of the call's own pre-activation
+    C within the reference's bounds, and the copies are the rules' value of that C; with q_only the same bytes."""
+    rng = np.random.default_rng(n + k + act)
+    case = rowmajor_case(ta, m, n, k, alpha=0.125, beta=0.0)
+    a, b, c = case.make_inputs(int(rng.integers(1 << 30)))
+    a.reshape(m, k)[1::2] ^= a.dtype.type(1 << (8 * a.itemsize - 1))  # sums of either sign
+    bias = rng.uniform(-2, 2, n).astype(np.float32)
+    start = np.array([-np.inf], np.float32)
+    anchor, _ = run_fused_gemm(gpu, "rc", case, a, b, c, bias, None, "device")
+    want = support.activation_reference(anchor, act)
+    for fmt in (2, 0):
+        scales = (rng.uniform(0.5, 2.0, n) * 60.0 / np.abs(want).max()).astype(np.float32)
+        rq = dict(q=np.zeros(m * n, np.int8), rsq=n, csq=1, scale=scales, per_column=True, zero=0 if fmt else -3, format=fmt)
+        got, top, q = run_fused_gemm(gpu, "rc", case, a, b, c, bias, start, "device", activation=act, requant=rq)
+        err = support.ulp_error_f32(got, want)
+        assert np.all(err <= support.activation_ulp_bound(anchor, act)), float(err.max())
+        _, want_top, want_q = fused_expectation(case, got, None, start, requant=rq)
+        assert np.array_equal(q, want_q) and top[0] == want_top[0] and len(np.unique(q)) > 20
+        _, _, q = run_fused_gemm(gpu, "rc", case, a, b, c, bias, start, "device", activation=act, requant=dict(rq, only=True))
+        assert np.array_equal(q, want_q)
 
 
 @pytest.mark.parametrize("ta,tb", (("i8", "i8"), ("bf16", "bf16"), ("f16", "f16"), ("f8e4m3", "f8e4m3"), ("f8e4m3", "f8e5m2")))
