@@ -9,9 +9,10 @@
 // keeps a tile of C in registers and walks K in slabs of 16 or 32 staged through LDS (two stages, the next slab's
 // global loads issued before the current slab's arithmetic, four elements per load along the operand's unit stride).
 // A thread's rows and columns are runs of up to four, a share of the tile apart, so that the lanes of a wave
-// read consecutive 16-byte pieces of the LDS rows. The last slab is filled past K with +0 in A and -0 in B: their
-// product is -0, and adding -0 leaves every accumulator as it is. (Adding +0 would not: a negative sum that underflows
-// when it is rounded to half is a -0, and so is C then if beta*C is one.)
+// read consecutive 16-byte pieces of the LDS rows. The last slab is filled past K with +0 in A and B: adding the product
+// +0 leaves an f32 or f64 accumulator unchanged, which started at +0 and is never -0. An f16 one can be: a negative sum
+// underflows when it is rounded to half, and C's sign shows it if beta*C is a -0 too. There B's fill is -0, and adding
+// the product -0 leaves every accumulator as it is.
 //
 // What bounds it: the order of the sum is fixed, so K cannot be shared out, and a wave alone on its SIMD issues one
 // vector instruction in five to six cycles where several waves together issue one in three. So a tile is split over
@@ -179,6 +180,7 @@ __global__ void __launch_bounds__((BM / TR) * (BN / TC)) gemm_tiled_kernel(Tiled
   using FA = Fetch<DT, BM, kSlab, kThreads, A_KC>;
   using FB = Fetch<DT, BN, kSlab, kThreads, B_KC>;
   constexpr int kUnrollK = TR * TC >= 64 ? 2 : 4;
+  constexpr Stage kPastB = DT == SKL_DT_F16H ? Stage(-0.0) : Stage(0.0);
   __shared__ __attribute__((aligned(16))) Stage As[2][kSlab][BM + 4];
   __shared__ __attribute__((aligned(16))) Stage Bs[2][kSlab][BN + 4];
 
@@ -197,7 +199,7 @@ __global__ void __launch_bounds__((BM / TR) * (BN / TC)) gemm_tiled_kernel(Tiled
   fb.init((const typename K::In *)g.b, g.b_s1, g.b_s0, g.b_sk, col0, g.n);
   Stage ra[FA::kGroups][4], rb[FB::kGroups][4];
   fa.load(ra, 0, g.k, Stage(0.0));
-  fb.load(rb, 0, g.k, Stage(-0.0));
+  fb.load(rb, 0, g.k, kPastB);
   fa.store(ra, As[0]);
   fb.store(rb, Bs[0]);
   __syncthreads();
@@ -206,7 +208,7 @@ __global__ void __launch_bounds__((BM / TR) * (BN / TC)) gemm_tiled_kernel(Tiled
     const size_t next = p0 + kSlab;
     if (next < g.k) {
       fa.load(ra, next, g.k - next, Stage(0.0));
-      fb.load(rb, next, g.k - next, Stage(-0.0));
+      fb.load(rb, next, g.k - next, kPastB);
     }
 #pragma unroll kUnrollK  // a full unroll makes the compiler fetch a whole slab into registers (256 + AGPRs)
     for (int kk = 0; kk < kSlab; ++kk) {
@@ -229,25 +231,57 @@ __global__ void __launch_bounds__((BM / TR) * (BN / TC)) gemm_tiled_kernel(Tiled
   using Wide = typename std::conditional<DT == SKL_DT_F16H, float, Out>::type;  // what alpha and beta are applied in
   Out *cbase = (Out *)g.c;
   const bool init = skl_beta_is_zero<Wide>(g.beta);
+  constexpr int W = TC < 4 ? TC : 4, kRuns = TC / W;
+  using CRun = typename Run<Out, W>::Type;
 #pragma unroll
   for (int r = 0; r < TR; ++r) {
     const size_t i = row0 + tiled_index<BM, TR>(ty, r);
     if (i >= g.m) continue;
     Out *crow = cbase + (i / 64) * g.rsc1 + (i % 64) * g.rsc0;
-    // a row's old values are requested together, ahead of its first store
-    Out *cp[TC];
+    // A row's old values are requested together, ahead of its first store. Where C's columns lie side by side a run of
+    // them is one access: dword by dword every store of a wave covers a quarter of each cache line (f32 2406 x 2003 x 16
+    // 21.5 -> 17.6 us, 13.7 with slabs of 16; 2048 x 2048 x 2048 unchanged).
+    Out *cp[kRuns];
     Wide old[TC];
 #pragma unroll
-    for (int c = 0; c < TC; ++c) {
-      const size_t j = col0 + tiled_index<BN, TC>(tx, c);
-      cp[c] = j < g.n ? crow + (j / 64) * g.csc1 + (j % 64) * g.csc0 : nullptr;
-      old[c] = Wide(0);
-      if (cp[c] && (!init || tiled_needs_c((Wide)acc[r][c], g.alpha, g.beta))) old[c] = (Wide)*cp[c];
+    for (int q = 0; q < kRuns; ++q) {
+      const size_t j = col0 + tiled_index<BN, TC>(tx, q * W);
+      cp[q] = crow + (j / 64) * g.csc1 + (j % 64) * g.csc0;
+      bool need[W], any = false;
+#pragma unroll
+      for (int e = 0; e < W; ++e) {
+        old[q * W + e] = Wide(0);
+        need[e] = j + e < g.n && (!init || tiled_needs_c((Wide)acc[r][q * W + e], g.alpha, g.beta));
+        any |= need[e];
+      }
+      if (g.csc0 == 1 && j + W <= g.n) {
+        if (any) {
+          const CRun v = *reinterpret_cast<const CRun *>(cp[q]);
+#pragma unroll
+          for (int e = 0; e < W; ++e) old[q * W + e] = need[e] ? (Wide)v[e] : Wide(0);
+        }
+      } else {
+#pragma unroll
+        for (int e = 0; e < W; ++e)
+          if (need[e]) old[q * W + e] = (Wide)cp[q][e * g.csc0];
+      }
     }
 #pragma unroll
-    for (int c = 0; c < TC; ++c) {
-      if (!cp[c]) continue;
-      *cp[c] = (Out)(init ? skl_initialise((Wide)acc[r][c], &old[c], g.alpha, g.beta) : skl_combine((Wide)acc[r][c], old[c], g.alpha, g.beta));
+    for (int q = 0; q < kRuns; ++q) {
+      const size_t j = col0 + tiled_index<BN, TC>(tx, q * W);
+      CRun v;
+#pragma unroll
+      for (int e = 0; e < W; ++e) {
+        const Wide sum = (Wide)acc[r][q * W + e];
+        v[e] = (Out)(init ? skl_initialise(sum, &old[q * W + e], g.alpha, g.beta) : skl_combine(sum, old[q * W + e], g.alpha, g.beta));
+      }
+      if (g.csc0 == 1 && j + W <= g.n) {
+        *reinterpret_cast<CRun *>(cp[q]) = v;
+      } else {
+#pragma unroll
+        for (int e = 0; e < W; ++e)
+          if (j + e < g.n) cp[q][e * g.csc0] = v[e];
+      }
     }
   }
 }
@@ -284,17 +318,23 @@ int launch(const skl_gemm_canon *g) {
 // f32, us, at K = 2048 (128 x 128 / 64 x 64 of 4 x 4 / 64 x 64 of 4 x 2 / 32 x 32 / 16 x 32 tiles):
 //   4096^2: 1243 / 1275 / 1356 / 2110 / 3066    2048^2: 347 / 349 / 364 / 532 / 779
 //   1024^2: 349 / 180 / 132 / 159 / 220          512^2: 338 / 170 / 121 / 78 / 70     256^2: 337 / 169 / 121 / 76 / 61
+//
+// Floats are staged in slabs of 32 from K = 512 on, of 16 below on the two larger tiles: half the LDS puts more
+// workgroups on a compute unit, which is what a short K lives on, and a K of 16 fills its slab (f32, over the time with
+// slabs of 32, K up to 16 / 32 / 64 / 128 / 256: 64 x 64 tiles 0.78 / 0.96 / 0.95 / 0.96 / 0.94, 128 x 128
+// 0.67 / 0.86 / 0.87 / 0.95 / 0.95; 2048^3 361 us with 32 and 367 with 16, f16 with A by columns 4096 x 4096 x 2048 2291 and 2404).
 template <int DT>
 int launch_sized(const skl_gemm_canon *g) {
-  constexpr int kSlab = sizeof(typename Kind<DT>::Stage) == 8 ? 16 : 32;  // 68 KiB of LDS for the largest tile of floats
+  constexpr bool kDoubles = sizeof(typename Kind<DT>::Stage) == 8;
+  constexpr int kSlab = kDoubles ? 16 : 32;  // 66 KiB of LDS for the largest tile of floats
   const auto tiles = [&](size_t bm, size_t bn) { return ((g->m + bm - 1) / bm) * ((g->n + bn - 1) / bn); };
   if (tiles(128, 128) >= 512) {
     // doubles: twice the bytes of LDS per step, so 8 x 8 per thread (4096 x 4096 x 2048: 8 x 4 2517 us, 8 x 8
     // 2203 us)
-    if constexpr (sizeof(typename Kind<DT>::Stage) == 8) return launch<DT, 128, 128, 8, 8, 8>(g);
-    else return launch<DT, 128, 128, 8, 4, kSlab>(g);
+    if constexpr (kDoubles) return launch<DT, 128, 128, 8, 8, 8>(g);
+    else return g->k < 512 ? launch<DT, 128, 128, 8, 4, 16>(g) : launch<DT, 128, 128, 8, 4, kSlab>(g);
   }
-  if (tiles(64, 64) >= 768) return launch<DT, 64, 64, 4, 4, kSlab>(g);
+  if (tiles(64, 64) >= 768) return g->k < 512 ? launch<DT, 64, 64, 4, 4, 16>(g) : launch<DT, 64, 64, 4, 4, kSlab>(g);
   if (tiles(64, 64) >= 176) return launch<DT, 64, 64, 4, 2, 16>(g);
   if (tiles(32, 32) > 256) return launch<DT, 32, 32, 2, 2, kSlab>(g);
   return launch<DT, 16, 32, 2, 1, kSlab>(g);

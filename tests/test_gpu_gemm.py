@@ -1125,6 +1125,22 @@ def test_register_tiled_kernel_at_the_edges_of_its_tiles(gpu, ta, m, n, k):
         assert np.array_equal(got.view(np.uint8), want.view(np.uint8)), (ta, i, vars(case))
 
 
+@pytest.mark.parametrize("ta", ("f32", "f64", "f16h"))
+@pytest.mark.parametrize("m,n", ((3, 65500), (5, 49203), (65501, 2), (49200, 7), (1025, 701), (70, 90)))
+def test_register_tiled_kernel_slabs_and_runs_of_c(gpu, ta, m, n):
+    """K on both sides of the change from slabs of 16 to slabs of 32, one off a slab, on every tile size; C by rows, whose
+    columns are written in runs, by columns, and in rows that begin at any element."""
+    for i, k in enumerate((513, 511) if max(m, n) > 2000 else (130, 512)):
+        for c_rows in (True, False):
+            rsc, csc = (n + i, 1) if c_rows else (1, m + 1)
+            case = support.GemmCase(ta, None, 1.5, (-0.5, 0.0)[i], m0=1, n0=1, k0=1, m1=m, n1=n, k1=k, rsa0=0, csa0=0, rsa1=k, csa1=1,
+                                    rsb0=0, csb0=0, rsb1=n, csb1=1, rsc0=0, csc0=0, rsc1=rsc, csc1=csc)
+            a, b, c = case.make_inputs(9950 + i)
+            want = run_oracle_gemm(case, a, b, c)
+            got = run_gemm(gpu, "rcprc", case, a, b, c, "device")
+            assert np.array_equal(got.view(np.uint8), want.view(np.uint8)), (ta, k, c_rows)
+
+
 @pytest.mark.parametrize("ta", ("f32", "f16h"))
 @pytest.mark.parametrize("m,n,k,a_rows,b_rows", ((2890, 2950, 67, True, True), (2944, 2944, 64, False, False), (2890, 2950, 97, False, True)))
 def test_register_tiled_kernel_walks_several_slabs_on_its_largest_tile(gpu, ta, m, n, k, a_rows, b_rows):
