@@ -640,7 +640,9 @@ __device__ __forceinline__ void write_wave_tile_staged(const MfmaArgs &p, const 
   const skl_fp8::Ofp8Format f8(p.rq.q_fmt);
   T running = skl_lowest<T>();
   const bool init = skl_beta_is_zero<T>(p.beta);
+  typedef T Rows4 __attribute__((ext_vector_type(4), aligned(4)));  // C by columns: a lane's four rows, on any element boundary
   T old[NI][16];
+  // The old values of strip i, if it needs any.
   auto request = [&](int i) {
     bool need = !init;
     skl_scalar alpha = p.alpha;  // a copy the compiler cannot identify with it: the products below are not kept
@@ -649,36 +651,52 @@ __device__ __forceinline__ void write_wave_tile_staged(const MfmaArgs &p, const 
 #pragma unroll
     for (int j = 0; j < NI; ++j)
 #pragma unroll
-      for (int r = 0; r < 16; ++r) {
-        old[j][r] = T(0);
-        need |= init && skl_initialise_needs_c(acc[i][j][r], alpha, p.beta);
+      for (int r = 0; r < 16; ++r) need |= init && skl_initialise_needs_c(acc[i][j][r], alpha, p.beta);
+    const bool any = __builtin_amdgcn_ballot_w64(need) != 0;
+    if (!any) return any;
+    const auto fetch = [&](auto by_rows) {
+#pragma unroll
+      for (int j = 0; j < NI; ++j) {
+        const size_t jc = col0 + (size_t)j * 32 + (lane & 31) + opaque;
+        const T *const c = reinterpret_cast<const T *>(p.c) + ((jc >> p.ccs) * p.csc1 + (jc & cmask) * p.csc0);
+#pragma unroll
+        for (int g = 0; g < 4; ++g) {
+          const size_t row = row0 + (size_t)i * 32 + g * 8 + (lane >> 5) * 4;  // four rows, in one block of C
+          const T *const from = c + ((row >> p.crs) * p.rsc1 + (row & rmask) * p.rsc0);
+          if constexpr (decltype(by_rows)::value) {
+            const Rows4 four = *reinterpret_cast<const Rows4 *>(from);
+#pragma unroll
+            for (int q = 0; q < 4; ++q) old[j][4 * g + q] = four[q];
+          } else {
+#pragma unroll
+            for (int q = 0; q < 4; ++q) old[j][4 * g + q] = !CHECK || (jc < p.n && row + q < p.m) ? from[q * p.rsc0] : T(0);
+          }
+          __builtin_amdgcn_sched_barrier(0);
+        }
       }
-    if (__builtin_amdgcn_ballot_w64(need) == 0) return;
-#pragma unroll
-    for (int j = 0; j < NI; ++j) {
-      const size_t jc = col0 + (size_t)j * 32 + (lane & 31) + opaque;
-      const T *const c = reinterpret_cast<const T *>(p.c) + ((jc >> p.ccs) * p.csc1 + (jc & cmask) * p.csc0);
-#pragma unroll
-      for (int g = 0; g < 4; ++g) {
-        const size_t row = row0 + (size_t)i * 32 + g * 8 + (lane >> 5) * 4;  // four rows, in one block of C
-        const T *const from = c + ((row >> p.crs) * p.rsc1 + (row & rmask) * p.rsc0);
-#pragma unroll
-        for (int q = 0; q < 4; ++q)
-          if (!CHECK || (jc < p.n && row + q < p.m)) old[j][4 * g + q] = from[q * p.rsc0];
-        __builtin_amdgcn_sched_barrier(0);
-      }
-    }
+    };
+    if (!CHECK && p.rsc0 == 1)
+      fetch(std::true_type{});
+    else
+      fetch(std::false_type{});
+    return any;
   };
-  request(0);
-#pragma unroll
-  for (int i = 0; i < MI; ++i) {
+  const auto put_strip = [&](int i, auto value) {
 #pragma unroll
     for (int j = 0; j < NI; ++j)
 #pragma unroll
-      for (int r = 0; r < 16; ++r)
-        stage_in[((r >> 2) * 8 + (r & 3)) * P + j * 32] =
-            init ? skl_initialise_with(acc[i][j][r], old[j][r], p.alpha, p.beta) : skl_combine(acc[i][j][r], old[j][r], p.alpha, p.beta);
-    if (i + 1 < MI) request(i + 1);
+      for (int r = 0; r < 16; ++r) stage_in[((r >> 2) * 8 + (r & 3)) * P + j * 32] = value(acc[i][j][r], j, r);
+  };
+  bool read_c = request(0);
+#pragma unroll
+  for (int i = 0; i < MI; ++i) {
+    if (!read_c)
+      put_strip(i, [&](T sum, int, int) { return skl_initialise_plain(sum, p.alpha, p.beta); });
+    else if (init)
+      put_strip(i, [&](T sum, int j, int r) { return skl_initialise_with(sum, old[j][r], p.alpha, p.beta); });
+    else
+      put_strip(i, [&](T sum, int j, int r) { return skl_combine(sum, old[j][r], p.alpha, p.beta); });
+    if (i + 1 < MI) read_c = request(i + 1);
     // the wave's own LDS accesses complete in order; the compiler must not move them across each other
     __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
     __builtin_amdgcn_wave_barrier();
@@ -1591,7 +1609,7 @@ constexpr size_t kRingMinSlicesPerSplit = 64;  // below 8 KiB of K per row the p
 // bytes: int8 behind an int32 C, fp8 behind an fp32 C); every other call with those steps takes the epilogue that loops
 // over rows in LDS (kStagedSteps).
 template <int TA, int TB>
-constexpr bool kRingCarriesExtraSteps = TA == TB;   // every kind but the mixed fp8 pairings
+constexpr bool kRingCarriesExtraSteps = TA == TB;   // every kind but the mixed fp8 pairings, which have no fused entry point
 
 // An int32 C the streaming kernel writes 16 bytes per lane: blocks of 4 to 16 columns with contiguous rows, a
 // multiple of four rows per block, everything on 16-byte boundaries, no fused steps.
@@ -1602,9 +1620,9 @@ inline bool c_in_row_quads(const MfmaArgs &p) {
 
 template <int TA, int TB, bool A_KC, bool B_KC, int BN, bool EDGE = false, int EXTRA = 0, bool CQUADS = false, bool SCAN = false, bool EXACT = false>
 int launch_ring(const MfmaArgs &args) {
-  if constexpr (EXTRA == 0 && !CQUADS && !SCAN) {
+  if constexpr (EXTRA == 0 && !CQUADS && !SCAN && kRingCarriesExtraSteps<TA, TB>) {
     using Steps = FusedSteps<decltype(typename Kind<TA>::Acc{}.x), 2>;
-    if ((args.rq.act || args.rq.q) && !(kRingCarriesExtraSteps<TA, TB> && !EDGE && !EXACT && Steps::dword_copy(args.rq)))
+    if ((args.rq.act || args.rq.q) && !(!EDGE && !EXACT && Steps::dword_copy(args.rq)))
       return launch_ring<TA, TB, A_KC, B_KC, BN, EDGE, kStagedSteps, false, false, EXACT>(args);
   }
   if constexpr (EXTRA == 0 && kRingCarriesExtraSteps<TA, TB> && !EDGE && !EXACT) {
@@ -1754,7 +1772,9 @@ int launch_whole_tiles(const MfmaArgs &p) {
   // 37.3 / 31.8, E4M3 36.1 / 33.6), nor for SiLU or GELU over several rounds of a K too short to outweigh them
   // (4096 x 8192 x 512: bf16 with GELU 106.7 / 109.8 us, E4M3 with SiLU 94.8 / 103.5; int8 with ReLU 52.0 / 49.4).
   using AccElem = decltype(typename Kind<TA>::Acc{}.x);
-  const bool staged = (p.rq.act || p.rq.q) && !(kRingCarriesExtraSteps<TA, TB> && !EXACT && FusedSteps<AccElem, 2>::dword_copy(p.rq));
+  const bool extra = p.rq.act || p.rq.q;
+  if (extra && !kRingCarriesExtraSteps<TA, TB>) return kNotWholeTiles;
+  const bool staged = extra && !(!EXACT && FusedSteps<AccElem, 2>::dword_copy(p.rq));
   if (staged && p.rq.act >= 2 && p.k * ES < 2048 && tiles_m * (p.n / 256) > 256) return kNotWholeTiles;
   if (p.n % 256 == 0 && tiles_m * (p.n / 256) >= 200) {
     // A last round that would fill at most half of the 256 compute units is run as 256 x 128 tiles
