@@ -1755,49 +1755,95 @@ int launch_one(const MfmaArgs &args) {
   return skl_check_launch("gemm_split_reduce");
 }
 
+// How well `tiles` workgroups, one at a time on each of the 256 compute units, fill the rounds they take, in per cent.
+// `tail`: the last round runs as 256 x 128 tiles, half as long.
+inline unsigned rounds_filled(size_t tiles, bool tail = false) {
+  const size_t half_rounds = tail ? tiles / 256 * 2 + 1 : (tiles + 255) / 256 * 2;
+  return (unsigned)(tiles * 200 / (256 * half_rounds));
+}
+
+// Whether the streaming kernel beats the bounds-checked ones on whole tiles where it has a handicap: the epilogue over
+// LDS rows (`staged`: an activation or a copy), which nothing overlaps while the bounds-checked kernels have several
+// workgroups on a compute unit, or the products of a short fp8 K, which are not long enough to outweigh a tile's start and
+// end. What decides is how full its last round is, how much K there is to gain on, and whether C is read, which it
+// requests earlier than the others do.
+// Its time over theirs, medians of some 1900 random problems of more than one round, by K in bytes and `filled`
+// (50-60 / 60-70 / 70-80 / 80-90 / 90-100 per cent); "-": no such problem was drawn:
+//   16 bits, SiLU or GELU, C read   below 1024  1.08 1.13 1.10 1.06 1.02   from 1024  1.12 1.08 1.07 0.91 0.95   from 2048  1.04 1.05 0.98 0.91 0.91   from 4096  0.99 0.97 0.90 0.90 0.80
+//                         not read  below 1024  1.22 1.20 1.29 1.03 1.07   from 1024    -  1.25 1.14 1.07 1.08   from 2048  1.16 1.06 1.12 0.92 1.01   from 4096  1.03 1.04 0.96 0.92 0.86
+//   16 bits, none or ReLU, C read   below 1024  0.73 1.00 0.95 0.94 0.89   from 1024  0.95 0.98 0.97 0.80 0.81   from 2048  1.01 0.91 0.90 0.87 0.79   from 4096  0.91 0.94 0.85 0.86 0.80
+//                         not read  below 1024  1.16 1.08 1.07 1.06 0.95   from 1024  1.05 1.15 0.93 0.91   -    from 2048  1.08 1.07 0.82   -  0.89   from 4096  0.97 0.88 0.96 0.82 0.81
+//   short fp8, SiLU or GELU, C read below 1024  1.19 1.22 1.17 1.07 1.02   from 1024  1.12 1.06 1.09 0.99 0.93
+//                         not read  below 1024  1.43 1.33 1.22 1.07 1.04   from 1024  1.31 1.21 1.13 1.03 0.96
+//   short fp8, none or ReLU, C read below 1024  1.01 1.01 0.92 0.90 0.91   from 1024  1.03 1.03 0.93 0.93 0.92
+//                         not read  below 1024  1.25 1.11 1.11 1.06 1.01   from 1024  1.09 1.15 1.07 0.97 0.90
+//   short fp8, no steps, C read     up to 1024  0.90 0.92 0.87 0.85 0.85   beyond     0.99 0.92 0.89 0.84 0.80
+//                         not read  up to 256   1.11 1.13 1.14 1.08 1.08   up to 1024 1.10 1.06 1.05 0.96 0.95   beyond 1.04 0.99 1.00 0.90 0.84
+//   int8                            C read 0.60 to 0.91, not read 0.67 to 0.99, at any K
+// A single round, full or nearly: 0.7 to 0.95 for all of them, short fp8 without steps 1.06 up to K = 256. With a K of 8 KiB
+// and more also 129 to 199 tiles, 0.82, and 65 to 128, which share K, 0.78; exactly 64 are 128 bounds-checked tiles, which
+// share it four ways: 1.12 to 1.24. (At 96 tiles of a shorter K f16 1024 x 3072 x 1024 with ReLU takes 23.3 us against 22.1.)
+template <typename AccElem, bool EXACT, bool A_KC, bool B_KC, bool FP8>
+bool ring_pays(const MfmaArgs &p, bool staged, size_t tiles, size_t k_bytes, bool long_k, unsigned filled) {
+  constexpr bool kInt = std::is_same<AccElem, int>::value;
+  constexpr bool kSlowOthers = FP8 && !EXACT && !(A_KC && B_KC);  // transposed fragments of 32 bytes: they take two to four times as long
+  constexpr unsigned kNever = 101;
+  const bool reads_c = kInt ? p.beta.i != 0 : !(p.beta.fz.skip_c_read && p.beta.f == 0.0f);
+  if (tiles < 200) return staged && long_k && (tiles > 64 || kSlowOthers);
+  if (tiles <= 256) return staged || reads_c || k_bytes > 256;
+  if (!staged) return reads_c || filled >= (k_bytes > 1024 ? 60 : k_bytes > 256 ? 80 : kNever);
+  if (kInt || kSlowOthers) return true;
+  if (!p.rq.q_only && p.csc0 != 1) return true;  // C written by columns: the others take three to four times as long
+  if (p.rq.act >= 2) {
+    if (reads_c) return filled >= (k_bytes >= 4096 ? 0 : k_bytes >= 2048 ? 70 : k_bytes >= 1024 ? 80 : kNever);
+    return filled >= (k_bytes >= 4096 ? 70 : k_bytes >= 2048 ? 80 : EXACT && k_bytes >= 1024 ? 90 : kNever);
+  }
+  if (reads_c) return !EXACT || filled >= 70;
+  if (EXACT) return filled >= (k_bytes >= 1024 ? 80 : kNever);
+  return filled >= (k_bytes >= 4096 ? 0 : k_bytes >= 1024 ? 70u : 90u);
+}
+
 // The streaming kernel takes problems that its tiles divide evenly: 256 x 256 tiles when those can fill the 256 compute
-// units, 256 x 128 tiles for the sizes below that. Returns kNotWholeTiles for the others.
+// units, 256 x 128 tiles for the sizes below that, from 96 tiles on, or from 64 when K is long enough to be shared between
+// two workgroups per tile. Returns kNotWholeTiles for the others, and where the bounds-checked kernels are faster.
 constexpr int kNotWholeTiles = 0x7FFFFFFF;
 template <int TA, int TB, bool A_KC, bool B_KC, bool EXACT>
 int launch_whole_tiles(const MfmaArgs &p) {
   constexpr int ES = Kind<TA>::ES;
   constexpr size_t kRing128FromTiles = 96;
+  using AccElem = decltype(typename Kind<TA>::Acc{}.x);
   const auto wide = [](const MfmaArgs &q) { return launch_ring<TA, TB, A_KC, B_KC, 256, false, 0, false, false, EXACT>(q); };
   const auto narrow = [](const MfmaArgs &q) { return launch_ring<TA, TB, A_KC, B_KC, 128, false, 0, false, false, EXACT>(q); };
-  if (p.m % 256 != 0 || (p.k * ES) % 128 != 0) return kNotWholeTiles;
-  const size_t tiles_m = p.m / 256;
-  // Steps that the epilogue over LDS rows applies: nothing overlaps it, where the bounds-checked kernels have several
-  // workgroups on a compute unit. So not for tiles that leave half of the chip idle (f16 1024 x 3072 x 1024 with ReLU 22.1
-  // against 23.3 us, E4M3 1024 x 4096 x 3072 with SiLU 36.6 / 42.9; 2048 x 4096 x 512 with SiLU, 256 narrow tiles: bf16
-  // 37.3 / 31.8, E4M3 36.1 / 33.6), nor for SiLU or GELU over several rounds of a K too short to outweigh them
-  // (4096 x 8192 x 512: bf16 with GELU 106.7 / 109.8 us, E4M3 with SiLU 94.8 / 103.5; int8 with ReLU 52.0 / 49.4).
-  using AccElem = decltype(typename Kind<TA>::Acc{}.x);
+  if (p.m % 256 != 0 || p.n % 128 != 0 || (p.k * ES) % 128 != 0) return kNotWholeTiles;
+  const size_t tiles_m = p.m / 256, slices = p.k * ES / kRingSlice;
+  const size_t tiles = p.n % 256 == 0 ? tiles_m * (p.n / 256) : 0, tiles128 = tiles_m * (p.n / 128);
+  // A last round of 256 x 256 tiles that would fill at most half of the 256 compute units is run as 256 x 128 tiles
+  // instead (a second launch on the trailing columns): twice the workgroups at half the length.
+  const size_t rest = tiles % 256;
+  const bool tail_round = rest != 0 && rest <= 128 && rest % tiles_m == 0;
+  const bool long_k = slices % 4 == 0 && slices / 2 >= kRingMinSlicesPerSplit;
   const bool extra = p.rq.act || p.rq.q;
   if (extra && !kRingCarriesExtraSteps<TA, TB>) return kNotWholeTiles;
   const bool staged = extra && !(!EXACT && FusedSteps<AccElem, 2>::dword_copy(p.rq));
-  if (staged && p.rq.act >= 2 && p.k * ES < 2048 && tiles_m * (p.n / 256) > 256) return kNotWholeTiles;
-  if (p.n % 256 == 0 && tiles_m * (p.n / 256) >= 200) {
-    // A last round that would fill at most half of the 256 compute units is run as 256 x 128 tiles
-    // instead (a second launch on the trailing columns): twice the workgroups at half the length.
-    const size_t tiles = tiles_m * (p.n / 256), rest = tiles % 256;
-    if (rest != 0 && rest <= 128 && rest % tiles_m == 0) {
-      const size_t tail_cols = rest / tiles_m * 256, head_cols = p.n - tail_cols;
-      MfmaArgs head = p, tail = p;
-      head.n = head_cols;
-      tail.n = tail_cols;
-      tail.b = p.b + (head_cols / 64) * p.b_s1 * ES;
-      tail.c = p.c + (head_cols >> p.ccs) * p.csc1 * sizeof(float);  // whole blocks; C elements are 4 bytes for every kind
-      if (p.bias) tail.bias = p.bias + head_cols * sizeof(float);
-      if (p.rq.q) tail.rq.q = p.rq.q + head_cols * p.rq.csq;
-      if (p.rq.q && p.rq.q_per_column) tail.rq.q_scale = p.rq.q_scale + head_cols;
-      const int rc = wide(head);
-      return rc != 0 ? rc : narrow(tail);
-    }
-    return wide(p);
+  if ((staged || EXACT) &&
+      !ring_pays<AccElem, EXACT, A_KC, B_KC, TA == SKL_DT_F8E4M3 || TA == SKL_DT_F8E5M2>(
+          p, staged, tiles >= 200 ? tiles : tiles128, p.k * ES, long_k, tiles >= 200 ? rounds_filled(tiles, tail_round) : rounds_filled(tiles128)))
+    return kNotWholeTiles;
+  if (tiles >= 200) {
+    if (!tail_round) return wide(p);
+    const size_t tail_cols = rest / tiles_m * 256, head_cols = p.n - tail_cols;
+    MfmaArgs head = p, tail = p;
+    head.n = head_cols;
+    tail.n = tail_cols;
+    tail.b = p.b + (head_cols / 64) * p.b_s1 * ES;
+    tail.c = p.c + (head_cols >> p.ccs) * p.csc1 * sizeof(float);  // whole blocks; C elements are 4 bytes for every kind
+    if (p.bias) tail.bias = p.bias + head_cols * sizeof(float);
+    if (p.rq.q) tail.rq.q = p.rq.q + head_cols * p.rq.csq;
+    if (p.rq.q && p.rq.q_per_column) tail.rq.q_scale = p.rq.q_scale + head_cols;
+    const int rc = wide(head);
+    return rc != 0 ? rc : narrow(tail);
   }
-  // ... from 96 tiles on, or from 64 when K is long enough to be shared between two workgroups per tile
-  const size_t tiles128 = p.n % 128 == 0 ? tiles_m * (p.n / 128) : 0, slices = p.k * ES / kRingSlice;
-  if (tiles128 >= (EXACT || staged ? 200 : kRing128FromTiles) || (tiles128 >= 64 && slices % 4 == 0 && slices / 2 >= kRingMinSlicesPerSplit)) return narrow(p);
+  if (tiles128 >= kRing128FromTiles || (tiles128 >= 64 && long_k)) return narrow(p);
   return kNotWholeTiles;
 }
 
@@ -1806,9 +1852,9 @@ int launch_tile(const MfmaArgs &p) {
   constexpr int ES = Kind<TA>::ES;
   constexpr bool kFp8 = TA == SKL_DT_F8E4M3 || TA == SKL_DT_F8E5M2;
   if constexpr (kFp8) {
-    // short K: exact products (see MmaF8Exact), on the streaming kernel when its tiles fill the chip (us, bounds-checked
-    // 128 x 128 / streaming: 2048 x 8192 x 2048 77 / 62, with GELU into E4M3 111 / 98; 2048 x 4096 x 2048 42 / 34, x 1024
-    // with GELU into E4M3 43 / 40; on 128 tiles, 512 x 8192 x 2048, 25.4 / 26.2)
+    // short K: exact products (see MmaF8Exact), on the streaming kernel when its tiles fill the chip and ring_pays() (us,
+    // bounds-checked 128 x 128 / streaming: 2048 x 8192 x 2048 77 / 62, with GELU into E4M3 111 / 94; 2048 x 4096 x 2048
+    // 42 / 34; on 128 tiles, 512 x 8192 x 2048, 25.4 / 26.2)
     if (p.k <= kF8ExactMaxK) {
       const int rc = launch_whole_tiles<TA, TB, A_KC, B_KC, true>(p);
       if (rc != kNotWholeTiles) return rc;
