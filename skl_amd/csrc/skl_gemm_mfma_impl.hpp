@@ -1776,7 +1776,7 @@ inline unsigned rounds_filled(size_t tiles, bool tail = false) {
 //   short fp8, SiLU or GELU, C read below 1024  1.19 1.22 1.17 1.07 1.02   from 1024  1.12 1.06 1.09 0.99 0.93
 //                         not read  below 1024  1.43 1.33 1.22 1.07 1.04   from 1024  1.31 1.21 1.13 1.03 0.96
 //   short fp8, none or ReLU, C read below 1024  1.01 1.01 0.92 0.90 0.91   from 1024  1.03 1.03 0.93 0.93 0.92
-//                         not read  below 1024  1.25 1.11 1.11 1.06 1.01   from 1024  1.09 1.15 1.07 0.97 0.90
+//                         not read  below 1024  1.25 1.11 1.11 1.06 1.01   from 1024  1.09 1.15 1.07 0.97 0.90   with an fp8 copy 0.97 to 1.02 from 512 on
 //   short fp8, no steps, C read     up to 1024  0.90 0.92 0.87 0.85 0.85   beyond     0.99 0.92 0.89 0.84 0.80
 //                         not read  up to 256   1.11 1.13 1.14 1.08 1.08   up to 1024 1.10 1.06 1.05 0.96 0.95   beyond 1.04 0.99 1.00 0.90 0.84
 //   int8                            C read 0.60 to 0.91, not read 0.67 to 0.99, at any K
@@ -1799,6 +1799,7 @@ bool ring_pays(const MfmaArgs &p, bool staged, size_t tiles, size_t k_bytes, boo
     return filled >= (k_bytes >= 4096 ? 70 : k_bytes >= 2048 ? 80 : EXACT && k_bytes >= 1024 ? 90 : kNever);
   }
   if (reads_c) return !EXACT || filled >= 70;
+  if (EXACT && p.rq.q && p.rq.q_fmt != 0) return k_bytes >= 512 || filled >= 70;
   if (EXACT) return filled >= (k_bytes >= 1024 ? 80 : kNever);
   return filled >= (k_bytes >= 4096 ? 0 : k_bytes >= 1024 ? 70u : 90u);
 }
