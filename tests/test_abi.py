@@ -115,7 +115,7 @@ def test_compat_header_agrees_with_the_reference_prototypes(tmp_path):
     import pytest
     ref = "/root/reference"
     clang = "/opt/rocm/lib/llvm/bin/clang"
-    if not (os.path.isdir(ref) and os.path.exists(clang)):
+    if not (os.path.isdir(os.path.join(ref, "include")) and os.path.exists(clang)):
         pytest.skip("needs the reference checkout and a compiler with __bf16 / _Float16")
     features = ("zve32x zve32f zve64d zvfh zvfbfwma zvfbfmin zvfofp8min zvfofp4min xsfmmbase xsfmm32a8i xsfmm32a8f "
                 "xsfmm32a16f xsfmm32a32f xsfvqdotq").split()
