@@ -26,7 +26,8 @@ extern "C" int skl_hip_gemm_mfma_supported(const skl_gemm_canon *g) {
 
 namespace {
 
-// Would the problem, as it lies in memory, run on the streaming kernel? (The rule of launch_tile.)
+// Would the problem, as it lies in memory, run on the streaming kernel? (The rule of launch_whole_tiles for calls without
+// activation or copy and beyond the short fp8 K; its callers decide about those themselves.)
 bool streams_in_place(const skl_gemm_canon *g, size_t es) {
   if (!skl_hip_gemm_mfma_supported(g) || g->m % 256 != 0 || (g->k * es) % 128 != 0) return false;
   const size_t tiles_m = g->m / 256;
@@ -62,14 +63,30 @@ extern "C" int skl_hip_gemm_mfma_padded_plan(const skl_gemm_canon *g, size_t *mp
   // With an activation or an 8-bit copy only where the operands would be copied anyway: the bounds-checked kernel, in
   // place, is the faster one for merely ragged sizes (bf16 2000 x 5000 x 3000 with SiLU 127 against 139 us, E4M3
   // 1027 x 8190 x 4096 into E4M3 87 against 114), the padded copies behind its own copies (int8 3001 x 4099 x 5003
-  // with ReLU into int8 172 against 124 us).
-  if ((g->rq.act || g->rq.q) && (skl_hip_gemm_mfma_supported(g) || (g->rq.act >= 2 && g->k * es < 2048))) return 0;
-  if (fp8a && g->k <= kF8ExactMaxK) return 0;  // short K: the exact fp8 product, which the streaming kernel does not have
+  // with ReLU into int8 172 against 124 us). Nor for whole tiles: the one operand that breaks the 16-byte rule is copied
+  // and the streaming kernel reads the other where it lies, with the epilogue without LDS rows and the trailing round of
+  // narrow tiles where those apply (padded copies take 1.25 times as long with a copy in dwords, 1.16 with other steps:
+  // medians of 42 and of 133 random layers). Only where both are copied, and padding N to 256 columns gives a chip full
+  // of the larger tiles, are padded copies as good or better (0.93, 14 layers).
+  const bool fused = g->rq.act || g->rq.q, wide_enough = (g->m + 255) / 256 * ((g->n + 255) / 256) >= 200;
+  const bool a_ok = operand_ok(g->a, es, g->a_s1, g->a_s0, g->a_sk, g->m, g->k), b_ok = operand_ok(g->b, es, g->b_s1, g->b_s0, g->b_sk, g->n, g->k);
+  if (fused) {
+    const bool whole = g->m % 256 == 0 && g->n % 128 == 0 && (g->k * es) % 128 == 0;
+    const bool dwords = g->ta == SKL_DT_I8 ? FusedSteps<int, 2>::dword_copy(g->rq) : FusedSteps<float, 2>::dword_copy(g->rq);
+    if (g->ta != g->tb || skl_hip_gemm_mfma_supported(g) || (g->rq.act >= 2 && g->k * es < 2048)) return 0;
+    if (whole && (dwords || a_ok || b_ok || !wide_enough || g->n % 256 == 0)) return 0;
+  }
+  if (fp8a && g->k <= kF8ExactMaxK) return 0;  // short K: the exact fp8 product, which the streaming kernel has for whole tiles only
   const size_t tiles_m = (g->m + 255) / 256;
   int tile_cols = 0;
-  if (tiles_m * ((g->n + 255) / 256) >= 200) tile_cols = 256;
-  else if (tiles_m * ((g->n + 127) / 128) >= (g->rq.act || g->rq.q ? 200 : 96)) tile_cols = 128;  // the rules of launch_whole_tiles
+  if (wide_enough) tile_cols = 256;
+  else if (tiles_m * ((g->n + 127) / 128) >= (fused ? 200 : 96)) tile_cols = 128;  // the rules of launch_whole_tiles
   if (!tile_cols) return 0;
+  // The epilogue of a fused call overlaps nothing, so its last round has to be fairly full (over the bounds-checked kernel
+  // behind its own copies: 0.86 from 70 per cent on, 1.02 and up to 1.6 below; medians of 130 random layers) - unless that
+  // kernel would read an fp8 operand across K where it lies (0.35 to 0.6), or for int8 of some K (0.8 to 0.95).
+  const bool across_k = fp8a && ((a_ok && g->a_sk != 1) || (b_ok && g->b_sk != 1));
+  if (fused && !across_k && !(g->ta == SKL_DT_I8 && g->k >= 1024) && rounds_filled(tiles_m * ((g->n + tile_cols - 1) / tile_cols)) < 70) return 0;
   *mp = tiles_m * 256;
   *np = (g->n + tile_cols - 1) / tile_cols * tile_cols;
   *kp = (g->k * es + 127) / 128 * 128 / es;

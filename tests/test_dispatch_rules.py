@@ -1,0 +1,75 @@
+"""The host side of the matrix-core dispatch, asked without a GPU: which problems go to the streaming kernel through copies
+of A and B padded to whole tiles (skl_hip_gemm_mfma_padded_plan)."""
+import ctypes as ct
+
+import pytest
+
+import skl_amd
+
+I8, BF16, F16, E4M3, E5M2 = range(5)
+
+
+class Requant(ct.Structure):  # skl_requant of skl_amd/csrc/skl_launch.h
+    _fields_ = [("act", ct.c_int), ("q_per_column", ct.c_int), ("q_only", ct.c_int), ("q_zero", ct.c_int32), ("q", ct.c_void_p),
+                ("rsq", ct.c_size_t), ("csq", ct.c_size_t), ("q_scale", ct.c_void_p), ("q_fmt", ct.c_int)]
+
+
+class Canon(ct.Structure):  # skl_gemm_canon
+    _fields_ = [("ta", ct.c_int), ("tb", ct.c_int), ("m", ct.c_size_t), ("n", ct.c_size_t), ("k", ct.c_size_t),
+                ("a", ct.c_void_p), ("a_s1", ct.c_size_t), ("a_s0", ct.c_size_t), ("a_sk", ct.c_size_t),
+                ("b", ct.c_void_p), ("b_s1", ct.c_size_t), ("b_s0", ct.c_size_t), ("b_sk", ct.c_size_t),
+                ("c", ct.c_void_p), ("rsc0", ct.c_size_t), ("csc0", ct.c_size_t), ("rsc1", ct.c_size_t), ("csc1", ct.c_size_t),
+                ("c_row_shift", ct.c_uint), ("c_col_shift", ct.c_uint), ("alpha", ct.c_double), ("beta", ct.c_double),
+                ("bias", ct.c_void_p), ("max", ct.c_void_p), ("rq", Requant)]
+
+
+def plan(kind, m, n, k, lda=None, ldb=None, act=0, q_fmt=None, b_rows=True):
+    """The tile width of the padded plan for row-major A (lda) and B (row-major, or [n][k]); 0: no padded copies."""
+    g = Canon(ta=kind, tb=kind, m=m, n=n, k=k, a=1 << 20, b=1 << 20, c=1 << 20, a_sk=1, c_row_shift=6, c_col_shift=6)
+    g.a_s0 = lda or k
+    g.a_s1 = 64 * g.a_s0
+    ldb = ldb or (n if b_rows else k)
+    g.b_s0, g.b_sk = (1, ldb) if b_rows else (ldb, 1)
+    g.b_s1 = 64 * g.b_s0
+    g.rsc0, g.csc0, g.rsc1, g.csc1 = n, 1, 64 * n, 64
+    g.rq.act = act
+    if q_fmt is not None:
+        g.rq.q, g.rq.rsq, g.rq.csq, g.rq.q_scale, g.rq.q_fmt = 1 << 20, (n + 3) // 4 * 4, 1, 1 << 20, q_fmt
+    fn = ct.CDLL(skl_amd.library_path()).skl_hip_gemm_mfma_padded_plan
+    fn.argtypes = [ct.POINTER(Canon)] + [ct.POINTER(ct.c_size_t)] * 3
+    padded = [ct.c_size_t(0) for _ in range(3)]
+    cols = fn(ct.byref(g), *(ct.byref(x) for x in padded))
+    if cols:
+        mp, np_, kp = (x.value for x in padded)
+        es = 2 if kind in (BF16, F16) else 1
+        assert mp % 256 == 0 and np_ % cols == 0 and kp * es % 128 == 0 and mp >= m and np_ >= n and kp >= k
+    return cols
+
+
+@pytest.mark.parametrize("kind,same_fmt", ((I8, 0), (BF16, 2), (E4M3, 2)))
+def test_fused_whole_tiles_copy_only_the_operand_that_needs_it(kind, same_fmt):
+    """A fused problem of whole tiles with one operand off the 16-byte rule is not padded; nor with both off it when the
+    8-bit copy goes out in dwords. The same problem without fused steps is, and so are ragged fused ones."""
+    for lda, ldb in ((4097, None), (None, 4097)):
+        assert plan(kind, 4096, 4096, 4096, lda, ldb, act=1, q_fmt=same_fmt) == 0
+        assert plan(kind, 4096, 4096, 4096, lda, ldb, act=1) == 0
+        assert plan(kind, 4096, 4096, 4096, lda, ldb) == 256
+    assert plan(kind, 4096, 4096, 4096, 4097, 4097, act=1, q_fmt=same_fmt) == 0
+    assert plan(kind, 4096, 4096 + 128, 4096, 4097, 4097 + 128, act=1, q_fmt=same_fmt) == 0
+    assert plan(kind, 4096, 4096, 4096, 4097, 4097, act=1) == 0
+    assert plan(kind, 4096, 3968, 4096, 4097, 3969, act=1) == 256  # both copied anyway, and 256 tiles of 256 columns
+    assert plan(kind, 4001, 4099, 5003, act=1, q_fmt=same_fmt) == (0 if kind != I8 else 256)  # 272 tiles: a last round of 16
+    assert plan(kind, 4001, 4099, 5003, ldb=4112, act=1, q_fmt=same_fmt) == (0 if kind == BF16 else 256)  # B read across K
+    assert plan(kind, 4001, 4051, 5003, act=1, q_fmt=same_fmt) == 256
+    assert plan(kind, 4001, 4051, 5008, lda=5008, ldb=4064, act=1, q_fmt=same_fmt) == 0  # aligned: ragged, read in place
+
+
+@pytest.mark.parametrize("m", (1, 100, 256, 300, 2048, 51200))
+@pytest.mark.parametrize("n", (1, 100, 130, 256, 6400))
+def test_every_size_has_an_answer(m, n):
+    for kind in range(5):
+        for k in (1, 128, 2304, 2432, 5003):
+            for act in (0, 1, 2):
+                if kind or act < 2:
+                    assert plan(kind, m, n, k, act=act) in (0, 128, 256)
+                    assert plan(kind, m, n, k, lda=k + 1, ldb=k + 3, act=act, b_rows=False) in (0, 128, 256)

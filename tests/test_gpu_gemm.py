@@ -1292,6 +1292,30 @@ def test_silu_and_gelu_looped_over_rows(gpu, ta, m, n, k, act):
         assert np.array_equal(q, want_q)
 
 
+@pytest.mark.parametrize("ta,n,k", (("i8", 6400, 256), ("i8", 3200, 256), ("bf16", 3200, 1024), ("f8e4m3", 6400, 2432), ("f8e4m3", 3200, 512)))
+@pytest.mark.parametrize("a_pad,b_pad", ((1, 0), (0, 1), (1, 1)))
+def test_fused_layers_of_whole_tiles_off_the_16_byte_rule(gpu, ta, n, k, a_pad, b_pad):
+    """Whole tiles with an operand (or both) in rows that begin anywhere: C, the copy and the maximum have the bits of the
+    same call on aligned rows, with a copy in dwords and one in bytes, and with the activation alone."""
+    m = 2048
+    rng = np.random.default_rng(n + k)
+    plain = rowmajor_case(ta, m, n, k, 1, 1)
+    case = rowmajor_case(ta, m, n, k, 1, 1, rsa=k + a_pad, rsb=n + b_pad)
+    a, b, c = plain.make_inputs(int(rng.integers(1 << 30)))
+    ua, ub = np.zeros(m * (k + a_pad), a.dtype), np.zeros(k * (n + b_pad), b.dtype)
+    ua.reshape(m, k + a_pad)[:, :k] = a.reshape(m, k)
+    ub.reshape(k, n + b_pad)[:, :n] = b.reshape(k, n)
+    bias = rng.integers(-99, 99, n).astype(np.int32) if ta == "i8" else rng.uniform(-4, 4, n).astype(np.float32)
+    start = np.array([-(1 << 31)], np.int32) if ta == "i8" else np.array([-np.inf], np.float32)
+    scale = np.array([0.002 if ta == "i8" else 0.5], np.float32)
+    for fmt, rsq, only in ((0, n, True), (2, n, False), (2, n + 1, False), (None, 0, False)):
+        rq = None if fmt is None else dict(q=np.zeros(m * rsq, np.int8), rsq=rsq, csq=1, scale=scale, format=fmt, only=only)
+        want = run_fused_gemm(gpu, "rc", plain, a, b, c, bias, start, "device", activation=1, requant=rq)
+        got = run_fused_gemm(gpu, "rc", case, ua, ub, c, bias, start, "device", activation=1, requant=rq)
+        for x, y in zip(got, want):
+            assert np.array_equal(x.view(np.uint8), y.view(np.uint8)), (ta, fmt, rsq)
+
+
 @pytest.mark.parametrize("ta,tb", (("i8", "i8"), ("bf16", "bf16"), ("f16", "f16"), ("f8e4m3", "f8e4m3"), ("f8e4m3", "f8e5m2")))
 def test_ragged_problems_on_padded_copies(gpu, ta, tb):
     """Ragged M, N and K (and odd leading dimensions) on a problem large enough to fill the chip: A and B are copied
