@@ -102,7 +102,8 @@ struct FusedSteps {
   // What a descriptor must look like for modes 2 and 3: a row-major copy on 4-byte boundaries, no activation beyond
   // ReLU (the others cost too much code in each of a lane's 128 elements), and the copy's format the one these
   // modes are built with for C's type - int8 behind an int32 C, OCP fp8 behind a floating-point C (an int8 product
-  // feeding an int8 layer, an fp8 product an fp8 layer; other pairings run on the bounds-checked kernels).
+  // feeding an int8 layer, an fp8 product an fp8 layer; other pairings take write_wave_tile_staged or the bounds-checked
+  // kernels).
   static constexpr bool kCopyIsFp8 = !std::is_same<T, int>::value;
   __host__ __device__ static bool dword_copy(const skl_requant &r) {
     return r.q && r.act <= 1 && (r.q_fmt != 0) == kCopyIsFp8 && r.csq == 1 && (r.rsq & 3) == 0 && ((uintptr_t)r.q & 3) == 0;
@@ -596,7 +597,7 @@ __device__ __forceinline__ void write_wave_tile(const MfmaArgs &p, const Acc (&a
 // Such calls ran on the bounds-checked 128 x 128 kernels: bf16 2048 x 8192 x 4096 with SiLU 188 -> 137 us, int8 4096^3
 // with ReLU 105 -> 72, E4M3 2048 x 8192 x 4096 with GELU into E4M3 125 -> 99 (110 while every lane multiplied out the
 // addresses of its rows); what is left of the last over the same call with ReLU, 37 us, is mostly the erfc of 16.8 million
-// elements. launch_whole_tiles says where the line lies.
+// elements. ring_pays says where the line lies.
 // alpha, beta and the old C are applied as a strip of 32 rows goes into LDS, and the old values of the next strip are
 // requested ahead of this one's stores: a load inside the loop waits for the stores of the pass before, every pass
 // (see write_wave_tile; C read, us, loads in the loop / ahead: E5M2 1024 x 14080 x 6272 with ReLU into int8 102 / 91, E4M3
@@ -1122,7 +1123,8 @@ constexpr int ceil_div(int a, int b) { return (a + b - 1) / b; }
 // EXACT: OCP fp8 operands multiplied exactly (MmaF8Exact). The bytes travel and are read like int8's; a fragment is
 // widened behind the MFMAs in front of its first use, B's NI and A's first at the top of the k-step. A wave widens
 // MI + NI fragments for MI x NI products - on the 128 x 128 kernels, with 64 x 32 per wave, three for two, which is
-// more vector work than the matrix cores take for the products; here six for eight. E4M3 2048 x 8192 x 2048: 77 us there,
+// more vector work than the matrix cores take for the products; here six for eight (256 columns) or four for four (128).
+// E4M3 2048 x 8192 x 2048: 77 us there,
 // 62 here (1.1 PFLOP/s, what the f16 kernel reaches).
 template <int TA, int TB, bool A_KC, bool B_KC, int BN, bool EDGE = false, int EXTRA = 0, bool CQUADS = false, bool SCAN = false, bool EXACT = false>
 __global__ void __launch_bounds__(512) gemm_mfma_ring_kernel(MfmaArgs p) {

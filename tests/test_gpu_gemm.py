@@ -407,9 +407,9 @@ EXTRA_STEP_SHAPES = (
     (130, 200, 64, 1, "64 x 64 bounds-checked tiles"),
     (300, 1100, 96, 0, "128 x 128 bounds-checked tiles"),
     (512, 768, 256, 1, "whole tiles, too few for the streaming kernel"),
-    (2048, 2048, 128, 1, "streaming kernel, 256 x 128 tiles (int8 with a row-major copy; everything else: bounds-checked kernels)"),
-    (2048, 9216, 128, 0, "streaming kernel, 256 x 256 tiles and a second launch of 256 x 128 on the last columns (int8)"),
-    (2048, 2048, 2560, 1, "streaming kernel, K beyond the exact fp8 kernels' range (int8 and fp8 kinds with a row-major copy)"),
+    (2048, 2048, 128, 1, "128 tiles of 256 x 128: streaming kernel where the copy goes out in dwords, else the bounds-checked kernels"),
+    (2048, 9216, 128, 0, "288 tiles of 256 x 256, a last round of 256 x 128: streaming kernel for int8 and where the copy goes out in dwords"),
+    (2048, 2048, 2560, 1, "128 tiles of a K beyond the exact fp8 kernels' range: streaming kernel where the copy goes out in dwords"),
     (1000, 1100, 520, 0, "ragged and large enough for padded copies: must stay on the bounds-checked kernels"),
     (16, 4096, 4096, 1, "a decode batch"),
     (40, 300, 8192, 1, "K shared between workgroups: the steps ride on the pass that adds the shares"),
@@ -586,7 +586,7 @@ def test_silu_and_gelu_values(gpu, act):
 
 @pytest.mark.parametrize("ta,m,n,k,what", (
     ("bf16", 300, 1100, 96, "bounds-checked tiles"),
-    ("f16", 2048, 2048, 128, "whole tiles: still the bounds-checked kernels, which carry the steps"),
+    ("f16", 2048, 2048, 128, "whole tiles, too few for the streaming kernel with these steps"),
     ("f8e4m3", 40, 300, 8192, "K shared between workgroups: the pass that adds the shares"),
     ("bf16", 16, 4096, 4096, "a decode batch: the pass that adds the planes"),
     ("f8e5m2", 1, 2048, 512, "M = 1"),
@@ -1076,7 +1076,7 @@ def test_blockings_no_kernel_reads_in_place(gpu, ta, tb):
 @pytest.mark.parametrize("ta", ("f32", "f64", "f16h"))
 def test_register_tiled_kernel_bit_identical(gpu, ta):
     """f32, f64 and f16 -> f16 on the register-tiled kernel: the same bits as the checker over the whole C buffer.
-    Both tile sizes (64 x 64; 128 x 128 from 512 tiles on), every pairing of row- and column-major operands, 64-row
+    Tiles of 16 x 32, 64 x 64 and (K below one slab) 128 x 128, every pairing of row- and column-major operands, 64-row
     panels, ragged edges in M, N and K, K shorter than one slab, beta == 0 and != 0."""
     from support import GemmCase
     te = support.TE
