@@ -318,6 +318,8 @@ int launch(const skl_gemm_canon *g) {
 // f32, us, at K = 2048 (128 x 128 / 64 x 64 of 4 x 4 / 64 x 64 of 4 x 2 / 32 x 32 / 16 x 32 tiles):
 //   4096^2: 1243 / 1275 / 1356 / 2110 / 3066    2048^2: 347 / 349 / 364 / 532 / 779
 //   1024^2: 349 / 180 / 132 / 159 / 220          512^2: 338 / 170 / 121 / 78 / 70     256^2: 337 / 169 / 121 / 76 / 61
+// The same limits serve f64 and f16: over 500 random problems the median time over that of 64 x 64 and 128 x 128 tiles alone
+// is, on the tiles from 64 x 64 of 4 x 2 down, f32 0.71 / 0.45 / 0.30, f64 0.81 / 0.56 / 0.40, f16 0.72 / 0.48 / 0.27.
 //
 // Floats are staged in slabs of 32 from K = 512 on, of 16 below on the two larger tiles: half the LDS puts more
 // workgroups on a compute unit, which is what a short K lives on, and a K of 16 fills its slab (f32, over the time with
