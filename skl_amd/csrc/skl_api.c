@@ -333,8 +333,8 @@ static int gemm_fast_path(const skl_gemm_canon *g, int fused, int launch) {
   return DECLINED;
 }
 
-/* An operand in a layout that none of the kernels reads - a leading dimension that is not a multiple of 16 bytes,
- * the row-major k x n matrix of a matrix-vector product, no unit stride at all - is copied into scratch memory as
+/* An operand in a layout that none of the kernels reads - no unit stride at all, rows shorter than 16 bytes, blocks off
+ * the 16-byte rule, or whole tiles that miss the streaming kernel by that rule - is copied into scratch memory as
  * rows contiguous in K, 16-byte aligned, and the problem runs on the copy: B alone, A alone, or both, whichever
  * the kernels accept first. Worth a copy only when the product is not tiny. */
 static int gemm_with_realigned_operands(const skl_gemm_canon *g, int fused) {

@@ -11,14 +11,34 @@ SKL_MFMA_DECLARE_KIND(f8e5m2)
 SKL_MFMA_DECLARE_KIND(f8e4m3_f8e5m2)
 SKL_MFMA_DECLARE_KIND(f8e5m2_f8e4m3)
 
+namespace {
+
+bool aligned_a(const skl_gemm_canon *g, size_t es) { return operand_ok(g->a, es, g->a_s1, g->a_s0, g->a_sk, g->m, g->k); }
+bool aligned_b(const skl_gemm_canon *g, size_t es) { return operand_ok(g->b, es, g->b_s1, g->b_s0, g->b_sk, g->n, g->k); }
+
+// Whole tiles enough for the streaming kernel, wherever the operands lie. (The rule of launch_whole_tiles for calls without
+// activation or copy and beyond the short fp8 K; its callers decide about those themselves.)
+bool tiles_to_stream(const skl_gemm_canon *g, size_t es) {
+  if (g->m % 256 != 0 || (g->k * es) % 128 != 0) return false;
+  const size_t tiles_m = g->m / 256;
+  return (g->n % 256 == 0 && tiles_m * (g->n / 256) >= 200) || (g->n % 128 == 0 && tiles_m * (g->n / 128) >= 96);
+}
+
+}  // namespace
+
 extern "C" int skl_hip_gemm_mfma_supported(const skl_gemm_canon *g) {
   if (g->m == 0 || g->n == 0 || g->k == 0) return 0;
   const bool fp8a = g->ta == SKL_DT_F8E4M3 || g->ta == SKL_DT_F8E5M2;
   const bool fp8b = g->tb == SKL_DT_F8E4M3 || g->tb == SKL_DT_F8E5M2;
   if (!(g->ta == g->tb || (fp8a && fp8b))) return 0;
   const size_t es = (g->ta == SKL_DT_BF16 || g->ta == SKL_DT_F16) ? 2 : 1;
-  if (!operand_ok(g->a, es, g->a_s1, g->a_s0, g->a_sk, g->m, g->k)) return 0;
-  if (!operand_ok(g->b, es, g->b_s1, g->b_s0, g->b_sk, g->n, g->k)) return 0;
+  const bool a_ok = aligned_a(g, es), b_ok = aligned_b(g, es);
+  if (!a_ok || !b_ok) {
+    // off the 16-byte rule: the bounds-checked kernels, in place, unless a copy of the operand lets the streaming kernel run
+    if (tiles_to_stream(g, es)) return 0;
+    if (!a_ok && !operand_loose_ok(es, g->a_s1, g->a_s0, g->a_sk, g->m, g->k)) return 0;
+    if (!b_ok && !operand_loose_ok(es, g->b_s1, g->b_s0, g->b_sk, g->n, g->k)) return 0;
+  }
   if (((uintptr_t)g->c & 3) != 0) return 0;
   if (g->c_row_shift < 2 || g->c_row_shift > 6 || g->c_col_shift < 1 || g->c_col_shift > 6) return 0;
   return 1;
@@ -26,12 +46,9 @@ extern "C" int skl_hip_gemm_mfma_supported(const skl_gemm_canon *g) {
 
 namespace {
 
-// Would the problem, as it lies in memory, run on the streaming kernel? (The rule of launch_whole_tiles for calls without
-// activation or copy and beyond the short fp8 K; its callers decide about those themselves.)
+// Would the problem, as it lies in memory, run on the streaming kernel?
 bool streams_in_place(const skl_gemm_canon *g, size_t es) {
-  if (!skl_hip_gemm_mfma_supported(g) || g->m % 256 != 0 || (g->k * es) % 128 != 0) return false;
-  const size_t tiles_m = g->m / 256;
-  return (g->n % 256 == 0 && tiles_m * (g->n / 256) >= 200) || (g->n % 128 == 0 && tiles_m * (g->n / 128) >= 96);
+  return skl_hip_gemm_mfma_supported(g) && aligned_a(g, es) && aligned_b(g, es) && tiles_to_stream(g, es);
 }
 
 }  // namespace
@@ -69,11 +86,11 @@ extern "C" int skl_hip_gemm_mfma_padded_plan(const skl_gemm_canon *g, size_t *mp
   // medians of 42 and of 133 random layers). Only where both are copied, and padding N to 256 columns gives a chip full
   // of the larger tiles, are padded copies as good or better (0.93, 14 layers).
   const bool fused = g->rq.act || g->rq.q, wide_enough = (g->m + 255) / 256 * ((g->n + 255) / 256) >= 200;
-  const bool a_ok = operand_ok(g->a, es, g->a_s1, g->a_s0, g->a_sk, g->m, g->k), b_ok = operand_ok(g->b, es, g->b_s1, g->b_s0, g->b_sk, g->n, g->k);
+  const bool a_ok = aligned_a(g, es), b_ok = aligned_b(g, es);
   if (fused) {
     const bool whole = g->m % 256 == 0 && g->n % 128 == 0 && (g->k * es) % 128 == 0;
     const bool dwords = g->ta == SKL_DT_I8 ? FusedSteps<int, 2>::dword_copy(g->rq) : FusedSteps<float, 2>::dword_copy(g->rq);
-    if (g->ta != g->tb || skl_hip_gemm_mfma_supported(g) || (g->rq.act >= 2 && g->k * es < 2048)) return 0;
+    if (g->ta != g->tb || (a_ok && b_ok) || (g->rq.act >= 2 && g->k * es < 2048)) return 0;
     if (whole && (dwords || a_ok || b_ok || !wide_enough || g->n % 256 == 0)) return 0;
   }
   if (fp8a && g->k <= kF8ExactMaxK) return 0;  // short K: the exact fp8 product, which the streaming kernel has for whole tiles only
@@ -213,6 +230,8 @@ extern "C" int skl_hip_launch_gemm_mfma(const skl_gemm_canon *g) {
   p.rq = g->rq;
   p.tiles_m = p.tiles_n = 0;
   p.splits = 1, p.slices_per_split = 0, p.partial = nullptr;
+  const size_t es = (g->ta == SKL_DT_BF16 || g->ta == SKL_DT_F16) ? 2 : 1;
+  p.a_loose = !aligned_a(g, es), p.b_loose = !aligned_b(g, es);
   switch (g->ta * 8 + g->tb) {
     case SKL_DT_I8 * 8 + SKL_DT_I8: return skl_mfma_launch_i8(p);
     case SKL_DT_BF16 * 8 + SKL_DT_BF16: return skl_mfma_launch_bf16(p);

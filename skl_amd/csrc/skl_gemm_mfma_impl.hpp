@@ -16,12 +16,9 @@
 // "K-contiguous" (row-major A, column-major B) or "MN-contiguous" (column-major
 // A, row-major B, and both panel formats); blocks of 64 along M / N may sit
 // anywhere (block stride), which is what the panel formats need. A workgroup
-// owns a BM x BN tile of C (256 x 256 on four waves of 128 x 128 each - the
-// largest accumulator block a wave's 512 registers hold, which minimises LDS
-// reads per MFMA - or 128 x 128 on eight waves for small or ragged problems); per 128-byte slice of K it copies the
-// A and B tiles global -> registers -> LDS in their native orientation with
-// 128-bit accesses (double-buffered: the next slice is in flight while the
-// current one is multiplied) and the waves read MFMA operands straight from
+// owns a BM x BN tile of C (128 x 128 on eight waves or 64 x 64 on four; the streaming kernel below has larger ones); per
+// 128-byte slice of K it copies the A and B tiles global -> registers -> LDS in their native orientation with
+// 128-bit accesses (up to four slices under way in registers, two in LDS) and the waves read MFMA operands straight from
 // LDS: ds_read_b128 for a K-contiguous tile (row pitch padded to 144 bytes),
 // ds_read_b64_tr_b8 / _tr_b16 - the LDS transpose loads - for an
 // MN-contiguous one (row pitch padded so the eight/four rows of one transpose
@@ -60,6 +57,7 @@ struct MfmaArgs {
   // sums to partial[split][m][n] (row-major, 4-byte elements) for gemm_split_reduce_kernel.
   unsigned splits, slices_per_split;
   char *partial;
+  bool a_loose = false, b_loose = false;  // bounds-checked kernel: the operand is off the 16-byte rule (Loader)
 };
 
 namespace {
@@ -308,98 +306,106 @@ struct Tile {
   static constexpr int kMnChunks = ROWS * ES / 16;   // chunks along MN of an MN-contiguous row
 };
 
-// 16 bytes from global memory with `valid` (<= CE) leading elements in range.
-template <int ES>
-__device__ __forceinline__ v4i load_chunk(const char *p, long valid) {
-  constexpr int CE = 16 / ES;
-  if (valid >= CE) return *reinterpret_cast<const v4i *>(p);
-  v4i v = {0, 0, 0, 0};
-  if (valid > 0) {
-    unsigned w[4] = {0, 0, 0, 0};
-    for (int e = 0; e < CE; ++e) {
-      if (e < valid) {
-        unsigned x = ES == 1 ? (unsigned)*reinterpret_cast<const uint8_t *>(p + e)
-                             : (unsigned)*reinterpret_cast<const uint16_t *>(p + 2 * e);
-        w[(e * ES) / 4] |= x << (8 * ((e * ES) % 4));
-      }
-    }
-    v = v4i{(int)w[0], (int)w[1], (int)w[2], (int)w[3]};
-  }
-  return v;
+// The low bytes of a 16-byte chunk moved down by `bytes` (0 to 15, its own for every lane), zeros above.
+__device__ __forceinline__ v4i chunk_shift_down(v4i v, unsigned bytes) {
+  const bool two = bytes & 8, one = bytes & 4;
+  int w0 = two ? v.z : v.x, w1 = two ? v.w : v.y, w2 = two ? 0 : v.z, w3 = two ? 0 : v.w;
+  w0 = one ? w1 : w0, w1 = one ? w2 : w1, w2 = one ? w3 : w2, w3 = one ? 0 : w3;
+  return v4i{(int)__builtin_amdgcn_alignbyte((unsigned)w1, (unsigned)w0, bytes), (int)__builtin_amdgcn_alignbyte((unsigned)w2, (unsigned)w1, bytes),
+             (int)__builtin_amdgcn_alignbyte((unsigned)w3, (unsigned)w2, bytes), (int)__builtin_amdgcn_alignbyte(0u, (unsigned)w3, bytes)};
+}
+// A chunk's first `bytes` (0 to 16) bytes, zeros above.
+__device__ __forceinline__ v4i chunk_keep(v4i v, int bytes) {
+  const auto keep = [&](int w, int b) { return b >= 4 ? w : b <= 0 ? 0 : (int)((unsigned)w & ((1u << (8 * b)) - 1u)); };
+  return v4i{keep(v.x, bytes), keep(v.y, bytes - 4), keep(v.z, bytes - 8), keep(v.w, bytes - 12)};
 }
 
-// Per-thread source bookkeeping for one operand. A chunk's address is a
-// workgroup-uniform 64-bit tile base (advanced by one slice per iteration) plus
-// a 32-bit per-thread offset, so the loop carries one scalar pointer instead of
-// a vector pointer per chunk.
+// One thread's share of the global loads of an operand, without a branch: a guard is a branch, and at a branch that is not
+// uniform every load in flight is waited for (guarded chunk by chunk, a slice of the 64 x 64 kernel cost four memory
+// latencies one after another: 2.2 us of it, 128 bytes of K). Chunks go through a buffer descriptor whose base follows K as a
+// scalar; a chunk that does not exist (rows or columns beyond the matrix, k beyond its end) gets an offset beyond the
+// descriptor's range, for which the load returns zeros and touches no memory.
+// `loose`: the operand is off the 16-byte rule, and what is loaded must not reach beyond it. Then a chunk of which only the
+// first elements exist is loaded from further down, so that it ends with the last of them, and its bytes are moved into place
+// on the way to LDS. (An operand on the rule has no such chunk in a 16-byte unit of its own: whatever follows the last element
+// there is cut off along K, and along M / N reaches rows and columns that do not exist.)
 template <int ES, int ROWS, bool KC, int NT>
 struct Loader {
   using T = Tile<ES, ROWS, KC, NT>;
-  const char *tile_base;         // uniform: first byte of the tile's first 64-block at k = 0
+  static constexpr unsigned kRange = 0xC0000000u, kOutside = 0xE0000000u;  // (offsets inside a tile stay below 0xA8000000, see operand_ok)
+  static constexpr unsigned kBias = 16;  // the base lies 16 bytes ahead of the tile, so that no offset is negative
+  static constexpr int kRowsPerPass = KC ? NT / 8 : NT / T::kMnChunks;
+  const char *base;              // uniform
   size_t k_step;                 // bytes between consecutive slices
-  unsigned off[T::kPerThread];   // byte offset of each chunk from tile_base
-  unsigned lds_off[T::kPerThread];
-  long mn_valid[T::kPerThread];  // guarded path - KC: row in range (1/0); MC: elements in range along MN
-  int k_off[T::kPerThread];      // guarded path - KC: k element offset of the chunk; MC: k row
+  unsigned off[T::kPerThread];   // byte offset of each chunk
+  unsigned lds_off;              // of the first chunk; the others follow kRowsPerPass rows apart
+  int k_first;                   // KC: k element of the chunks in the slice; MC: k row of the first chunk
+  unsigned back;                 // MC: bytes by which the chunks are loaded too low
+  bool loose, mn_shift;          // uniform
 
-  __device__ void init(const char *base, size_t mn0, size_t mn_dim, size_t s1, size_t s0, size_t sk) {
+  __device__ __forceinline__ void init(const char *operand, size_t mn0, size_t mn_dim, size_t s1, size_t s0, size_t sk, bool is_loose) {
     const int t = threadIdx.x;
-    tile_base = base + (mn0 >> 6) * s1 * ES;  // mn0 is a multiple of 64
+    loose = is_loose;
+    base = operand + (mn0 >> 6) * s1 * ES - kBias;  // mn0 is a multiple of 64
+    back = 0;
+    mn_shift = false;
+    if constexpr (KC) {
+      const int c = t & 7;
+      k_first = c * T::CE;
+      lds_off = (t >> 3) * kPitchKC + c * 16;
 #pragma unroll
-    for (int i = 0; i < T::kPerThread; ++i) {
-      const int q = t + NT * i;
-      if (KC) {
-        const int row = q >> 3, c = q & 7;
-        off[i] = (unsigned)(((size_t)(row >> 6) * s1 + (size_t)(row & 63) * s0 + (size_t)c * T::CE) * ES);
-        mn_valid[i] = mn0 + row < mn_dim ? 1 : 0;
-        k_off[i] = c * T::CE;
-        lds_off[i] = row * kPitchKC + c * 16;
-      } else {
-        const int mc = q % T::kMnChunks, kr = q / T::kMnChunks;
-        const int r = mc * T::CE;
-        off[i] = (unsigned)(((size_t)(r >> 6) * s1 + (size_t)(r & 63) + (size_t)kr * sk) * ES);
-        mn_valid[i] = (long)mn_dim - (long)(mn0 + r);
-        k_off[i] = kr;
-        lds_off[i] = kr * T::kPitchMC + mc * 16;
+      for (int i = 0; i < T::kPerThread; ++i) {
+        const int row = (t >> 3) + i * kRowsPerPass;
+        off[i] = mn0 + row < mn_dim ? (unsigned)(((size_t)(row >> 6) * s1 + (size_t)(row & 63) * s0) * ES + c * 16) + kBias : kOutside;
       }
+    } else {
+      const int mc = t % T::kMnChunks, r = mc * T::CE;
+      k_first = t / T::kMnChunks;
+      lds_off = k_first * T::kPitchMC + mc * 16;
+      const long there = (long)mn_dim - (long)(mn0 + r);  // elements from the chunk's first on
+      if (loose && there > 0 && there < T::CE) back = (unsigned)((T::CE - there) * ES);
+      mn_shift = loose && mn_dim - mn0 < ROWS && mn_dim % T::CE != 0;
+#pragma unroll
+      for (int i = 0; i < T::kPerThread; ++i)
+        off[i] = there > 0 ? (unsigned)(((size_t)(r >> 6) * s1 + (size_t)(r & 63) + (size_t)(k_first + i * kRowsPerPass) * sk) * ES) + kBias - back : kOutside;
     }
     k_step = KC ? (size_t)kSliceBytes : (size_t)T::KE * sk * ES;
   }
 
-  // Interior tiles of problems whose extents are multiples of the tile: every chunk is whole.
-  __device__ __forceinline__ void fetch_whole(v4i (&regs)[T::kPerThread], size_t slice) const {
-    const char *b = tile_base + slice * k_step;
-#pragma unroll
-    for (int i = 0; i < T::kPerThread; ++i) regs[i] = *reinterpret_cast<const v4i *>(b + off[i]);
-  }
-
-  // Any extents: chunks that stick out of the matrix are zero-filled (zeros along
-  // K add nothing; rows/columns beyond M/N are never stored).
-  __device__ __forceinline__ void fetch_guarded(v4i (&regs)[T::kPerThread], size_t slice, size_t k_dim) const {
-    const long k0 = (long)(slice * T::KE);
-    const char *b = tile_base + slice * k_step;
+  // `left`: elements of K from the slice's first on, none or fewer beyond the last slice.
+  __device__ __forceinline__ void fetch(v4i (&regs)[T::kPerThread], size_t slice, int left) const {
+    const __amdgpu_buffer_rsrc_t rsrc = __builtin_amdgcn_make_buffer_rsrc((void *)(base + slice * k_step), 0, (int)kRange, 0x00027000);
+    unsigned tail = 0;
+    if (KC && loose) {
+      const int over = k_first + T::CE - left;  // elements of the chunk beyond K
+      tail = over > 0 ? (unsigned)(over * ES) : 0u;
+    }
 #pragma unroll
     for (int i = 0; i < T::kPerThread; ++i) {
-      long valid;
-      if (KC)
-        valid = mn_valid[i] ? (long)k_dim - (k0 + k_off[i]) : 0;
-      else
-        valid = (k0 + k_off[i] < (long)k_dim) ? mn_valid[i] : 0;
-      regs[i] = load_chunk<ES>(b + off[i], valid);
+      const bool there = (KC ? k_first : k_first + i * kRowsPerPass) < left;
+      const unsigned o = there ? off[i] - tail : kOutside;
+      regs[i] = __builtin_bit_cast(v4i, __builtin_amdgcn_raw_buffer_load_b128(rsrc, (int)o, 0, 0));
     }
   }
 
-  template <bool GUARDED>
-  __device__ __forceinline__ void fetch(v4i (&regs)[T::kPerThread], size_t slice, size_t k_dim) const {
-    if constexpr (GUARDED)
-      fetch_guarded(regs, slice, k_dim);
-    else
-      fetch_whole(regs, slice);
-  }
-
-  __device__ __forceinline__ void stash(char *tile, const v4i (&regs)[T::kPerThread]) const {
+  // Into LDS, the chunks that end inside 16 bytes put right first (along K: LAST, the share's last slice may be among them).
+  template <bool LAST>
+  __device__ __forceinline__ void stash(char *tile, v4i (&regs)[T::kPerThread], int left) const {
+    if constexpr (KC) {
+      if (LAST && left < T::KE && left % T::CE != 0) {  // uniform: the last slice of a K that ends inside a chunk
+        const int bytes = (left - k_first) * ES;
 #pragma unroll
-    for (int i = 0; i < T::kPerThread; ++i) *reinterpret_cast<v4i *>(tile + lds_off[i]) = regs[i];
+        for (int i = 0; i < T::kPerThread; ++i)
+          regs[i] = loose ? chunk_shift_down(regs[i], bytes > 0 && bytes < 16 ? 16u - (unsigned)bytes : 0u) : chunk_keep(regs[i], bytes);
+      }
+    } else {
+      if (mn_shift) {
+#pragma unroll
+        for (int i = 0; i < T::kPerThread; ++i) regs[i] = chunk_shift_down(regs[i], back);
+      }
+    }
+#pragma unroll
+    for (int i = 0; i < T::kPerThread; ++i) *reinterpret_cast<v4i *>(tile + lds_off + i * kRowsPerPass * (KC ? kPitchKC : T::kPitchMC)) = regs[i];
   }
 };
 
@@ -755,12 +761,16 @@ __device__ __forceinline__ void write_wave_tile_staged(const MfmaArgs &p, const 
 // (eight of them, each with its own L2), so ids are first regrouped per XCD into
 // contiguous ranges, then walked in column-major groups of kGroupM tile rows so
 // that the tiles resident on one XCD at a time share A and B panels.
+// ANY: also when the tiles are not a multiple of eight. The bounds-checked kernels gain by it (bf16 6409 x 14591 x 1344 on
+// 5814 tiles of 128 x 128: 458 -> 398 us); the streaming kernel with its larger tiles does not (int8 5169 x 15488 x 704 on
+// 1281 tiles: 362 -> 389 us): its eight XCDs then read eight tile rows of the same columns.
+template <bool ANY>
 __device__ __forceinline__ void tile_of_block(unsigned bid, unsigned tiles_m, unsigned tiles_n, unsigned &tm,
                                               unsigned &tn) {
   constexpr unsigned kXcd = 8, kGroupM = 8;
-  const unsigned total = tiles_m * tiles_n;
+  const unsigned total = tiles_m * tiles_n, xcd = bid % kXcd, longer = total % kXcd;  // the first `longer` ranges hold one tile more
   unsigned t = bid;
-  if (total % kXcd == 0) t = (bid % kXcd) * (total / kXcd) + bid / kXcd;
+  if (ANY || longer == 0) t = xcd * (total / kXcd) + (xcd < longer ? xcd : longer) + bid / kXcd;
   const unsigned per_group = kGroupM * tiles_n;
   const unsigned group = t / per_group, first_m = group * kGroupM;
   const unsigned rows = tiles_m - first_m < kGroupM ? tiles_m - first_m : kGroupM;
@@ -769,8 +779,13 @@ __device__ __forceinline__ void tile_of_block(unsigned bid, unsigned tiles_m, un
   tn = in_group / rows;
 }
 
-template <int TA, int TB, bool A_KC, bool B_KC, int BM, int BN, int WAVES_M, int WAVES_N, bool GUARDED, bool EXACT = false, bool EXTRA = false>
-__global__ void __launch_bounds__(WAVES_M *WAVES_N * 64, (BM == 128 ? 4 : 6)) gemm_mfma_kernel(MfmaArgs p) {
+// The kernel for ragged and small problems: any M, N and K, operands on any boundary. A problem of few tiles is bound by the
+// time from one slice to the next (requests, their memory latency, LDS, barrier), so several slices of loads are under way, and
+// the loads are never guarded (Loader). Guarded loads, a slice ahead -> this, us: int8 512^3 5.9 -> 5.0, bf16 16 x 11008 x 4096
+// 28.4 -> 23.7 with its second pass, int8 136 x 704 x 2207 51 -> 12.4 (no copy of A in front), f16 427 x 5901 x 1805 93 -> 33;
+// over 120 random problems 0.70.
+template <int TA, int TB, bool A_KC, bool B_KC, int BM, int BN, int WAVES_M, int WAVES_N, bool EXACT = false, bool EXTRA = false>
+__global__ void __launch_bounds__(WAVES_M *WAVES_N * 64, 4) gemm_mfma_kernel(MfmaArgs p) {
   constexpr int NT = WAVES_M * WAVES_N * 64;
   using KA = Kind<TA>;
   using M = typename std::conditional<EXACT, MmaF8Exact<TA, TB>, Mma<TA, TB>>::type;
@@ -784,20 +799,22 @@ __global__ void __launch_bounds__(WAVES_M *WAVES_N * 64, (BM == 128 ? 4 : 6)) ge
   using TileA = Tile<ES, BM, A_KC, NT>;
   using TileB = Tile<ES, BN, B_KC, NT>;
   constexpr int kStage = TileA::kBytes + TileB::kBytes;
+  // Slices under way, 16 registers each, of the 128 a thread has (the 32-byte fragments of the fp8 kinds take twice the room).
+  constexpr int kAhead = BM == 128 ? (FRB == 32 ? 1 : 2) : FRB == 32 || EXACT ? 3 : 4;
 
   extern __shared__ __attribute__((aligned(16))) char smem[];
 
   unsigned tm, tn;
   const unsigned tiles = p.tiles_m * p.tiles_n, split = blockIdx.x / tiles;
-  tile_of_block(blockIdx.x % tiles, p.tiles_m, p.tiles_n, tm, tn);
+  tile_of_block<true>(blockIdx.x % tiles, p.tiles_m, p.tiles_n, tm, tn);
   const size_t m0 = (size_t)tm * BM, n0 = (size_t)tn * BN;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;  // the wave index as a scalar: nothing derived from it occupies a vector register across the main loop
   const int wm = (wave / WAVES_N) * WM, wn = (wave % WAVES_N) * WN;
 
   Loader<ES, BM, A_KC, NT> la;
   Loader<ES, BN, B_KC, NT> lb;
-  la.init(p.a, m0, p.m, p.a_s1, p.a_s0, p.a_sk);
-  lb.init(p.b, n0, p.n, p.b_s1, p.b_s0, p.b_sk);
+  la.init(p.a, m0, p.m, p.a_s1, p.a_s0, p.a_sk, p.a_loose);
+  lb.init(p.b, n0, p.n, p.b_s1, p.b_s0, p.b_sk, p.b_loose);
 
   Acc acc[MI][NI];
 #pragma unroll
@@ -807,36 +824,39 @@ __global__ void __launch_bounds__(WAVES_M *WAVES_N * 64, (BM == 128 ? 4 : 6)) ge
 #pragma unroll
       for (int r = 0; r < 16; ++r) acc[i][j][r] = 0;
 
-  const size_t all_slices = (p.k * ES + kSliceBytes - 1) / kSliceBytes;
+  // This workgroup's share of K: whole slices, and the elements from slice s on that belong to it (as a number of at most 31
+  // bits; negative beyond the end).
+  constexpr int KE = TileA::KE;
+  const size_t all_slices = (p.k + KE - 1) / KE;
   const size_t s_begin = (size_t)split * p.slices_per_split;  // the host makes every split non-empty
-  const size_t slices = all_slices - s_begin < p.slices_per_split ? all_slices : s_begin + p.slices_per_split;
-  v4i ra[TileA::kPerThread], rb[TileB::kPerThread];
-  la.template fetch<GUARDED>(ra, s_begin, p.k);
-  lb.template fetch<GUARDED>(rb, s_begin, p.k);
-  la.stash(smem, ra);
-  lb.stash(smem + TileA::kBytes, rb);
+  const size_t s_end = all_slices - s_begin < p.slices_per_split ? all_slices : s_begin + p.slices_per_split;
+  const unsigned count = (unsigned)(s_end - s_begin);
+  const int last_left = (int)((s_end == all_slices ? p.k : s_end * KE) - (s_end - 1) * KE);  // elements in the last slice
+  const auto left = [&](unsigned s) __attribute__((always_inline)) { return s + 1 < count ? KE : s + 1 == count ? last_left : 0; };
+
+  // Slices s + 1 to s + kAhead are on their way, global -> registers, while slice s is multiplied from LDS.
+  v4i ra[kAhead][TileA::kPerThread], rb[kAhead][TileB::kPerThread];
+#pragma unroll
+  for (int d = 0; d < kAhead; ++d) {
+    la.fetch(ra[d], s_begin + d, left(d));
+    lb.fetch(rb[d], s_begin + d, left(d));
+  }
+  la.template stash<true>(smem, ra[0], left(0));
+  lb.template stash<true>(smem + TileA::kBytes, rb[0], left(0));
+  la.fetch(ra[0], s_begin + kAhead, left(kAhead));
+  lb.fetch(rb[0], s_begin + kAhead, left(kAhead));
+  __builtin_amdgcn_sched_barrier(0);
   __syncthreads();
 
   constexpr int kSteps = kSliceBytes / KB;  // MFMA k-steps per slice
   typename M::Frag fa[2][MI], fb[2][NI];    // operand fragments, double-buffered across k-steps
-#pragma unroll
-  for (int i = 0; i < MI; ++i) fa[0][i] = read_frag<ES, BM, A_KC, FRB>(smem, wm + i * 32, 0);
-#pragma unroll
-  for (int j = 0; j < NI; ++j) fb[0][j] = read_frag<ES, BN, B_KC, FRB>(smem + TileA::kBytes, wn + j * 32, 0);
-
-  for (size_t s = s_begin; s < slices; ++s) {
-    const char *ta = smem + ((s - s_begin) & 1) * kStage;
+  const auto multiply = [&](unsigned s) __attribute__((always_inline)) {
+    const char *ta = smem + (s & 1) * kStage;
     const char *tb = ta + TileA::kBytes;
-    char *na = smem + ((s - s_begin + 1) & 1) * kStage;
-    // Next slice: global -> registers while this one is multiplied. The last
-    // iteration fetches its own slice again (in range, never consumed) so that
-    // the loop body has no branch around the loads.
-    const size_t nxt = s + 1 < slices ? s + 1 : s;
-    la.template fetch<GUARDED>(ra, nxt, p.k);
-    lb.template fetch<GUARDED>(rb, nxt, p.k);
-    // Keep the loads up here: left alone, the scheduler sinks them to just before
-    // the LDS stores below and the whole memory latency lands on every slice.
-    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int i = 0; i < MI; ++i) fa[0][i] = read_frag<ES, BM, A_KC, FRB>(ta, wm + i * 32, 0);
+#pragma unroll
+    for (int j = 0; j < NI; ++j) fb[0][j] = read_frag<ES, BN, B_KC, FRB>(tb, wn + j * 32, 0);
 #pragma unroll
     for (int ks = 0; ks < kSteps; ++ks) {
       const int cur = ks & 1, nx = cur ^ 1;
@@ -865,15 +885,33 @@ __global__ void __launch_bounds__(WAVES_M *WAVES_N * 64, (BM == 128 ? 4 : 6)) ge
       }
       __builtin_amdgcn_sched_barrier(0);
     }
-    la.stash(na, ra);
-    lb.stash(na + TileA::kBytes, rb);
+  };
+  // Slice s, whose loads have been under way for kAhead slices, into LDS; slice s + kAhead requested in its registers (not
+  // by the last slices: LAST).
+  const auto advance = [&](auto last, unsigned s, v4i (&next_a)[TileA::kPerThread], v4i (&next_b)[TileB::kPerThread]) __attribute__((always_inline)) {
+    constexpr bool LAST = decltype(last)::value;
+    char *na = smem + (s & 1) * kStage;
+    la.template stash<LAST>(na, next_a, left(s));
+    lb.template stash<LAST>(na + TileA::kBytes, next_b, left(s));
+    if constexpr (!LAST) {
+      la.fetch(next_a, s_begin + s + kAhead, left(s + kAhead));
+      lb.fetch(next_b, s_begin + s + kAhead, left(s + kAhead));
+      __builtin_amdgcn_sched_barrier(0);  // the loads stay up here, not next to the stores that use them
+    }
     __syncthreads();
-    // First fragments of the next slice (kSteps is even, so they land in buffer 0 again).
-#pragma unroll
-    for (int i = 0; i < MI; ++i) fa[0][i] = read_frag<ES, BM, A_KC, FRB>(na, wm + i * 32, 0);
-#pragma unroll
-    for (int j = 0; j < NI; ++j) fb[0][j] = read_frag<ES, BN, B_KC, FRB>(na + TileA::kBytes, wn + j * 32, 0);
+  };
+  // The compiler counts the loads in flight along every path into a block: a loop with a way out after each slice, or around
+  // one, makes it wait for the youngest of them. So the loop runs whole rounds of kAhead slices, up to the last kAhead + 1.
+  unsigned s = 0;
+  for (; s + kAhead + 1 < count; s += kAhead) {
+    [&]<int... Us>(std::integer_sequence<int, Us...>) __attribute__((always_inline)) {
+      ((multiply(s + Us), advance(std::false_type{}, s + Us + 1, ra[(Us + 1) % kAhead], rb[(Us + 1) % kAhead])), ...);
+    }(std::make_integer_sequence<int, kAhead>{});
   }
+  multiply(s);
+  [&]<int... Us>(std::integer_sequence<int, Us...>) __attribute__((always_inline)) {
+    (void)((++s < count && (advance(std::true_type{}, s, ra[(Us + 1) % kAhead], rb[(Us + 1) % kAhead]), multiply(s), true)) && ...);
+  }(std::make_integer_sequence<int, kAhead>{});
 
   // Lane l of a 32x32 block holds column l%32 and rows 8*(r/4) + 4*(l/32) + r%4.
   if (p.splits > 1) {  // a share of K: the raw sums go to this split's M x N plane
@@ -892,7 +930,7 @@ __global__ void __launch_bounds__(WAVES_M *WAVES_N * 64, (BM == 128 ? 4 : 6)) ge
     }
     return;
   }
-  write_wave_tile<MI, NI, GUARDED, EXTRA ? 1 : 0>(p, acc, m0 + wm, n0 + wn);
+  write_wave_tile<MI, NI, true, EXTRA ? 1 : 0>(p, acc, m0 + wm, n0 + wn);
 }
 
 // ===========================================================================
@@ -1204,7 +1242,7 @@ __global__ void __launch_bounds__(512) gemm_mfma_ring_kernel(MfmaArgs p) {
   // starts s shares into K and leaves its raw sums in plane s of the workspace.
   unsigned tm, tn;
   const unsigned tiles = p.tiles_m * p.tiles_n, split = blockIdx.x / tiles;
-  tile_of_block(blockIdx.x % tiles, p.tiles_m, p.tiles_n, tm, tn);
+  tile_of_block<false>(blockIdx.x % tiles, p.tiles_m, p.tiles_n, tm, tn);
   const size_t m0 = (size_t)tm * BM, n0 = (size_t)tn * BN;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;  // the wave index as a scalar: nothing derived from it occupies a vector register across the main loop
   const int wm = (wave / WAVES_N) * WM, wn = (wave % WAVES_N) * WN;
@@ -1709,15 +1747,15 @@ inline unsigned splits_for(size_t tiles, size_t slices, size_t m, size_t n) {
   return (unsigned)(want < 1 ? 1 : want);
 }
 
-template <int TA, int TB, bool A_KC, bool B_KC, int BM, int BN, int WAVES_M, int WAVES_N, bool GUARDED, bool EXACT = false, bool EXTRA = false>
+template <int TA, int TB, bool A_KC, bool B_KC, int BM, int BN, int WAVES_M, int WAVES_N, bool EXACT = false, bool EXTRA = false>
 int launch_one(const MfmaArgs &args) {
   if constexpr (!EXTRA) {  // calls with an activation or a requantised copy take the kernels that carry those steps
-    if (args.rq.act || args.rq.q) return launch_one<TA, TB, A_KC, B_KC, BM, BN, WAVES_M, WAVES_N, GUARDED, EXACT, true>(args);
+    if (args.rq.act || args.rq.q) return launch_one<TA, TB, A_KC, B_KC, BM, BN, WAVES_M, WAVES_N, EXACT, true>(args);
   }
   constexpr int ES = Kind<TA>::ES;
   constexpr int NT = WAVES_M * WAVES_N * 64;
   constexpr int lds = 2 * (Tile<ES, BM, A_KC, NT>::kBytes + Tile<ES, BN, B_KC, NT>::kBytes);
-  auto kernel = gemm_mfma_kernel<TA, TB, A_KC, B_KC, BM, BN, WAVES_M, WAVES_N, GUARDED, EXACT, EXTRA>;
+  auto kernel = gemm_mfma_kernel<TA, TB, A_KC, B_KC, BM, BN, WAVES_M, WAVES_N, EXACT, EXTRA>;
   static std::atomic<bool> configured{false};  // per instantiation; racing threads set the same value
   if (!configured.load(std::memory_order_acquire)) {
     int rc = skl_check_hip(hipFuncSetAttribute(reinterpret_cast<const void *>(kernel),
@@ -1817,7 +1855,7 @@ int launch_whole_tiles(const MfmaArgs &p) {
   using AccElem = decltype(typename Kind<TA>::Acc{}.x);
   const auto wide = [](const MfmaArgs &q) { return launch_ring<TA, TB, A_KC, B_KC, 256, false, 0, false, false, EXACT>(q); };
   const auto narrow = [](const MfmaArgs &q) { return launch_ring<TA, TB, A_KC, B_KC, 128, false, 0, false, false, EXACT>(q); };
-  if (p.m % 256 != 0 || p.n % 128 != 0 || (p.k * ES) % 128 != 0) return kNotWholeTiles;
+  if (p.m % 256 != 0 || p.n % 128 != 0 || (p.k * ES) % 128 != 0 || p.a_loose || p.b_loose) return kNotWholeTiles;
   const size_t tiles_m = p.m / 256, slices = p.k * ES / kRingSlice;
   const size_t tiles = p.n % 256 == 0 ? tiles_m * (p.n / 256) : 0, tiles128 = tiles_m * (p.n / 128);
   // A last round of 256 x 256 tiles that would fill at most half of the 256 compute units is run as 256 x 128 tiles
@@ -1862,8 +1900,8 @@ int launch_tile(const MfmaArgs &p) {
       const int rc = launch_whole_tiles<TA, TB, A_KC, B_KC, true>(p);
       if (rc != kNotWholeTiles) return rc;
       if (skl_div_up(p.m, 128) * (size_t)skl_div_up(p.n, 128) < 64)
-        return launch_one<TA, TB, A_KC, B_KC, 64, 64, 2, 2, true, true>(p);
-      return launch_one<TA, TB, A_KC, B_KC, 128, 128, 2, 4, true, true>(p);
+        return launch_one<TA, TB, A_KC, B_KC, 64, 64, 2, 2, true>(p);
+      return launch_one<TA, TB, A_KC, B_KC, 128, 128, 2, 4, true>(p);
     }
   }
   const int rc = launch_whole_tiles<TA, TB, A_KC, B_KC, false>(p);
@@ -1872,8 +1910,8 @@ int launch_tile(const MfmaArgs &p) {
   // ... and for the 16-bit kinds up to 64 rows of A: a 128-row tile would fetch and multiply rows that do not exist
   // (bf16 64 x 11008 x 4096: 36 -> 28 us; the 8-bit kinds are faster on the larger tile, 23 against 25 us).
   if ((ES == 2 && p.m <= 64) || skl_div_up(p.m, 128) * (size_t)skl_div_up(p.n, 128) < 64)
-    return launch_one<TA, TB, A_KC, B_KC, 64, 64, 2, 2, true>(p);
-  return launch_one<TA, TB, A_KC, B_KC, 128, 128, 2, 4, true>(p);
+    return launch_one<TA, TB, A_KC, B_KC, 64, 64, 2, 2>(p);
+  return launch_one<TA, TB, A_KC, B_KC, 128, 128, 2, 4>(p);
 }
 
 template <int TA, int TB>
@@ -1900,6 +1938,15 @@ inline bool operand_ok(const void *base, size_t es, size_t s1, size_t s0, size_t
     if (s1 * es * 4 >= limit || sk * es * 128 >= limit) return false;
     return (k <= 1 || mult16(sk * es)) && (mn <= 64 || mult16(s1 * es));
   }
+  return false;
+}
+
+// What the bounds-checked kernels read besides: an operand off the 16-byte rule whose rows (K-contiguous), or whose runs along
+// M / N, hold at least one chunk that can be loaded in a place further down (Loader).
+inline bool operand_loose_ok(size_t es, size_t s1, size_t s0, size_t sk, size_t mn, size_t k) {
+  const size_t limit = size_t(1) << 31, chunk = 16 / es;
+  if (sk == 1) return s1 * es * 4 < limit && s0 * es * 64 < limit && k >= chunk;
+  if (s0 == 1) return s1 * es * 4 < limit && sk * es * 128 < limit && (mn % chunk == 0 || (mn >= chunk && (mn <= 64 || s1 == 64)));
   return false;
 }
 

@@ -73,3 +73,29 @@ def test_every_size_has_an_answer(m, n):
                 if kind or act < 2:
                     assert plan(kind, m, n, k, act=act) in (0, 128, 256)
                     assert plan(kind, m, n, k, lda=k + 1, ldb=k + 3, act=act, b_rows=False) in (0, 128, 256)
+
+
+def in_place(kind, m, n, k, a=1 << 20, a_s0=None, a_sk=1, b_s0=1, b_sk=None, b_s1=None):
+    g = Canon(ta=kind, tb=kind, m=m, n=n, k=k, a=a, b=1 << 20, c=1 << 20, c_row_shift=6, c_col_shift=6)
+    g.a_s0, g.a_sk = a_s0 or k, a_sk
+    g.b_s0, g.b_sk = b_s0, b_sk or n
+    g.a_s1, g.b_s1 = 64 * g.a_s0, b_s1 or 64 * g.b_s0
+    g.rsc0, g.csc0, g.rsc1, g.csc1 = n, 1, 64 * n, 64
+    fn = ct.CDLL(skl_amd.library_path()).skl_hip_gemm_mfma_supported
+    fn.argtypes = [ct.POINTER(Canon)]
+    return fn(ct.byref(g))
+
+
+@pytest.mark.parametrize("kind", range(5))
+def test_operands_off_the_16_byte_rule_the_kernels_read_in_place(kind):
+    """Any base and leading dimension, as long as a row along K, or a run along M / N, holds 16 bytes; strided along both
+    dimensions, or whole tiles that a copy of the operand sends to the streaming kernel: not in place."""
+    chunk = 8 if kind in (BF16, F16) else 16
+    assert in_place(kind, 100, 100, chunk + 1) and in_place(kind, 100, 100, 999, a=(1 << 20) + 2)
+    assert not in_place(kind, 100, 100, chunk - 1)
+    assert in_place(kind, 100, chunk + 1, 100) and not in_place(kind, 100, chunk - 1, 100)
+    assert not in_place(kind, 100, 100, 100, b_s0=2, b_sk=301)
+    assert in_place(kind, 100, 2 * chunk + 1, 100, b_sk=64, b_s1=6400)  # one panel: its rows are on the rule
+    assert not in_place(kind, 100, 64 + chunk + 1, 100, b_sk=65, b_s1=6501)  # blocks apart: a run's start has no bytes in front
+    assert in_place(kind, 100, 64 + chunk, 100, b_sk=65, b_s1=6501)
+    assert not in_place(kind, 4096, 4096, 4096, a_s0=4097) and in_place(kind, 4095, 4096, 4096, a_s0=4097)

@@ -1,0 +1,73 @@
+"""The matrix-core kernels that check bounds, on operands read where they lie: sizes at the edges of their tiles and of the
+slices of K they keep under way, leading dimensions and bases off the 16-byte rule. What surrounds an operand - ahead of it,
+behind it and in the gaps between its rows - is filled with the kind's largest or non-finite codes, so that an element taken
+from there shows."""
+import numpy as np
+import pytest
+
+import skl_amd
+import support
+from skl_amd import DeviceBuffer
+from support import GemmCase, run_oracle_gemm
+
+pytestmark = pytest.mark.gpu
+
+POISON = {"i8": 127, "bf16": 0x7FC0, "f16": 0x7E00, "f8e4m3": 0x7F, "f8e5m2": 0x7E}
+GUARD = 64
+
+
+def in_place(gpu, ta, m, n, k, a_rows, b_rows, a_pad, b_pad, a_off, b_off, beta):
+    """A row-major or by columns, B row-major or by columns, `pad` elements between rows, the base `off` elements off."""
+    lda, ldb = (k if a_rows else m) + a_pad, (n if b_rows else k) + b_pad
+    case = GemmCase(ta, None, 2 if ta == "i8" else 1.5, beta, m0=1, n0=1, k0=1, m1=m, n1=n, k1=k, rsa0=0, csa0=0,
+                    rsa1=lda if a_rows else 1, csa1=1 if a_rows else lda, rsb0=0, csb0=0, rsb1=ldb if b_rows else 1,
+                    csb1=1 if b_rows else ldb, rsc0=0, csc0=0, rsc1=n + 3, csc1=1)
+    a, b, c = case.make_inputs(m + 31 * n + 977 * k + 7 * a_pad + 3 * b_pad + a_off)
+
+    def poisoned(x, rows, run, ld):
+        keep = np.zeros(x.size, bool)
+        for r in range(rows):
+            keep[r * ld:r * ld + run] = True
+        x = x.copy()
+        x[~keep] = POISON[ta]
+        return x
+
+    a, b = poisoned(a, m if a_rows else k, k if a_rows else m, lda), poisoned(b, k if b_rows else n, n if b_rows else k, ldb)
+    guard = np.full(2 * GUARD, POISON[ta], a.dtype)
+    es = a.itemsize
+    da = DeviceBuffer.from_array(np.concatenate([guard[:GUARD // es + a_off], a, guard]))
+    db = DeviceBuffer.from_array(np.concatenate([guard[:GUARD // es + b_off], b, guard]))
+    dc = DeviceBuffer.from_array(c)
+    getattr(gpu, f"skl_gemm_{ta}rc_{ta}rc_{case.ctag}rc_gfx950")(
+        m, n, k, case.alpha, da.offset((GUARD // es + a_off) * es), case.rsa1, case.csa1, db.offset((GUARD // es + b_off) * es), case.rsb1, case.csb1,
+        case.beta, dc, case.rsc1, 1)
+    gpu.skl_hip_synchronize()
+    skl_amd.check_error()
+    got = dc.download(c.dtype, c.size)
+    for d in (da, db, dc):
+        d.free()
+    if case.is_int:
+        assert np.array_equal(got, run_oracle_gemm(case, a, b, c)), vars(case)
+    else:
+        support.assert_fp_gemm_close(case, a, b, c, got, extra_rel=support.FP8_MFMA_REL if ta.startswith("f8") else 0.0)
+
+
+# one chunk, one tile less, exactly and more; K of a chunk, of one to eight slices of 128 bytes and what sticks out of them
+SIZES = ((65, 63, 16), (64, 64, 127), (17, 130, 128), (129, 64, 257), (63, 129, 385), (128, 127, 520), (66, 200, 641), (300, 65, 1031))
+
+
+@pytest.mark.parametrize("ta", ("i8", "bf16", "f8e4m3"))
+@pytest.mark.parametrize("m,n,k", SIZES)
+def test_operands_off_the_16_byte_rule_in_place(gpu, ta, m, n, k):
+    for a_rows in (True, False):
+        for b_rows in (True, False):
+            for a_pad, b_pad, a_off, b_off in ((1, 0, 0, 0), (0, 3, 1, 5), (16, 16, 0, 0)):
+                in_place(gpu, ta, m, n, k, a_rows, b_rows, a_pad, b_pad, a_off, b_off, (a_pad + b_rows) % 2)
+
+
+@pytest.mark.parametrize("ta,k", (("f8e5m2", 2500), ("f8e4m3", 4097), ("f16", 1283), ("i8", 8191)))
+def test_large_tiles_and_shared_k_off_the_16_byte_rule(gpu, ta, k):
+    """Tiles of 128 x 128, the fp8 instructions' fragments of 32 bytes, and K shared between workgroups."""
+    for a_rows, b_rows in ((True, False), (False, False), (True, True)):
+        in_place(gpu, ta, 1025, 1031, k, a_rows, b_rows, 1, 2, 3, 0, 1)
+        in_place(gpu, ta, 40, 333, k, a_rows, b_rows, 5, 0, 0, 1, 0)
