@@ -375,7 +375,7 @@ static int gemm_with_realigned_operands(const skl_gemm_canon *g, int fused) {
   return DECLINED;
 }
 
-/* Ragged or misaligned problems large enough for the streaming kernel: A and B copied into scratch memory padded
+/* Misaligned problems large enough for the streaming kernel: A and B copied into scratch memory padded
  * to whole tiles (the rows beyond M and N are never written and what they hold only reaches elements of C that do
  * not exist; K is zero-filled), C updated in place. */
 static int gemm_padded_to_tiles(const skl_gemm_canon *g) {
@@ -543,7 +543,7 @@ static int gemm_on_device(const skl_gemm_desc *d) {
         if (fused && r == DECLINED && skl_hip_gemv_kc_rows_supported(&g)) r = outcome(skl_hip_launch_gemv_kc_rows(&g));
         if (fused && r == DECLINED && g.m == 1 && skl_hip_gemv_supported(&g, 0)) r = outcome(skl_hip_launch_gemv(&g, 0));
         if (fused && r == DECLINED) r = gemv_then_epilogue(&g); /* uses the operand scratch itself: only here, on the caller's own operands */
-        if (r == DECLINED) r = gemm_padded_to_tiles(&g);
+        if (r == DECLINED && !skl_hip_gemm_mfma_in_place_pays(&g)) r = gemm_padded_to_tiles(&g);
         if (r == DECLINED) r = gemm_fast_path(&g, fused, 1);
         if (r == DECLINED) r = gemm_with_realigned_operands(&g, fused);
       } else {

@@ -53,6 +53,18 @@ bool streams_in_place(const skl_gemm_canon *g, size_t es) {
 
 }  // namespace
 
+// Whether a ragged problem, or one off the 16-byte rule, is best run where its operands lie. Copies padded to whole tiles pay
+// only when neither operand is on the rule, both have K contiguous, and K is long on rounds of tiles that are more than half
+// full: 0.81 to 1.03 of the time in place there (28 of 260 random problems), 1 to 3 times it elsewhere (us, padded copies / in
+// place: f16 4179 x 1024 x 10624 with A by columns 290 / 189, E4M3 5184 x 3310 x 6434 273 / 194, bf16 1600 x 4731 x 896 81 / 33).
+extern "C" int skl_hip_gemm_mfma_in_place_pays(const skl_gemm_canon *g) {
+  if (!skl_hip_gemm_mfma_supported(g)) return 0;
+  const size_t es = (g->ta == SKL_DT_BF16 || g->ta == SKL_DT_F16) ? 2 : 1;
+  if (aligned_a(g, es) || aligned_b(g, es) || g->a_sk != 1 || g->b_sk != 1 || g->k * es < 4096) return 1;
+  const size_t tiles_m = (g->m + 255) / 256, wide = tiles_m * ((g->n + 255) / 256);
+  return rounds_filled(wide >= 200 ? wide : tiles_m * ((g->n + 127) / 128)) < 60;
+}
+
 // Would the streaming kernel take this int8 problem as it lies and write its C 16 bytes per lane (C in blocks of 4
 // to 16 columns with contiguous rows)? Then a blocked C costs no more than a row-major one.
 extern "C" int skl_hip_gemm_mfma_streams_c_quads(const skl_gemm_canon *g) {

@@ -984,9 +984,14 @@ struct STile {
 
 // Global -> LDS loads of one operand, this wave's share. `unit` below is a slice
 // for an MN-contiguous operand and a pair of slices for a K-contiguous one.
-template <int ES, bool KC, int WAVES, int ROWS, int NS>
+// EDGE: the operand ends inside the tile, along M / N or along K. Its loads go through a buffer descriptor whose base follows K
+// as a scalar; a lane whose 16 bytes do not exist holds an offset beyond the descriptor's range, for which the load writes zeros
+// to LDS and touches no memory. The offsets of rows beyond M / N are so from the start; those of k beyond the end become so
+// with the first unit that holds any (mask()).
+template <int ES, bool KC, int WAVES, int ROWS, int NS, bool EDGE>
 struct SLoader {
   using T = STile<ES, KC, ROWS, NS>;
+  static constexpr unsigned kRange = 0xC0000000u, kOutside = 0xE0000000u;  // (the host checks that offsets stay below kRange)
   static constexpr int kUnitBytes = KC ? 2 * T::kBytes : T::kBytes;
   static constexpr int kBlocks = kUnitBytes / 1024 / WAVES;  // KiB blocks per wave and unit
   static_assert(kBlocks >= 1, "every wave loads at least one block per unit");
@@ -994,12 +999,18 @@ struct SLoader {
   size_t k_step;           // bytes from one unit to the next
   unsigned off[kBlocks];   // global byte offsets of this lane
   unsigned lds[kBlocks];   // LDS byte offsets (inside the operand's region, stage 0) of the blocks
+  unsigned k_lane;         // EDGE: where along K the lane's 16 bytes of block 0 lie in a unit - KC: bytes, MC: k rows
+  unsigned k_total;        // EDGE: bytes / k rows of K
 
-  __device__ void init(const char *base, size_t mn0, size_t s1, size_t s0, size_t sk) {
+  __device__ __forceinline__ void init(const char *base, size_t mn0, size_t mn_dim, size_t k, size_t s1, size_t s0, size_t sk) {
     // The wave index as a scalar: the LDS address of a block (which goes into M0) is then scalar arithmetic, not a
     // vector add and a v_readfirstlane per load, and lds[] lives in scalar registers.
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
     tile_base = base + (mn0 >> 6) * s1 * ES;
+    if constexpr (EDGE) {  // spelled out as scalars, like the step below: a descriptor in vector registers costs a loop over the lanes per load
+      const uintptr_t at = (uintptr_t)tile_base;
+      tile_base = (const char *)(((uintptr_t)(unsigned)__builtin_amdgcn_readfirstlane((int)(at >> 32)) << 32) | (unsigned)__builtin_amdgcn_readfirstlane((int)at));
+    }
 #pragma unroll
     for (int i = 0; i < kBlocks; ++i) {
       const int b = wave * kBlocks + i;
@@ -1008,18 +1019,39 @@ struct SLoader {
         const int c = pos ^ ((row >> 2) & 3);
         off[i] = (unsigned)(((size_t)(row >> 6) * s1 + (size_t)(row & 63) * s0) * ES + half * 64 + c * 16);
         lds[i] = b * T::kGroup;
+        if constexpr (EDGE) {
+          static_assert(kBlocks % 2 == 0, "c of block i is that of block 0 with its second bit turned for odd i");
+          if (i == 0) k_lane = half * 64 + c * 16;
+          if (mn0 + row >= mn_dim) off[i] = kOutside;
+        }
       } else {
         constexpr int kLanesPerRow = T::kRowBytes / 16, kRowsPerBlock = 1024 / T::kRowBytes;
         const int kr = kRowsPerBlock * b + lane / kLanesPerRow, pos = lane % kLanesPerRow;
         const int mn = ((T::chunk(kr, pos) - kr * T::kRowBytes) >> 4) * (16 / ES);  // the chunk stored at position `pos`
         off[i] = (unsigned)(((size_t)(mn >> 6) * s1 + (size_t)(mn & 63) + (size_t)kr * sk) * ES);
         lds[i] = b * 1024;
+        if constexpr (EDGE) {
+          if (i == 0) k_lane = kr;
+          if (mn0 + mn >= mn_dim) off[i] = kOutside;
+        }
       }
     }
+    if constexpr (EDGE) k_total = (unsigned)(KC ? k * ES : k);
     // (spelled out as a scalar: as a member next to per-lane offsets it otherwise ends up in a vector register, and
     // every load of an MN-contiguous operand pays a 64-bit vector multiply-add for its address)
     const size_t step = KC ? (size_t)(2 * kRingSlice) : (size_t)(kRingSlice / ES) * sk * ES;
     k_step = ((size_t)(unsigned)__builtin_amdgcn_readfirstlane((int)(step >> 32)) << 32) | (unsigned)__builtin_amdgcn_readfirstlane((int)step);
+  }
+
+  // EDGE: the first unit that K ends in (or ends before), and the offsets from `unit` on, one after another from that one.
+  static constexpr unsigned kUnitK = KC ? 2 * kRingSlice : kRingSlice / ES;
+  __device__ __forceinline__ unsigned first_masked() const { return k_total / kUnitK; }
+  __device__ __forceinline__ void mask(unsigned unit) {
+#pragma unroll
+    for (int i = 0; i < kBlocks; ++i) {
+      const unsigned at = unit * kUnitK + (KC ? k_lane ^ (unsigned)(i & 1) * 32u : k_lane + (unsigned)i * (1024 / T::kRowBytes));
+      off[i] = at < k_total ? off[i] : kOutside;
+    }
   }
 
   // Requests block `i` of `unit`; it lands in stage `stage` (the even one of the pair for KC) of `region`.
@@ -1030,9 +1062,13 @@ struct SLoader {
     // takes the scalar base and the 32-bit offset as they are.
     unsigned o = off[i];
     asm volatile("" : "+v"(o));
-    __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void *)(g + o),
-                                     (__attribute__((address_space(3))) void *)(region + stage * T::kStageStep + lds[i]),
-                                     16, 0, 0);
+    if constexpr (EDGE)
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(__builtin_amdgcn_make_buffer_rsrc((void *)g, 0, (int)kRange, 0x00027000),
+                                               (__attribute__((address_space(3))) void *)(region + stage * T::kStageStep + lds[i]), 16, (int)o, 0, 0, 0);
+    else
+      __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void *)(g + o),
+                                       (__attribute__((address_space(3))) void *)(region + stage * T::kStageStep + lds[i]),
+                                       16, 0, 0);
   }
   __device__ __forceinline__ void issue(char *region, int stage, size_t unit) const {
 #pragma unroll
@@ -1141,8 +1177,8 @@ __device__ __forceinline__ Frag join_pieces(const Piece (&pc)[N]) {
 
 constexpr int ceil_div(int a, int b) { return (a + b - 1) / b; }
 
-// EDGE: the operands are copies padded to whole tiles, C is not - its last tile rows / columns end at p.m / p.n and
-// the epilogue touches nothing beyond them.
+// EDGE: problems that are not whole tiles, or whole pairs of slices along K: the loads take nothing from beyond the operands
+// (SLoader), and the epilogue touches no row or column beyond p.m / p.n.
 // CQUADS: an int32 C in small blocks with contiguous rows (the 4 x 4 blocks of src/gemm/packed-gemm.md:270-298, up to
 // 16 columns), no fused steps - see the epilogue.
 // SCAN (floating-point row-major C, beta == 0 evaluated like the reference's loops, whole tiles, K of at least 64
@@ -1194,8 +1230,8 @@ __global__ void __launch_bounds__(512) gemm_mfma_ring_kernel(MfmaArgs p) {
   constexpr int kEachAhead = STAGES - 1 + kExtra, kPairAhead = STAGES - 2 + kExtra;
   constexpr int kPairU = kPairAhead & 1;             // parity of the slices that issue pair loads
   constexpr int kPairsPrologue = (kPairU + kPairAhead) / 2;
-  using LA = SLoader<ES, A_KC, WAVES, BM, NSA>;
-  using LB = SLoader<ES, B_KC, WAVES, BN, NSB>;
+  using LA = SLoader<ES, A_KC, WAVES, BM, NSA, EDGE>;
+  using LB = SLoader<ES, B_KC, WAVES, BN, NSB, EDGE>;
   using TileA = STile<ES, A_KC, BM, NSA>;
   using TileB = STile<ES, B_KC, BN, NSB>;
   // Load `it` of a slice's kLoads goes out behind MFMA slot it * kSlots / kLoads, pair loads first.
@@ -1249,8 +1285,8 @@ __global__ void __launch_bounds__(512) gemm_mfma_ring_kernel(MfmaArgs p) {
 
   LA la;
   LB lb;
-  la.init(p.a + (size_t)split * p.k * p.a_sk * ES, m0, p.a_s1, p.a_s0, p.a_sk);
-  lb.init(p.b + (size_t)split * p.k * p.b_sk * ES, n0, p.b_s1, p.b_s0, p.b_sk);
+  la.init(p.a + (size_t)split * p.k * p.a_sk * ES, m0, p.m, p.k, p.a_s1, p.a_s0, p.a_sk);
+  lb.init(p.b + (size_t)split * p.k * p.b_sk * ES, n0, p.n, p.k, p.b_s1, p.b_s0, p.b_sk);
   RA ra;
   RB rb;
   ra.init(wm);
@@ -1264,11 +1300,12 @@ __global__ void __launch_bounds__(512) gemm_mfma_ring_kernel(MfmaArgs p) {
 #pragma unroll
       for (int r = 0; r < 16; ++r) acc[i][j][r] = 0;
 
-  // K is a whole number of slice pairs. Units beyond the end are requested as the last unit
+  // K is a whole number of slice pairs (EDGE: what is missing is zeros). Units beyond the end are requested as the last unit
   // again: in range, and the stage they land in is never read, which keeps the load counts static.
   // (32-bit counters - the host refuses a K of 2^31 slices or more: a 64-bit "less than" of two scalars is a vector
   // compare and two vector registers)
-  const unsigned slices = (unsigned)(p.k * ES / SB), pairs = slices / 2;
+  const unsigned slices = EDGE ? (unsigned)((p.k * ES + 2 * SB - 1) / (2 * SB)) * 2 : (unsigned)(p.k * ES / SB), pairs = slices / 2;
+  [[maybe_unused]] const unsigned mask_a = EDGE ? la.first_masked() : 0, mask_b = EDGE ? lb.first_masked() : 0;
 
   // SCAN: the tile's old C, 1 KiB per wave and two slices (the host has checked that K has the slices for it and
   // that C is row-major with 16-byte aligned rows).
@@ -1319,17 +1356,41 @@ __global__ void __launch_bounds__(512) gemm_mfma_ring_kernel(MfmaArgs p) {
 
   if constexpr (A_KC) {
 #pragma unroll
-    for (int i = 0; i < kPairsPrologue; ++i) la.issue(region_a, 2 * i, (unsigned)i < pairs ? (unsigned)i : pairs - 1);
+    for (int i = 0; i < kPairsPrologue; ++i) {
+      const unsigned unit = (unsigned)i < pairs ? (unsigned)i : pairs - 1;
+      if constexpr (EDGE) {
+        if (unit >= mask_a) la.mask(unit);
+      }
+      la.issue(region_a, 2 * i, unit);
+    }
   } else {
 #pragma unroll
-    for (int i = 0; i < kEachAhead; ++i) la.issue(region_a, i, (unsigned)i < slices ? (unsigned)i : slices - 1);
+    for (int i = 0; i < kEachAhead; ++i) {
+      const unsigned unit = (unsigned)i < slices ? (unsigned)i : slices - 1;
+      if constexpr (EDGE) {
+        if (unit >= mask_a) la.mask(unit);
+      }
+      la.issue(region_a, i, unit);
+    }
   }
   if constexpr (B_KC) {
 #pragma unroll
-    for (int i = 0; i < kPairsPrologue; ++i) lb.issue(region_b, 2 * i, (unsigned)i < pairs ? (unsigned)i : pairs - 1);
+    for (int i = 0; i < kPairsPrologue; ++i) {
+      const unsigned unit = (unsigned)i < pairs ? (unsigned)i : pairs - 1;
+      if constexpr (EDGE) {
+        if (unit >= mask_b) lb.mask(unit);
+      }
+      lb.issue(region_b, 2 * i, unit);
+    }
   } else {
 #pragma unroll
-    for (int i = 0; i < kEachAhead; ++i) lb.issue(region_b, i, (unsigned)i < slices ? (unsigned)i : slices - 1);
+    for (int i = 0; i < kEachAhead; ++i) {
+      const unsigned unit = (unsigned)i < slices ? (unsigned)i : slices - 1;
+      if constexpr (EDGE) {
+        if (unit >= mask_b) lb.mask(unit);
+      }
+      lb.issue(region_b, i, unit);
+    }
   }
   if constexpr (SCAN) {  // the slots start as zeros: the first slices read slots that no load has filled yet
 #pragma unroll
@@ -1376,16 +1437,16 @@ __global__ void __launch_bounds__(512) gemm_mfma_ring_kernel(MfmaArgs p) {
       for (int w = 0; w < PB; ++w) asm volatile("" : "+v"(pb[buf][j][w]));
   };
 
-  [&]<int... Rs>(std::integer_sequence<int, Rs...>) {
+  [&]<int... Rs>(std::integer_sequence<int, Rs...>) __attribute__((always_inline)) {
     (read_item(std::integral_constant<int, Rs>{}, std::integral_constant<int, 0>{}, 0, addr_a, addr_b), ...);
   }(std::make_integer_sequence<int, kReads>{});
 
   // Two slices per trip: the parity of the slice decides which loads it issues, and (for the
   // operand kinds with one k-step per slice) which fragment buffer a k-step uses.
   for (unsigned s0 = 0; s0 < slices; s0 += 2) {
-    [&]<int... Us>(std::integer_sequence<int, Us...>) {
+    [&]<int... Us>(std::integer_sequence<int, Us...>) __attribute__((always_inline)) {
       (
-          [&](auto uc) {
+          [&](auto uc) __attribute__((always_inline)) {
             constexpr int U = decltype(uc)::value;
             constexpr int kLoads = kLoadsOfU[U];
             const unsigned s = s0 + U;
@@ -1394,9 +1455,9 @@ __global__ void __launch_bounds__(512) gemm_mfma_ring_kernel(MfmaArgs p) {
             const unsigned s32 = s;
             const int cur_a = (int)(s32 % NSA), nxt_a = (int)((s32 + 1) % NSA), cur_b = (int)(s32 % NSB), nxt_b = (int)((s32 + 1) % NSB);
             const int fill_a = (int)((s32 + (A_KC ? kPairAhead : kEachAhead)) % NSA), fill_b = (int)((s32 + (B_KC ? kPairAhead : kEachAhead)) % NSB);
-            [&]<int... KSs>(std::integer_sequence<int, KSs...>) {
+            [&]<int... KSs>(std::integer_sequence<int, KSs...>) __attribute__((always_inline)) {
               (
-                  [&](auto ksc) {
+                  [&](auto ksc) __attribute__((always_inline)) {
                     constexpr int KS = decltype(ksc)::value;
                     constexpr bool kLast = KS == kSteps - 1;
                     constexpr int KSN = kLast ? 0 : KS + 1;  // k-step whose fragments are read during this one
@@ -1430,9 +1491,9 @@ __global__ void __launch_bounds__(512) gemm_mfma_ring_kernel(MfmaArgs p) {
                     const unsigned sa = addr_a + (kLast ? nxt_a : cur_a) * TileA::kStageStep;
                     const unsigned sb = addr_b + (kLast ? nxt_b : cur_b) * TileB::kStageStep;
                     __builtin_amdgcn_sched_barrier(0);
-                    [&]<int... Qs>(std::integer_sequence<int, Qs...>) {
+                    [&]<int... Qs>(std::integer_sequence<int, Qs...>) __attribute__((always_inline)) {
                       (
-                          [&](auto qc) {
+                          [&](auto qc) __attribute__((always_inline)) {
                             constexpr int Q = decltype(qc)::value, kSlot = KS * kMfmas + Q;
                             constexpr int i = Q / NI, j = Q % NI;
                             acc[i][j] = M::run(wa[i], wb[j], acc[i][j]);
@@ -1443,15 +1504,23 @@ __global__ void __launch_bounds__(512) gemm_mfma_ring_kernel(MfmaArgs p) {
                             // extra instructions of SCAN the difference between +43 and +14 us).
                             __builtin_amdgcn_sched_barrier(0);
                             if constexpr (EXACT && j == 0 && i + 1 < MI) wa[i + 1] = prep_a<M>(fa[i + 1]);
+                            if constexpr (EDGE && kSlot == 0) {  // what this slice requests may reach the end of K
+                              if constexpr (!A_KC || U == kPairU) {
+                                if ((A_KC ? fill_pair : fill_slice) >= mask_a) la.mask(A_KC ? fill_pair : fill_slice);
+                              }
+                              if constexpr (!B_KC || U == kPairU) {
+                                if ((B_KC ? fill_pair : fill_slice) >= mask_b) lb.mask(B_KC ? fill_pair : fill_slice);
+                              }
+                            }
                             if constexpr (SCAN && U == 0 && kSlot == 0) scan_issue(s);
                             if constexpr (SCAN && kSlot == 1) scan_check();  // what the last slot of the k-step before has read, behind this k-step's lgkmcnt(0)
                             // Behind the barrier of slice 2q + 3 the rows requested in slice 2q have landed: half of them is
                             // read back in that slice, half in the next (the first slices find zeros).
                             if constexpr (SCAN && kSlot == kSlots - 1) scan_read(((s32 >> 1) + kScanSlots - (U == 1 ? 1 : 2)) % kScanSlots, U == 1 ? 0 : 1);
                             // this slot's share of the next k-step's reads
-                            [&]<int... Rs>(std::integer_sequence<int, Rs...>) {
+                            [&]<int... Rs>(std::integer_sequence<int, Rs...>) __attribute__((always_inline)) {
                               (
-                                  [&](auto rc) {
+                                  [&](auto rc) __attribute__((always_inline)) {
                                     constexpr int R = decltype(rc)::value;
                                     if constexpr (R * kReadSlots / kReads == Q)
                                       read_item(rc, std::integral_constant<int, KSN>{}, nx, sa, sb);
@@ -1459,9 +1528,9 @@ __global__ void __launch_bounds__(512) gemm_mfma_ring_kernel(MfmaArgs p) {
                                   ...);
                             }(std::make_integer_sequence<int, kReads>{});
                             // and this slot's share of the slice's loads
-                            [&]<int... Ls>(std::integer_sequence<int, Ls...>) {
+                            [&]<int... Ls>(std::integer_sequence<int, Ls...>) __attribute__((always_inline)) {
                               (
-                                  [&](auto lc) {
+                                  [&](auto lc) __attribute__((always_inline)) {
                                     constexpr int L = decltype(lc)::value;
                                     if constexpr (L * kSlots / kLoads == kSlot) {
                                       constexpr int kPairsNow = U == kPairU ? kPairs : 0;
@@ -1710,7 +1779,7 @@ int launch_ring(const MfmaArgs &args) {
     skl_hip_record_error(-2, "gemm_mfma: K too long");
     return -2;
   }
-  p.splits = (tiles <= 128 && slices % 4 == 0 && slices / 2 >= kRingMinSlicesPerSplit) ? 2 : 1;
+  p.splits = (tiles <= 128 && p.k * ES % (4 * kRingSlice) == 0 && slices / 2 >= kRingMinSlicesPerSplit) ? 2 : 1;
   SequenceGuard sequence(p.splits > 1);
   if (p.splits > 1) {
     p.partial = (char *)skl_workspace((size_t)p.splits * p.m * p.n * 4);
@@ -1888,6 +1957,34 @@ int launch_whole_tiles(const MfmaArgs &p) {
   return kNotWholeTiles;
 }
 
+// The streaming kernel on problems that are not whole tiles (EDGE): the tile's columns, or 0 where the bounds-checked kernels
+// are as good. Those have 512 tiles of 128 x 128 on the chip at a time and waste little of a last round; a round of 256 x 256
+// tiles takes as long as about 745 of theirs, from 4 KiB of K on (below, starts and ends of the larger tiles show: bf16
+// 6016 x 6848 x 896 with SiLU 176 against 153 us). The 256 x 128 tiles gain nothing on full rounds; a single round of them
+// does, over 353 tiles and more that are one long round there too, where C is read, which they request earlier, or where
+// operands read across K are long. Bounds-checked / streaming, us: bf16 3000 x 5000 x 7000 267 / 207, int8 2176 x 2816 x 512
+// reading C 33.8 / 19.9, bf16 2880 x 2176 x 5425 with A by columns 98 / 71; over 367 random problems the rule takes 22, at
+// 0.82 of the bounds-checked kernels' time, the worst 1.10.
+template <int TA, int TB, bool A_KC, bool B_KC>
+int ragged_tile_cols(const MfmaArgs &p) {
+  constexpr size_t ES = Kind<TA>::ES, limit = 0xB0000000u;
+  if (p.a_loose || p.b_loose) return 0;
+  // 16 bytes along K that K ends in would need zeros behind it; the offsets inside a tile stay in the descriptor's range
+  if (p.k * ES % 16 != 0 && (A_KC || B_KC)) return 0;
+  if ((3 * p.a_s1 + (A_KC ? 63 * p.a_s0 : 64 * p.a_sk)) * ES >= limit || (3 * p.b_s1 + (B_KC ? 63 * p.b_s0 : 64 * p.b_sk)) * ES >= limit) return 0;
+  const size_t tiles_m = (p.m + 255) / 256, wide = tiles_m * ((p.n + 255) / 256), narrow = tiles_m * ((p.n + 127) / 128);
+  const size_t small = (size_t)skl_div_up(p.m, 128) * skl_div_up(p.n, 128), k_bytes = p.k * ES;
+  if (k_bytes >= 4096 && small >= (wide + 255) / 256 * 745) return 256;
+  const bool reads_c = std::is_same<decltype(typename Kind<TA>::Acc{}.x), int>::value ? p.beta.i != 0 : !(p.beta.fz.skip_c_read && p.beta.f == 0.0f);
+  const bool plain = !p.rq.act && !p.rq.q;
+  if (plain && narrow <= 256 && small >= 353 && (reads_c || (k_bytes >= 8192 && !(A_KC && B_KC)))) return 128;
+  return 0;
+}
+template <int TA, int TB, bool A_KC, bool B_KC>
+int launch_ragged(const MfmaArgs &p, int tile_cols) {
+  return tile_cols == 256 ? launch_ring<TA, TB, A_KC, B_KC, 256, true>(p) : launch_ring<TA, TB, A_KC, B_KC, 128, true>(p);
+}
+
 template <int TA, int TB, bool A_KC, bool B_KC>
 int launch_tile(const MfmaArgs &p) {
   constexpr int ES = Kind<TA>::ES;
@@ -1906,6 +2003,7 @@ int launch_tile(const MfmaArgs &p) {
   }
   const int rc = launch_whole_tiles<TA, TB, A_KC, B_KC, false>(p);
   if (rc != kNotWholeTiles) return rc;
+  if (const int cols = ragged_tile_cols<TA, TB, A_KC, B_KC>(p)) return launch_ragged<TA, TB, A_KC, B_KC>(p, cols);
   // Small problems: 64 x 64 tiles put four times as many workgroups on the chip.
   // ... and for the 16-bit kinds up to 64 rows of A: a 128-row tile would fetch and multiply rows that do not exist
   // (bf16 64 x 11008 x 4096: 36 -> 28 us; the 8-bit kinds are faster on the larger tile, 23 against 25 us).

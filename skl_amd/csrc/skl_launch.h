@@ -109,9 +109,11 @@ int skl_hip_launch_gemm_generic(const skl_gemm_desc *d);
  * canonical form, no fused steps. */
 int skl_hip_gemm_tiled_supported(const skl_gemm_canon *g);
 int skl_hip_launch_gemm_tiled(const skl_gemm_canon *g);
-/* Returns 1 if the canonical problem meets the matrix-core kernels' alignment
- * rules (16-byte aligned bases and strides along the non-unit dimensions). */
+/* Returns 1 if the matrix-core kernels read the canonical problem's operands where they lie: one unit stride each, the
+ * other strides and the base on 16-byte boundaries or, for the bounds-checked kernels, on any (skl_gemm_mfma.hip). */
 int skl_hip_gemm_mfma_supported(const skl_gemm_canon *g);
+/* ... and whether that beats copies padded to whole tiles. */
+int skl_hip_gemm_mfma_in_place_pays(const skl_gemm_canon *g);
 int skl_hip_launch_gemm_mfma(const skl_gemm_canon *g);
 
 /* The streaming kernel on copies of A and B padded to whole tiles (see skl_gemm_mfma.hip): the plan returns the tile

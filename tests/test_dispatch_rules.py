@@ -99,3 +99,26 @@ def test_operands_off_the_16_byte_rule_the_kernels_read_in_place(kind):
     assert not in_place(kind, 100, 64 + chunk + 1, 100, b_sk=65, b_s1=6501)  # blocks apart: a run's start has no bytes in front
     assert in_place(kind, 100, 64 + chunk, 100, b_sk=65, b_s1=6501)
     assert not in_place(kind, 4096, 4096, 4096, a_s0=4097) and in_place(kind, 4095, 4096, 4096, a_s0=4097)
+
+
+def pays(kind, m, n, k, lda=None, ldb=None, b_rows=True):
+    g = Canon(ta=kind, tb=kind, m=m, n=n, k=k, a=1 << 20, b=1 << 20, c=1 << 20, a_sk=1, c_row_shift=6, c_col_shift=6)
+    g.a_s0 = lda or k
+    ldb = ldb or (n if b_rows else k)
+    g.b_s0, g.b_sk = (1, ldb) if b_rows else (ldb, 1)
+    g.a_s1, g.b_s1 = 64 * g.a_s0, 64 * g.b_s0
+    g.rsc0, g.csc0, g.rsc1, g.csc1 = n, 1, 64 * n, 64
+    fn = ct.CDLL(skl_amd.library_path()).skl_hip_gemm_mfma_in_place_pays
+    fn.argtypes = [ct.POINTER(Canon)]
+    return fn(ct.byref(g))
+
+
+@pytest.mark.parametrize("kind", (I8, BF16, E4M3))
+def test_copies_padded_to_tiles_only_where_both_operands_need_them(kind):
+    k = 4500 if kind != BF16 else 2500
+    assert pays(kind, 4000, 4000, 5008, ldb=4000) and pays(kind, 4000, 4000, 5008, lda=5009)
+    assert pays(kind, 4000, 4000, k + 1, lda=k + 1, ldb=4001)                          # B read across K
+    assert not pays(kind, 4000, 4000, k + 1, b_rows=False)                             # 256 tiles, a full round
+    assert pays(kind, 4000, 4000, k // 2 + 1, lda=k // 2 + 1, b_rows=False)            # short K
+    assert pays(kind, 300, 300, k + 1, b_rows=False)                                   # six tiles
+    assert not pays(kind, 4096, 4096, 4096, lda=4097) and pays(kind, 4096, 4096, 4096)  # whole tiles: one copy streams

@@ -8,6 +8,7 @@ import pytest
 import skl_amd
 import support
 from skl_amd import DeviceBuffer
+from gpu_support import run_fused_gemm, run_gemm
 from support import GemmCase, run_oracle_gemm
 
 pytestmark = pytest.mark.gpu
@@ -71,3 +72,52 @@ def test_large_tiles_and_shared_k_off_the_16_byte_rule(gpu, ta, k):
     for a_rows, b_rows in ((True, False), (False, False), (True, True)):
         in_place(gpu, ta, 1025, 1031, k, a_rows, b_rows, 1, 2, 3, 0, 1)
         in_place(gpu, ta, 40, 333, k, a_rows, b_rows, 5, 0, 0, 1, 0)
+
+
+def ragged_large(gpu, ta, m, n, k, a_rows, b_rows, beta, relu=False):
+    """Operands on the 16-byte rule with poisoned gaps between their rows, against the product in fp64."""
+    es = support.ETYPES[ta].dtype.itemsize
+    pad = 32 // es
+    lda, ldb = (k if a_rows else m) + pad, (n if b_rows else k) + pad
+    case = GemmCase(ta, None, 2 if ta == "i8" else 1.5, beta, m0=1, n0=1, k0=1, m1=m, n1=n, k1=k, rsa0=0, csa0=0,
+                    rsa1=lda if a_rows else 1, csa1=1 if a_rows else lda, rsb0=0, csb0=0, rsb1=ldb if b_rows else 1,
+                    csb1=1 if b_rows else ldb, rsc0=0, csc0=0, rsc1=n, csc1=1)
+    rng = np.random.default_rng(m + n + k + a_rows + 2 * b_rows)
+    gen, widen = support.ETYPES[ta].gen, support.ETYPES[ta].widen
+    a = np.full((m if a_rows else k, lda), POISON[ta], support.ETYPES[ta].dtype)
+    b = np.full((k if b_rows else n, ldb), POISON[ta], support.ETYPES[ta].dtype)
+    a[:, :lda - pad] = gen(rng, a.shape[0] * (lda - pad)).reshape(a.shape[0], -1)
+    b[:, :ldb - pad] = gen(rng, b.shape[0] * (ldb - pad)).reshape(b.shape[0], -1)
+    c = rng.integers(-100, 100, (m, n)).astype(case.cdtype)
+    A, B = widen(a[:, :lda - pad]), widen(b[:, :ldb - pad])
+    A, B = A if a_rows else A.T, B if b_rows else B.T
+    exact = case.alpha * (A @ B) + beta * c
+    if relu:
+        got, _ = run_fused_gemm(gpu, "rc", case, a.reshape(-1)[:a.size - pad], b.reshape(-1)[:b.size - pad], c.reshape(-1), None, None, "device", activation=1)
+        exact = np.maximum(exact, 0)
+    else:
+        got = run_gemm(gpu, "rc", case, a.reshape(-1)[:a.size - pad], b.reshape(-1)[:b.size - pad], c.reshape(-1), "device")
+    got = got.reshape(m, n)
+    if case.is_int:
+        assert np.array_equal(got, (exact.astype(np.int64) & 0xFFFFFFFF).astype(np.uint32).view(np.int32))
+        return
+    gamma = 2.0 * np.expm1((k + 2) * np.log1p(2.0 ** -24))
+    extra = support.FP8_MFMA_REL if ta.startswith("f8") else 0.0
+    bound = (gamma + extra) * 1.5 * (np.abs(A) @ np.abs(B)) + gamma * abs(beta) * np.abs(c)
+    assert np.all(np.abs(got - exact) <= bound + np.abs(exact) * 2.0 ** -22)
+
+
+@pytest.mark.parametrize("ta,k", (("i8", 272), ("i8", 65), ("bf16", 264), ("bf16", 129), ("f8e4m3", 2416), ("f8e5m2", 2433)))
+@pytest.mark.parametrize("a_rows,b_rows", ((True, True), (True, False), (False, True), (False, False)))
+def test_streaming_kernel_on_ragged_tiles(gpu, ta, k, a_rows, b_rows):
+    """One round of 256 x 128 tiles that reads C, every operand layout; a K that ends inside a slice, in an odd slice, and -
+    where no operand has K contiguous - anywhere; the last tiles 16 rows and columns wide."""
+    if k % 8 and (a_rows or not b_rows):
+        pytest.skip("16 bytes along K that end inside: the bounds-checked kernels")
+    ragged_large(gpu, ta, 2320, 2832, k, a_rows, b_rows, 1 if ta == "i8" else 0.5)
+
+
+@pytest.mark.parametrize("ta,k,relu", (("i8", 4112, False), ("bf16", 2088, True), ("f8e4m3", 4240, False)))
+@pytest.mark.parametrize("a_rows,b_rows", ((True, True), (False, True), (True, False)))
+def test_streaming_kernel_on_ragged_wide_tiles(gpu, ta, k, relu, a_rows, b_rows):
+    ragged_large(gpu, ta, 3856, 3104, k, a_rows, b_rows, 0, relu)
