@@ -1051,6 +1051,7 @@ static int run_large_cases(void) {
   run_rowmajor_fused(1, 4096, 1536, 1, 0, 1, "fused int8 GEMV (product into scratch, then the epilogue pass) differs");
   run_rowmajor_fused(6, 2048, 2048, -1, 2, 0, "fused int8 decode batch (product into scratch, then the epilogue pass) differs");
   run_rowmajor(SKL_DT_I8, 1500, 2100, 120, 1, 5, 3, 2, -1, "large ragged int8 GEMM (tile-padded copies) differs");
+  run_rowmajor(SKL_DT_I8, 2304, 1408, 128, 5, 3, 2, 3, -1, "int8 GEMM of whole tiles off the 16-byte rule (tile-padded copies) differs");
   run_rowmajor(SKL_DT_BF16, 500, 600, 72, 8, 16, 1, 1, 1, "ragged mid-size bf16 GEMM differs");
   run_rowmajor(SKL_DT_I8, 3, 256, 100, 0, 0, 0, 1, 0, "int8 GEMM with three rows (few-rows kernel) differs");
   run_rowmajor(SKL_DT_I8, 6, 2048, 2048, 0, 0, 0, -1, 2, "int8 GEMM with six rows (decode batch) differs");
