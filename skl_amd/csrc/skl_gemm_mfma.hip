@@ -210,15 +210,13 @@ int launch_epilogue(const skl_gemm_canon *g, const void *product, bool zeroing) 
   p.rq = g->rq;
   p.tiles_m = p.tiles_n = 0;
   p.splits = 1, p.slices_per_split = 0, p.partial = (char *)product;
+  if (!zeroing) return launch_split_reduce<int>(p, "gemm_epilogue");
   const size_t blocks = (p.m * p.n + 255) / 256;
   if (blocks > 0x7FFFFFFFu) {
     skl_hip_record_error(-2, "gemm_epilogue: grid too large");
     return -2;
   }
-  if (zeroing)
-    gemm_epilogue_zeroing_kernel<<<(unsigned)blocks, 256, 0, skl_current_stream()>>>(p);
-  else
-    gemm_split_reduce_kernel<int><<<(unsigned)blocks, 256, 0, skl_current_stream()>>>(p);
+  gemm_epilogue_zeroing_kernel<<<(unsigned)blocks, 256, 0, skl_current_stream()>>>(p);
   return skl_check_launch("gemm_epilogue");
 }
 }  // namespace

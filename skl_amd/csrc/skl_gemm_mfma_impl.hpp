@@ -52,8 +52,9 @@ struct MfmaArgs {
   char *max;
   skl_requant rq;    // ... activation and requantised int8 copy
   unsigned tiles_m, tiles_n;
-  // Split along K (bounds-checked kernel only): workgroup b works on tile b % (tiles_m * tiles_n) and on the
-  // slices [split * slices_per_split, ...) with split = b / (tiles_m * tiles_n); splits > 1 stores the raw
+  unsigned by_group = 0, by_rest = 0;  // tile_of_block's divisions as multiplications (set_tiles), 0: too many tiles for that
+  // Split along K (bounds-checked kernel only): workgroup (b, split) works on tile b and on the
+  // slices [split * slices_per_split, ...); splits > 1 stores the raw
   // sums to partial[split][m][n] (row-major, 4-byte elements) for gemm_split_reduce_kernel.
   unsigned splits, slices_per_split;
   char *partial;
@@ -73,8 +74,10 @@ typedef _Float16 v8h __attribute__((ext_vector_type(8)));
 
 #define LDS_PTR(T, p) ((__attribute__((address_space(3))) T *)(p))
 
-constexpr int kSliceBytes = 128;    // bytes of K per LDS stage and operand row
-constexpr int kPitchKC = 144;       // LDS row pitch of a K-contiguous tile
+// Bytes of K per LDS stage and operand row in the bounds-checked kernels. The 64 x 64 tiles serve problems too small to fill the
+// chip, whose time is a chain - LDS stores, a barrier, fragment reads, products - per slice, most of it latency: 256 bytes to
+// a slice halve the chain. (The 128 x 128 tiles keep two workgroups on a compute unit with 128.)
+constexpr int slice_bytes(int tile) { return tile == 64 ? 256 : 128; }
 
 
 // The fused steps behind the alpha/beta step, for one lane: bias of the lane's column, activation, running maximum,
@@ -289,19 +292,29 @@ __device__ __forceinline__ auto prep_b(F f) {
 }
 
 // ---------------------------------------------------------------------------
-// LDS tile geometry of one operand: ROWS along M or N, 128 bytes of K.
+// LDS tile geometry of one operand: ROWS along M or N, a slice of K.
 // ---------------------------------------------------------------------------
 template <int ES, int ROWS, bool KC, int NT>
 struct Tile {
+  static constexpr int kSlice = slice_bytes(ROWS);
+  static constexpr int kRowChunks = kSlice / 16;
   static constexpr int CE = 16 / ES;                 // elements per 16-byte chunk
-  static constexpr int KE = kSliceBytes / ES;        // k elements per slice
+  static constexpr int KE = kSlice / ES;             // k elements per slice
+  static constexpr int kPitchKC = kSlice + 16;       // 16 rows of 16 bytes fill the 64 banks once
   // MN-contiguous tile: KE rows of ROWS*ES bytes. A transpose load is served 32
   // lanes at a time: 8 rows x 32 B (8-bit) or 4 rows x 64 B (16-bit). Skewing
   // consecutive rows by that width spreads them over all 64 banks (measured:
   // zero bank conflicts with 32 / 64 bytes of padding, conflicts with 16 / 32).
-  static constexpr int kPitchMC = ROWS * ES + (ES == 1 ? 32 : 64);
+  // The tiles of 64 rows do it without padding - four (two) rows fill the banks, the next ones swap their halves -,
+  // which lets two workgroups share a compute unit.
+  static constexpr bool kSwizzled = ROWS == 64;
+  static constexpr int kPitchMC = ROWS * ES + (kSwizzled ? 0 : ES == 1 ? 32 : 64);
+  __device__ static __forceinline__ int mc(int r, int byte) {  // byte `byte` of k-row r
+    if constexpr (!kSwizzled) return r * kPitchMC + byte;
+    return r * kPitchMC + (ES == 1 ? byte ^ ((r >> 2 & 1) << 5) : byte ^ ((r >> 1 & 1) << 6));
+  }
   static constexpr int kBytes = KC ? ROWS * kPitchKC : KE * kPitchMC;
-  static constexpr int kChunks = ROWS * 8;           // 16-byte chunks per slice
+  static constexpr int kChunks = ROWS * kRowChunks;  // 16-byte chunks per slice
   static constexpr int kPerThread = kChunks / NT;    // chunks each of the NT threads moves
   static constexpr int kMnChunks = ROWS * ES / 16;   // chunks along MN of an MN-contiguous row
 };
@@ -334,7 +347,8 @@ struct Loader {
   using T = Tile<ES, ROWS, KC, NT>;
   static constexpr unsigned kRange = 0xC0000000u, kOutside = 0xE0000000u;  // (offsets inside a tile stay below 0xA8000000, see operand_ok)
   static constexpr unsigned kBias = 16;  // the base lies 16 bytes ahead of the tile, so that no offset is negative
-  static constexpr int kRowsPerPass = KC ? NT / 8 : NT / T::kMnChunks;
+  static constexpr int kRowsPerPass = KC ? NT / T::kRowChunks : NT / T::kMnChunks;
+  static_assert(KC || kRowsPerPass % 8 == 0, "the swizzle of a thread's chunks is that of its first");
   const char *base;              // uniform
   size_t k_step;                 // bytes between consecutive slices
   unsigned off[T::kPerThread];   // byte offset of each chunk
@@ -343,33 +357,36 @@ struct Loader {
   unsigned back;                 // MC: bytes by which the chunks are loaded too low
   bool loose, mn_shift;          // uniform
 
+  // A thread's chunks lie kRowsPerPass rows (or k-rows) apart: their offsets are that of its first one plus scalars. (All in 32
+  // bits: instructions ahead of the first load are time that a small problem has nothing to hide under.)
   __device__ __forceinline__ void init(const char *operand, size_t mn0, size_t mn_dim, size_t s1, size_t s0, size_t sk, bool is_loose) {
-    const int t = threadIdx.x;
+    const unsigned t = threadIdx.x, extent = mn_dim - mn0 < (size_t)ROWS ? (unsigned)(mn_dim - mn0) : (unsigned)ROWS;
     loose = is_loose;
     base = operand + (mn0 >> 6) * s1 * ES - kBias;  // mn0 is a multiple of 64
     back = 0;
     mn_shift = false;
     if constexpr (KC) {
-      const int c = t & 7;
-      k_first = c * T::CE;
-      lds_off = (t >> 3) * kPitchKC + c * 16;
+      static_assert(64 % kRowsPerPass == 0, "a pass lies in one block of 64 rows");
+      const unsigned c = t % T::kRowChunks, first_row = t / T::kRowChunks, mine = first_row * (unsigned)(s0 * ES) + c * 16 + kBias;
+      k_first = (int)(c * T::CE);
+      lds_off = first_row * T::kPitchKC + c * 16;
 #pragma unroll
       for (int i = 0; i < T::kPerThread; ++i) {
-        const int row = (t >> 3) + i * kRowsPerPass;
-        off[i] = mn0 + row < mn_dim ? (unsigned)(((size_t)(row >> 6) * s1 + (size_t)(row & 63) * s0) * ES + c * 16) + kBias : kOutside;
+        constexpr int R = kRowsPerPass;
+        off[i] = first_row + i * R < extent ? mine + (unsigned)(((size_t)(i * R >> 6) * s1 + (size_t)(i * R & 63) * s0) * ES) : kOutside;
       }
     } else {
-      const int mc = t % T::kMnChunks, r = mc * T::CE;
-      k_first = t / T::kMnChunks;
-      lds_off = k_first * T::kPitchMC + mc * 16;
-      const long there = (long)mn_dim - (long)(mn0 + r);  // elements from the chunk's first on
+      const unsigned mc = t % T::kMnChunks, r = mc * T::CE, row = t / T::kMnChunks;
+      k_first = (int)row;
+      lds_off = T::mc((int)row, (int)mc * 16);
+      const int there = (int)extent - (int)r;  // elements from the chunk's first on
       if (loose && there > 0 && there < T::CE) back = (unsigned)((T::CE - there) * ES);
-      mn_shift = loose && mn_dim - mn0 < ROWS && mn_dim % T::CE != 0;
+      mn_shift = loose && extent < (unsigned)ROWS && extent % T::CE != 0;
+      const unsigned mine = (ROWS > 64 ? (r >> 6) * (unsigned)(s1 * ES) : 0u) + (r & 63) * ES + row * (unsigned)(sk * ES) + kBias - back;
 #pragma unroll
-      for (int i = 0; i < T::kPerThread; ++i)
-        off[i] = there > 0 ? (unsigned)(((size_t)(r >> 6) * s1 + (size_t)(r & 63) + (size_t)(k_first + i * kRowsPerPass) * sk) * ES) + kBias - back : kOutside;
+      for (int i = 0; i < T::kPerThread; ++i) off[i] = there > 0 ? mine + (unsigned)((size_t)(i * kRowsPerPass) * sk * ES) : kOutside;
     }
-    k_step = KC ? (size_t)kSliceBytes : (size_t)T::KE * sk * ES;
+    k_step = KC ? (size_t)T::kSlice : (size_t)T::KE * sk * ES;
   }
 
   // `left`: elements of K from the slice's first on, none or fewer beyond the last slice.
@@ -405,7 +422,7 @@ struct Loader {
       }
     }
 #pragma unroll
-    for (int i = 0; i < T::kPerThread; ++i) *reinterpret_cast<v4i *>(tile + lds_off + i * kRowsPerPass * (KC ? kPitchKC : T::kPitchMC)) = regs[i];
+    for (int i = 0; i < T::kPerThread; ++i) *reinterpret_cast<v4i *>(tile + lds_off + i * kRowsPerPass * (KC ? T::kPitchKC : T::kPitchMC)) = regs[i];
   }
 };
 
@@ -417,7 +434,7 @@ __device__ __forceinline__ auto read_frag(const char *tile, int row0, int kb) {
   const int lane = threadIdx.x & 63;
   const int h = lane >> 5;  // which half of the k-step this lane feeds
   if constexpr (KC) {
-    const char *p = tile + (row0 + (lane & 31)) * kPitchKC + kb + h * FRB;
+    const char *p = tile + (row0 + (lane & 31)) * T::kPitchKC + kb + h * FRB;
     if constexpr (FRB == 16) {
       return *reinterpret_cast<const v4i *>(p);
     } else {
@@ -428,7 +445,7 @@ __device__ __forceinline__ auto read_frag(const char *tile, int row0, int kb) {
     // ds_read_b64_tr_b8: 16 lanes read an 8 (k) x 16 (mn) byte block; lane j receives column j.
     const int g16 = (lane >> 4) & 1, j = lane & 15;
     const int kfirst = kb + h * FRB + (j >> 1);
-    const char *p = tile + kfirst * T::kPitchMC + row0 + g16 * 16 + (j & 1) * 8;
+    const char *p = tile + T::mc(kfirst, row0 + g16 * 16 + (j & 1) * 8);
     v2i r[FRB / 8];
 #pragma unroll
     for (int s = 0; s < FRB / 8; ++s) r[s] = __builtin_amdgcn_ds_read_tr8_b64_v2i32(LDS_PTR(v2i, p + s * 8 * T::kPitchMC));
@@ -442,7 +459,7 @@ __device__ __forceinline__ auto read_frag(const char *tile, int row0, int kb) {
     static_assert(FRB == 16, "16-bit fragments are 16 bytes");
     const int g16 = (lane >> 4) & 1, j = lane & 15;
     const int kfirst = kb / 2 + h * 8 + (j >> 2);
-    const char *p = tile + kfirst * T::kPitchMC + (row0 + g16 * 16 + (j & 3) * 4) * 2;
+    const char *p = tile + T::mc(kfirst, (row0 + g16 * 16 + (j & 3) * 4) * 2);
     const v4s r0 = __builtin_amdgcn_ds_read_tr16_b64_v4i16(LDS_PTR(v4s, p));
     const v4s r1 = __builtin_amdgcn_ds_read_tr16_b64_v4i16(LDS_PTR(v4s, p + 4 * T::kPitchMC));
     const v2i a = __builtin_bit_cast(v2i, r0), b = __builtin_bit_cast(v2i, r1);
@@ -565,7 +582,13 @@ __device__ __forceinline__ void write_wave_tile(const MfmaArgs &p, const Acc (&a
         constexpr int j = B / MI, i = B % MI;
         const Where w = where(j, i);
 #pragma unroll
-        for (int r = 0; r < 16; ++r) old[B % (kAhead + 1)][r] = inside(j, i, r) ? w.out[r >> 2][(r & 3) * p.rsc0] : AccElem(0);
+        for (int r = 0; r < 16; ++r) {
+          // beyond the edge the first element of C is read in place of one that does not exist: a guard would be a branch, at
+          // which the loads in flight are waited for (int8 3584 x 1266 x 768 reading C: 33.4 -> 21.2 us)
+          const AccElem *from = w.out[r >> 2] + (r & 3) * p.rsc0;
+          if (CHECK) from = inside(j, i, r) ? from : c;
+          old[B % (kAhead + 1)][r] = *from;
+        }
         __builtin_amdgcn_sched_barrier(0);
       }
     };
@@ -639,10 +662,10 @@ __device__ __forceinline__ void write_wave_tile_staged(const MfmaArgs &p, const 
   // the copy's four bytes on a dword
   const bool c_run = cols == 4 && p.csc0 == 1 && p.ccs >= 2 && (((uintptr_t)p.c | (p.csc1 * 4) | (p.rsc0 * 4) | (p.rsc1 * 4)) & 15) == 0;
   const bool q_run = cols == 4 && p.rq.csq == 1 && (p.rq.rsq & 3) == 0 && ((uintptr_t)p.rq.q & 3) == 0;
-  // A pass covers four rows from a multiple of four on, which lie in one block of C: where they start is the same for the
-  // whole wave (scalar arithmetic), the lane's row among them a constant.
-  static_assert(kRowsPerPass == 4, "four rows per pass");
-  T *const c_lane = reinterpret_cast<T *>(p.c) + (size_t)r_first * p.rsc0;
+  // A pass covers four (eight) rows from a multiple of four (eight) on, whole blocks of C or part of one: where they start is
+  // the same for the whole wave (scalar arithmetic), the lane's row among them a constant.
+  static_assert(kRowsPerPass == 4 || kRowsPerPass == 8, "blocks of C have a power of two of rows, at least four");
+  T *const c_lane = reinterpret_cast<T *>(p.c) + ((size_t)r_first >> p.crs) * p.rsc1 + ((size_t)r_first & rmask) * p.rsc0;
   int8_t *const q_lane = reinterpret_cast<int8_t *>(p.rq.q) + (size_t)r_first * p.rq.rsq + col * p.rq.csq;
   const skl_fp8::Ofp8Format f8(p.rq.q_fmt);
   T running = skl_lowest<T>();
@@ -676,7 +699,11 @@ __device__ __forceinline__ void write_wave_tile_staged(const MfmaArgs &p, const 
             for (int q = 0; q < 4; ++q) old[j][4 * g + q] = four[q];
           } else {
 #pragma unroll
-            for (int q = 0; q < 4; ++q) old[j][4 * g + q] = !CHECK || (jc < p.n && row + q < p.m) ? from[q * p.rsc0] : T(0);
+            for (int q = 0; q < 4; ++q) {  // (no guard, see write_wave_tile)
+              const T *at = from + q * p.rsc0;
+              if (CHECK) at = jc < p.n && row + q < p.m ? at : reinterpret_cast<const T *>(p.c);
+              old[j][4 * g + q] = *at;
+            }
           }
           __builtin_amdgcn_sched_barrier(0);
         }
@@ -710,7 +737,7 @@ __device__ __forceinline__ void write_wave_tile_staged(const MfmaArgs &p, const 
 #pragma unroll 2
     for (int pass = 0; pass < 32 / kRowsPerPass; ++pass) {
       const V4 sum = *reinterpret_cast<const V4 *>(stage_out + pass * kRowsPerPass * P);
-      const size_t four = row0 + (size_t)(i * 32 + pass * kRowsPerPass);  // a scalar
+      const size_t four = row0 + (size_t)(i * 32 + pass * kRowsPerPass);  // the first of them: a scalar
       if (CHECK && (four + r_first >= p.m || cols == 0)) continue;
       T *const c_row = c_lane + ((four >> p.crs) * p.rsc1 + (four & rmask) * p.rsc0);
       V4 v;
@@ -765,18 +792,20 @@ __device__ __forceinline__ void write_wave_tile_staged(const MfmaArgs &p, const 
 // 5814 tiles of 128 x 128: 458 -> 398 us); the streaming kernel with its larger tiles does not (int8 5169 x 15488 x 704 on
 // 1281 tiles: 362 -> 389 us): its eight XCDs then read eight tile rows of the same columns.
 template <bool ANY>
-__device__ __forceinline__ void tile_of_block(unsigned bid, unsigned tiles_m, unsigned tiles_n, unsigned &tm,
-                                              unsigned &tn) {
+__device__ __forceinline__ void tile_of_block(unsigned bid, const MfmaArgs &p, unsigned &tm, unsigned &tn) {
   constexpr unsigned kXcd = 8, kGroupM = 8;
+  const unsigned tiles_m = p.tiles_m, tiles_n = p.tiles_n;
   const unsigned total = tiles_m * tiles_n, xcd = bid % kXcd, longer = total % kXcd;  // the first `longer` ranges hold one tile more
   unsigned t = bid;
   if (ANY || longer == 0) t = xcd * (total / kXcd) + (xcd < longer ? xcd : longer) + bid / kXcd;
   const unsigned per_group = kGroupM * tiles_n;
-  const unsigned group = t / per_group, first_m = group * kGroupM;
-  const unsigned rows = tiles_m - first_m < kGroupM ? tiles_m - first_m : kGroupM;
-  const unsigned in_group = t % per_group;
-  tm = first_m + in_group % rows;
-  tn = in_group / rows;
+  const unsigned group = p.by_group ? __umulhi(t, p.by_group) : t / per_group, first_m = group * kGroupM;
+  const unsigned in_group = t - group * per_group;
+  const bool full = tiles_m - first_m >= kGroupM;
+  const unsigned rows = full ? kGroupM : tiles_m - first_m;  // of the last group: tiles_m % 8
+  const unsigned column = full ? in_group / kGroupM : rows == 1 ? in_group : p.by_group ? __umulhi(in_group, p.by_rest) : in_group / rows;
+  tm = first_m + in_group - column * rows;
+  tn = column;
 }
 
 // The kernel for ragged and small problems: any M, N and K, operands on any boundary. A problem of few tiles is bound by the
@@ -785,7 +814,7 @@ __device__ __forceinline__ void tile_of_block(unsigned bid, unsigned tiles_m, un
 // 28.4 -> 23.7 with its second pass, int8 136 x 704 x 2207 51 -> 12.4 (no copy of A in front), f16 427 x 5901 x 1805 93 -> 33;
 // over 120 random problems 0.70.
 template <int TA, int TB, bool A_KC, bool B_KC, int BM, int BN, int WAVES_M, int WAVES_N, bool EXACT = false, bool EXTRA = false>
-__global__ void __launch_bounds__(WAVES_M *WAVES_N * 64, 4) gemm_mfma_kernel(MfmaArgs p) {
+__global__ void __launch_bounds__(WAVES_M *WAVES_N * 64, (BM == 64 ? 2 : 4)) gemm_mfma_kernel(MfmaArgs p) {
   constexpr int NT = WAVES_M * WAVES_N * 64;
   using KA = Kind<TA>;
   using M = typename std::conditional<EXACT, MmaF8Exact<TA, TB>, Mma<TA, TB>>::type;
@@ -799,14 +828,15 @@ __global__ void __launch_bounds__(WAVES_M *WAVES_N * 64, 4) gemm_mfma_kernel(Mfm
   using TileA = Tile<ES, BM, A_KC, NT>;
   using TileB = Tile<ES, BN, B_KC, NT>;
   constexpr int kStage = TileA::kBytes + TileB::kBytes;
-  // Slices under way, 16 registers each, of the 128 a thread has (the 32-byte fragments of the fp8 kinds take twice the room).
-  constexpr int kAhead = BM == 128 ? (FRB == 32 ? 1 : 2) : FRB == 32 || EXACT ? 3 : 4;
+  // Slices under way: 16 registers each, of the 128 a thread has (the 32-byte fragments of the fp8 kinds take twice the room);
+  // 64 x 64: 32 of 256.
+  constexpr int kAhead = BM == 128 ? (FRB == 32 ? 1 : 2) : 2;
 
   extern __shared__ __attribute__((aligned(16))) char smem[];
 
   unsigned tm, tn;
-  const unsigned tiles = p.tiles_m * p.tiles_n, split = blockIdx.x / tiles;
-  tile_of_block<true>(blockIdx.x % tiles, p.tiles_m, p.tiles_n, tm, tn);
+  const unsigned split = blockIdx.y;
+  tile_of_block<true>(blockIdx.x, p, tm, tn);
   const size_t m0 = (size_t)tm * BM, n0 = (size_t)tn * BN;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;  // the wave index as a scalar: nothing derived from it occupies a vector register across the main loop
   const int wm = (wave / WAVES_N) * WM, wn = (wave % WAVES_N) * WN;
@@ -848,43 +878,30 @@ __global__ void __launch_bounds__(WAVES_M *WAVES_N * 64, 4) gemm_mfma_kernel(Mfm
   __builtin_amdgcn_sched_barrier(0);
   __syncthreads();
 
-  constexpr int kSteps = kSliceBytes / KB;  // MFMA k-steps per slice
-  typename M::Frag fa[2][MI], fb[2][NI];    // operand fragments, double-buffered across k-steps
-  const auto multiply = [&](unsigned s) __attribute__((always_inline)) {
+  constexpr int kSteps = TileA::kSlice / KB;  // MFMA k-steps per slice
+  // Operand fragments: read a k-step ahead of their use, or, 64 x 64, all of a slice at once.
+  constexpr bool kAllAtOnce = BM == 64;
+  constexpr int kSets = kAllAtOnce ? kSteps : 2;
+  typename M::Frag fa[kSets][MI], fb[kSets][NI];
+  const auto read_step = [&](unsigned s, int ks, int set) __attribute__((always_inline)) {
     const char *ta = smem + (s & 1) * kStage;
     const char *tb = ta + TileA::kBytes;
 #pragma unroll
-    for (int i = 0; i < MI; ++i) fa[0][i] = read_frag<ES, BM, A_KC, FRB>(ta, wm + i * 32, 0);
+    for (int i = 0; i < MI; ++i) fa[set][i] = read_frag<ES, BM, A_KC, FRB>(ta, wm + i * 32, ks * KB);
 #pragma unroll
-    for (int j = 0; j < NI; ++j) fb[0][j] = read_frag<ES, BN, B_KC, FRB>(tb, wn + j * 32, 0);
+    for (int j = 0; j < NI; ++j) fb[set][j] = read_frag<ES, BN, B_KC, FRB>(tb, wn + j * 32, ks * KB);
+  };
+  const auto products = [&](int set) __attribute__((always_inline)) {
+    decltype(prep_a<M>(fa[set][0])) wa[MI];
+    decltype(prep_b<M>(fb[set][0])) wb[NI];
 #pragma unroll
-    for (int ks = 0; ks < kSteps; ++ks) {
-      const int cur = ks & 1, nx = cur ^ 1;
-      if (ks + 1 < kSteps) {  // fragments of the next k-step are requested before this step's MFMAs
+    for (int i = 0; i < MI; ++i) wa[i] = prep_a<M>(fa[set][i]);
 #pragma unroll
-        for (int i = 0; i < MI; ++i) fa[nx][i] = read_frag<ES, BM, A_KC, FRB>(ta, wm + i * 32, (ks + 1) * KB);
+    for (int j = 0; j < NI; ++j) wb[j] = prep_b<M>(fb[set][j]);
 #pragma unroll
-        for (int j = 0; j < NI; ++j) fb[nx][j] = read_frag<ES, BN, B_KC, FRB>(tb, wn + j * 32, (ks + 1) * KB);
-      }
-      // The LDS reads above are all issued before the first MFMA below and are
-      // not needed until the next k-step: the scheduler must not pull them
-      // down next to their uses (with one wave per SIMD nothing else would
-      // hide their latency).
-      __builtin_amdgcn_sched_barrier(0);
-      {
-        decltype(prep_a<M>(fa[cur][0])) wa[MI];
-        decltype(prep_b<M>(fb[cur][0])) wb[NI];
+    for (int i = 0; i < MI; ++i)
 #pragma unroll
-        for (int i = 0; i < MI; ++i) wa[i] = prep_a<M>(fa[cur][i]);
-#pragma unroll
-        for (int j = 0; j < NI; ++j) wb[j] = prep_b<M>(fb[cur][j]);
-#pragma unroll
-        for (int i = 0; i < MI; ++i)
-#pragma unroll
-          for (int j = 0; j < NI; ++j) acc[i][j] = M::run(wa[i], wb[j], acc[i][j]);
-      }
-      __builtin_amdgcn_sched_barrier(0);
-    }
+      for (int j = 0; j < NI; ++j) acc[i][j] = M::run(wa[i], wb[j], acc[i][j]);
   };
   // Slice s, whose loads have been under way for kAhead slices, into LDS; slice s + kAhead requested in its registers (not
   // by the last slices: LAST).
@@ -898,20 +915,43 @@ __global__ void __launch_bounds__(WAVES_M *WAVES_N * 64, 4) gemm_mfma_kernel(Mfm
       lb.fetch(next_b, s_begin + s + kAhead, left(s + kAhead));
       __builtin_amdgcn_sched_barrier(0);  // the loads stay up here, not next to the stores that use them
     }
-    __syncthreads();
+  };
+  // Slice s is multiplied and, if there are `more`, the next one put into the other half of LDS, which every wave has left.
+  const auto slice = [&](auto last, bool more, unsigned s, v4i (&next_a)[TileA::kPerThread], v4i (&next_b)[TileB::kPerThread]) __attribute__((always_inline)) {
+    read_step(s, 0, 0);
+    if constexpr (kAllAtOnce) {  // the next slice's stores land under this one's products
+#pragma unroll
+      for (int ks = 1; ks < kSteps; ++ks) read_step(s, ks, ks);
+      if (more) advance(last, s + 1, next_a, next_b);
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int ks = 0; ks < kSteps; ++ks) products(ks);
+    } else {
+#pragma unroll
+      for (int ks = 0; ks < kSteps; ++ks) {
+        // The next k-step's LDS reads are all issued before the first MFMA below and are not needed until then: the scheduler
+        // must not pull them down next to their uses.
+        if (ks + 1 < kSteps) read_step(s, ks + 1, (ks + 1) & 1);
+        __builtin_amdgcn_sched_barrier(0);
+        products(ks & 1);
+        __builtin_amdgcn_sched_barrier(0);
+      }
+      if (more) advance(last, s + 1, next_a, next_b);
+    }
+    if (more) __syncthreads();
   };
   // The compiler counts the loads in flight along every path into a block: a loop with a way out after each slice, or around
   // one, makes it wait for the youngest of them. So the loop runs whole rounds of kAhead slices, up to the last kAhead + 1.
   unsigned s = 0;
   for (; s + kAhead + 1 < count; s += kAhead) {
     [&]<int... Us>(std::integer_sequence<int, Us...>) __attribute__((always_inline)) {
-      ((multiply(s + Us), advance(std::false_type{}, s + Us + 1, ra[(Us + 1) % kAhead], rb[(Us + 1) % kAhead])), ...);
+      (slice(std::false_type{}, true, s + Us, ra[(Us + 1) % kAhead], rb[(Us + 1) % kAhead]), ...);
     }(std::make_integer_sequence<int, kAhead>{});
   }
-  multiply(s);
   [&]<int... Us>(std::integer_sequence<int, Us...>) __attribute__((always_inline)) {
-    (void)((++s < count && (advance(std::true_type{}, s, ra[(Us + 1) % kAhead], rb[(Us + 1) % kAhead]), multiply(s), true)) && ...);
+    (void)((slice(std::true_type{}, s + 1 < count, s, ra[(Us + 1) % kAhead], rb[(Us + 1) % kAhead]), ++s < count) && ...);
   }(std::make_integer_sequence<int, kAhead>{});
+  if (s < count) slice(std::true_type{}, false, s, ra[0], rb[0]);
 
   // Lane l of a 32x32 block holds column l%32 and rows 8*(r/4) + 4*(l/32) + r%4.
   if (p.splits > 1) {  // a share of K: the raw sums go to this split's M x N plane
@@ -930,7 +970,18 @@ __global__ void __launch_bounds__(WAVES_M *WAVES_N * 64, 4) gemm_mfma_kernel(Mfm
     }
     return;
   }
-  write_wave_tile<MI, NI, true, EXTRA ? 1 : 0>(p, acc, m0 + wm, n0 + wn);
+  if constexpr (EXTRA) {
+    __syncthreads();  // the last slice has been read by every wave
+    write_wave_tile_staged<MI, NI, true>(p, acc, m0 + wm, n0 + wn, smem + wave * 32 * staged_pitch<NI>() * 4);
+  } else {
+    if constexpr (BM == 64) {  // a tile that lies inside C is written without a test per element
+      if (m0 + BM <= p.m && n0 + BN <= p.n) {
+        write_wave_tile<MI, NI, false, 0>(p, acc, m0 + wm, n0 + wn);
+        return;
+      }
+    }
+    write_wave_tile<MI, NI, true, 0>(p, acc, m0 + wm, n0 + wn);
+  }
 }
 
 // ===========================================================================
@@ -1278,7 +1329,7 @@ __global__ void __launch_bounds__(512) gemm_mfma_ring_kernel(MfmaArgs p) {
   // starts s shares into K and leaves its raw sums in plane s of the workspace.
   unsigned tm, tn;
   const unsigned tiles = p.tiles_m * p.tiles_n, split = blockIdx.x / tiles;
-  tile_of_block<false>(blockIdx.x % tiles, p.tiles_m, p.tiles_n, tm, tn);
+  tile_of_block<false>(blockIdx.x % tiles, p, tm, tn);
   const size_t m0 = (size_t)tm * BM, n0 = (size_t)tn * BN;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;  // the wave index as a scalar: nothing derived from it occupies a vector register across the main loop
   const int wm = (wave / WAVES_N) * WM, wn = (wave % WAVES_N) * WN;
@@ -1671,38 +1722,106 @@ __global__ void __launch_bounds__(512) gemm_mfma_ring_kernel(MfmaArgs p) {
 }
 
 // C = beta*C + alpha * (sum of the splits' planes, in split order), then the fused steps: the second
-// half of a GEMM whose K range was shared out between workgroups.
-template <typename T>
+// half of a GEMM whose K range was shared out between workgroups. A thread takes V neighbouring columns of a row; what the
+// pass costs is its launch and one trip to memory, so everything it needs is requested at once and the row is found with one
+// 32-bit division (one element per thread and 64-bit divisions: 4.7 us for 3 planes of 16 x 11008, now 3.0).
+template <typename T, int V>
 __global__ void __launch_bounds__(256) gemm_split_reduce_kernel(MfmaArgs p) {
-  const size_t idx = (size_t)blockIdx.x * 256 + threadIdx.x;
-  if (idx >= p.m * p.n) return;
-  const size_t row = idx / p.n, col = idx % p.n;
+  typedef T Run __attribute__((ext_vector_type(4)));
+  const size_t idx = (size_t)blockIdx.x * 256 + threadIdx.x, per_row = p.n / V;
+  if (idx >= p.m * per_row) return;
+  const size_t row = p.m * per_row >> 32 ? idx / per_row : (size_t)((unsigned)idx / (unsigned)per_row), col = (idx - row * per_row) * V;
+  const size_t mn = p.m * p.n;
+  const T *plane = reinterpret_cast<const T *>(p.partial) + row * p.n + col;
+  const auto load = [](const T *at, T (&v)[V]) __attribute__((always_inline)) {
+    if constexpr (V == 4) {
+      const Run r = *reinterpret_cast<const Run *>(at);
+#pragma unroll
+      for (int e = 0; e < V; ++e) v[e] = r[e];
+    } else {
+      v[0] = *at;
+    }
+  };
+  // V columns of C: they lie in one block of C if its columns come in multiples of V, else each is found by itself.
+  T *const c_row = reinterpret_cast<T *>(p.c) + (row >> p.crs) * p.rsc1 + (row & ((size_t(1) << p.crs) - 1)) * p.rsc0;
+  T *c[V];
+  T bias[V], old[V];
+  const bool init = skl_beta_is_zero<T>(p.beta);
+#pragma unroll
+  for (int e = 0; e < V; ++e) {
+    c[e] = c_row + ((col + e) >> p.ccs) * p.csc1 + ((col + e) & ((size_t(1) << p.ccs) - 1)) * p.csc0;
+    bias[e] = p.bias ? reinterpret_cast<const T *>(p.bias)[col + e] : T(0);
+    old[e] = init ? T(0) : *c[e];
+  }
   // Eight planes are requested before the first is used (one memory round trip per eight, not per plane); the
   // sum still runs over the planes in order, starting from plane 0 itself.
-  const T *plane = reinterpret_cast<const T *>(p.partial) + idx;
-  const size_t mn = p.m * p.n;
-  T sum = plane[0];
+  T sum[V];
+  load(plane, sum);
   for (unsigned q0 = 1; q0 < p.splits; q0 += 8) {
-    T v[8];
+    T v[8][V];
 #pragma unroll
-    for (unsigned u = 0; u < 8; ++u) v[u] = q0 + u < p.splits ? plane[(size_t)(q0 + u) * mn] : T(0);
+    for (unsigned u = 0; u < 8; ++u)
+      if (q0 + u < p.splits) load(plane + (size_t)(q0 + u) * mn, v[u]);
 #pragma unroll
     for (unsigned u = 0; u < 8; ++u) {
       if (q0 + u >= p.splits) continue;
-      if constexpr (std::is_same<T, int>::value)
-        sum = (int)((unsigned)sum + (unsigned)v[u]);
-      else
-        sum = __fadd_rn(sum, v[u]);
+#pragma unroll
+      for (int e = 0; e < V; ++e) {
+        if constexpr (std::is_same<T, int>::value)
+          sum[e] = (int)((unsigned)sum[e] + (unsigned)v[u][e]);
+        else
+          sum[e] = __fadd_rn(sum[e], v[u][e]);
+      }
     }
   }
-  T *c = reinterpret_cast<T *>(p.c) + (row >> p.crs) * p.rsc1 + (row & ((size_t(1) << p.crs) - 1)) * p.rsc0 +
-         (col >> p.ccs) * p.csc1 + (col & ((size_t(1) << p.ccs) - 1)) * p.csc0;
-  T v = skl_beta_is_zero<T>(p.beta) ? skl_initialise(sum, c, p.alpha, p.beta) : skl_combine(sum, *c, p.alpha, p.beta);
-  if (p.bias) v = skl_add_bias(v, reinterpret_cast<const T *>(p.bias)[col]);
-  v = skl_activate(v, p.rq.act);
-  if (!p.rq.q_only) *c = v;
-  skl_emit_requantised(p.rq, v, row, col);
-  if (p.max && v > skl_lowest<T>()) skl_atomic_max(reinterpret_cast<T *>(p.max), v);
+  T best = skl_lowest<T>();
+  Run out;
+#pragma unroll
+  for (int e = 0; e < V; ++e) {
+    T v = init ? skl_initialise(sum[e], c[e], p.alpha, p.beta) : skl_combine(sum[e], old[e], p.alpha, p.beta);
+    if (p.bias) v = skl_add_bias(v, bias[e]);
+    v = skl_activate(v, p.rq.act);
+    out[e] = v;
+    if (v > best) best = v;
+  }
+  if (!p.rq.q_only) {
+    if (V == 4 && p.csc0 == 1 && p.ccs >= 2 && ((uintptr_t)c[0] & 15) == 0) {
+      *reinterpret_cast<Run *>(c[0]) = out;
+    } else {
+#pragma unroll
+      for (int e = 0; e < V; ++e) *c[e] = out[e];
+    }
+  }
+#pragma unroll
+  for (int e = 0; e < V; ++e) skl_emit_requantised(p.rq, (T)out[e], row, col + e);
+  if (p.max && best > skl_lowest<T>()) skl_atomic_max(reinterpret_cast<T *>(p.max), best);
+}
+
+// The tiles of a launch. t / d is the high word of t * (2^32 / d + 1) as long as t * d < 2^32 (the remainder of 2^32 / d, at
+// most d, times t stays below 2^32).
+inline void set_tiles(MfmaArgs &p, unsigned tiles_m, unsigned tiles_n) {
+  p.tiles_m = tiles_m, p.tiles_n = tiles_n;
+  p.by_group = p.by_rest = 0;
+  const size_t total = (size_t)tiles_m * tiles_n, per_group = (size_t)8 * tiles_n, rest = tiles_m % 8 ? tiles_m % 8 : 8;
+  if (total < (size_t(1) << 31) && (total + 8) * per_group < (size_t(1) << 32)) {
+    p.by_group = (unsigned)((size_t(1) << 32) / per_group + 1);
+    p.by_rest = rest == 1 ? 0 : (unsigned)((size_t(1) << 32) / rest + 1);
+  }
+}
+
+template <typename T>
+int launch_split_reduce(const MfmaArgs &p, const char *who) {
+  const int v = p.n % 4 == 0 && ((uintptr_t)p.partial & 15) == 0 ? 4 : 1;
+  const size_t blocks = (p.m * (p.n / v) + 255) / 256;
+  if (blocks > 0x7FFFFFFFu) {
+    skl_hip_record_error(-2, "gemm_mfma: grid too large");
+    return -2;
+  }
+  if (v == 4)
+    gemm_split_reduce_kernel<T, 4><<<(unsigned)blocks, 256, 0, skl_current_stream()>>>(p);
+  else
+    gemm_split_reduce_kernel<T, 1><<<(unsigned)blocks, 256, 0, skl_current_stream()>>>(p);
+  return skl_check_launch(who);
 }
 
 struct SequenceGuard {
@@ -1794,24 +1913,26 @@ int launch_ring(const MfmaArgs &args) {
   kernel<<<(unsigned)grid, 512, lds, skl_current_stream()>>>(p);
   int rc = skl_check_launch("gemm_mfma_ring");
   if (rc != 0 || p.splits == 1) return rc;
-  const size_t blocks = (p.m * p.n + 255) / 256;
-  if (blocks > 0x7FFFFFFFu) {
-    skl_hip_record_error(-2, "gemm_mfma: grid too large");
-    return -2;
-  }
-  gemm_split_reduce_kernel<AccElem><<<(unsigned)blocks, 256, 0, skl_current_stream()>>>(p);
-  return skl_check_launch("gemm_split_reduce");
+  return launch_split_reduce<AccElem>(p, "gemm_split_reduce");
 }
 
-// How many ways K is shared out when a problem has too few tiles for the chip: enough to put about two
-// workgroups on every compute unit, each share at least kMinSlicesPerSplit slices long, planes within 64 MiB.
-// (Four slices: the reference's benchmark shapes of one 128 x 128 tile - 8192 k of int8, 4096 k of bf16 - 10.2 -> 8.9 us
-// and 10.0 -> 9.0 us against shares of eight; two slices measure the same.)
-constexpr size_t kMinSlicesPerSplit = 4, kSplitFromSlices = 32, kSplitPlaneLimit = size_t(64) << 20;
-inline unsigned splits_for(size_t tiles, size_t slices, size_t m, size_t n) {
-  if (tiles >= 256 || slices < kSplitFromSlices) return 1;
-  size_t want = (512 + tiles - 1) / tiles;
-  if (want > slices / kMinSlicesPerSplit) want = slices / kMinSlicesPerSplit;
+// How many ways K is shared out when a problem has too few tiles for the chip: each share at least kMinBytesPerSplit of K per
+// row, planes within 64 MiB. (512 bytes: the reference's benchmark shapes of one 128 x 128 tile - 8192 k of int8, 4096 k of
+// bf16 - 10.2 -> 8.9 us and 10.0 -> 9.0 us against twice that; half of it measures the same.) The pass over the planes costs
+// 3.5 us, so K is shared from 4 KiB on, and where few workgroups leave a slice's chain of latencies uncovered from 2 KiB, or
+// 1 KiB where fp8 is widened for exact products (us, whole / shared: bf16 32 x 320 x 1920 11.9 / 9.1, E4M3 97 x 1920 x 1280
+// 12.3 / 10.3; with more tiles the other way, f16 105 x 3712 x 1216 9.5 / 15.4). The number depends on nothing but the sizes
+// and the operand kind, so that a call gives the same sums with and without fused steps.
+constexpr size_t kMinBytesPerSplit = 512, kSplitFromBytes = 4096, kSplitEarlyTiles = 96, kSplitPlaneLimit = size_t(64) << 20;
+inline unsigned splits_for(size_t tiles, size_t slices, size_t m, size_t n, size_t slice, bool exact) {
+  const size_t from = tiles > kSplitEarlyTiles ? kSplitFromBytes : exact ? kSplitFromBytes / 4 : kSplitFromBytes / 2;
+  if (tiles >= 256 || slices * slice < from) return 1;
+  // 512 workgroups run at a time: a few more than that would be a round of their own. Of the larger problems' fewer are
+  // enough, and fewer planes.
+  size_t want = 512 / tiles;
+  if (!(slice == 256 && tiles < kSplitEarlyTiles) && want > (384 + tiles - 1) / tiles) want = (384 + tiles - 1) / tiles;
+  const size_t most = slices * slice / kMinBytesPerSplit;
+  if (want > most) want = most;
   while (want > 1 && want * m * n * 4 > kSplitPlaneLimit) --want;
   return (unsigned)(want < 1 ? 1 : want);
 }
@@ -1834,11 +1955,11 @@ int launch_one(const MfmaArgs &args) {
     configured.store(true, std::memory_order_release);
   }
   MfmaArgs p = args;
-  p.tiles_m = skl_div_up(p.m, BM);
-  p.tiles_n = skl_div_up(p.n, BN);
+  set_tiles(p, skl_div_up(p.m, BM), skl_div_up(p.n, BN));
   const size_t tiles = (size_t)p.tiles_m * p.tiles_n;
-  const size_t slices = (p.k * ES + kSliceBytes - 1) / kSliceBytes;
-  p.splits = splits_for(tiles, slices, p.m, p.n);
+  constexpr int kSlice = slice_bytes(BM);
+  const size_t slices = (p.k * ES + kSlice - 1) / kSlice;
+  p.splits = splits_for(tiles, slices, p.m, p.n, kSlice, EXACT);
   p.slices_per_split = (unsigned)((slices + p.splits - 1) / p.splits);
   p.splits = (unsigned)((slices + p.slices_per_split - 1) / p.slices_per_split);  // no empty share
   SequenceGuard sequence(p.splits > 1);  // the partial sums travel from this kernel to the next through the workspace
@@ -1846,22 +1967,15 @@ int launch_one(const MfmaArgs &args) {
     p.partial = (char *)skl_workspace((size_t)p.splits * p.m * p.n * 4);
     if (!p.partial) return -4;
   }
-  const size_t grid = tiles * p.splits;
-  if (grid > 0x7FFFFFFFu) {
+  if (tiles > 0x7FFFFFFFu || p.splits > 0xFFFFu) {
     skl_hip_record_error(-2, "gemm_mfma: grid too large");
     return -2;
   }
-  kernel<<<(unsigned)grid, NT, lds, skl_current_stream()>>>(p);
+  kernel<<<dim3((unsigned)tiles, p.splits), NT, lds, skl_current_stream()>>>(p);
   int rc = skl_check_launch("gemm_mfma");
   if (rc != 0 || p.splits == 1) return rc;
   using AccElem = decltype(typename Kind<TA>::Acc{}.x);
-  const size_t blocks = (p.m * p.n + 255) / 256;
-  if (blocks > 0x7FFFFFFFu) {
-    skl_hip_record_error(-2, "gemm_mfma: grid too large");
-    return -2;
-  }
-  gemm_split_reduce_kernel<AccElem><<<(unsigned)blocks, 256, 0, skl_current_stream()>>>(p);
-  return skl_check_launch("gemm_split_reduce");
+  return launch_split_reduce<AccElem>(p, "gemm_split_reduce");
 }
 
 // How well `tiles` workgroups, one at a time on each of the 256 compute units, fill the rounds they take, in per cent.
@@ -1985,6 +2099,23 @@ int launch_ragged(const MfmaArgs &p, int tile_cols) {
   return tile_cols == 256 ? launch_ring<TA, TB, A_KC, B_KC, 256, true>(p) : launch_ring<TA, TB, A_KC, B_KC, 128, true>(p);
 }
 
+// Whether the 64 x 64 tiles take a problem: where 128 x 128 ones are few - fewer than 128 as long as K is short and they are
+// not to be shared, fewer than 256 where C is read or there are steps behind the product, which one workgroup to a compute unit
+// leaves uncovered - and for the 16-bit kinds up to 64 rows of A, of which the larger tile would fetch and multiply as many
+// again that do not exist. Us, 128 x 128 / 64 x 64 tiles: int8 64 tiles of 128 x 128, 256 x 4096 x 1344 with GELU 24.8 / 13.2,
+// f16 448 x 1932 x 1024 reading C 20.0 / 11.1, int8 1664 x 1536 x 832 reading C 21.4 / 13.0; the other way, int8 256 x 11520 x 896
+// 8.9 / 11.2, E5M2 128 x 10240 x 12608 53 / 96.
+// (Their slices are up to 256 rows of an operand read across K: offsets inside a tile stay in 32 bits.)
+template <int ES, bool INT, bool A_KC, bool B_KC>
+bool small_tiles(const MfmaArgs &p) {
+  constexpr size_t limit = size_t(1) << 31;
+  if ((!A_KC && p.a_sk * ES * 256 >= limit) || (!B_KC && p.b_sk * ES * 256 >= limit)) return false;
+  const size_t large = skl_div_up(p.m, 128) * (size_t)skl_div_up(p.n, 128), k_bytes = p.k * ES;
+  if ((ES == 2 && p.m <= 64) || large < 64) return true;
+  const bool reads_c = INT ? p.beta.i != 0 : !(p.beta.fz.skip_c_read && p.beta.f == 0.0f);
+  return k_bytes < (large < 128 ? 5120 : large < 256 && (reads_c || p.rq.act || p.rq.q) ? 4096 : 0);
+}
+
 template <int TA, int TB, bool A_KC, bool B_KC>
 int launch_tile(const MfmaArgs &p) {
   constexpr int ES = Kind<TA>::ES;
@@ -1996,7 +2127,7 @@ int launch_tile(const MfmaArgs &p) {
     if (p.k <= kF8ExactMaxK) {
       const int rc = launch_whole_tiles<TA, TB, A_KC, B_KC, true>(p);
       if (rc != kNotWholeTiles) return rc;
-      if (skl_div_up(p.m, 128) * (size_t)skl_div_up(p.n, 128) < 64)
+      if (small_tiles<ES, TA == SKL_DT_I8, A_KC, B_KC>(p))
         return launch_one<TA, TB, A_KC, B_KC, 64, 64, 2, 2, true>(p);
       return launch_one<TA, TB, A_KC, B_KC, 128, 128, 2, 4, true>(p);
     }
@@ -2004,10 +2135,7 @@ int launch_tile(const MfmaArgs &p) {
   const int rc = launch_whole_tiles<TA, TB, A_KC, B_KC, false>(p);
   if (rc != kNotWholeTiles) return rc;
   if (const int cols = ragged_tile_cols<TA, TB, A_KC, B_KC>(p)) return launch_ragged<TA, TB, A_KC, B_KC>(p, cols);
-  // Small problems: 64 x 64 tiles put four times as many workgroups on the chip.
-  // ... and for the 16-bit kinds up to 64 rows of A: a 128-row tile would fetch and multiply rows that do not exist
-  // (bf16 64 x 11008 x 4096: 36 -> 28 us; the 8-bit kinds are faster on the larger tile, 23 against 25 us).
-  if ((ES == 2 && p.m <= 64) || skl_div_up(p.m, 128) * (size_t)skl_div_up(p.n, 128) < 64)
+  if (small_tiles<ES, TA == SKL_DT_I8, A_KC, B_KC>(p))
     return launch_one<TA, TB, A_KC, B_KC, 64, 64, 2, 2>(p);
   return launch_one<TA, TB, A_KC, B_KC, 128, 128, 2, 4>(p);
 }

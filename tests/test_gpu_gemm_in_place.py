@@ -10,6 +10,7 @@ import support
 from skl_amd import DeviceBuffer
 from gpu_support import run_fused_gemm, run_gemm
 from support import GemmCase, run_oracle_gemm
+from test_oracle_gemm import fused_expectation
 
 pytestmark = pytest.mark.gpu
 
@@ -121,3 +122,33 @@ def test_streaming_kernel_on_ragged_tiles(gpu, ta, k, a_rows, b_rows):
 @pytest.mark.parametrize("a_rows,b_rows", ((True, True), (False, True), (True, False)))
 def test_streaming_kernel_on_ragged_wide_tiles(gpu, ta, k, relu, a_rows, b_rows):
     ragged_large(gpu, ta, 3856, 3104, k, a_rows, b_rows, 0, relu)
+
+
+@pytest.mark.parametrize("ta", ("i8", "bf16", "f8e4m3"))
+@pytest.mark.parametrize("m,n,k,block", ((70, 90, 200, 0), (64, 128, 96, 0), (257, 300, 160, 0), (1029, 1040, 160, 0), (72, 92, 80, 2), (132, 200, 96, 4), (1032, 1040, 96, 4),
+                                         (40, 100, 4400, 0), (40, 101, 4400, 0)))
+def test_fused_steps_of_the_bounds_checked_kernels(gpu, ta, m, n, k, block):
+    """Tiles of 64 x 64 and 128 x 128 whose edges cut rows and columns, C row-major (`block` 0), by columns and in blocks of four rows,
+    reading C; K whole and shared. The call with bias alone is the anchor: the steps make of its C what the rules say, bit for bit."""
+    rng = np.random.default_rng(m + n + k)
+    bias = rng.integers(-999, 999, n).astype(np.int32) if ta == "i8" else rng.uniform(-4, 4, n).astype(np.float32)
+    start = np.array([-(1 << 31)], np.int32) if ta == "i8" else np.array([-np.inf], np.float32)
+    for by_columns in ((False,) if block else (False, True)):
+        if block:
+            n1 = n // block
+            case = GemmCase(ta, None, 2, -1, m0=4, n0=block, k0=1, m1=m // 4, n1=n1, k1=k, rsa0=k, csa0=0, rsa1=4 * k, csa1=1, rsb0=0, csb0=1, rsb1=n,
+                            csb1=block, rsc0=block, csc0=1, rsc1=4 * block * n1 + 2, csc1=4 * block)
+        else:
+            case = GemmCase(ta, None, 1, 1, m0=1, n0=1, k0=1, m1=m, n1=n, k1=k, rsa0=0, csa0=0, rsa1=k, csa1=1, rsb0=0, csb0=0, rsb1=n, csb1=1,
+                            rsc0=0, csc0=0, rsc1=1 if by_columns else n + 2, csc1=m + 1 if by_columns else 1)
+        kind = "rcprc" if block else "rc"
+        a, b, c = case.make_inputs(int(rng.integers(1 << 30)))
+        anchor, _ = run_fused_gemm(gpu, kind, case, a, b, c, bias, None, "device")
+        scales = (rng.uniform(0.5, 2.0, n) * 100.0 / float(np.abs(anchor.astype(np.float64)).max())).astype(np.float32)
+        for rsq, csq, only in ((n + (-n) % 4, 1, False), (n + 5, 1, True), (1, m + 5, False)):
+            rq = dict(q=np.full((m - 1) * rsq + (n - 1) * csq + 1, 0x55, np.int8), rsq=rsq, csq=csq, scale=scales, per_column=True, zero=3, only=only,
+                      format=0 if ta == "i8" else 2)
+            got, top, q = run_fused_gemm(gpu, kind, case, a, b, c, bias, start, "device", activation=1, requant=rq)
+            want_c, want_top, want_q = fused_expectation(case, anchor, None, start, activation=1, requant=rq)
+            assert np.array_equal(q, want_q) and top[0] == want_top[0], (by_columns, rsq, csq)
+            assert np.array_equal(got.view(np.uint8), (c if only else want_c).view(np.uint8)), (by_columns, rsq, csq)
