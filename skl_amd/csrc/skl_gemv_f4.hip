@@ -24,12 +24,16 @@
 // added in wave order: no sums between workgroups, no scratch, the same bits on every run.
 #include <hip/hip_runtime.h>
 
+#include <atomic>
+
 #include "skl_device.hpp"
 #include "skl_fp8.hpp"
+#include "skl_kcstream.hpp"
 
 namespace {
 
-typedef int v4i __attribute__((ext_vector_type(4)));
+using skl_kcstream::v2i;
+using skl_kcstream::v4i;
 typedef int v8i __attribute__((ext_vector_type(8)));
 typedef float v4f __attribute__((ext_vector_type(4)));
 typedef __bf16 v2bf __attribute__((ext_vector_type(2)));
@@ -70,6 +74,7 @@ __device__ __forceinline__ v8bf widen_e4m3(unsigned lo, unsigned hi) {
   return v8bf{p0.x, p0.y, p1.x, p1.y, p2.x, p2.y, p3.x, p3.y};
 }
 
+// K up to 2304 (and what does not fit gemv_f4_stream_kernel's offsets and scale space).
 // CG groups of 16 columns per workgroup: a wave's pieces of A serve CG instructions each. With one group, 16 rows of
 // A make every workgroup pull 64 KB of A through its L1 for 32 KB of weights (12.2 us for 16 x 4096 x 11008 against
 // 7.2 us for one row); four groups quarter that. Loads are clamped into the operands rather than guarded (a guard is
@@ -188,7 +193,7 @@ __global__ void __launch_bounds__(kWaves * 64) gemv_f4_kernel(F4Args p) {
   }
 }
 
-// 17 to 128 rows of A: the same decomposition with B held in registers for 4096 k (one pass of the K loop above:
+// 17 (33 beyond K = 2304) to 128 rows of A: the same decomposition with B held in registers for 4096 k (one pass of the K loop above:
 // four chunks per wave; a longer K takes one launch per 4096 k, the later ones adding to C) while up to eight groups of 16 rows take their turns - the 4-bit weights cross
 // HBM once and never exist as a converted copy (which cost 22.5 MB read, 45 MB written and a tile GEMM behind it:
 // 37 / 40 / 45 us for 32 / 64 / 128 x 4096 x 11008). Two groups of 16 columns per workgroup; a row group's pieces of A
@@ -307,6 +312,165 @@ __global__ void __launch_bounds__(kWaves * 64) gemv_f4_rows_kernel(F4Args p) {
   }
 }
 
+// Long K on the scaled instruction, up to 32 rows of A: the weights and A through LDS, a ring per wave, as skl_kcstream.hpp has
+// it. A unit is a line of every column, 256 k, and two lines of each row of A; lane group g takes the 32 k of B's piece 4 h + g and
+// the FP8 operand's pieces g and 4 + g of A's line h. The scales of all of K - a byte per 32 k and column, which a lane would
+// gather one by one - are put next to the ring first, eight bytes per unit and column, while the first units are under way.
+// us, operands and scales straight into registers / here: 4096 x 11008 with scales, 1 / 16 rows 8.4 / 6.5, 12.6 / 7.1, without
+// 7.0 / 5.7, 10.4 / 6.6; 11008 x 14336 with scales, 5 rows 35.9 / 17.3; 14336 x 1024, 12 rows 13.2 / 6.7.
+constexpr int kStreamRows = 32;
+constexpr size_t kScaleSpace = 32 * 1024;
+
+template <int RG, int CG, bool SCALED>
+__global__ void __launch_bounds__((skl_kcstream::Shape<RG, CG, 2>::kWaves * 64)) gemv_f4_stream_kernel(F4Args p) {
+  using Shape = skl_kcstream::Shape<RG, CG, 2>;
+  constexpr int kRingWaves = Shape::kWaves, kTileCols = 16 * CG, kPitch = Shape::kPitch, kThreads = kRingWaves * 64;
+  extern __shared__ __attribute__((aligned(1024))) char f4_ring[];
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
+  const int jl = lane & 15, g = lane >> 4;
+  const size_t col0 = (size_t)blockIdx.x * kTileCols;
+  const unsigned units = (unsigned)((p.k + 255) / 256), steps = (units + kRingWaves - 1) / kRingWaves;
+  const unsigned ring = (unsigned)(uintptr_t)(__attribute__((address_space(3))) char *)f4_ring, scales = ring + Shape::kRingBytes;
+  // The scales of 4096 k at a time, four to a lane, two columns to a wave and load; those of a column's end are loaded from
+  // further down and moved into place.
+  constexpr int kEach = kTileCols / (2 * kRingWaves);
+  const unsigned count = (unsigned)(p.k / 32);  // of a column: at least 4
+  const size_t cols_here = p.n - col0;
+  unsigned word[kEach];
+  auto load_scales = [&](unsigned block) {
+    const __amdgpu_buffer_rsrc_t rsrc = __builtin_amdgcn_make_buffer_rsrc((void *)(p.s + col0 * p.s_col), 0, (int)skl_kcstream::kRange, 0x00027000);
+    const unsigned d = block * 32 + (unsigned)(lane & 31), from = 4 * d + 4 <= count ? 4 * d : count - 4, over = 4 * d - from;
+#pragma unroll
+    for (int q = 0; q < kEach; ++q) {
+      const unsigned cl = (unsigned)(q * kRingWaves + wave) * 2u + (unsigned)(lane >> 5), col = cl < cols_here ? cl : (unsigned)cols_here - 1u;
+      const unsigned off = over < 4 ? col * (unsigned)p.s_col + from : skl_kcstream::kOutside;
+      word[q] = (unsigned)__builtin_amdgcn_raw_buffer_load_b32(rsrc, (int)off, 0, 0) >> ((8 * over) & 31);
+    }
+  };
+  auto keep_scales = [&](unsigned block) {
+    const unsigned d = block * 32 + (unsigned)(lane & 31);
+#pragma unroll
+    for (int q = 0; q < kEach; ++q) {
+      const unsigned cl = (unsigned)(q * kRingWaves + wave) * 2u + (unsigned)(lane >> 5);
+      // (spelled out: the compiler makes a store to LDS wait for the loads into LDS under way)
+      asm volatile("ds_write_b32 %0, %1" ::"v"(scales + ((d >> 1) * kTileCols + cl) * 8 + (d & 1) * 4), "v"(word[q]) : "memory");
+    }
+  };
+  if constexpr (SCALED) load_scales(0);
+  skl_kcstream::Requests<RG, 2> ra;
+  skl_kcstream::Requests<CG, 1> rb;
+  ra.template set<false>(p.a, p.a_row, p.m, (unsigned)p.k, lane);
+  rb.template set<true>(p.b + col0 * p.b_col, p.b_col, p.n - col0, (unsigned)(p.k / 2), lane);
+  __attribute__((address_space(3))) char *mine = (__attribute__((address_space(3))) char *)f4_ring + wave * Shape::kUnits * Shape::kUnitBytes;
+  const unsigned at0 = (unsigned)(uintptr_t)mine + (unsigned)jl * skl_kcstream::kLine + (unsigned)(g ^ (jl & 7)) * 16u;
+  auto request = [&](unsigned step) {
+    __attribute__((address_space(3))) char *to = mine + (step % Shape::kUnits) * Shape::kUnitBytes;
+    rb.template issue<2>(to, step * kRingWaves + (unsigned)wave);
+    ra.template issue<0>(to + 2048 * CG, step * kRingWaves + (unsigned)wave);
+  };
+  __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+  for (unsigned s = 0; s < (unsigned)Shape::kUnits; ++s) request(s);
+  __builtin_amdgcn_sched_barrier(0);
+  if constexpr (SCALED) {
+    keep_scales(0);
+    for (unsigned block = 1; block * 128 < count; ++block) {
+      load_scales(block);
+      keep_scales(block);
+    }
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+    __builtin_amdgcn_s_barrier();
+  }
+  v4f acc[RG][CG];
+#pragma unroll
+  for (int rg = 0; rg < RG; ++rg)
+#pragma unroll
+    for (int cg = 0; cg < CG; ++cg) acc[rg][cg] = v4f{0.0f, 0.0f, 0.0f, 0.0f};
+  for (unsigned step = 0; step < steps; ++step) {
+    skl_kcstream::wait_loads<(Shape::kUnits - 1) * Shape::kLoads>();
+    const unsigned at = at0 + (step % Shape::kUnits) * Shape::kUnitBytes, unit = step * kRingWaves + (unsigned)wave;
+    v2i sc[CG];
+    if constexpr (SCALED) skl_kcstream::read_scales<CG>(sc, scales + ((unit < units ? unit : 0u) * kTileCols + (unsigned)jl) * 8);
+    v4i a[2][2 * RG], b[2][CG];  // a[x][h * RG + rg]: the lane's piece x of line h
+    skl_kcstream::read_operands<CG, 2 * RG>(b[0], a[0], at, at + 2048 * CG);
+    skl_kcstream::read_operands<CG, 2 * RG>(b[1], a[1], at ^ 64u, (at ^ 64u) + 2048 * CG);
+    request(step + Shape::kUnits);
+#pragma unroll
+    for (int h = 0; h < 2; ++h)
+#pragma unroll
+      for (int cg = 0; cg < CG; ++cg) {
+        const int scale = SCALED ? (int)__builtin_amdgcn_ubfe((unsigned)(h ? sc[cg].y : sc[cg].x), 8u * (unsigned)g, 8u) : 127;
+        const v8i bv = {b[h][cg].x, b[h][cg].y, b[h][cg].z, b[h][cg].w, 0, 0, 0, 0};
+#pragma unroll
+        for (int rg = 0; rg < RG; ++rg) {
+          const v4i lo = a[0][h * RG + rg], hi = a[1][h * RG + rg];
+          const v8i av = {lo.x, lo.y, lo.z, lo.w, hi.x, hi.y, hi.z, hi.w};
+          // A: E4M3 (format 0) with scale 2^0, B: E2M1 (format 4) with this lane's scale for its 32 values
+          acc[rg][cg] = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(av, bv, acc[rg][cg], 0, 4, 0, 127, 0, scale);
+        }
+      }
+  }
+  skl_kcstream::wait_loads<0>();  // the requests behind the last unit write zeros into the ring
+  __syncthreads();
+  float(*red)[RG * 16][kPitch] = reinterpret_cast<float(*)[RG * 16][kPitch]>(f4_ring);
+#pragma unroll
+  for (int rg = 0; rg < RG; ++rg)
+#pragma unroll
+    for (int cg = 0; cg < CG; ++cg)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) red[wave][16 * rg + 4 * g + r][cg * 16 + jl] = acc[rg][cg][r];
+  __syncthreads();
+  const unsigned rows = p.m < (size_t)(16 * RG) ? (unsigned)p.m : (unsigned)(16 * RG);
+  for (unsigned at = threadIdx.x; at < rows * kTileCols; at += kThreads) {
+    const unsigned i = at / kTileCols, tc = at % kTileCols;
+    const size_t j = col0 + tc;
+    if (j >= p.n) continue;
+    float sum = red[0][i][tc];
+#pragma unroll
+    for (int w = 1; w < kRingWaves; ++w) sum = __fadd_rn(sum, red[w][i][tc]);
+    skl_update(sum, p.c + (size_t)i * p.c_row + j * p.c_col, p.alpha, p.beta);
+  }
+}
+
+template <int RG, int CG, bool SCALED>
+int launch_stream_as(const F4Args &p, unsigned grid) {
+  using Shape = skl_kcstream::Shape<RG, CG, 2>;
+  constexpr int kMost = Shape::kRingBytes + (SCALED ? (int)kScaleSpace : 0);
+  static std::atomic<bool> configured{false};  // per instantiation; racing threads set the same value
+  if (!configured.load(std::memory_order_acquire)) {
+    int rc = skl_check_hip(hipFuncSetAttribute(reinterpret_cast<const void *>(gemv_f4_stream_kernel<RG, CG, SCALED>),
+                                               hipFuncAttributeMaxDynamicSharedMemorySize, kMost), "gemv_f4_stream: LDS size");
+    if (rc != 0) return rc;
+    configured.store(true, std::memory_order_release);
+  }
+  const size_t bytes = (size_t)Shape::kRingBytes + (SCALED ? (p.k + 4095) / 4096 * 2048 * CG : 0);
+  gemv_f4_stream_kernel<RG, CG, SCALED><<<grid, Shape::kWaves * 64, bytes, skl_current_stream()>>>(p);
+  return skl_check_launch("gemv_f4_stream");
+}
+
+// Takes the problem if a workgroup's rows, columns and scales fit its offsets and LDS.
+bool streams(const F4Args &p) {
+  const size_t most = (size_t(1) << 31) - 4096, cg = (size_t)skl_kcstream::column_groups(p.n);
+  return p.m <= (size_t)kStreamRows && p.k > kExactMaxK && p.k <= most && p.a_row <= most / 32 && p.b_col <= most / 64 &&
+         (!p.s || ((p.k + 4095) / 4096 * 2048 * cg <= kScaleSpace && p.s_col <= most / 64));
+}
+
+int launch_stream(const F4Args &p) {
+  const int cg = skl_kcstream::column_groups(p.n);
+  const size_t grid = (p.n + 16 * (size_t)cg - 1) / (16 * (size_t)cg);
+  if (grid > 0x7FFFFFFFu) {
+    skl_hip_record_error(-2, "gemv_f4: grid too large");
+    return -2;
+  }
+#define SKL_F4_STREAM(RG, CG)                                                                             \
+  if (cg == CG && p.m <= 16 * RG)                                                                         \
+    return p.s ? launch_stream_as<RG, CG, true>(p, (unsigned)grid) : launch_stream_as<RG, CG, false>(p, (unsigned)grid);
+  SKL_F4_STREAM(1, 1) SKL_F4_STREAM(1, 2) SKL_F4_STREAM(1, 3) SKL_F4_STREAM(1, 4)
+  SKL_F4_STREAM(2, 1) SKL_F4_STREAM(2, 2) SKL_F4_STREAM(2, 3) SKL_F4_STREAM(2, 4)
+#undef SKL_F4_STREAM
+  return -2;
+}
+
 inline bool aligned16(const void *p) { return ((uintptr_t)p & 15) == 0; }
 
 }  // namespace
@@ -329,6 +493,9 @@ extern "C" int skl_hip_launch_gemv_f4(size_t m, size_t n, size_t k, skl_scalar a
     skl_hip_record_error(-2, "gemv_f4: unsupported problem");
     return -2;
   }
+  const int s_pairs = scales && (k % 64) == 0 && ((uintptr_t)scales & 1) == 0 && (n == 1 || (lds & 1) == 0);
+  const F4Args whole = {(const char *)a, rsa, (const char *)b, ldb / 2, scales, lds, s_pairs, c, rsc, csc, m, n, k, alpha, beta};
+  if (streams(whole)) return launch_stream(whole);
   if (m > (size_t)kMaxRows) {
     const size_t grid = (n + (size_t)kRowsCG * kCols - 1) / ((size_t)kRowsCG * kCols);
     if (grid > 0x7FFFFFFFu) {
@@ -371,8 +538,7 @@ extern "C" int skl_hip_launch_gemv_f4(size_t m, size_t n, size_t k, skl_scalar a
     skl_hip_record_error(-2, "gemv_f4: grid too large");
     return -2;
   }
-  const int s_pairs = scales && (k % 64) == 0 && ((uintptr_t)scales & 1) == 0 && (n == 1 || (lds & 1) == 0);
-  F4Args p = {(const char *)a, rsa, (const char *)b, ldb / 2, scales, lds, s_pairs, c, rsc, csc, m, n, k, alpha, beta};
+  const F4Args &p = whole;
   hipStream_t st = skl_current_stream();
   if (k <= kExactMaxK) {
     if (cg == 4) gemv_f4_kernel<true, 4><<<(unsigned)grid, kWaves * 64, 0, st>>>(p);
