@@ -73,11 +73,12 @@ __global__ void __launch_bounds__((skl_kcstream::Shape<RG, CG, 1>::kWaves * 64))
   };
 #pragma unroll
   for (unsigned s = 0; s < (unsigned)Shape::kUnits; ++s) request(s);
-  v4acc acc[RG][CG];
+  constexpr int kChains = KIND != kI8 && kWaves < 8 ? 2 : 1;  // eight sums per output, whatever the waves: shorter chains of roundings
+  v4acc acc2[kChains][RG][CG];
 #pragma unroll
   for (int rg = 0; rg < RG; ++rg)
 #pragma unroll
-    for (int cg = 0; cg < CG; ++cg) acc[rg][cg] = v4acc{0, 0, 0, 0};
+    for (int cg = 0; cg < CG; ++cg) acc2[0][rg][cg] = acc2[kChains - 1][rg][cg] = v4acc{0, 0, 0, 0};
   for (unsigned step = 0; step < steps; ++step) {
     skl_kcstream::wait_loads<(Shape::kUnits - 1) * Shape::kLoads>();
     const unsigned at = at0 + (step % Shape::kUnits) * Shape::kUnitBytes;
@@ -87,6 +88,7 @@ __global__ void __launch_bounds__((skl_kcstream::Shape<RG, CG, 1>::kWaves * 64))
     request(step + Shape::kUnits);
 #pragma unroll
     for (int h = 0; h < 2; ++h) {
+      auto &acc = acc2[h % kChains];
       if constexpr (KIND == kI8 || KIND == kBF16 || KIND == kF16) {
 #pragma unroll
         for (int rg = 0; rg < RG; ++rg)
@@ -121,14 +123,18 @@ __global__ void __launch_bounds__((skl_kcstream::Shape<RG, CG, 1>::kWaves * 64))
   }
   skl_kcstream::wait_loads<0>();  // the requests behind the last unit write zeros into the ring
   __syncthreads();
-  // acc[rg][cg][r] is row 16 rg + 4 g + r of C, column 16 cg + jl of the workgroup's.
+  // acc2[.][rg][cg][r] is row 16 rg + 4 g + r of C, column 16 cg + jl of the workgroup's.
   Acc(*red)[RG * 16][kPitch] = reinterpret_cast<Acc(*)[RG * 16][kPitch]>(kc_ring);
 #pragma unroll
   for (int rg = 0; rg < RG; ++rg)
 #pragma unroll
     for (int cg = 0; cg < CG; ++cg)
 #pragma unroll
-      for (int r = 0; r < 4; ++r) red[wave][16 * rg + 4 * g + r][cg * 16 + jl] = acc[rg][cg][r];
+      for (int r = 0; r < 4; ++r) {
+        Acc sum = acc2[0][rg][cg][r];
+        if constexpr (kChains == 2) sum = __fadd_rn(sum, acc2[1][rg][cg][r]);
+        red[wave][16 * rg + 4 * g + r][cg * 16 + jl] = sum;
+      }
   __syncthreads();
   const bool fused = p.bias || p.max || p.rq.act || p.rq.q;  // the same for every thread
   Acc largest = skl_lowest<Acc>();                           // what this thread wrote, for the maximum
