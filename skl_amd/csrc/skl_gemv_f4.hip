@@ -193,7 +193,8 @@ __global__ void __launch_bounds__(kWaves * 64) gemv_f4_kernel(F4Args p) {
   }
 }
 
-// 17 (33 beyond K = 2304) to 128 rows of A: the same decomposition with B held in registers for 4096 k (one pass of the K loop above:
+// 17 to 128 rows of A where K is at most 2304, or 65 rows and more of a wide B at most 4096 (and what gemv_f4_stream_kernel
+// cannot hold): the same decomposition with B held in registers for 4096 k (one pass of the K loop above:
 // four chunks per wave; a longer K takes one launch per 4096 k, the later ones adding to C) while up to eight groups of 16 rows take their turns - the 4-bit weights cross
 // HBM once and never exist as a converted copy (which cost 22.5 MB read, 45 MB written and a tile GEMM behind it:
 // 37 / 40 / 45 us for 32 / 64 / 128 x 4096 x 11008). Two groups of 16 columns per workgroup; a row group's pieces of A
@@ -312,13 +313,16 @@ __global__ void __launch_bounds__(kWaves * 64) gemv_f4_rows_kernel(F4Args p) {
   }
 }
 
-// Long K on the scaled instruction, up to 32 rows of A: the weights and A through LDS, a ring per wave, as skl_kcstream.hpp has
+// Long K on the scaled instruction, up to 128 rows of A: the weights and A through LDS, a ring per wave, as skl_kcstream.hpp has
 // it. A unit is a line of every column, 256 k, and two lines of each row of A; lane group g takes the 32 k of B's piece 4 h + g and
 // the FP8 operand's pieces g and 4 + g of A's line h. The scales of all of K - a byte per 32 k and column, which a lane would
 // gather one by one - are put next to the ring first, eight bytes per unit and column, while the first units are under way.
 // us, operands and scales straight into registers / here: 4096 x 11008 with scales, 1 / 16 rows 8.4 / 6.5, 12.6 / 7.1, without
-// 7.0 / 5.7, 10.4 / 6.6; 11008 x 14336 with scales, 5 rows 35.9 / 17.3; 14336 x 1024, 12 rows 13.2 / 6.7.
-constexpr int kStreamRows = 32;
+// 7.0 / 5.7, 10.4 / 6.6; 11008 x 14336 with scales, 5 rows 35.9 / 17.3; 14336 x 1024, 12 rows 13.2 / 6.7. Against B in registers:
+// 4096 x 11008 with scales, 20 / 48 rows 13.1 / 8.4, 16.9 / 13.4; 14336 x 4096, 33 rows 86.0 / 51.5, of which the exact last
+// 2048 k take two thirds.
+// More than 64 rows go to two workgroups per column tile, the second half of the grid for the rows from 64 on.
+constexpr int kStreamRowGroups = 4, kStreamRows = 2 * 16 * kStreamRowGroups;
 constexpr size_t kScaleSpace = 32 * 1024;
 
 template <int RG, int CG, bool SCALED>
@@ -328,7 +332,7 @@ __global__ void __launch_bounds__((skl_kcstream::Shape<RG, CG, 2>::kWaves * 64))
   extern __shared__ __attribute__((aligned(1024))) char f4_ring[];
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
   const int jl = lane & 15, g = lane >> 4;
-  const size_t col0 = (size_t)blockIdx.x * kTileCols;
+  const size_t col0 = (size_t)blockIdx.x * kTileCols, row0 = (size_t)blockIdx.y * (16 * RG);
   const unsigned units = (unsigned)((p.k + 255) / 256), steps = (units + kRingWaves - 1) / kRingWaves;
   const unsigned ring = (unsigned)(uintptr_t)(__attribute__((address_space(3))) char *)f4_ring, scales = ring + Shape::kRingBytes;
   // The scales of 4096 k at a time, four to a lane, two columns to a wave and load; those of a column's end are loaded from
@@ -359,7 +363,7 @@ __global__ void __launch_bounds__((skl_kcstream::Shape<RG, CG, 2>::kWaves * 64))
   if constexpr (SCALED) load_scales(0);
   skl_kcstream::Requests<RG, 2> ra;
   skl_kcstream::Requests<CG, 1> rb;
-  ra.template set<false>(p.a, p.a_row, p.m, (unsigned)p.k, lane);
+  ra.template set<false>(p.a + row0 * p.a_row, p.a_row, p.m - row0, (unsigned)p.k, lane);
   rb.template set<true>(p.b + col0 * p.b_col, p.b_col, p.n - col0, (unsigned)(p.k / 2), lane);
   __attribute__((address_space(3))) char *mine = (__attribute__((address_space(3))) char *)f4_ring + wave * Shape::kUnits * Shape::kUnitBytes;
   const unsigned at0 = (unsigned)(uintptr_t)mine + (unsigned)jl * skl_kcstream::kLine + (unsigned)(g ^ (jl & 7)) * 16u;
@@ -381,19 +385,21 @@ __global__ void __launch_bounds__((skl_kcstream::Shape<RG, CG, 2>::kWaves * 64))
     asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
     __builtin_amdgcn_s_barrier();
   }
-  v4f acc[RG][CG];
+  constexpr int kChains = kRingWaves == 2 ? 2 : 1;  // at least four sums per output: no longer a chain of roundings than four waves have
+  v4f acc[kChains][RG][CG];
 #pragma unroll
   for (int rg = 0; rg < RG; ++rg)
 #pragma unroll
-    for (int cg = 0; cg < CG; ++cg) acc[rg][cg] = v4f{0.0f, 0.0f, 0.0f, 0.0f};
+    for (int cg = 0; cg < CG; ++cg) acc[0][rg][cg] = acc[kChains - 1][rg][cg] = v4f{0.0f, 0.0f, 0.0f, 0.0f};
   for (unsigned step = 0; step < steps; ++step) {
     skl_kcstream::wait_loads<(Shape::kUnits - 1) * Shape::kLoads>();
     const unsigned at = at0 + (step % Shape::kUnits) * Shape::kUnitBytes, unit = step * kRingWaves + (unsigned)wave;
     v2i sc[CG];
     if constexpr (SCALED) skl_kcstream::read_scales<CG>(sc, scales + ((unit < units ? unit : 0u) * kTileCols + (unsigned)jl) * 8);
-    v4i a[2][2 * RG], b[2][CG];  // a[x][h * RG + rg]: the lane's piece x of line h
-    skl_kcstream::read_operands<CG, 2 * RG>(b[0], a[0], at, at + 2048 * CG);
-    skl_kcstream::read_operands<CG, 2 * RG>(b[1], a[1], at ^ 64u, (at ^ 64u) + 2048 * CG);
+    v4i a[2][2][RG], b[2][CG];  // a[h][x][rg]: the lane's piece x of line h
+    skl_kcstream::read_operands<CG, RG>(b[0], a[0][0], at, at + 2048 * CG);
+    skl_kcstream::read_operands<CG, RG>(b[1], a[0][1], at ^ 64u, (at ^ 64u) + 2048 * CG);
+    skl_kcstream::read_operands<RG, RG>(a[1][0], a[1][1], at + 2048 * (CG + RG), (at ^ 64u) + 2048 * (CG + RG));
     request(step + Shape::kUnits);
 #pragma unroll
     for (int h = 0; h < 2; ++h)
@@ -403,10 +409,10 @@ __global__ void __launch_bounds__((skl_kcstream::Shape<RG, CG, 2>::kWaves * 64))
         const v8i bv = {b[h][cg].x, b[h][cg].y, b[h][cg].z, b[h][cg].w, 0, 0, 0, 0};
 #pragma unroll
         for (int rg = 0; rg < RG; ++rg) {
-          const v4i lo = a[0][h * RG + rg], hi = a[1][h * RG + rg];
+          const v4i lo = a[h][0][rg], hi = a[h][1][rg];
           const v8i av = {lo.x, lo.y, lo.z, lo.w, hi.x, hi.y, hi.z, hi.w};
           // A: E4M3 (format 0) with scale 2^0, B: E2M1 (format 4) with this lane's scale for its 32 values
-          acc[rg][cg] = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(av, bv, acc[rg][cg], 0, 4, 0, 127, 0, scale);
+          acc[h % kChains][rg][cg] = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(av, bv, acc[h % kChains][rg][cg], 0, 4, 0, 127, 0, scale);
         }
       }
   }
@@ -418,9 +424,10 @@ __global__ void __launch_bounds__((skl_kcstream::Shape<RG, CG, 2>::kWaves * 64))
 #pragma unroll
     for (int cg = 0; cg < CG; ++cg)
 #pragma unroll
-      for (int r = 0; r < 4; ++r) red[wave][16 * rg + 4 * g + r][cg * 16 + jl] = acc[rg][cg][r];
+      for (int r = 0; r < 4; ++r)
+        red[wave][16 * rg + 4 * g + r][cg * 16 + jl] = kChains == 2 ? __fadd_rn(acc[0][rg][cg][r], acc[1][rg][cg][r]) : acc[0][rg][cg][r];
   __syncthreads();
-  const unsigned rows = p.m < (size_t)(16 * RG) ? (unsigned)p.m : (unsigned)(16 * RG);
+  const unsigned rows = p.m - row0 < (size_t)(16 * RG) ? (unsigned)(p.m - row0) : (unsigned)(16 * RG);
   for (unsigned at = threadIdx.x; at < rows * kTileCols; at += kThreads) {
     const unsigned i = at / kTileCols, tc = at % kTileCols;
     const size_t j = col0 + tc;
@@ -428,7 +435,7 @@ __global__ void __launch_bounds__((skl_kcstream::Shape<RG, CG, 2>::kWaves * 64))
     float sum = red[0][i][tc];
 #pragma unroll
     for (int w = 1; w < kRingWaves; ++w) sum = __fadd_rn(sum, red[w][i][tc]);
-    skl_update(sum, p.c + (size_t)i * p.c_row + j * p.c_col, p.alpha, p.beta);
+    skl_update(sum, p.c + (row0 + i) * p.c_row + j * p.c_col, p.alpha, p.beta);
   }
 }
 
@@ -444,14 +451,16 @@ int launch_stream_as(const F4Args &p, unsigned grid) {
     configured.store(true, std::memory_order_release);
   }
   const size_t bytes = (size_t)Shape::kRingBytes + (SCALED ? (p.k + 4095) / 4096 * 2048 * CG : 0);
-  gemv_f4_stream_kernel<RG, CG, SCALED><<<grid, Shape::kWaves * 64, bytes, skl_current_stream()>>>(p);
+  gemv_f4_stream_kernel<RG, CG, SCALED><<<dim3(grid, (unsigned)((p.m + 16 * RG - 1) / (16 * RG))), Shape::kWaves * 64, bytes, skl_current_stream()>>>(p);
   return skl_check_launch("gemv_f4_stream");
 }
 
-// Takes the problem if a workgroup's rows, columns and scales fit its offsets and LDS.
+// Takes the problem if a workgroup's rows, columns and scales fit its offsets and LDS. More than 64 rows of a wide B are two rounds of
+// workgroups, while the kernel with B in registers makes one up to K = 4096 (4096 x 11008, us here / there: 96 rows 25.8 / 23.7,
+// 128 rows 26.1 / 26.5; 4096 x 4096, 65 rows 12.9 / 17.9).
 bool streams(const F4Args &p) {
   const size_t most = (size_t(1) << 31) - 4096, cg = (size_t)skl_kcstream::column_groups(p.n);
-  return p.m <= (size_t)kStreamRows && p.k > kExactMaxK && p.k <= most && p.a_row <= most / 32 && p.b_col <= most / 64 &&
+  return p.m <= (size_t)kStreamRows && (p.m <= (size_t)(16 * kStreamRowGroups) || p.k > kRowsMaxK || p.n < 8192) && p.k > kExactMaxK && p.k <= most && p.a_row <= most / 64 && p.b_col <= most / 64 &&
          (!p.s || ((p.k + 4095) / 4096 * 2048 * cg <= kScaleSpace && p.s_col <= most / 64));
 }
 
@@ -463,10 +472,11 @@ int launch_stream(const F4Args &p) {
     return -2;
   }
 #define SKL_F4_STREAM(RG, CG)                                                                             \
-  if (cg == CG && p.m <= 16 * RG)                                                                         \
+  if (cg == CG && (p.m <= 16 * RG || RG == kStreamRowGroups))                                                                         \
     return p.s ? launch_stream_as<RG, CG, true>(p, (unsigned)grid) : launch_stream_as<RG, CG, false>(p, (unsigned)grid);
   SKL_F4_STREAM(1, 1) SKL_F4_STREAM(1, 2) SKL_F4_STREAM(1, 3) SKL_F4_STREAM(1, 4)
   SKL_F4_STREAM(2, 1) SKL_F4_STREAM(2, 2) SKL_F4_STREAM(2, 3) SKL_F4_STREAM(2, 4)
+  SKL_F4_STREAM(4, 1) SKL_F4_STREAM(4, 2) SKL_F4_STREAM(4, 3) SKL_F4_STREAM(4, 4)
 #undef SKL_F4_STREAM
   return -2;
 }
@@ -495,7 +505,17 @@ extern "C" int skl_hip_launch_gemv_f4(size_t m, size_t n, size_t k, skl_scalar a
   }
   const int s_pairs = scales && (k % 64) == 0 && ((uintptr_t)scales & 1) == 0 && (n == 1 || (lds & 1) == 0);
   const F4Args whole = {(const char *)a, rsa, (const char *)b, ldb / 2, scales, lds, s_pairs, c, rsc, csc, m, n, k, alpha, beta};
-  if (streams(whole)) return launch_stream(whole);
+  // More than 16 rows and K beyond 4096: a last part of at most 2304 k is multiplied exactly, in a pass of its own behind the stream,
+  // as the kernel with B in registers does with every K.
+  const size_t part = k % kRowsMaxK;
+  const size_t streamed = m > (size_t)kMaxRows && k > kRowsMaxK && part <= kExactMaxK ? k - part : k;
+  F4Args first = whole;
+  first.k = streamed;
+  const bool stream = streams(first);
+  if (stream) {
+    const int rc = launch_stream(first);
+    if (rc != 0 || streamed == k) return rc;
+  }
   if (m > (size_t)kMaxRows) {
     const size_t grid = (n + (size_t)kRowsCG * kCols - 1) / ((size_t)kRowsCG * kCols);
     if (grid > 0x7FFFFFFFu) {
@@ -506,7 +526,7 @@ extern "C" int skl_hip_launch_gemv_f4(size_t m, size_t n, size_t k, skl_scalar a
     const unsigned blocks = (unsigned)grid, threads = kWaves * 64;
     // A K beyond what the registers hold goes in passes of 4096 k: the first applies the caller's beta, the others
     // add to C (beta = 1) - launches on one stream, in order; the same bits on every run.
-    for (size_t k0 = 0; k0 < k; k0 += kRowsMaxK) {
+    for (size_t k0 = stream ? streamed : 0; k0 < k; k0 += kRowsMaxK) {
       const size_t kk = k - k0 < kRowsMaxK ? k - k0 : kRowsMaxK;
       skl_scalar pass_beta = beta;
       if (k0 != 0) pass_beta.fz.value = 1.0f, pass_beta.fz.skip_c_read = 0;

@@ -36,13 +36,13 @@ inline int column_groups(size_t n) {
 }
 
 // The ring's shape for RG groups of 16 rows, CG groups of 16 columns, and A_LINES lines of A per row and unit: eight waves
-// with at least two units each where 160 KiB hold that, else four.
+// with at least two units each where 160 KiB hold that, else four, else two.
 template <int RG, int CG, int A_LINES>
 struct Shape {
   static constexpr int kUnitBytes = 16 * (int)kLine * (CG + RG * A_LINES);
   static constexpr int kLoads = 2 * (CG + RG * A_LINES);  // per unit and wave
-  static constexpr int kWaves = A_LINES == 1 && 16 * kUnitBytes <= kMaxLds ? 8 : 4;
   static constexpr int kSpace = A_LINES == 1 ? kMaxLds : kMaxLds - 32 * 1024;  // 4-bit weights keep their scales next to the ring
+  static constexpr int kWaves = A_LINES == 1 && 16 * kUnitBytes <= kSpace ? 8 : 8 * kUnitBytes <= kSpace ? 4 : 2;
   static constexpr int kFit = kSpace / (kWaves * kUnitBytes);
   static constexpr int kUnits = kFit < 4 ? kFit : 4;
   static constexpr int kRingBytes = kWaves * kUnits * kUnitBytes;

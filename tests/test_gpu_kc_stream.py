@@ -73,9 +73,10 @@ def test_fused_steps_follow_the_plain_call(gpu, ta, act):
         assert np.all(np.abs(got[rows] - want) <= 4 * 2.0 ** -23 * np.abs(want) + 1e-37)
 
 
-# one to four column groups, the last one ragged; one and two row groups; K one block of scales beyond 2304, one beyond the 4096
+# one to four column groups, the last one ragged; one to four row groups, and two workgroups' rows; K one block of scales beyond 2304, one beyond the 4096
 # k whose scales are fetched at once, beyond what the scales' space holds (the kernel without it); columns of scales at every alignment
-@pytest.mark.parametrize("m,n,k", ((1, 1040, 2336), (16, 4100, 4128), (17, 12300, 2336), (32, 8200, 2400), (31, 260, 14368), (3, 37, 65568)))
+@pytest.mark.parametrize("m,n,k", ((1, 1040, 2336), (16, 4100, 4128), (17, 12300, 2336), (32, 8200, 2400), (31, 260, 14368), (3, 37, 65568),
+                                   (33, 8200, 2368), (64, 4100, 2592), (65, 1040, 4128), (128, 12290, 2336)))
 def test_block_scaled_4_bit_weights(gpu, m, n, k):
     """Inside the bound of the reference's fp8 GEMM test around the exact product of the decoded operands, without allowance."""
     for alpha, beta in ((1.0, 0.0), (-1.5, 0.5)):
