@@ -59,6 +59,7 @@ struct MfmaArgs {
   unsigned splits, slices_per_split;
   char *partial;
   bool a_loose = false, b_loose = false;  // bounds-checked kernel: the operand is off the 16-byte rule (Loader)
+  bool blocked_sums = false;              // 64 x 64 tiles: K is added up in blocks (see the kernel)
 };
 
 namespace {
@@ -916,6 +917,33 @@ __global__ void __launch_bounds__(WAVES_M *WAVES_N * 64, (BM == 64 ? 2 : 4)) gem
       __builtin_amdgcn_sched_barrier(0);  // the loads stay up here, not next to the stores that use them
     }
   };
+  // How the products of a floating-point kind are added up on the 64 x 64 tiles. Every product of the chain in `acc` rounds at the
+  // size of the sum so far, so one chain over a long K loses what short ones keep.
+  // blocked_sums, a K that the larger tile would share between workgroups: the products of two slices, 512 bytes of K as in the
+  // shortest share there is, are a sum of their own, and `sum` adds those (bf16 1024 x 1024 x 2048, error against 64 bits: one chain
+  // 2.7e-7, eight shares 1.0e-7, blocks 1.0e-7).
+  // (Not for the fp8 instructions: what they lose in aligning products, 1.3e-5, does not depend on the sums.)
+  constexpr bool kSums = BM == 64 && ES == 2;
+  [[maybe_unused]] Acc sum[kSums ? MI : 1][kSums ? NI : 1];
+  [[maybe_unused]] const auto settle = [&]() __attribute__((always_inline)) {
+    if constexpr (kSums) {
+#pragma unroll
+      for (int i = 0; i < MI; ++i)
+#pragma unroll
+        for (int j = 0; j < NI; ++j)
+#pragma unroll
+          for (int r = 0; r < 16; ++r) {
+            sum[i][j][r] = __fadd_rn(sum[i][j][r], acc[i][j][r]);
+            acc[i][j][r] = 0;
+          }
+    }
+  };
+  if constexpr (kSums) {
+#pragma unroll
+    for (int i = 0; i < MI; ++i)
+#pragma unroll
+      for (int j = 0; j < NI; ++j) sum[i][j] = acc[i][j];
+  }
   // Slice s is multiplied and, if there are `more`, the next one put into the other half of LDS, which every wave has left.
   const auto slice = [&](auto last, bool more, unsigned s, v4i (&next_a)[TileA::kPerThread], v4i (&next_b)[TileB::kPerThread]) __attribute__((always_inline)) {
     read_step(s, 0, 0);
@@ -942,16 +970,30 @@ __global__ void __launch_bounds__(WAVES_M *WAVES_N * 64, (BM == 64 ? 2 : 4)) gem
   };
   // The compiler counts the loads in flight along every path into a block: a loop with a way out after each slice, or around
   // one, makes it wait for the youngest of them. So the loop runs whole rounds of kAhead slices, up to the last kAhead + 1.
+  static_assert(!kSums || kAhead == 2, "a round is a block");
   unsigned s = 0;
   for (; s + kAhead + 1 < count; s += kAhead) {
     [&]<int... Us>(std::integer_sequence<int, Us...>) __attribute__((always_inline)) {
       (slice(std::false_type{}, true, s + Us, ra[(Us + 1) % kAhead], rb[(Us + 1) % kAhead]), ...);
     }(std::make_integer_sequence<int, kAhead>{});
+    if (kSums && p.blocked_sums) settle();
   }
   [&]<int... Us>(std::integer_sequence<int, Us...>) __attribute__((always_inline)) {
     (void)((slice(std::true_type{}, s + 1 < count, s, ra[(Us + 1) % kAhead], rb[(Us + 1) % kAhead]), ++s < count) && ...);
   }(std::make_integer_sequence<int, kAhead>{});
-  if (s < count) slice(std::true_type{}, false, s, ra[0], rb[0]);
+  if (s < count) {
+    if (kSums && p.blocked_sums) settle();
+    slice(std::true_type{}, false, s, ra[0], rb[0]);
+  }
+  if constexpr (kSums) {
+    if (p.blocked_sums) {
+      settle();
+#pragma unroll
+      for (int i = 0; i < MI; ++i)
+#pragma unroll
+        for (int j = 0; j < NI; ++j) acc[i][j] = sum[i][j];
+    }
+  }
 
   // Lane l of a 32x32 block holds column l%32 and rows 8*(r/4) + 4*(l/32) + r%4.
   if (p.splits > 1) {  // a share of K: the raw sums go to this split's M x N plane
@@ -1753,8 +1795,8 @@ __global__ void __launch_bounds__(256) gemm_split_reduce_kernel(MfmaArgs p) {
     bias[e] = p.bias ? reinterpret_cast<const T *>(p.bias)[col + e] : T(0);
     old[e] = init ? T(0) : *c[e];
   }
-  // Eight planes are requested before the first is used (one memory round trip per eight, not per plane); the
-  // sum still runs over the planes in order, starting from plane 0 itself.
+  // Eight planes are requested before the first is used (one memory round trip per eight, not per plane); they are added in
+  // order, the first nine to each other, then each eight by themselves: shorter chains of roundings than one over all planes.
   T sum[V];
   load(plane, sum);
   for (unsigned q0 = 1; q0 < p.splits; q0 += 8) {
@@ -1762,17 +1804,21 @@ __global__ void __launch_bounds__(256) gemm_split_reduce_kernel(MfmaArgs p) {
 #pragma unroll
     for (unsigned u = 0; u < 8; ++u)
       if (q0 + u < p.splits) load(plane + (size_t)(q0 + u) * mn, v[u]);
-#pragma unroll
-    for (unsigned u = 0; u < 8; ++u) {
-      if (q0 + u >= p.splits) continue;
+    const auto add = [](T (&to)[V], const T (&by)[V]) __attribute__((always_inline)) {
 #pragma unroll
       for (int e = 0; e < V; ++e) {
-        if constexpr (std::is_same<T, int>::value)
-          sum[e] = (int)((unsigned)sum[e] + (unsigned)v[u][e]);
-        else
-          sum[e] = __fadd_rn(sum[e], v[u][e]);
+        if constexpr (std::is_same<T, int>::value) to[e] = (int)((unsigned)to[e] + (unsigned)by[e]);
+        else to[e] = __fadd_rn(to[e], by[e]);
       }
+    };
+    if (q0 == 1) add(sum, v[0]);
+#pragma unroll
+    for (unsigned u = 1; u < 8; ++u) {
+      if (q0 + u >= p.splits) continue;
+      if (q0 == 1) add(sum, v[u]);
+      else add(v[0], v[u]);
     }
+    if (q0 != 1) add(sum, v[0]);
   }
   T best = skl_lowest<T>();
   Run out;
@@ -1916,21 +1962,27 @@ int launch_ring(const MfmaArgs &args) {
   return launch_split_reduce<AccElem>(p, "gemm_split_reduce");
 }
 
+constexpr size_t kMinBytesPerSplit = 512, kSplitFromBytes = 4096, kSplitEarlyTiles = 96, kSplitPlaneLimit = size_t(64) << 20;
+inline size_t bytes_in_lines(size_t k_bytes) { return (k_bytes + 127) / 128 * 128; }
+
 // How many ways K is shared out when a problem has too few tiles for the chip: each share at least kMinBytesPerSplit of K per
 // row, planes within 64 MiB. (512 bytes: the reference's benchmark shapes of one 128 x 128 tile - 8192 k of int8, 4096 k of
 // bf16 - 10.2 -> 8.9 us and 10.0 -> 9.0 us against twice that; half of it measures the same.) The pass over the planes costs
 // 3.5 us, so K is shared from 4 KiB on, and where few workgroups leave a slice's chain of latencies uncovered from 2 KiB, or
 // 1 KiB where fp8 is widened for exact products (us, whole / shared: bf16 32 x 320 x 1920 11.9 / 9.1, E4M3 97 x 1920 x 1280
-// 12.3 / 10.3; with more tiles the other way, f16 105 x 3712 x 1216 9.5 / 15.4). The number depends on nothing but the sizes
-// and the operand kind, so that a call gives the same sums with and without fused steps.
-constexpr size_t kMinBytesPerSplit = 512, kSplitFromBytes = 4096, kSplitEarlyTiles = 96, kSplitPlaneLimit = size_t(64) << 20;
-inline unsigned splits_for(size_t tiles, size_t slices, size_t m, size_t n, size_t slice, bool exact) {
-  const size_t from = tiles > kSplitEarlyTiles ? kSplitFromBytes : exact ? kSplitFromBytes / 4 : kSplitFromBytes / 2;
-  if (tiles >= 256 || slices * slice < from) return 1;
-  // 512 workgroups run at a time: a few more than that would be a round of their own. Of the larger problems' fewer are
-  // enough, and fewer planes.
+// 12.3 / 10.3; with more tiles the other way, f16 105 x 3712 x 1216 9.5 / 15.4).
+// 512 workgroups run at a time: a few more than that would be a round of their own, and of larger problems' fewer are enough,
+// with fewer planes. But a sum of rounded products is the more exact the more parts it is made of: `many`, the 16-bit kinds on the
+// 128 x 128 tiles, take the next number above 512 workgroups (bf16 300 x 4096 x 4096, six shares instead of four: error against
+// 64 bits 1.9e-7 -> 1.6e-7, 28 -> 31 us; 3648 x 320 x 13056 59 -> 73), and two shares also at 256 tiles, from 8 KiB of K on
+// (2001 x 2001 x 8192: 5.7e-7 -> 4.0e-7, 85 -> 97 us).
+inline unsigned splits_for(size_t tiles, size_t slices, size_t m, size_t n, size_t k_bytes, int slice, bool exact, bool many) {
+  const bool early = tiles <= kSplitEarlyTiles;
+  const size_t from = !early ? kSplitFromBytes : exact ? kSplitFromBytes / 4 : kSplitFromBytes / 2;
+  if (tiles >= 256 || slices * slice < from) return many && tiles == 256 && k_bytes >= 8192 ? 2 : 1;
   size_t want = 512 / tiles;
-  if (!(slice == 256 && tiles < kSplitEarlyTiles) && want > (384 + tiles - 1) / tiles) want = (384 + tiles - 1) / tiles;
+  if (many) want = (512 + tiles - 1) / tiles;
+  else if (!(slice == 256 && tiles < kSplitEarlyTiles) && want > (384 + tiles - 1) / tiles) want = (384 + tiles - 1) / tiles;
   const size_t most = slices * slice / kMinBytesPerSplit;
   if (want > most) want = most;
   while (want > 1 && want * m * n * 4 > kSplitPlaneLimit) --want;
@@ -1942,6 +1994,7 @@ int launch_one(const MfmaArgs &args) {
   if constexpr (!EXTRA) {  // calls with an activation or a requantised copy take the kernels that carry those steps
     if (args.rq.act || args.rq.q) return launch_one<TA, TB, A_KC, B_KC, BM, BN, WAVES_M, WAVES_N, EXACT, true>(args);
   }
+  using AccElem = decltype(typename Kind<TA>::Acc{}.x);
   constexpr int ES = Kind<TA>::ES;
   constexpr int NT = WAVES_M * WAVES_N * 64;
   constexpr int lds = 2 * (Tile<ES, BM, A_KC, NT>::kBytes + Tile<ES, BN, B_KC, NT>::kBytes);
@@ -1959,7 +2012,8 @@ int launch_one(const MfmaArgs &args) {
   const size_t tiles = (size_t)p.tiles_m * p.tiles_n;
   constexpr int kSlice = slice_bytes(BM);
   const size_t slices = (p.k * ES + kSlice - 1) / kSlice;
-  p.splits = splits_for(tiles, slices, p.m, p.n, kSlice, EXACT);
+  p.splits = splits_for(tiles, slices, p.m, p.n, p.k * ES, kSlice, EXACT, ES == 2 && BM == 128);
+  p.blocked_sums = bytes_in_lines(p.k * ES) >= kSplitFromBytes;
   p.slices_per_split = (unsigned)((slices + p.splits - 1) / p.splits);
   p.splits = (unsigned)((slices + p.slices_per_split - 1) / p.slices_per_split);  // no empty share
   SequenceGuard sequence(p.splits > 1);  // the partial sums travel from this kernel to the next through the workspace
@@ -1974,7 +2028,6 @@ int launch_one(const MfmaArgs &args) {
   kernel<<<dim3((unsigned)tiles, p.splits), NT, lds, skl_current_stream()>>>(p);
   int rc = skl_check_launch("gemm_mfma");
   if (rc != 0 || p.splits == 1) return rc;
-  using AccElem = decltype(typename Kind<TA>::Acc{}.x);
   return launch_split_reduce<AccElem>(p, "gemm_split_reduce");
 }
 
@@ -2102,9 +2155,10 @@ int launch_ragged(const MfmaArgs &p, int tile_cols) {
 // Whether the 64 x 64 tiles take a problem: where 128 x 128 ones are few - fewer than 128 as long as K is short and they are
 // not to be shared, fewer than 256 where C is read or there are steps behind the product, which one workgroup to a compute unit
 // leaves uncovered - and for the 16-bit kinds up to 64 rows of A, of which the larger tile would fetch and multiply as many
-// again that do not exist. Us, 128 x 128 / 64 x 64 tiles: int8 64 tiles of 128 x 128, 256 x 4096 x 1344 with GELU 24.8 / 13.2,
-// f16 448 x 1932 x 1024 reading C 20.0 / 11.1, int8 1664 x 1536 x 832 reading C 21.4 / 13.0; the other way, int8 256 x 11520 x 896
-// 8.9 / 11.2, E5M2 128 x 10240 x 12608 53 / 96.
+// again that do not exist. Where C and the steps decide, floating point has a K that neither tile shares (kSplitFromBytes), so that
+// the sums, which both then make in the same order, are the same with and without fused steps. Us, 128 x 128 / 64 x 64 tiles: int8
+// 64 tiles of 128 x 128, 256 x 4096 x 1344 with GELU 24.8 / 13.2, f16 448 x 1932 x 1024 reading C 20.0 / 11.1, int8 1664 x 1536 x 832
+// reading C 21.4 / 13.0; the other way, int8 256 x 11520 x 896 8.9 / 11.2, E5M2 128 x 10240 x 12608 53 / 96.
 // (Their slices are up to 256 rows of an operand read across K: offsets inside a tile stay in 32 bits.)
 template <int ES, bool INT, bool A_KC, bool B_KC>
 bool small_tiles(const MfmaArgs &p) {
@@ -2113,6 +2167,7 @@ bool small_tiles(const MfmaArgs &p) {
   const size_t large = skl_div_up(p.m, 128) * (size_t)skl_div_up(p.n, 128), k_bytes = p.k * ES;
   if ((ES == 2 && p.m <= 64) || large < 64) return true;
   const bool reads_c = INT ? p.beta.i != 0 : !(p.beta.fz.skip_c_read && p.beta.f == 0.0f);
+  if (!INT && large >= 128 && bytes_in_lines(k_bytes) >= kSplitFromBytes) return false;
   return k_bytes < (large < 128 ? 5120 : large < 256 && (reads_c || p.rq.act || p.rq.q) ? 4096 : 0);
 }
 
