@@ -28,6 +28,14 @@ static inline int skl_check_launch(const char *what) { return skl_check_hip(hipG
 
 static inline unsigned skl_div_up(size_t a, size_t b) { return (unsigned)((a + b - 1) / b); }
 
+// sum + part, with what the rounding of that addition loses carried in `lost` and taken off the next part (compensated
+// summation, Kahan 1965). An infinite or undefined loss is none: a sum that has become infinite or NaN stays what it is.
+__device__ __forceinline__ float skl_add_keeping_loss(float sum, float part, float &lost) {
+  const float y = __fsub_rn(part, lost), t = __fadd_rn(sum, y), l = __fsub_rn(__fsub_rn(t, sum), y);
+  lost = __builtin_fabsf(l) < __builtin_inff() ? l : 0.0f;
+  return t;
+}
+
 // ---------------------------------------------------------------------------
 // C = beta*C + alpha*acc for one element, as the reference's C computes it: two
 // products and a sum, each rounded on its own (the translation units are built

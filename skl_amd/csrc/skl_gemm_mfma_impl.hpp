@@ -809,12 +809,14 @@ __device__ __forceinline__ void tile_of_block(unsigned bid, const MfmaArgs &p, u
   tn = column;
 }
 
+enum Few { kFewRows = 1, kFewest = 2 };  // gemm_mfma_kernel's FEW
+
 // The kernel for ragged and small problems: any M, N and K, operands on any boundary. A problem of few tiles is bound by the
 // time from one slice to the next (requests, their memory latency, LDS, barrier), so several slices of loads are under way, and
 // the loads are never guarded (Loader). Guarded loads, a slice ahead -> this, us: int8 512^3 5.9 -> 5.0, bf16 16 x 11008 x 4096
 // 28.4 -> 23.7 with its second pass, int8 136 x 704 x 2207 51 -> 12.4 (no copy of A in front), f16 427 x 5901 x 1805 93 -> 33;
 // over 120 random problems 0.70.
-template <int TA, int TB, bool A_KC, bool B_KC, int BM, int BN, int WAVES_M, int WAVES_N, bool EXACT = false, bool EXTRA = false>
+template <int TA, int TB, bool A_KC, bool B_KC, int BM, int BN, int WAVES_M, int WAVES_N, bool EXACT = false, bool EXTRA = false, int FEW = 0>
 __global__ void __launch_bounds__(WAVES_M *WAVES_N * 64, (BM == 64 ? 2 : 4)) gemm_mfma_kernel(MfmaArgs p) {
   constexpr int NT = WAVES_M * WAVES_N * 64;
   using KA = Kind<TA>;
@@ -922,9 +924,13 @@ __global__ void __launch_bounds__(WAVES_M *WAVES_N * 64, (BM == 64 ? 2 : 4)) gem
   // blocked_sums, a K that the larger tile would share between workgroups: the products of two slices, 512 bytes of K as in the
   // shortest share there is, are a sum of their own, and `sum` adds those (bf16 1024 x 1024 x 2048, error against 64 bits: one chain
   // 2.7e-7, eight shares 1.0e-7, blocks 1.0e-7).
+  // FEW, a few rows in place of a streaming kernel, with sums as exact as its many short ones: half a slice is a block and, kFewest,
+  // what its addition to `sum` loses is carried along in `lost`: seven instructions per element and four products, for the rows
+  // that exist.
   // (Not for the fp8 instructions: what they lose in aligning products, 1.3e-5, does not depend on the sums.)
-  constexpr bool kSums = BM == 64 && ES == 2;
-  [[maybe_unused]] Acc sum[kSums ? MI : 1][kSums ? NI : 1];
+  constexpr bool kSums = BM == 64 && (EXACT || ES == 2);
+  static_assert(kSums || !FEW);
+  [[maybe_unused]] Acc sum[kSums ? MI : 1][kSums ? NI : 1], lost[FEW == kFewest ? MI : 1][FEW == kFewest ? NI : 1];
   [[maybe_unused]] const auto settle = [&]() __attribute__((always_inline)) {
     if constexpr (kSums) {
 #pragma unroll
@@ -938,11 +944,36 @@ __global__ void __launch_bounds__(WAVES_M *WAVES_N * 64, (BM == 64 ? 2 : 4)) gem
           }
     }
   };
+  [[maybe_unused]] const auto settle_rows = [&](auto from, auto to) __attribute__((always_inline)) {
+    if constexpr (FEW) {
+      static_assert(MI == 1 && NI == 1);
+#pragma unroll
+      for (int r = decltype(from)::value; r < decltype(to)::value; ++r) {
+        if constexpr (FEW == kFewest) {
+          float l = lost[0][0][r];
+          sum[0][0][r] = skl_add_keeping_loss(sum[0][0][r], acc[0][0][r], l);
+          lost[0][0][r] = l;
+        } else {
+          sum[0][0][r] = __fadd_rn(sum[0][0][r], acc[0][0][r]);
+        }
+        acc[0][0][r] = 0;
+      }
+    }
+  };
+  [[maybe_unused]] const auto settle_existing = [&]() __attribute__((always_inline)) {  // registers 0 to 3 hold rows 0 to 7 of the wave's, 4 to 7 rows 8 to 15
+    if (m0 + wm >= p.m) return;
+    settle_rows(std::integral_constant<int, 0>{}, std::integral_constant<int, 4>{});
+    if (p.m > 8) settle_rows(std::integral_constant<int, 4>{}, std::integral_constant<int, 8>{});
+    if (p.m > 16) settle_rows(std::integral_constant<int, 8>{}, std::integral_constant<int, 16>{});
+  };
   if constexpr (kSums) {
 #pragma unroll
     for (int i = 0; i < MI; ++i)
 #pragma unroll
-      for (int j = 0; j < NI; ++j) sum[i][j] = acc[i][j];
+      for (int j = 0; j < NI; ++j) {
+        sum[i][j] = acc[i][j];
+        if constexpr (FEW == kFewest) lost[i][j] = acc[i][j];
+      }
   }
   // Slice s is multiplied and, if there are `more`, the next one put into the other half of LDS, which every wave has left.
   const auto slice = [&](auto last, bool more, unsigned s, v4i (&next_a)[TileA::kPerThread], v4i (&next_b)[TileB::kPerThread]) __attribute__((always_inline)) {
@@ -953,7 +984,10 @@ __global__ void __launch_bounds__(WAVES_M *WAVES_N * 64, (BM == 64 ? 2 : 4)) gem
       if (more) advance(last, s + 1, next_a, next_b);
       __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-      for (int ks = 0; ks < kSteps; ++ks) products(ks);
+      for (int ks = 0; ks < kSteps; ++ks) {
+        products(ks);
+        if (FEW && ks % (kSteps / 2) == kSteps / 2 - 1) settle_existing();
+      }
     } else {
 #pragma unroll
       for (int ks = 0; ks < kSteps; ++ks) {
@@ -976,18 +1010,18 @@ __global__ void __launch_bounds__(WAVES_M *WAVES_N * 64, (BM == 64 ? 2 : 4)) gem
     [&]<int... Us>(std::integer_sequence<int, Us...>) __attribute__((always_inline)) {
       (slice(std::false_type{}, true, s + Us, ra[(Us + 1) % kAhead], rb[(Us + 1) % kAhead]), ...);
     }(std::make_integer_sequence<int, kAhead>{});
-    if (kSums && p.blocked_sums) settle();
+    if (kSums && !FEW && p.blocked_sums) settle();
   }
   [&]<int... Us>(std::integer_sequence<int, Us...>) __attribute__((always_inline)) {
     (void)((slice(std::true_type{}, s + 1 < count, s, ra[(Us + 1) % kAhead], rb[(Us + 1) % kAhead]), ++s < count) && ...);
   }(std::make_integer_sequence<int, kAhead>{});
   if (s < count) {
-    if (kSums && p.blocked_sums) settle();
+    if (kSums && !FEW && p.blocked_sums) settle();
     slice(std::true_type{}, false, s, ra[0], rb[0]);
   }
   if constexpr (kSums) {
-    if (p.blocked_sums) {
-      settle();
+    if (!FEW && p.blocked_sums) settle();
+    if (FEW || p.blocked_sums) {
 #pragma unroll
       for (int i = 0; i < MI; ++i)
 #pragma unroll
@@ -1965,19 +1999,33 @@ int launch_ring(const MfmaArgs &args) {
 constexpr size_t kMinBytesPerSplit = 512, kSplitFromBytes = 4096, kSplitEarlyTiles = 96, kSplitPlaneLimit = size_t(64) << 20;
 inline size_t bytes_in_lines(size_t k_bytes) { return (k_bytes + 127) / 128 * 128; }
 
+// A few rows of A, or columns of B, off the 16-byte rule, of a floating-point kind. Copied into aligned rows contiguous in K they
+// would be the streaming kernels' - fp8 also a decode batch, with K up to 4096 or against a wide B -, whose sums are many and short
+// and whose fp8 products are exact for any K. Read in place they keep both, on the 64 x 64 tiles: exact products, and sums
+// compensated up to four rows (or few columns), beyond that in blocks (us and error against 64 bits, copies / one chain of the fp8
+// instructions or of 16-bit products in place / this: E4M3 2 x 1755 x 3408 27.9, 7.4, 8.3 and 2.7e-8, 1.3e-5, 3.0e-8; E5M2 89 x 7045 x 3440
+// 100, 19.9, 25.3 and 4.7e-8, 9.0e-6, 4.5e-8; bf16 4 x 6614 x 1400 30.6, 10.7, 13.0 and 5.0e-8, 1.3e-7, 4.2e-8).
+template <int ES>
+bool few_off_rule(const MfmaArgs &p) {
+  if (!p.a_loose && !p.b_loose) return false;
+  if (p.n <= 8 && p.n < p.m) return true;
+  if (ES == 2) return p.m <= 4 || (p.m <= 16 && p.b_sk != 1);
+  return p.m <= 4 || (p.m <= 96 && p.n * p.k >= (size_t(1) << 20) && (p.k <= 4096 || p.n >= 8192));
+}
+
 // How many ways K is shared out when a problem has too few tiles for the chip: each share at least kMinBytesPerSplit of K per
 // row, planes within 64 MiB. (512 bytes: the reference's benchmark shapes of one 128 x 128 tile - 8192 k of int8, 4096 k of
 // bf16 - 10.2 -> 8.9 us and 10.0 -> 9.0 us against twice that; half of it measures the same.) The pass over the planes costs
 // 3.5 us, so K is shared from 4 KiB on, and where few workgroups leave a slice's chain of latencies uncovered from 2 KiB, or
 // 1 KiB where fp8 is widened for exact products (us, whole / shared: bf16 32 x 320 x 1920 11.9 / 9.1, E4M3 97 x 1920 x 1280
-// 12.3 / 10.3; with more tiles the other way, f16 105 x 3712 x 1216 9.5 / 15.4).
+// 12.3 / 10.3; with more tiles the other way, f16 105 x 3712 x 1216 9.5 / 15.4), as are exact products of a longer K.
 // 512 workgroups run at a time: a few more than that would be a round of their own, and of larger problems' fewer are enough,
 // with fewer planes. But a sum of rounded products is the more exact the more parts it is made of: `many`, the 16-bit kinds on the
 // 128 x 128 tiles, take the next number above 512 workgroups (bf16 300 x 4096 x 4096, six shares instead of four: error against
 // 64 bits 1.9e-7 -> 1.6e-7, 28 -> 31 us; 3648 x 320 x 13056 59 -> 73), and two shares also at 256 tiles, from 8 KiB of K on
 // (2001 x 2001 x 8192: 5.7e-7 -> 4.0e-7, 85 -> 97 us).
 inline unsigned splits_for(size_t tiles, size_t slices, size_t m, size_t n, size_t k_bytes, int slice, bool exact, bool many) {
-  const bool early = tiles <= kSplitEarlyTiles;
+  const bool early = tiles <= kSplitEarlyTiles || (exact && k_bytes > kF8ExactMaxK);
   const size_t from = !early ? kSplitFromBytes : exact ? kSplitFromBytes / 4 : kSplitFromBytes / 2;
   if (tiles >= 256 || slices * slice < from) return many && tiles == 256 && k_bytes >= 8192 ? 2 : 1;
   size_t want = 512 / tiles;
@@ -1989,16 +2037,24 @@ inline unsigned splits_for(size_t tiles, size_t slices, size_t m, size_t n, size
   return (unsigned)(want < 1 ? 1 : want);
 }
 
-template <int TA, int TB, bool A_KC, bool B_KC, int BM, int BN, int WAVES_M, int WAVES_N, bool EXACT = false, bool EXTRA = false>
+template <int TA, int TB, bool A_KC, bool B_KC, int BM, int BN, int WAVES_M, int WAVES_N, bool EXACT = false, bool EXTRA = false, int FEW = 0>
 int launch_one(const MfmaArgs &args) {
   if constexpr (!EXTRA) {  // calls with an activation or a requantised copy take the kernels that carry those steps
     if (args.rq.act || args.rq.q) return launch_one<TA, TB, A_KC, B_KC, BM, BN, WAVES_M, WAVES_N, EXACT, true>(args);
+  }
+  if constexpr (!FEW && BM == 64 && (EXACT || Kind<TA>::ES == 2)) {
+    if (few_off_rule<Kind<TA>::ES>(args) && (args.m <= 4 || args.n <= 8))
+      return launch_one<TA, TB, A_KC, B_KC, BM, BN, WAVES_M, WAVES_N, EXACT, EXTRA, kFewest>(args);
+    if constexpr (Kind<TA>::ES == 2) {
+      if (few_off_rule<2>(args))
+        return launch_one<TA, TB, A_KC, B_KC, BM, BN, WAVES_M, WAVES_N, EXACT, EXTRA, kFewRows>(args);
+    }
   }
   using AccElem = decltype(typename Kind<TA>::Acc{}.x);
   constexpr int ES = Kind<TA>::ES;
   constexpr int NT = WAVES_M * WAVES_N * 64;
   constexpr int lds = 2 * (Tile<ES, BM, A_KC, NT>::kBytes + Tile<ES, BN, B_KC, NT>::kBytes);
-  auto kernel = gemm_mfma_kernel<TA, TB, A_KC, B_KC, BM, BN, WAVES_M, WAVES_N, EXACT, EXTRA>;
+  auto kernel = gemm_mfma_kernel<TA, TB, A_KC, B_KC, BM, BN, WAVES_M, WAVES_N, EXACT, EXTRA, FEW>;
   static std::atomic<bool> configured{false};  // per instantiation; racing threads set the same value
   if (!configured.load(std::memory_order_acquire)) {
     int rc = skl_check_hip(hipFuncSetAttribute(reinterpret_cast<const void *>(kernel),
@@ -2013,7 +2069,7 @@ int launch_one(const MfmaArgs &args) {
   constexpr int kSlice = slice_bytes(BM);
   const size_t slices = (p.k * ES + kSlice - 1) / kSlice;
   p.splits = splits_for(tiles, slices, p.m, p.n, p.k * ES, kSlice, EXACT, ES == 2 && BM == 128);
-  p.blocked_sums = bytes_in_lines(p.k * ES) >= kSplitFromBytes;
+  p.blocked_sums = few_off_rule<ES>(p) || bytes_in_lines(p.k * ES) >= kSplitFromBytes;
   p.slices_per_split = (unsigned)((slices + p.splits - 1) / p.splits);
   p.splits = (unsigned)((slices + p.slices_per_split - 1) / p.slices_per_split);  // no empty share
   SequenceGuard sequence(p.splits > 1);  // the partial sums travel from this kernel to the next through the workspace
@@ -2165,7 +2221,7 @@ bool small_tiles(const MfmaArgs &p) {
   constexpr size_t limit = size_t(1) << 31;
   if ((!A_KC && p.a_sk * ES * 256 >= limit) || (!B_KC && p.b_sk * ES * 256 >= limit)) return false;
   const size_t large = skl_div_up(p.m, 128) * (size_t)skl_div_up(p.n, 128), k_bytes = p.k * ES;
-  if ((ES == 2 && p.m <= 64) || large < 64) return true;
+  if ((ES == 2 && p.m <= 64) || large < 64 || (!INT && few_off_rule<ES>(p))) return true;
   const bool reads_c = INT ? p.beta.i != 0 : !(p.beta.fz.skip_c_read && p.beta.f == 0.0f);
   if (!INT && large >= 128 && bytes_in_lines(k_bytes) >= kSplitFromBytes) return false;
   return k_bytes < (large < 128 ? 5120 : large < 256 && (reads_c || p.rq.act || p.rq.q) ? 4096 : 0);
@@ -2179,8 +2235,8 @@ int launch_tile(const MfmaArgs &p) {
     // short K: exact products (see MmaF8Exact), on the streaming kernel when its tiles fill the chip and ring_pays() (us,
     // bounds-checked 128 x 128 / streaming: 2048 x 8192 x 2048 77 / 62, with GELU into E4M3 111 / 94; 2048 x 4096 x 2048
     // 42 / 34; on 128 tiles, 512 x 8192 x 2048, 25.4 / 26.2)
-    if (p.k <= kF8ExactMaxK) {
-      const int rc = launch_whole_tiles<TA, TB, A_KC, B_KC, true>(p);
+    if (p.k <= kF8ExactMaxK || few_off_rule<ES>(p)) {
+      const int rc = launch_whole_tiles<TA, TB, A_KC, B_KC, true>(p);  // (not of operands off the 16-byte rule)
       if (rc != kNotWholeTiles) return rc;
       if (small_tiles<ES, TA == SKL_DT_I8, A_KC, B_KC>(p))
         return launch_one<TA, TB, A_KC, B_KC, 64, 64, 2, 2, true>(p);

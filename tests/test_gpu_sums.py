@@ -60,3 +60,35 @@ def test_fused_steps_on_the_sums_of_the_plain_call(gpu, ta, k):
     assert np.array_equal(run_fused_gemm(*args, activation=1)[0], np.maximum(anchor, 0))
     rq = dict(q=np.zeros(m * n, np.int8), rsq=n, csq=1, scale=np.ones(1, np.float32), per_column=False, zero=0, only=False, format=0)
     assert np.array_equal(run_fused_gemm(*args, requant=rq)[0], anchor)
+
+
+# B or A off the 16-byte rule: one row, a few, the most that count as few, and few columns; K beyond the fp8 kinds' exact products.
+# `roundings`: one per eight products of a block, one per block unless their sum is compensated, one per share of K.
+@pytest.mark.parametrize("ta,m,n,k,roundings", (("f8e4m3", 2, 1755, 3408, 16 + 1 + 7), ("f8e4m3", 89, 705, 3441, 64 + 1 + 7), ("f8e5m2", 1, 91, 2425, 16 + 1 + 5),
+                                                ("f8e4m3", 300, 5, 4801, 16 + 1 + 9), ("bf16", 1, 1957, 593, 8 + 1 + 1), ("bf16", 4, 6614, 1401, 8 + 1 + 1),
+                                                ("bf16", 9, 333, 4097, 8 + 4 + 16), ("f16", 16, 1157, 2817, 8 + 4 + 11)))
+def test_few_rows_off_the_16_byte_rule_keep_exact_products_and_short_sums(gpu, ta, m, n, k, roundings):
+    a, b = operands(ta, m, n, k)
+    got = product(gpu, ta, a, b)
+    widen = support.ETYPES[ta].widen
+    exact = widen(a) @ widen(b)
+    assert np.linalg.norm(got - exact) <= 2.0 ** -24 / np.sqrt(3) * np.sqrt(roundings / 2) * np.linalg.norm(exact)
+
+
+@pytest.mark.parametrize("ta", ("bf16", "f16", "f8e4m3"))
+def test_few_rows_with_infinities_and_nan(gpu, ta):
+    """An infinite sum stays infinite, also when finite blocks of K follow it; opposite infinities and NaN give NaN."""
+    m, n, k = 3, 33, 1025
+    a, b = operands(ta, m, n, k)
+    big = {"bf16": 0x7F80, "f16": 0x7C00}.get(ta)
+    if big is None:
+        a[:, 5], nan = 0x7F, True          # E4M3 has no infinity: NaN
+    else:
+        one = support.ETYPES[ta]
+        b[5], b[700], nan = (0x3F80 if ta == "bf16" else 0x3C00), (0x3F80 if ta == "bf16" else 0x3C00), False
+        a[0, 5], a[1, 5], a[1, 700] = big, big, big | 0x8000
+    got = product(gpu, ta, a, b)
+    if nan:
+        assert np.isnan(got).all()
+    else:
+        assert np.isposinf(got[0]).all() and np.isnan(got[1]).all() and np.isfinite(got[2]).all()
