@@ -73,12 +73,28 @@ __global__ void __launch_bounds__((skl_kcstream::Shape<RG, CG, 1>::kWaves * 64))
   };
 #pragma unroll
   for (unsigned s = 0; s < (unsigned)Shape::kUnits; ++s) request(s);
-  constexpr int kChains = KIND != kI8 && kWaves < 8 ? 2 : 1;  // eight sums per output, whatever the waves: shorter chains of roundings
+  // Floating point: the units of a block of products (settle()). Up to 16 rows every unit is one, and what the sum over the waves
+  // loses is carried along, so that few rows are as exact as by the dot products of skl_gemv.hip; beyond that every four, or, with half
+  // as many waves, every eight in two sums (error against 64 bits, one chain per wave / blocks: bf16 2 x 4096 x 14336 2.5e-7 / 1.1e-7,
+  // 16 x 11008 x 4096 1.4e-7 / 7.8e-8, 96 x 11008 x 4096 1.3e-7 / 1.0e-7, E4M3 16 x 11008 x 14336 5.8e-8 / 3.7e-8; 29.3 -> 31.0 us for the 96
+  // rows, nothing for 16).
+  constexpr int kChains = KIND != kI8 && RG > 1 && kWaves < 8 && RG * CG < 24 ? 2 : 1;  // (6 x 4 groups leave no registers for two)
+  constexpr unsigned kBlock = RG == 1 ? 1 : 4 * kChains;
   v4acc acc2[kChains][RG][CG];
+  [[maybe_unused]] v4acc sums[KIND == kI8 ? 1 : RG][CG];
 #pragma unroll
   for (int rg = 0; rg < RG; ++rg)
 #pragma unroll
-    for (int cg = 0; cg < CG; ++cg) acc2[0][rg][cg] = acc2[kChains - 1][rg][cg] = v4acc{0, 0, 0, 0};
+    for (int cg = 0; cg < CG; ++cg) {
+      acc2[0][rg][cg] = acc2[kChains - 1][rg][cg] = v4acc{0, 0, 0, 0};
+      if constexpr (KIND != kI8) sums[rg][cg] = acc2[0][rg][cg];
+    }
+  [[maybe_unused]] const auto settle_all = [&]() __attribute__((always_inline)) {
+    if constexpr (KIND != kI8) {
+#pragma unroll
+      for (int c = 0; c < kChains; ++c) skl_kcstream::settle(sums, acc2[c]);
+    }
+  };
   for (unsigned step = 0; step < steps; ++step) {
     skl_kcstream::wait_loads<(Shape::kUnits - 1) * Shape::kLoads>();
     const unsigned at = at0 + (step % Shape::kUnits) * Shape::kUnitBytes;
@@ -120,10 +136,14 @@ __global__ void __launch_bounds__((skl_kcstream::Shape<RG, CG, 1>::kWaves * 64))
         }
       }
     }
+    if constexpr (KIND != kI8) {
+      if (step % kBlock == kBlock - 1) settle_all();
+    }
   }
+  if constexpr (KIND != kI8 && kBlock != 1) settle_all();
   skl_kcstream::wait_loads<0>();  // the requests behind the last unit write zeros into the ring
   __syncthreads();
-  // acc2[.][rg][cg][r] is row 16 rg + 4 g + r of C, column 16 cg + jl of the workgroup's.
+  // acc2[0][rg][cg][r], or sums[rg][cg][r], is row 16 rg + 4 g + r of C, column 16 cg + jl of the workgroup's.
   Acc(*red)[RG * 16][kPitch] = reinterpret_cast<Acc(*)[RG * 16][kPitch]>(kc_ring);
 #pragma unroll
   for (int rg = 0; rg < RG; ++rg)
@@ -131,9 +151,8 @@ __global__ void __launch_bounds__((skl_kcstream::Shape<RG, CG, 1>::kWaves * 64))
     for (int cg = 0; cg < CG; ++cg)
 #pragma unroll
       for (int r = 0; r < 4; ++r) {
-        Acc sum = acc2[0][rg][cg][r];
-        if constexpr (kChains == 2) sum = __fadd_rn(sum, acc2[1][rg][cg][r]);
-        red[wave][16 * rg + 4 * g + r][cg * 16 + jl] = sum;
+        if constexpr (KIND == kI8) red[wave][16 * rg + 4 * g + r][cg * 16 + jl] = acc2[0][rg][cg][r];
+        else red[wave][16 * rg + 4 * g + r][cg * 16 + jl] = sums[rg][cg][r];
       }
   __syncthreads();
   const bool fused = p.bias || p.max || p.rq.act || p.rq.q;  // the same for every thread
@@ -145,9 +164,11 @@ __global__ void __launch_bounds__((skl_kcstream::Shape<RG, CG, 1>::kWaves * 64))
     const size_t j = col0 + tc;
     if (j >= p.n) continue;
     Acc sum = red[0][i][tc];
+    [[maybe_unused]] Acc loss = 0;
 #pragma unroll
     for (int w = 1; w < kWaves; ++w) {
       if constexpr (KIND == kI8) sum = (int)((unsigned)sum + (unsigned)red[w][i][tc]);
+      else if constexpr (RG == 1) sum = skl_add_keeping_loss(sum, red[w][i][tc], loss);
       else sum = __fadd_rn(sum, red[w][i][tc]);
     }
     Acc *c = cbase + (size_t)i * p.c_row + j * p.c_col;

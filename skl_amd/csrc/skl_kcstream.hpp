@@ -141,6 +141,21 @@ struct Requests {
   }
 };
 
+// Every product of a matrix-core instruction rounds at the size of the sum it is added to, so one chain over a wave's share of a
+// long K loses what short chains keep. The products of a few units are a block of their own; here it is added to the running
+// sums and starts again from zero.
+template <typename V, int RG, int CG>
+__device__ __forceinline__ void settle(V (&sum)[RG][CG], V (&block)[RG][CG]) {
+#pragma unroll
+  for (int rg = 0; rg < RG; ++rg)
+#pragma unroll
+    for (int cg = 0; cg < CG; ++cg) {
+#pragma unroll
+      for (int r = 0; r < 4; ++r) sum[rg][cg][r] = __fadd_rn(sum[rg][cg][r], block[rg][cg][r]);
+      block[rg][cg] = V{0, 0, 0, 0};
+    }
+}
+
 // Waits until at most N of the wave's loads are under way.
 template <int N>
 __device__ __forceinline__ void wait_loads() {

@@ -5,7 +5,7 @@ import pytest
 
 import support
 from gpu_support import run_fused_gemm, run_gemm
-from support import rowmajor_case
+from support import GemmCase, rowmajor_case
 
 pytestmark = pytest.mark.gpu
 
@@ -92,3 +92,27 @@ def test_few_rows_with_infinities_and_nan(gpu, ta):
         assert np.isnan(got).all()
     else:
         assert np.isposinf(got[0]).all() and np.isnan(got[1]).all() and np.isfinite(got[2]).all()
+
+
+def k_contiguous_product(gpu, ta, a, bt):
+    """A * B with B stored column by column."""
+    (m, k), n = a.shape, bt.shape[0]
+    case = GemmCase(ta, None, 1.0, 0.0, m0=1, n0=1, k0=1, m1=m, n1=n, k1=k, rsa0=0, csa0=0, rsa1=k, csa1=1, rsb0=0, csb0=0, rsb1=1, csb1=k,
+                    rsc0=0, csc0=0, rsc1=n, csc1=1)
+    return run_gemm(gpu, "rc", case, a.reshape(-1), bt.reshape(-1), np.zeros(m * n, np.float32), "device").reshape(m, n)
+
+
+# few rows: blocks of 128 bytes of K in eight waves; many: of 512 bytes in eight or four; fp8 with K beyond 4096 and beyond the
+# exact products of the tile kernels, on a chip not full of workgroups
+@pytest.mark.parametrize("ta,m,n,k", (("bf16", 2, 64, 14336), ("bf16", 4, 4112, 4096), ("f16", 16, 1024, 8192), ("bf16", 20, 3072, 8192), ("f16", 70, 4096, 4096),
+                                      ("f8e4m3", 4, 4112, 8192), ("f8e4m3", 16, 8208, 14336), ("f8e5m2", 48, 9168, 8192), ("f8e4m3", 96, 8208, 4096)))
+def test_k_contiguous_decode_batches_add_up_blocks(gpu, ta, m, n, k):
+    rng = np.random.default_rng(m + n + k)
+    gen, widen = support.ETYPES[ta].gen, support.ETYPES[ta].widen
+    a, bt = gen(rng, m * k).reshape(m, k), gen(rng, n * k).reshape(n, k)
+    got = k_contiguous_product(gpu, ta, a, bt)
+    exact = widen(a) @ widen(bt).T
+    line = 128 if ta.startswith("f8") else 64
+    block, waves = (line if m <= 16 else 4 * line), (8 if m <= 32 else 4)
+    roundings = block / 8 + k / waves / block + waves
+    assert np.linalg.norm(got - exact) <= 2.0 ** -24 / np.sqrt(3) * np.sqrt(roundings / 2) * np.linalg.norm(exact)
