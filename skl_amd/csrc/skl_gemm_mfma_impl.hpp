@@ -2012,6 +2012,13 @@ bool few_off_rule(const MfmaArgs &p) {
   if (ES == 2) return p.m <= 4 || (p.m <= 16 && p.b_sk != 1);
   return p.m <= 4 || (p.m <= 96 && p.n * p.k >= (size_t(1) << 20) && (p.k <= 4096 || p.n >= 8192));
 }
+// Decode batches of the 16-bit kinds with a short K, from 1 MiB of B on: what the streaming kernel for operands with K contiguous
+// leaves to the tiles. Their sums are as short chains there: half slices up to 2816 bytes of K, where those become more than two
+// slices to a block are, then blocks.
+constexpr size_t kHalfSlicesBelow = 2816;
+inline bool short_decode_batch(const MfmaArgs &p, size_t k_bytes) {
+  return p.a_sk == 1 && p.b_sk == 1 && p.m > 4 && p.m <= 96 && k_bytes * p.n >= (size_t(1) << 20) && bytes_in_lines(k_bytes) < kSplitFromBytes;
+}
 
 // How many ways K is shared out when a problem has too few tiles for the chip: each share at least kMinBytesPerSplit of K per
 // row, planes within 64 MiB. (512 bytes: the reference's benchmark shapes of one 128 x 128 tile - 8192 k of int8, 4096 k of
@@ -2046,7 +2053,7 @@ int launch_one(const MfmaArgs &args) {
     if (few_off_rule<Kind<TA>::ES>(args) && (args.m <= 4 || args.n <= 8))
       return launch_one<TA, TB, A_KC, B_KC, BM, BN, WAVES_M, WAVES_N, EXACT, EXTRA, kFewest>(args);
     if constexpr (Kind<TA>::ES == 2) {
-      if (few_off_rule<2>(args))
+      if (few_off_rule<2>(args) || (args.k * 2 < kHalfSlicesBelow && short_decode_batch(args, args.k * 2)))
         return launch_one<TA, TB, A_KC, B_KC, BM, BN, WAVES_M, WAVES_N, EXACT, EXTRA, kFewRows>(args);
     }
   }
@@ -2069,7 +2076,7 @@ int launch_one(const MfmaArgs &args) {
   constexpr int kSlice = slice_bytes(BM);
   const size_t slices = (p.k * ES + kSlice - 1) / kSlice;
   p.splits = splits_for(tiles, slices, p.m, p.n, p.k * ES, kSlice, EXACT, ES == 2 && BM == 128);
-  p.blocked_sums = few_off_rule<ES>(p) || bytes_in_lines(p.k * ES) >= kSplitFromBytes;
+  p.blocked_sums = few_off_rule<ES>(p) || short_decode_batch(p, p.k * ES) || bytes_in_lines(p.k * ES) >= kSplitFromBytes;
   p.slices_per_split = (unsigned)((slices + p.splits - 1) / p.splits);
   p.splits = (unsigned)((slices + p.slices_per_split - 1) / p.slices_per_split);  // no empty share
   SequenceGuard sequence(p.splits > 1);  // the partial sums travel from this kernel to the next through the workspace

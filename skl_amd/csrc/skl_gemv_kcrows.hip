@@ -238,13 +238,44 @@ int kind_of(const skl_gemm_canon *g) {
 
 inline bool aligned16(const void *p) { return ((uintptr_t)p & 15) == 0; }
 
-// A workgroup streams its columns and all of A at 60 to 70 KB per microsecond; with fewer workgroups than compute units a long
-// K is better shared out by the tile kernels, two launches as that takes (us here / there: int8 16 x 1024 x 14336, 459 KB a
-// workgroup, 10.4 / 10.9; int8 96 x 1024 x 8192 and bf16 48 x 2048 x 8192, 1 MB, 16.0 / 12.2 and 19.0 / 13.8; f16
-// 32 x 3072 x 14336 on 192 workgroups, 1.4 MB, 28.5 / 27.8). Up to four rows the other kernel is the one of dot products, slower still.
-bool chip_too_empty(size_t m, size_t n, size_t k_bytes) {
-  const size_t cg = (size_t)skl_kcstream::column_groups(n), groups = (n + 16 * cg - 1) / (16 * cg), bytes = (16 * cg + m) * k_bytes;
-  return m > 4 && ((groups < 192 && bytes > (size_t(512) << 10)) || (groups < 224 && bytes > (size_t(1280) << 10)));
+// Whether another kernel is the better one: the tile kernels, which share K or have more rows and columns to a workgroup, or up to
+// three rows the dot products of skl_gemv.hip. Not for fp8 with K up to 4096, or a B of 8192 columns and more: beyond K = 2304 the
+// tile kernels multiply fp8 with instructions that align the products (error 1.3e-5 against 5e-8 here).
+// A workgroup streams its columns and all of A at 60 to 70 KB per microsecond, at two thirds of that if the columns start inside
+// lines. With fewer workgroups than compute units a long K is better shared out (us here / there: int8 48 x 2048 x 8192 on 128
+// workgroups, 512 KiB each, 11.1 / 9.4; int8 96 x 1024 x 8192, 896 KiB, 16.0 / 12.2; f16 64 x 448 x 2688, 420 KiB, 10.3 / 8.8; int8
+// 28 x 153 x 11312, 486 KiB and columns inside lines, 13.0 / 9.6; the other way, with a ring of four units, int8 16 x 128 x 14336,
+// 448 KiB, 5.9 / 9.1). Medians over some 2000 random problems, by KiB per workgroup, here over there: up to 80 workgroups 0.69 at
+// 128, 0.90 at 256, 1.07 at 384, inside lines 0.78, 1.05 and 1.28; 129 to 191 workgroups 0.62, 0.77, 0.88 and 0.72, 0.90, 1.02.
+// On a full chip the 16-bit kinds' ring gets short as rows and columns are many: bf16 96 x 8192 x 14336 75 / 49, 48 x 4096 x 14336
+// 35 / 28, 64 x 4096 x 8192 22.5 / 20.6; with a short K the sums' way through LDS is what takes the time: bf16 64 x 11008 x 512
+// 1.5 times theirs, 48 x 8192 x 256 1.08. More than 16384 columns are more than one round of workgroups, each with its own start and
+// end: 32 rows of bf16 at K = 1024 / 2048 / 4096 / 8192 take 1.35 / 1.33 / 1.27 / 1.05 of the tile kernels' time at 32000 columns, 16 rows 1.04,
+// 1.06, 1.13 and 0.89; two rows 1.0 to 1.2 of the dot products' up to 24576 columns. From 65 rows on the tile kernels' sums would be
+// longer chains than the ones here (they are the faster ones there too: bf16 96 x 50257 x 2048 85 / 43).
+bool others_are_faster(int kind, size_t m, size_t n, size_t k, size_t k_bytes, size_t b_pitch) {
+  constexpr size_t kib = 1024;
+  const size_t cg = (size_t)skl_kcstream::column_groups(n), groups = (n + 16 * cg - 1) / (16 * cg);
+  const bool half = kind >= kBF16, fp8 = kind != kI8 && !half, lines = b_pitch % skl_kcstream::kLine == 0;
+  size_t bytes = (16 * cg + m) * k_bytes;
+  if (m <= 4) {
+    if (n <= 16384 || k < (half ? lines ? 2048u : 1024u : 4096u)) return false;
+    return lines ? !fp8 && m == 2 && n <= 24576 : m <= (kind == kI8 ? 3u : 2u);
+  }
+  const bool starved = (groups < 192 && bytes > 512 * kib) || (groups < 224 && bytes > 1280 * kib);
+  if (fp8) return k > 4096 && n < 8192 && starved;
+  if (starved || (half && m > 64 && n > 8192)) return starved;
+  if (!lines) bytes = bytes / 2 * 3;  // what they take the time of
+  if (kind == kI8 && k <= 4096) return false;
+  if (groups < 224 && (m > 16 || !lines) && bytes >= (groups <= 80 && (half || !lines) ? 384 : groups < 192 ? 512 : 960) * kib) return true;
+  if (!half) return n <= 4096 && k > 4096 && bytes > 800 * kib;
+  if (cg == 1) return bytes > 960 * kib;
+  if (cg == 2) return m > 32 && (bytes > 1416 * kib || (m > 48 && m <= 64 && k < 768));
+  if (m > 64) return false;
+  if (cg == 3) return m > 32 && k < 1024;
+  if (n <= 14336) return m > 16 && k < (m > 48 ? 2048u : 640u);
+  if (n <= 16384) return m > 16 && k < (m > 48 ? 12288u : m > 32 ? 2048u : 1024u);
+  return k < (m > 16 ? 8192u : 2048u);
 }
 
 }  // namespace
@@ -259,7 +290,7 @@ extern "C" int skl_hip_gemv_kc_rows_supported(const skl_gemm_canon *g) {
   if (g->m < (size_t)kMinRows || g->m > (size_t)(16 * kMaxRowGroups) || g->n == 0 || g->k == 0) return 0;
   const size_t es = kind >= kBF16 ? 2 : 1, most = (size_t(1) << 31) - 4096;
   if (((g->k * es) % 16) != 0 || g->k * es > most || g->k * es * g->n < (size_t(1) << 20)) return 0;
-  if (g->a_sk != 1 || g->b_sk != 1 || chip_too_empty(g->m, g->n, g->k * es)) return 0;
+  if (g->a_sk != 1 || g->b_sk != 1 || others_are_faster(kind, g->m, g->n, g->k, g->k * es, g->b_s0 * es)) return 0;
   if (!aligned16(g->a) || ((g->a_s0 * es) % 16) != 0 || (g->m > 64 && g->a_s1 != 64 * g->a_s0)) return 0;
   if (!aligned16(g->b) || ((g->b_s0 * es) % 16) != 0 || (g->n > 64 && g->b_s1 != 64 * g->b_s0)) return 0;
   if (g->a_s0 * es > most / 96 || g->b_s0 * es > most / 64) return 0;

@@ -122,3 +122,35 @@ def test_copies_padded_to_tiles_only_where_both_operands_need_them(kind):
     assert pays(kind, 4000, 4000, k // 2 + 1, lda=k // 2 + 1, b_rows=False)            # short K
     assert pays(kind, 300, 300, k + 1, b_rows=False)                                   # six tiles
     assert not pays(kind, 4096, 4096, 4096, lda=4097) and pays(kind, 4096, 4096, 4096)  # whole tiles: one copy streams
+
+
+def streams_k_contiguous(kind, m, n, k, pitch=None):
+    """Whether a decode batch against weights with K contiguous, columns `pitch` apart, is the streaming kernel's."""
+    g = Canon(ta=kind, tb=kind, m=m, n=n, k=k, a=1 << 20, b=1 << 20, c=1 << 20, a_sk=1, b_sk=1, c_row_shift=6, c_col_shift=6)
+    g.a_s0, g.b_s0 = k, pitch or k
+    g.a_s1, g.b_s1 = 64 * g.a_s0, 64 * g.b_s0
+    g.rsc0, g.csc0, g.rsc1, g.csc1 = n, 1, 64 * n, 64
+    fn = ct.CDLL(skl_amd.library_path()).skl_hip_gemv_kc_rows_supported
+    fn.argtypes = [ct.POINTER(Canon)]
+    return bool(fn(ct.byref(g)))
+
+
+@pytest.mark.parametrize("kind", (E4M3, E5M2))
+def test_fp8_decode_batches_that_only_the_streaming_kernel_multiplies_exactly(kind):
+    """K up to 4096, or 8192 columns and more: however few workgroups there are."""
+    for m, n, k in ((96, 9216, 14336), (16, 8208, 14336), (5, 8192, 16384), (96, 9168, 4096), (48, 1024, 4096), (96, 320, 4096), (70, 50000, 8192)):
+        assert streams_k_contiguous(kind, m, n, k), (m, n, k)
+    assert not streams_k_contiguous(kind, 48, 1024, 14336) and streams_k_contiguous(kind, 16, 1024, 14336)
+
+
+def test_where_k_contiguous_decode_batches_leave_the_streaming_kernel():
+    yes = ((BF16, 16, 32000, 8192), (BF16, 4, 20480, 4096), (BF16, 64, 11008, 4096), (BF16, 96, 50000, 2048), (F16, 16, 8208, 4096), (F16, 32, 4096, 8192),
+           (I8, 16, 128, 14336), (I8, 48, 9168, 4096), (I8, 2, 32000, 8192), (I8, 64, 50000, 256))
+    no = ((BF16, 64, 50000, 2048), (BF16, 16, 32000, 1024), (BF16, 2, 20480, 4096), (BF16, 64, 11008, 512), (BF16, 96, 8192, 14336), (F16, 48, 4096, 14336),
+          (F16, 64, 448, 2688), (I8, 48, 2048, 8192), (I8, 2, 20480, 8192), (I8, 96, 1024, 8192))
+    for case in yes:
+        assert streams_k_contiguous(*case), case
+    for case in no:
+        assert not streams_k_contiguous(*case), case
+    # columns that start inside lines take half as long again
+    assert streams_k_contiguous(I8, 16, 256, 14336) and not streams_k_contiguous(I8, 16, 256, 14336, pitch=14352)
