@@ -385,7 +385,9 @@ __global__ void __launch_bounds__((skl_kcstream::Shape<RG, CG, 2>::kWaves * 64))
     asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
     __builtin_amdgcn_s_barrier();
   }
-  constexpr int kChains = kRingWaves == 2 ? 2 : 1;  // at least four sums per output: no longer a chain of roundings than four waves have
+  // Sums per output: four up to 16 rows; beyond that one per half line and wave, eight or (two waves) four, as the kernel with B in
+  // registers starts new ones every 4096 k.
+  constexpr int kChains = RG > 1 ? 2 : 1;
   v4f acc[kChains][RG][CG];
 #pragma unroll
   for (int rg = 0; rg < RG; ++rg)
