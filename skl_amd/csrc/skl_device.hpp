@@ -12,8 +12,9 @@
 hipStream_t skl_current_stream();
 
 // Scratch of the current stream (on the current device) used by split reductions. Grows on
-// demand; contents are only meaningful inside one launch sequence.
-void *skl_workspace(size_t bytes);
+// demand; contents are only meaningful inside one launch sequence. `optional`: the caller does without as well; then
+// nothing is recorded when there is none, and nothing is allocated while the stream is being captured into a graph.
+void *skl_workspace(size_t bytes, bool optional = false);
 
 // A block of the current stream (on the current device) that is zero when a kernel starts and
 // that every kernel leaves zero again: sums and counters shared by the workgroups of a launch.

@@ -2081,8 +2081,11 @@ int launch_one(const MfmaArgs &args) {
   p.splits = (unsigned)((slices + p.slices_per_split - 1) / p.slices_per_split);  // no empty share
   SequenceGuard sequence(p.splits > 1);  // the partial sums travel from this kernel to the next through the workspace
   if (p.splits > 1) {
-    p.partial = (char *)skl_workspace((size_t)p.splits * p.m * p.n * 4);
-    if (!p.partial) return -4;
+    // A K below kSplitFromBytes is shared for speed alone: without scratch memory one workgroup per tile takes all of it.
+    const bool optional = bytes_in_lines(p.k * ES) < kSplitFromBytes;
+    p.partial = (char *)skl_workspace((size_t)p.splits * p.m * p.n * 4, optional);
+    if (!p.partial && !optional) return -4;
+    if (!p.partial) p.splits = 1, p.slices_per_split = (unsigned)slices;
   }
   if (tiles > 0x7FFFFFFFu || p.splits > 0xFFFFu) {
     skl_hip_record_error(-2, "gemm_mfma: grid too large");

@@ -116,11 +116,11 @@ DeviceState *current_device_state() {
 
 // Under g_mutex: the scratch of the calling thread's stream on this device; nullptr when every slot belongs to
 // another stream (two streams on one slot would mix their partial sums and counters).
-StreamState *current_stream_state(DeviceState &st) {
+StreamState *current_stream_state(DeviceState &st, bool record = true) {
   for (StreamState &s : st.streams)
     if (s.stream == t_stream) return &s;
   if (st.streams.size() >= kMaxStreamStates) {
-    skl_hip_record_error(SKL_HIP_ERR_STREAM_SLOTS, "scratch memory: 32 streams hold a slot on this device - release one (skl_hip_release_stream)");
+    if (record) skl_hip_record_error(SKL_HIP_ERR_STREAM_SLOTS, "scratch memory: 32 streams hold a slot on this device - release one (skl_hip_release_stream)");
     return nullptr;
   }
   st.streams.emplace_back();
@@ -130,12 +130,20 @@ StreamState *current_stream_state(DeviceState &st) {
 
 }  // namespace
 
-void *skl_workspace(size_t bytes) {
+void *skl_workspace(size_t bytes, bool optional) {
   DeviceState *st = current_device_state();
   if (!st) return nullptr;
   std::lock_guard<std::mutex> lock(g_mutex);
-  StreamState *ss = current_stream_state(*st);
-  return ss ? grow(*ss, ss->workspace, bytes, kWorkspaceBytes, "skl_workspace", true) : nullptr;
+  StreamState *ss = current_stream_state(*st, !optional);
+  if (!ss) return nullptr;
+  if (optional && (!ss->workspace.ptr || ss->workspace.bytes < bytes)) {
+    hipStreamCaptureStatus status = hipStreamCaptureStatusNone;
+    if (hipStreamIsCapturing(t_stream, &status) != hipSuccess || status != hipStreamCaptureStatusNone) {
+      (void)hipGetLastError();
+      return nullptr;
+    }
+  }
+  return grow(*ss, ss->workspace, bytes, kWorkspaceBytes, "skl_workspace", !optional);
 }
 
 void *skl_zeroed_scratch(size_t bytes) {
