@@ -2183,6 +2183,9 @@ int launch_whole_tiles(const MfmaArgs &p) {
     if (p.bias) tail.bias = p.bias + head_cols * sizeof(float);
     if (p.rq.q) tail.rq.q = p.rq.q + head_cols * p.rq.csq;
     if (p.rq.q && p.rq.q_per_column) tail.rq.q_scale = p.rq.q_scale + head_cols;
+    // The tail may be tiles few enough to share K (launch_ring): what it needs for that is there before the head has written
+    // its columns of C, which no other kernel could then start from.
+    if (tiles_m * (tail_cols / 128) <= 128 && long_k && !skl_workspace((size_t)2 * p.m * tail_cols * 4)) return -4;
     const int rc = wide(head);
     return rc != 0 ? rc : narrow(tail);
   }

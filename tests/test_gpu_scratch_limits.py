@@ -28,7 +28,8 @@ def _streams_until_the_slots_are_gone(gpu, hip, ct):
 
 
 @pytest.mark.parametrize("ta,m,n,k,beta,code", (("bf16", 40, 300, 1200, 1, 0),      # a K that is shared for speed alone: in one share, without a word
-                                                ("f8e4m3", 64, 520, 1100, 0, 0)))
+                                                ("f8e4m3", 64, 520, 1100, 0, 0),
+                                                ("i8", 2048, 8448, 8192, 3, -5)))   # 33 tile columns of 256: the trailing ones would share K
 def test_without_a_scratch_slot(gpu, ta, m, n, k, beta, code):
     """A stream beyond the 32 that hold scratch: the results of the others, each element of C updated once."""
     import ctypes as ct
