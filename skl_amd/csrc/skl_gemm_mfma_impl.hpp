@@ -2204,7 +2204,7 @@ int launch_whole_tiles(const MfmaArgs &p) {
 template <int TA, int TB, bool A_KC, bool B_KC>
 int ragged_tile_cols(const MfmaArgs &p) {
   constexpr size_t ES = Kind<TA>::ES, limit = 0xB0000000u;
-  if (p.a_loose || p.b_loose) return 0;
+  if (p.a_loose || p.b_loose || ((p.rq.act || p.rq.q) && !kRingCarriesExtraSteps<TA, TB>)) return 0;
   // 16 bytes along K that K ends in would need zeros behind it; the offsets inside a tile stay in the descriptor's range
   if (p.k * ES % 16 != 0 && (A_KC || B_KC)) return 0;
   if ((3 * p.a_s1 + (A_KC ? 63 * p.a_s0 : 64 * p.a_sk)) * ES >= limit || (3 * p.b_s1 + (B_KC ? 63 * p.b_s0 : 64 * p.b_sk)) * ES >= limit) return 0;
