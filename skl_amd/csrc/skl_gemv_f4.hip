@@ -498,6 +498,18 @@ extern "C" int skl_hip_gemv_f4_supported(size_t m, size_t n, size_t k, const voi
   return 1;
 }
 
+// How many k of a supported problem gemv_f4_stream_kernel multiplies: all, none, or - more than 16 rows and K beyond 4096 - all but a
+// last part of at most 2304, which is multiplied exactly, in a pass of its own behind the stream, as the kernel with B in registers
+// does with every K.
+extern "C" size_t skl_hip_gemv_f4_streamed_k(size_t m, size_t n, size_t k, size_t rsa, size_t ldb, int scaled, size_t lds) {
+  const size_t part = k % kRowsMaxK;
+  F4Args p = {};
+  p.m = m, p.n = n, p.a_row = rsa, p.b_col = ldb / 2, p.s_col = lds;
+  p.s = scaled ? reinterpret_cast<const uint8_t *>(16) : nullptr;  // asked for, not read
+  p.k = m > (size_t)kMaxRows && k > kRowsMaxK && part <= kExactMaxK ? k - part : k;
+  return streams(p) ? p.k : 0;
+}
+
 extern "C" int skl_hip_launch_gemv_f4(size_t m, size_t n, size_t k, skl_scalar alpha, const void *a, size_t rsa, size_t csa,
                                       const void *b, size_t ldb, const uint8_t *scales, size_t lds, skl_scalar beta, float *c,
                                       size_t rsc, size_t csc) {
@@ -507,14 +519,10 @@ extern "C" int skl_hip_launch_gemv_f4(size_t m, size_t n, size_t k, skl_scalar a
   }
   const int s_pairs = scales && (k % 64) == 0 && ((uintptr_t)scales & 1) == 0 && (n == 1 || (lds & 1) == 0);
   const F4Args whole = {(const char *)a, rsa, (const char *)b, ldb / 2, scales, lds, s_pairs, c, rsc, csc, m, n, k, alpha, beta};
-  // More than 16 rows and K beyond 4096: a last part of at most 2304 k is multiplied exactly, in a pass of its own behind the stream,
-  // as the kernel with B in registers does with every K.
-  const size_t part = k % kRowsMaxK;
-  const size_t streamed = m > (size_t)kMaxRows && k > kRowsMaxK && part <= kExactMaxK ? k - part : k;
-  F4Args first = whole;
-  first.k = streamed;
-  const bool stream = streams(first);
-  if (stream) {
+  const size_t streamed = skl_hip_gemv_f4_streamed_k(m, n, k, rsa, ldb, scales != nullptr, lds);
+  if (streamed != 0) {
+    F4Args first = whole;
+    first.k = streamed;
     const int rc = launch_stream(first);
     if (rc != 0 || streamed == k) return rc;
   }
@@ -528,7 +536,7 @@ extern "C" int skl_hip_launch_gemv_f4(size_t m, size_t n, size_t k, skl_scalar a
     const unsigned blocks = (unsigned)grid, threads = kWaves * 64;
     // A K beyond what the registers hold goes in passes of 4096 k: the first applies the caller's beta, the others
     // add to C (beta = 1) - launches on one stream, in order; the same bits on every run.
-    for (size_t k0 = stream ? streamed : 0; k0 < k; k0 += kRowsMaxK) {
+    for (size_t k0 = streamed; k0 < k; k0 += kRowsMaxK) {
       const size_t kk = k - k0 < kRowsMaxK ? k - k0 : kRowsMaxK;
       skl_scalar pass_beta = beta;
       if (k0 != 0) pass_beta.fz.value = 1.0f, pass_beta.fz.skip_c_read = 0;

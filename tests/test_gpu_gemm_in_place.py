@@ -152,3 +152,42 @@ def test_fused_steps_of_the_bounds_checked_kernels(gpu, ta, m, n, k, block):
             want_c, want_top, want_q = fused_expectation(case, anchor, None, start, activation=1, requant=rq)
             assert np.array_equal(q, want_q) and top[0] == want_top[0], (by_columns, rsq, csq)
             assert np.array_equal(got.view(np.uint8), (c if only else want_c).view(np.uint8)), (by_columns, rsq, csq)
+
+
+@pytest.mark.parametrize("ta,k", (("i8", 4112), ("bf16", 2056), ("f8e4m3", 4240)))
+@pytest.mark.parametrize("c_form", ("rows", "columns", "blocks"))
+def test_fused_steps_of_the_streaming_kernel_on_ragged_tiles(gpu, ta, k, c_form):
+    """Bias per column, ReLU, maximum and an 8-bit copy - off the dword rule, by columns, and alone - where tiles of 256 x 256 end inside
+    rows and columns, C row-major, by columns and in blocks of four. The call with bias alone is the anchor, which holds the product."""
+    m, n = 3856, 3104
+    rng = np.random.default_rng(k)
+    bias = rng.integers(-999, 999, n).astype(np.int32) if ta == "i8" else rng.uniform(-4, 4, n).astype(np.float32)
+    start = np.array([-(1 << 31)], np.int32) if ta == "i8" else np.array([-np.inf], np.float32)
+    if c_form == "blocks":
+        kind = "rcprc"
+        case = GemmCase(ta, None, 1, 1, m0=4, n0=4, k0=1, m1=m // 4, n1=n // 4, k1=k, rsa0=k, csa0=0, rsa1=4 * k, csa1=1, rsb0=0, csb0=k, rsb1=1, csb1=4 * k,
+                        rsc0=4, csc0=1, rsc1=4 * n + 4, csc1=16)
+    else:
+        kind = "rc"
+        case = GemmCase(ta, None, 1, 0, m0=1, n0=1, k0=1, m1=m, n1=n, k1=k, rsa0=0, csa0=0, rsa1=k, csa1=1, rsb0=0, csb0=0, rsb1=1, csb1=k, rsc0=0, csc0=0,
+                        rsc1=1 if c_form == "columns" else n, csc1=m + 1 if c_form == "columns" else 1)
+    a, b, c = case.make_inputs(int(rng.integers(1 << 30)))
+    anchor, _ = run_fused_gemm(gpu, kind, case, a, b, c, bias, None, "device")
+    if c_form == "rows":
+        widen = support.ETYPES[ta].widen
+        A, B = widen(a[:m * k]).reshape(m, k), widen(b[:n * k]).reshape(n, k)
+        exact = A @ B.T + bias
+        if ta == "i8":
+            assert np.array_equal(anchor.reshape(m, n), exact.astype(np.int64).astype(np.int32))
+        else:
+            gamma = 2.0 * np.expm1((k + 2) * np.log1p(2.0 ** -24))
+            assert np.all(np.abs(anchor.reshape(m, n) - exact) <= gamma * (np.abs(A) @ np.abs(B).T + np.abs(bias)))
+    scales = (rng.uniform(0.5, 2.0, n) * 100.0 / float(np.abs(anchor.astype(np.float64)).max())).astype(np.float32)
+    forms = {"rows": ((n + 5, 1, False), (n + (-n) % 4, 1, True)), "columns": ((1, m + 5, False),), "blocks": ((n + 5, 1, False),)}[c_form]
+    for rsq, csq, only in forms:
+        rq = dict(q=np.full((m - 1) * rsq + (n - 1) * csq + 1, 0x55, np.int8), rsq=rsq, csq=csq, scale=scales, per_column=True, zero=3, only=only,
+                  format=0 if ta == "i8" else 2)
+        got, top, q = run_fused_gemm(gpu, kind, case, a, b, c, bias, start, "device", activation=1, requant=rq)
+        want_c, want_top, want_q = fused_expectation(case, anchor, None, start, activation=1, requant=rq)
+        assert np.array_equal(q, want_q) and top[0] == want_top[0], (rsq, csq, only)
+        assert np.array_equal(got.view(np.uint8), (c if only else want_c).view(np.uint8)), (rsq, csq, only)
