@@ -17,8 +17,8 @@
 // A, row-major B, and both panel formats); blocks of 64 along M / N may sit
 // anywhere (block stride), which is what the panel formats need. A workgroup
 // owns a BM x BN tile of C (128 x 128 on eight waves or 64 x 64 on four; the streaming kernel below has larger ones); per
-// 128-byte slice of K it copies the A and B tiles global -> registers -> LDS in their native orientation with
-// 128-bit accesses (up to four slices under way in registers, two in LDS) and the waves read MFMA operands straight from
+// slice of K (128 or 256 bytes) it copies the A and B tiles global -> registers -> LDS in their native orientation with
+// 128-bit accesses (up to two slices under way in registers, two in LDS) and the waves read MFMA operands straight from
 // LDS: ds_read_b128 for a K-contiguous tile (row pitch padded to 144 bytes),
 // ds_read_b64_tr_b8 / _tr_b16 - the LDS transpose loads - for an
 // MN-contiguous one (row pitch padded so the eight/four rows of one transpose

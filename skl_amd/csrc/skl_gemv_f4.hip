@@ -197,7 +197,7 @@ __global__ void __launch_bounds__(kWaves * 64) gemv_f4_kernel(F4Args p) {
 // cannot hold): the same decomposition with B held in registers for 4096 k (one pass of the K loop above:
 // four chunks per wave; a longer K takes one launch per 4096 k, the later ones adding to C) while up to eight groups of 16 rows take their turns - the 4-bit weights cross
 // HBM once and never exist as a converted copy (which cost 22.5 MB read, 45 MB written and a tile GEMM behind it:
-// 37 / 40 / 45 us for 32 / 64 / 128 x 4096 x 11008). Two groups of 16 columns per workgroup; a row group's pieces of A
+// 37 / 40 / 45 us for 32 / 64 / 128 x 4096 x 11008). Four groups of 16 columns per workgroup; a row group's pieces of A
 // are requested two groups ahead; its sums go through one of two LDS blocks, added in wave order (one barrier per
 // group: the next group's barrier stands between this group's readers and the writers of the group after it).
 constexpr int kRowsCG = 4, kMaxRowGroups = 8;

@@ -162,7 +162,7 @@ int skl_hip_launch_gemv_kc_rows(const skl_gemm_canon *g);
 int skl_hip_noalloc_setup(void);
 size_t skl_hip_noalloc_max_sums(void);
 int skl_hip_launch_gemv_noalloc(const skl_gemm_canon *g);
-/* E4M3 A (1 to 16 rows, K contiguous) times OFP4 B (columns contiguous in K, two values per byte, `ldb` elements
+/* E4M3 A (1 to 128 rows, K contiguous) times OFP4 B (columns contiguous in K, two values per byte, `ldb` elements
  * apart): skl_gemv_f4.hip. */
 int skl_hip_gemv_f4_supported(size_t m, size_t n, size_t k, const void *a, size_t rsa, size_t csa, const void *b, size_t ldb);
 int skl_hip_launch_gemv_f4(size_t m, size_t n, size_t k, skl_scalar alpha, const void *a, size_t rsa, size_t csa, const void *b,
