@@ -101,7 +101,7 @@ extern "C" int skl_hip_gemm_mfma_padded_plan(const skl_gemm_canon *g, size_t *mp
   const bool a_ok = aligned_a(g, es), b_ok = aligned_b(g, es);
   if (fused) {
     const bool whole = g->m % 256 == 0 && g->n % 128 == 0 && (g->k * es) % 128 == 0;
-    const bool dwords = g->ta == SKL_DT_I8 ? FusedSteps<int, 2>::dword_copy(g->rq) : FusedSteps<float, 2>::dword_copy(g->rq);
+    const bool dwords = g->ta == SKL_DT_I8 ? dword_copy<int>(g->rq) : dword_copy<float>(g->rq);
     if (g->ta != g->tb || (a_ok && b_ok) || (g->rq.act >= 2 && g->k * es < 2048)) return 0;
     if (whole && (dwords || a_ok || b_ok || !wide_enough || g->n % 256 == 0)) return 0;
   }

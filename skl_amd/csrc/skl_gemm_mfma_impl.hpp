@@ -68,6 +68,7 @@ typedef int v2i __attribute__((ext_vector_type(2)));
 typedef int v4i __attribute__((ext_vector_type(4)));
 typedef int v8i __attribute__((ext_vector_type(8)));
 typedef int v16i __attribute__((ext_vector_type(16)));
+typedef float v4f __attribute__((ext_vector_type(4)));
 typedef float v16f __attribute__((ext_vector_type(16)));
 typedef short v4s __attribute__((ext_vector_type(4)));
 typedef __bf16 v8bf __attribute__((ext_vector_type(8)));
@@ -81,105 +82,40 @@ typedef _Float16 v8h __attribute__((ext_vector_type(8)));
 constexpr int slice_bytes(int tile) { return tile == 64 ? 256 : 128; }
 
 
-// The fused steps behind the alpha/beta step, for one lane: bias of the lane's column, activation, running maximum,
-// requantised copy.
-// EXTRA: with the activation and the requantised copy (kernels are instantiated with and without: the two steps cost
-// code in every one of a lane's 128 stores, which calls without them should not carry). 1: any descriptor, decided
-// element by element at run time. 2 and 3: for kernels that hand every lane's elements to rows4() with all lanes
-// active - a row-major copy on 4-byte boundaries, written as dwords, without (2, q_only) or with (3) C; no
-// branches inside the epilogue, which with 128 accumulators live is what keeps the registers from spilling (the
-// run-time form in the streaming kernel: 240 spilled registers, an 8192^3 call 45 % longer).
-template <typename T, int EXTRA = 0>
+// A block of sums, fetched from its accumulation (IN_A) or vector registers here: left to itself the compiler copies all of a wave's
+// 256 to vector registers ahead of the first use, and spills.
+template <bool IN_A, typename Acc>
+__device__ __forceinline__ Acc fetched(Acc acc) {
+  if constexpr (IN_A) asm volatile("" : "+a"(acc)); else asm volatile("" : "+v"(acc));
+  return acc;
+}
+
+// A row-major copy on 4-byte boundaries with no activation beyond ReLU, in the format that goes with C's type (int8 behind an int32
+// C, OCP fp8 behind a floating-point one): steps of a few instructions per element.
+template <typename T>
+bool dword_copy(const skl_requant &r) {
+  return r.q && r.act <= 1 && (r.q_fmt != 0) == !std::is_same<T, int>::value && r.csq == 1 && (r.rsq & 3) == 0 && ((uintptr_t)r.q & 3) == 0;
+}
+
+// The steps behind the alpha/beta step that need no more than a lane's column: its bias, and the running maximum.
+template <typename T>
 struct FusedSteps {
   const T *bias;
   T *max;
-  const skl_requant rq;
   T bias_j, running;
-  size_t col;
-  float q_scale_j;  // EXTRA: the current column's scale
-  const skl_fp8::Ofp8Format f8;  // modes 2 and 3: the constants of an fp8 copy (uniform; unused for an int8 copy)
   __device__ explicit FusedSteps(const MfmaArgs &p)
-      : bias(reinterpret_cast<const T *>(p.bias)), max(reinterpret_cast<T *>(p.max)), rq(p.rq), bias_j(0), running(skl_lowest<T>()), col(0),
-        q_scale_j(0.0f), f8(p.rq.q_fmt) {}
-  // What a descriptor must look like for modes 2 and 3: a row-major copy on 4-byte boundaries, no activation beyond
-  // ReLU (the others cost too much code in each of a lane's 128 elements), and the copy's format the one these
-  // modes are built with for C's type - int8 behind an int32 C, OCP fp8 behind a floating-point C (an int8 product
-  // feeding an int8 layer, an fp8 product an fp8 layer; other pairings take write_wave_tile_staged or the bounds-checked
-  // kernels).
-  static constexpr bool kCopyIsFp8 = !std::is_same<T, int>::value;
-  __host__ __device__ static bool dword_copy(const skl_requant &r) {
-    return r.q && r.act <= 1 && (r.q_fmt != 0) == kCopyIsFp8 && r.csq == 1 && (r.rsq & 3) == 0 && ((uintptr_t)r.q & 3) == 0;
-  }
+      : bias(reinterpret_cast<const T *>(p.bias)), max(reinterpret_cast<T *>(p.max)), bias_j(0), running(skl_lowest<T>()) {}
   // What the steps need to know about column c, fetched ahead of the stores (a load issued behind a store has to
   // wait for that store's acknowledgement before its value can be used) ...
-  struct Column {
-    T bias;
-    float q_scale;
-  };
-  __device__ __forceinline__ Column fetch(size_t c) const {
-    Column k{T(0), 0.0f};
-    if (bias) k.bias = bias[c];
-    if constexpr (EXTRA >= 2) k.q_scale = rq.q_scale[rq.q_per_column ? c : 0];
-    if constexpr (EXTRA == 1) {
-      if (rq.q) k.q_scale = rq.q_scale[rq.q_per_column ? c : 0];
-    }
-    return k;
-  }
+  __device__ __forceinline__ T fetch(size_t c) const { return bias ? bias[c] : T(0); }
   // ... and made current.
-  __device__ __forceinline__ void column(size_t c, const Column &k) {
-    col = c;
-    bias_j = k.bias;
-    q_scale_j = k.q_scale;
-  }
-  __device__ __forceinline__ void column(size_t c) { column(c, fetch(c)); }
-  __device__ __forceinline__ T apply(T v) {
+  __device__ __forceinline__ void column(T k) { bias_j = k; }
+  // An element of the current column: the steps, then C (written once and not read again: a non-temporal store keeps it out of
+  // the operands' caches).
+  __device__ __forceinline__ void put(T v, T *dst) {
     if (bias) v = skl_add_bias(v, bias_j);
-    if constexpr (EXTRA == 1) v = skl_activate(v, rq.act);
-    if constexpr (EXTRA >= 2) v = skl_activate(v, rq.act != 0);  // none or ReLU
     if (max && v > running) running = v;
-    return v;
-  }
-  // The element of logical row `row` in the current column: the steps, then C (written once and not read again: a
-  // non-temporal store keeps it out of the operands' caches) and, in mode 1, the requantised copy. Returns what
-  // was written.
-  __device__ __forceinline__ T put(T v, T *dst, size_t row) {
-    v = apply(v);
-    if constexpr (EXTRA == 1) {
-      if (!rq.q_only) __builtin_nontemporal_store(v, dst);
-      if (rq.q) rq.q[row * rq.rsq + col * rq.csq] = skl_quantise((float)v, q_scale_j, rq.q_zero, rq.q_fmt);
-    } else {
-      (void)row;
-      if constexpr (EXTRA != 2) __builtin_nontemporal_store(v, dst);
-    }
-    return v;
-  }
-  // Modes 2 and 3: the requantised copy of rows row0 .. row0 + 3 of the current column, v as put() returned them.
-  // A lane's four values are one column of a 4 x 4 block of bytes whose other columns its quad's lanes hold (four
-  // neighbouring columns, the first a multiple of four); the block is transposed across the quad (four broadcasts
-  // and three byte permutes per lane), and lane q stores row row0 + q of it as one dword - a quarter of the store
-  // instructions and address arithmetic of single bytes.
-  __device__ __forceinline__ void rows4(const T (&v)[4], size_t row0) {
-    if constexpr (EXTRA >= 2) {
-      unsigned packed = 0;
-#pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        if constexpr (kCopyIsFp8)
-          packed |= skl_fp8::encode_ofp8_hw(__fmul_rn((float)v[i], q_scale_j), f8) << (8 * i);
-        else
-          packed |= ((unsigned)skl_requantise_int((float)v[i], q_scale_j, rq.q_zero) & 0xFFu) << (8 * i);
-      }
-      const unsigned p0 = (unsigned)__builtin_amdgcn_update_dpp(0, (int)packed, 0x00, 0xF, 0xF, true);  // quad_perm: lane 0 of the quad
-      const unsigned p1 = (unsigned)__builtin_amdgcn_update_dpp(0, (int)packed, 0x55, 0xF, 0xF, true);
-      const unsigned p2 = (unsigned)__builtin_amdgcn_update_dpp(0, (int)packed, 0xAA, 0xF, 0xF, true);
-      const unsigned p3 = (unsigned)__builtin_amdgcn_update_dpp(0, (int)packed, 0xFF, 0xF, 0xF, true);
-      const unsigned q = threadIdx.x & 3u;
-      const unsigned sel = 0x0C0C0400u + q * 0x0101u;  // byte q of the second operand, byte q of the first, zeros
-      const unsigned lo = __builtin_amdgcn_perm(p1, p0, sel), hi = __builtin_amdgcn_perm(p3, p2, sel);
-      const unsigned out = __builtin_amdgcn_perm(hi, lo, 0x05040100u);
-      *reinterpret_cast<unsigned *>(rq.q + (row0 + q) * rq.rsq + (col - q)) = out;
-    } else {
-      (void)v, (void)row0;
-    }
+    __builtin_nontemporal_store(v, dst);
   }
   // Every lane of the wave calls this once, after its last element.
   __device__ __forceinline__ void finish() {
@@ -281,6 +217,85 @@ struct MmaF8Exact {
 // K up to which the fp8 kinds run on MmaF8Exact: the reference's bound 2((1 + 2^-24)^(K+2) - 1) passes the fp8
 // instructions' 2^-11.9 at K = 2193.
 constexpr size_t kF8ExactMaxK = 2304;
+
+// What the streaming kernel multiplies with: blocks of SIDE x SIDE, 64 bytes of K. The instructions take B's columns as their
+// first operand, A's rows as their second, so that a lane holds four consecutive columns of a row of C: 16 bytes of a row-major C.
+// 16 x 16 blocks take the device a seventh less energy per product than 32 x 32 ones (instructions alone on random operands, P/s for
+// 32 x 32 / 16 x 16: bf16 1.67 / 1.86, f16 1.55 / 1.75, int8 3.18 / 3.69), with the same error against 64 bits.
+// Written in assembly for the registers' sake: a wave's operands are vector registers that LDS reads under way will write, its sums
+// accumulation registers, and left to itself the compiler moves both about. Of the 256 sums per lane of a 256 x 256 tile a few are
+// vector registers (IN_A false): where all accumulation registers are taken the compiler copies a block out and back around a
+// product, which it does not know to be under way.
+// run() with a load: also 16 bytes per lane from g + off to LDS at `lds` + AT (a load to LDS takes its place there from M0, which is
+// to be written an instruction ahead).
+#define SKL_RING_PRODUCT(IN_, INSN, MODS) asm volatile("v_mfma_" INSN " %0, %1, %2, %0" MODS : "+" IN_(c) : "v"(b), "v"(a))
+#define SKL_RING_PRODUCT_LOAD(IN_, INSN, MODS)                                                                       \
+  asm volatile("s_add_u32 m0, %3, %6\n\tv_mfma_" INSN " %0, %1, %2, %0" MODS "\n\tglobal_load_lds_dwordx4 %4, %5"   \
+               : "+" IN_(c) : "v"(b), "v"(a), "s"(lds), "v"(off), "s"(g), "n"(AT) : "memory", "scc")
+#define SKL_RING_MMA(INSN, MODS, FRAG)                                                                                            \
+  template <bool IN_A>                                                                                                            \
+  __device__ static __forceinline__ void run(FRAG a, FRAG b, Acc &c) {                                                            \
+    if constexpr (IN_A) SKL_RING_PRODUCT("a", INSN, MODS); else SKL_RING_PRODUCT("v", INSN, MODS);                                \
+  }                                                                                                                               \
+  template <bool IN_A, unsigned AT>                                                                                               \
+  __device__ static __forceinline__ void run(FRAG a, FRAG b, Acc &c, unsigned lds, const char *g, unsigned off) {                 \
+    if constexpr (IN_A) SKL_RING_PRODUCT_LOAD("a", INSN, MODS); else SKL_RING_PRODUCT_LOAD("v", INSN, MODS);                      \
+  }
+template <int TA, int TB, bool EXACT>
+struct RingMma;
+#define SKL_RING_F8(TA_, TB_, MODS)                   \
+  template <>                                         \
+  struct RingMma<TA_, TB_, false> {                   \
+    using Frag = v8i;                                 \
+    static constexpr int kSide = 32, kFrag = 32;      \
+    using Acc = v16f;                                 \
+    SKL_RING_MMA("f32_32x32x64_f8f6f4", MODS, v8i)    \
+  };
+SKL_RING_F8(SKL_DT_F8E4M3, SKL_DT_F8E4M3, "")
+SKL_RING_F8(SKL_DT_F8E4M3, SKL_DT_F8E5M2, " cbsz:1")
+SKL_RING_F8(SKL_DT_F8E5M2, SKL_DT_F8E4M3, " blgp:1")
+SKL_RING_F8(SKL_DT_F8E5M2, SKL_DT_F8E5M2, " cbsz:1 blgp:1")
+#undef SKL_RING_F8
+template <>
+struct RingMma<SKL_DT_I8, SKL_DT_I8, false> {
+  using Frag = v4i;
+  static constexpr int kSide = 16, kFrag = 16;
+  using Acc = v4i;
+  SKL_RING_MMA("i32_16x16x64_i8", "", v4i)
+};
+template <>
+struct RingMma<SKL_DT_BF16, SKL_DT_BF16, false> {
+  using Frag = v4i;
+  static constexpr int kSide = 16, kFrag = 16;
+  using Acc = v4f;
+  SKL_RING_MMA("f32_16x16x32_bf16", "", v4i)
+};
+template <>
+struct RingMma<SKL_DT_F16, SKL_DT_F16, false> {
+  using Frag = v4i;
+  static constexpr int kSide = 16, kFrag = 16;
+  using Acc = v4f;
+  SKL_RING_MMA("f32_16x16x32_f16", "", v4i)
+};
+template <int TA, int TB>
+struct RingMma<TA, TB, true> {  // a lane's 16 bytes of K are two products' worth (see FragReader): its first eight, its last eight
+  using Frag = v4i;
+  static constexpr int kSide = 16, kFrag = 16;
+  using Acc = v4f;
+  template <int DT>
+  __device__ static v8h widen(v4i f, int half) {
+    return half ? skl_fp8::widen8_to_f16<DT == SKL_DT_F8E5M2>((unsigned)f.z, (unsigned)f.w) : skl_fp8::widen8_to_f16<DT == SKL_DT_F8E5M2>((unsigned)f.x, (unsigned)f.y);
+  }
+  __device__ static v8h widen_a(v4i f, int half) { return widen<TA>(f, half); }
+  __device__ static v8h widen_b(v4i f, int half) { return widen<TB>(f, half); }
+  SKL_RING_MMA("f32_16x16x32_f16", "", v8h)
+};
+#undef SKL_RING_MMA
+#undef SKL_RING_PRODUCT
+#undef SKL_RING_PRODUCT_LOAD
+// Whether block (i, j) of a wave's MI x NI lies in accumulation registers: all but half a row of blocks where there are 256 sums.
+template <int MI, int NI, typename Acc>
+constexpr bool ring_sum_in_a(int i, int j) { return MI * NI * sizeof(Acc) < 1024 || i < MI - 1 || j < NI / 2; }
 
 // A fragment as the multiply wants it: widened where the operand kind asks for that, else as it was read.
 template <typename M, typename F>
@@ -484,10 +499,9 @@ __device__ __forceinline__ auto read_frag(const char *tile, int row0, int kb) {
 // any element of the wave's tile is one is decided once, for the whole wave, before the first store.
 // CHECK: rows / columns beyond p.m / p.n are left alone.
 // ---------------------------------------------------------------------------
-template <int MI, int NI, bool CHECK, int EXTRA, typename Acc>
+template <int MI, int NI, bool CHECK, typename Acc>
 __device__ __forceinline__ void write_wave_tile(const MfmaArgs &p, const Acc (&acc)[MI][NI], size_t row0, size_t col0) {
   using AccElem = decltype(Acc{}.x);
-  using Steps = FusedSteps<AccElem, EXTRA>;
   constexpr int kBlocks = MI * NI;            // block b: j = b / MI, i = b % MI (a column strip at a time)
   constexpr int kAhead = (kBlocks < 2 || CHECK) ? 1 : 2;  // the bounds-checked kernels run four waves per SIMD: 128 registers
   // The lane index from the execution mask rather than from threadIdx: nothing the epilogue needs is then computed
@@ -535,10 +549,10 @@ __device__ __forceinline__ void write_wave_tile(const MfmaArgs &p, const Acc (&a
     }
     return w;
   };
-  Steps fused(p);
-  typename Steps::Column columns[NI];
+  FusedSteps<AccElem> fused(p);
+  AccElem columns[NI];
 #pragma unroll
-  for (int j = 0; j < NI; ++j) columns[j] = (!CHECK || col_of(j) < p.n) ? fused.fetch(col_of(j)) : typename Steps::Column{AccElem(0), 0.0f};
+  for (int j = 0; j < NI; ++j) columns[j] = (!CHECK || col_of(j) < p.n) ? fused.fetch(col_of(j)) : AccElem(0);
 
   // Block B. MODE 0: C is not read; 1: with the old values `old` (C is updated, or beta == 0 and they decide the sign of
   // zeros); 2: C is not read and there is no fused step (no bias, no maximum, no copy).
@@ -546,15 +560,13 @@ __device__ __forceinline__ void write_wave_tile(const MfmaArgs &p, const Acc (&a
   auto write_block = [&](auto mode, auto bc, const AccElem (&old)[16]) {
     constexpr int MODE = decltype(mode)::value, B = decltype(bc)::value;
     constexpr int j = B / MI, i = B % MI;
-    fused.column(col_of(j), columns[j]);
+    fused.column(columns[j]);
     const Where w = where(j, i);
 #pragma unroll
     for (int g = 0; g < 4; ++g) {
-      AccElem four[4];
 #pragma unroll
       for (int q = 0; q < 4; ++q) {
         const int r = 4 * g + q;
-        four[q] = AccElem(0);
         if (inside(j, i, r)) {
           AccElem v;
           if constexpr (MODE == 0 || MODE == 2) v = skl_initialise_plain(acc[i][j][r], p.alpha, p.beta);
@@ -562,15 +574,12 @@ __device__ __forceinline__ void write_wave_tile(const MfmaArgs &p, const Acc (&a
             const AccElem vi = skl_initialise_with(acc[i][j][r], old[r], p.alpha, p.beta), vc = skl_combine(acc[i][j][r], old[r], p.alpha, p.beta);
             v = init ? vi : vc;
           }
-          if constexpr (MODE == 2) {  // no fused step at all: the value as it is
+          if constexpr (MODE == 2)  // no fused step at all: the value as it is
             __builtin_nontemporal_store(v, w.out[g] + q * p.rsc0);
-            four[q] = v;
-          } else {
-            four[q] = fused.put(v, w.out[g] + q * p.rsc0, first_row(i, g) + q);
-          }
+          else
+            fused.put(v, w.out[g] + q * p.rsc0);
         }
       }
-      fused.rows4(four, first_row(i, g));
     }
     __builtin_amdgcn_sched_barrier(0);  // a block at a time: the addresses of later blocks are not computed (and held) early
   };
@@ -600,7 +609,7 @@ __device__ __forceinline__ void write_wave_tile(const MfmaArgs &p, const Acc (&a
   };
   if (!read_c) {
     const AccElem none[16] = {};
-    if (EXTRA == 0 && !p.bias && !p.max) {  // the plain product: two or three instructions and a store per element
+    if (!p.bias && !p.max) {  // the plain product: two or three instructions and a store per element
       [&]<int... Bs>(std::integer_sequence<int, Bs...>) {
         (write_block(std::integral_constant<int, 2>{}, std::integral_constant<int, Bs>{}, none), ...);
       }(std::make_integer_sequence<int, kBlocks>{});
@@ -783,6 +792,309 @@ __device__ __forceinline__ void write_wave_tile_staged(const MfmaArgs &p, const 
     const T best = skl_wave_max(running);
     if (lane == 0 && best > skl_lowest<T>()) skl_atomic_max(reinterpret_cast<T *>(p.max), best);
   }
+}
+
+// ---------------------------------------------------------------------------
+// The streaming kernel's epilogue: one wave writes its MI x NI blocks, of which a lane holds four consecutive columns of a row at a
+// time (acc[i][j][4 g + e]: row S i + lane % S, column S j + 8 g + 4 (lane / S) + e). The operands' ring being over, the rows of one row
+// of blocks at a time go to LDS as they are, and a loop takes them from there in the order that C wants: a wave's rows of 128 (64)
+// columns in whole lines, 16 bytes per lane. A loop, because what is behind it - a GELU is some fifty instructions - cannot be written
+// out for each of a lane's 256 sums: eight copies of the loop, one behind every row of blocks, are 250 KB of code and were three times
+// as slow (E4M3 2048 x 8192 x 2048 with GELU into E4M3, all of it 137 us). And whole lines, because the sums as they lie make pieces of 64
+// bytes (32 x 32 blocks: 32 bytes), which took 17.5 us for the 64 MiB of 4096^2 (with 32 x 32 blocks 35).
+// C by columns is written from LDS by columns, 16 bytes of a column per lane.
+// The old values of C are requested a batch ahead: one counter covers loads and stores, in issue order, so that a value used
+// right behind its load has waited for every store in front of it. beta == 0 in floating point reads C only where alpha * acc is the
+// negative zero (skl_initialise_needs_c), decided for a batch at a time.
+// CHECK: rows and columns beyond p.m / p.n are left alone; a lane at the edge reads its old values from the last four columns.
+// `stage`: this wave's S x (COLS + 4) elements.
+// ---------------------------------------------------------------------------
+template <int COLS>
+constexpr int wave_rows_pitch() { return COLS + 4; }
+template <int MI, int NI, bool CHECK, bool STEPS, typename Acc>
+__device__ __forceinline__ void write_wave_rows(const MfmaArgs &p, const Acc (&acc)[MI][NI], size_t row0, size_t col0, char *stage_bytes) {
+  using T = decltype(Acc{}.x);
+  typedef T V4 __attribute__((ext_vector_type(4)));
+  typedef T Run4 __attribute__((ext_vector_type(4), aligned(4)));
+  constexpr int S = sizeof(Acc) == 64 ? 32 : 16, G = S == 32 ? 4 : 1, COLS = NI * S, P = wave_rows_pitch<COLS>();
+  // A pass: 8 rows by 32 columns, whole lines; by columns: S rows by 256 / S columns. A batch: four passes, side by side first.
+  constexpr int kPasses = S * COLS / 256, kBatch = 4, kSide = COLS / 32, kColsDown = 256 / S;
+  static_assert(kPasses % kBatch == 0 && kBatch % kSide == 0);
+  const int lane = (int)__builtin_amdgcn_mbcnt_hi(~0u, __builtin_amdgcn_mbcnt_lo(~0u, 0u));  // (not from threadIdx, see write_wave_tile)
+  T *const stage = reinterpret_cast<T *>(stage_bytes);
+  T *const c = reinterpret_cast<T *>(p.c);
+  const size_t rmask = (size_t(1) << p.crs) - 1, cmask = (size_t(1) << p.ccs) - 1;
+  const auto row_at = [&](size_t row) { return (row >> p.crs) * p.rsc1 + (row & rmask) * p.rsc0; };
+  const auto col_at = [&](size_t col) { return (col >> p.ccs) * p.csc1 + (col & cmask) * p.csc0; };
+  const T *const bias = reinterpret_cast<const T *>(p.bias);
+  const skl_fp8::Ofp8Format f8(p.rq.q_fmt);
+  // A single round of tiles ends all at once, and its stores go faster through the caches; with more rounds the operands of the next
+  // one need the room (bf16, us, kept / past the caches: 4096^3 97.5 / 100.2, 8192^3 743 / 721).
+  const bool kept = p.tiles_m * p.tiles_n <= 256;
+
+  // RUN: four columns lie side by side in C. Otherwise, `down`, a lane's four elements are four rows of a column: side by side in a C by
+  // columns, and in any other C as good as four columns. UPDATE: C is read (not only where a zero's sign asks for it). FUSED: there are
+  // steps behind the alpha/beta step.
+  const auto write = [&](auto run, auto update, auto fused) __attribute__((always_inline)) {
+    constexpr bool RUN = decltype(run)::value, UPDATE = decltype(update)::value, FUSED = decltype(fused)::value;
+    // the lane's first row and column in a pass, from those of the pass
+    const int r_lane = RUN ? lane / 8 : lane % (S / 4) * 4, c_lane = RUN ? lane % 8 * 4 : lane / (S / 4);
+    // C's place of the lane's elements in a pass: that of the pass, a scalar, and this (passes begin at multiples of 8 rows and 16 or
+    // more columns, blocks of C are powers of two)
+    T *const c_lane_at = c + row_at(r_lane) + col_at(c_lane);
+    const auto cols_in = [&](size_t col) -> int {  // of four columns from `col` on
+      if constexpr (!CHECK) return 4;
+      return col >= p.n ? 0 : p.n - col < 4 ? (int)(p.n - col) : 4;
+    };
+    const auto column_at = [&](size_t k) { return !CHECK || k < p.n ? k : 0; };
+    T bias_of[RUN ? kSide : 1][4];
+    float scale_of[RUN ? kSide : 1][4];
+    if constexpr (RUN && FUSED) {
+#pragma unroll
+      for (int t = 0; t < kSide; ++t)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          const size_t k = column_at(col0 + t * 32 + c_lane + e);
+          bias_of[t][e] = bias ? bias[k] : T(0);
+          scale_of[t][e] = STEPS && p.rq.q ? p.rq.q_scale[p.rq.q_per_column ? k : 0] : 0.0f;
+        }
+      __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0): in the loop they would be waited for with every batch, and its stores with them
+    }
+    const bool q_run = STEPS && RUN && p.rq.csq == 1 && (p.rq.rsq & 3) == 0 && ((uintptr_t)p.rq.q & 3) == 0;
+    T running = skl_lowest<T>();
+
+    // Pass x of a row of blocks that begins at row `top`: its first row and column.
+    const auto first_row = [&](size_t top, unsigned x) { return top + (RUN ? x / kSide * 8 : 0); };
+    const auto first_col = [&](unsigned x) { return col0 + (RUN ? x % kSide * 32 : x * kColsDown); };
+    const auto request = [&](size_t top, unsigned x, V4 (&old)[kBatch]) __attribute__((always_inline)) {
+#pragma unroll
+      for (int t = 0; t < kBatch; ++t) {
+        const size_t row = first_row(top, x + t) + r_lane, k = first_col(x + t) + c_lane;
+        if constexpr (RUN && !CHECK) {
+          old[t] = *reinterpret_cast<const Run4 *>(c_lane_at + row_at(first_row(top, x + t)) + col_at(first_col(x + t)));
+        } else if constexpr (RUN) {  // (rows and columns that do not exist: some that do)
+          old[t] = *reinterpret_cast<const Run4 *>(c + row_at(row < p.m ? row : p.m - 1) + col_at(k + 4 > p.n ? p.n - 4 : k));
+        } else {
+#pragma unroll
+          for (int e = 0; e < 4; ++e) old[t][e] = c[!CHECK || (row + e < p.m && k < p.n) ? row_at(row) + e * p.rsc0 + col_at(k) : 0];
+        }
+      }
+    };
+    const auto moved = [&](size_t k, V4 o) __attribute__((always_inline)) {  // the last four columns, moved down to the lane's own
+      if constexpr (CHECK && RUN) {
+        const int by = cols_in(k) > 0 ? 4 - cols_in(k) : 0;
+        if (by & 1) o = V4{o.y, o.z, o.w, o.w};
+        if (by & 2) o = V4{o.z, o.w, o.w, o.w};
+      }
+      return o;
+    };
+
+    V4 next[kBatch];
+    if constexpr (UPDATE) request(row0, 0, next);
+#pragma clang loop unroll(disable)
+    for (unsigned i = 0; i < (unsigned)MI; ++i) {
+      // this row of blocks' sums (accumulators cannot be indexed: a branch for each)
+      T *const to = stage + lane % S * P + lane / S * 4;
+      [&]<int... Is>(std::integer_sequence<int, Is...>) __attribute__((always_inline)) {
+        (
+            [&](auto ic) __attribute__((always_inline)) {
+              constexpr int I = decltype(ic)::value;
+              if (i == I) {
+#pragma unroll
+                for (int j = 0; j < NI; ++j) {
+                  const Acc sums = j < NI / 2 ? fetched<ring_sum_in_a<MI, NI, Acc>(I, 0)>(acc[I][j]) : fetched<ring_sum_in_a<MI, NI, Acc>(I, NI - 1)>(acc[I][j]);
+#pragma unroll
+                  for (int g = 0; g < G; ++g) *reinterpret_cast<V4 *>(to + j * S + g * 8) = V4{sums[4 * g], sums[4 * g + 1], sums[4 * g + 2], sums[4 * g + 3]};
+                }
+              }
+            }(std::integral_constant<int, Is>{}),
+            ...);
+      }(std::make_integer_sequence<int, MI>{});
+      // the wave's own LDS accesses complete in order; the compiler must not move them across each other
+      __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+      __builtin_amdgcn_wave_barrier();
+      const size_t top = row0 + i * S;
+#pragma clang loop unroll(disable)
+      for (unsigned x = 0; x < (unsigned)kPasses; x += kBatch) {
+        V4 v[kBatch];
+#pragma unroll
+        for (int t = 0; t < kBatch; ++t) {
+          const unsigned y = x + t;
+          if constexpr (RUN) {
+            v[t] = *reinterpret_cast<const V4 *>(stage + (y / kSide * 8 + r_lane) * P + y % kSide * 32 + c_lane);
+          } else {
+#pragma unroll
+            for (int e = 0; e < 4; ++e) v[t][e] = stage[(r_lane + e) * P + y * kColsDown + c_lane];
+          }
+        }
+        if constexpr (UPDATE) {
+#pragma unroll
+          for (int t = 0; t < kBatch; ++t) {
+            const V4 old = moved(first_col(x + t) + c_lane, next[t]);
+#pragma unroll
+            for (int e = 0; e < 4; ++e) v[t][e] = skl_combine(v[t][e], old[e], p.alpha, p.beta);
+          }
+          __builtin_amdgcn_sched_barrier(0);  // the next batch's take these registers
+          const bool more = x + kBatch < (unsigned)kPasses, end = !more && i + 1 == (unsigned)MI;  // (the end: once more, not used)
+          request(more || end ? top : top + S, more ? x + kBatch : end ? x : 0, next);
+        } else {
+          bool need = false;
+#pragma unroll
+          for (int t = 0; t < kBatch; ++t)
+#pragma unroll
+            for (int e = 0; e < 4; ++e) need |= skl_initialise_needs_c(v[t][e], p.alpha, p.beta);
+          if (!std::is_same<T, int>::value && __builtin_amdgcn_ballot_w64(need) != 0) {  // the old values decide the sign of some zeros
+            V4 signs[kBatch];
+            request(top, x, signs);
+#pragma unroll
+            for (int t = 0; t < kBatch; ++t) {
+              const V4 o = moved(first_col(x + t) + c_lane, signs[t]);
+#pragma unroll
+              for (int e = 0; e < 4; ++e) v[t][e] = skl_initialise_with(v[t][e], o[e], p.alpha, p.beta);
+            }
+          } else {
+#pragma unroll
+            for (int t = 0; t < kBatch; ++t)
+#pragma unroll
+              for (int e = 0; e < 4; ++e) v[t][e] = skl_initialise_plain(v[t][e], p.alpha, p.beta);
+          }
+        }
+        if constexpr (FUSED) {
+          if (bias) {
+#pragma unroll
+            for (int t = 0; t < kBatch; ++t) {
+              const T by_column = RUN ? T(0) : bias[column_at(first_col(x + t) + c_lane)];
+#pragma unroll
+              for (int e = 0; e < 4; ++e) v[t][e] = skl_add_bias(v[t][e], RUN ? bias_of[t % kSide][e] : by_column);
+            }
+          }
+          if constexpr (STEPS) {  // (the choice outside of the elements: a batch's chains of instructions then run side by side)
+            const auto activate = [&](auto act) __attribute__((always_inline)) {
+#pragma unroll
+              for (int t = 0; t < kBatch; ++t)
+#pragma unroll
+                for (int e = 0; e < 4; ++e) v[t][e] = skl_activate(v[t][e], decltype(act)::value);
+            };
+            if (p.rq.act == 1) activate(std::integral_constant<int, 1>{});
+            if constexpr (!std::is_same<T, int>::value) {
+              if (p.rq.act == 2) activate(std::integral_constant<int, 2>{});
+              if (p.rq.act >= 3) activate(std::integral_constant<int, 3>{});
+            }
+          }
+          if (p.max) {
+#pragma unroll
+            for (int t = 0; t < kBatch; ++t) {
+              const size_t row = first_row(top, x + t) + r_lane, k = first_col(x + t) + c_lane;
+#pragma unroll
+              for (int e = 0; e < 4; ++e)
+                if ((!CHECK || (row + (RUN ? 0 : e) < p.m && k + (RUN ? e : 0) < p.n)) && v[t][e] > running) running = v[t][e];
+            }
+          }
+        }
+        if (!STEPS || !p.rq.q_only) {
+#pragma unroll
+          for (int t = 0; t < kBatch; ++t) {
+            const size_t row = first_row(top, x + t) + r_lane, k = first_col(x + t) + c_lane;
+            if constexpr (RUN) {
+              if (!CHECK || (row < p.m && cols_in(k) == 4)) {
+                Run4 *const at = reinterpret_cast<Run4 *>(c_lane_at + row_at(first_row(top, x + t)) + col_at(first_col(x + t)));
+                if (kept) *at = v[t];
+                else __builtin_nontemporal_store((Run4)v[t], at);
+              } else if (row < p.m) {
+#pragma unroll
+                for (int e = 0; e < 3; ++e)
+                  if (k + e < p.n) c[row_at(row) + col_at(k + e)] = v[t][e];
+              }
+            } else {
+              T *const at = c + row_at(row) + col_at(k);
+              if (p.rsc0 == 1 && (!CHECK || (row + 4 <= p.m && k < p.n))) {
+                *reinterpret_cast<Run4 *>(at) = v[t];
+              } else {
+#pragma unroll
+                for (int e = 0; e < 4; ++e)
+                  if (!CHECK || (row + e < p.m && k < p.n)) at[e * p.rsc0] = v[t][e];
+              }
+            }
+          }
+        }
+        if constexpr (STEPS) {
+          if (p.rq.q) {
+#pragma unroll
+            for (int t = 0; t < kBatch; ++t) {
+              const size_t row = first_row(top, x + t) + r_lane, k = first_col(x + t) + c_lane;
+              const float by_column = RUN ? 0.0f : p.rq.q_scale[p.rq.q_per_column ? column_at(k) : 0];
+              unsigned packed = 0;
+#pragma unroll
+              for (int e = 0; e < 4; ++e) {
+                const float scale = RUN ? scale_of[t % kSide][e] : by_column;
+                const unsigned byte = p.rq.q_fmt == 0 ? (unsigned)skl_requantise_int((float)v[t][e], scale, p.rq.q_zero) & 0xFFu
+                                                      : skl_fp8::encode_ofp8_hw(__fmul_rn((float)v[t][e], scale), f8) & 0xFFu;
+                packed |= byte << (8 * e);
+              }
+              int8_t *const q = reinterpret_cast<int8_t *>(p.rq.q) + row * p.rq.rsq + k * p.rq.csq;
+              if (q_run && (!CHECK || (row < p.m && cols_in(k) == 4))) {
+                *reinterpret_cast<unsigned *>(q) = packed;
+              } else {
+#pragma unroll
+                for (int e = 0; e < 4; ++e)
+                  if (!CHECK || (row + (RUN ? 0 : e) < p.m && k + (RUN ? e : 0) < p.n)) q[e * (RUN ? p.rq.csq : p.rq.rsq)] = (int8_t)(packed >> (8 * e));
+              }
+            }
+          }
+        }
+      }
+      __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+      __builtin_amdgcn_wave_barrier();
+    }
+    if (FUSED && p.max) {
+      const T best = skl_wave_max(running);
+      if (lane == 0 && best > skl_lowest<T>()) skl_atomic_max(reinterpret_cast<T *>(p.max), best);
+    }
+  };
+  // any row-major C, blocks of four columns and more (a lane at the edge reads its old values from the last four columns)
+  const bool run = p.csc0 == 1 && p.ccs >= 2 && (!CHECK || (p.n >= 4 && (p.n % 4 == 0 || p.csc1 == (size_t(1) << p.ccs))));
+  const bool update = !skl_beta_is_zero<T>(p.beta);
+  if (run && (STEPS || p.bias || p.max)) {
+    if (update) write(std::true_type{}, std::true_type{}, std::true_type{});
+    else write(std::true_type{}, std::false_type{}, std::true_type{});
+  } else if (run) {
+    if constexpr (!STEPS) {
+      if (update) write(std::true_type{}, std::true_type{}, std::false_type{});
+      else write(std::true_type{}, std::false_type{}, std::false_type{});
+    }
+  } else {
+    if (update) write(std::false_type{}, std::true_type{}, std::true_type{});
+    else write(std::false_type{}, std::false_type{}, std::true_type{});
+  }
+}
+
+// The raw sums of one share of K, held as in write_wave_rows, to the share's M x N plane.
+template <int MI, int NI, bool CHECK, typename Acc>
+__device__ __forceinline__ void write_wave_plane(const MfmaArgs &p, const Acc (&acc)[MI][NI], size_t row0, size_t col0, unsigned split) {
+  using T = decltype(Acc{}.x);
+  typedef T Run4 __attribute__((ext_vector_type(4), aligned(4)));
+  constexpr int S = sizeof(Acc) == 64 ? 32 : 16, G = S == 32 ? 4 : 1;
+  const int lane = threadIdx.x & 63;
+  T *const plane = reinterpret_cast<T *>(p.partial) + (size_t)split * p.m * p.n;
+#pragma unroll
+  for (int i = 0; i < MI; ++i)
+#pragma unroll
+    for (int j = 0; j < NI; ++j) {
+      const Acc sums = i < MI - 1 || j < NI / 2 ? fetched<true>(acc[i][j]) : fetched<ring_sum_in_a<MI, NI, Acc>(MI - 1, NI - 1)>(acc[i][j]);
+#pragma unroll
+      for (int g = 0; g < G; ++g) {
+        const size_t row = row0 + i * S + lane % S, col = col0 + j * S + g * 8 + lane / S * 4;
+        const Run4 v = {sums[4 * g], sums[4 * g + 1], sums[4 * g + 2], sums[4 * g + 3]};
+        T *const to = plane + row * p.n + col;
+        if (!CHECK || (row < p.m && col + 4 <= p.n)) {
+          *reinterpret_cast<Run4 *>(to) = v;
+        } else if (row < p.m) {
+#pragma unroll
+          for (int e = 0; e < 4; ++e)
+            if (col + e < p.n) to[e] = v[e];
+        }
+      }
+    }
 }
 
 // Tile index of a workgroup. Consecutive workgroup ids go to different XCDs
@@ -1052,11 +1364,11 @@ __global__ void __launch_bounds__(WAVES_M *WAVES_N * 64, (BM == 64 ? 2 : 4)) gem
   } else {
     if constexpr (BM == 64) {  // a tile that lies inside C is written without a test per element
       if (m0 + BM <= p.m && n0 + BN <= p.n) {
-        write_wave_tile<MI, NI, false, 0>(p, acc, m0 + wm, n0 + wn);
+        write_wave_tile<MI, NI, false>(p, acc, m0 + wm, n0 + wn);
         return;
       }
     }
-    write_wave_tile<MI, NI, true, 0>(p, acc, m0 + wm, n0 + wn);
+    write_wave_tile<MI, NI, true>(p, acc, m0 + wm, n0 + wn);
   }
 }
 
@@ -1079,15 +1391,11 @@ __global__ void __launch_bounds__(WAVES_M *WAVES_N * 64, (BM == 64 ? 2 : 4)) gem
 // halves of such a load next to each other: one KiB, as the load writes it.
 // ===========================================================================
 constexpr int kRingSlice = 64;   // bytes of K per stage
-constexpr int kStagedSteps = 4;  // EXTRA: any fused steps, by write_wave_tile_staged
-constexpr int kRingStages = 4;
-// Stages of the ring for tiles of BN columns. The kernel's load schedule is written for any even number of stages;
-// four it is for both tile widths: six stages for the 256 x 128 tile (144 KiB; its slices take half the time, so
-// the same number of slices ahead is half the time ahead) measured no faster - bf16 2048 x 4096 x 4096 without its
-// epilogue 75 us against 71-74 us - i.e. that kernel does not wait for its loads.
-constexpr int ring_stages(int /*bn*/) { return kRingStages; }
-
-template <int ES, bool KC, int ROWS, int NS = kRingStages>
+constexpr int kRingWaves = 4;
+// Stages of an operand's ring: four, or six of an operand with K contiguous where 160 KiB of LDS hold them (see the kernel's loads).
+constexpr int ring_stages_a(bool a_kc, bool b_kc, int bn, bool scan) { return !a_kc || (bn == 256 && (b_kc || scan)) ? 4 : 6; }
+constexpr int ring_stages_b(bool, bool b_kc, int bn, bool scan) { return !b_kc || (bn == 256 && scan) ? 4 : 6; }
+template <int ES, bool KC, int ROWS, int NS, int SIDE>
 struct STile {
   static constexpr int kStages = NS;
   static constexpr int kBytes = ROWS * kRingSlice;            // one stage
@@ -1095,17 +1403,24 @@ struct STile {
   static constexpr int kRowBytes = ROWS * ES;                 // a k-row of an MN-contiguous tile
   static constexpr int kStageStep = KC ? 512 : kBytes;        // from one stage to the next
   static constexpr int kGroup = NS * 512;                     // K-contiguous: from 8 rows to the next 8
+  // K-contiguous: a b128 read is served 16 lanes at a time - 0-3, 12-15 and 20-27, then 4-11, 16-19 and 28-31, and so in the upper
+  // half (found from the conflicts of other arrangements) -, which in 16 x 4 chunks are the 16 rows, eight of them with the next chunk.
+  __device__ static constexpr int turn(int r) { return (r >> 2 & 3) ^ (r >> 1 & 2); }
   // Byte offset (inside stage 0) of 16-byte chunk `c` of line `r`. A line is an M/N row
   // holding 64 bytes of K (KC), or a k-row holding ROWS elements along M/N (MC).
   __device__ static __forceinline__ int chunk(int r, int c) {
     if constexpr (KC)  // 4 chunks: rows r and r+4 share banks, the XOR parts them; 16 rows fill the banks once
-      return (r >> 3) * kGroup + (r & 7) * 64 + ((c ^ ((r >> 2) & 3)) << 4);
-    else if constexpr (ES == 1 && kRowBytes == 256)
+      return (r >> 3) * kGroup + (r & 7) * 64 + ((c ^ turn(r)) << 4);
+    else if constexpr (ES == 2)  // 32 or 16 chunks; 32 lanes of a tr16 read take k-rows r .. r + 3 and r + 8 .. r + 11, 32 B of each
+      return r * kRowBytes + ((c ^ ((r & 3) << 1 | (r & 8))) << 4);
+    else if constexpr (SIDE == 32 && kRowBytes == 256)
       return r * 256 + ((c ^ ((r & 7) << 1)) << 4);   // 16 chunks; tr8 reads take 8 k-rows x 32 B
-    else if constexpr (ES == 1)
+    else if constexpr (SIDE == 32)
       return r * 128 + ((c ^ (((r >> 1) & 3) << 1)) << 4);  // 8 chunks: two k-rows fill the banks once
+    else if constexpr (kRowBytes == 256)  // 32 lanes of a tr8 read take k-rows r .. r + 7 and r + 16 .. r + 23, 16 B of each
+      return r * 256 + ((c ^ ((r & 7) | (r >> 1 & 8))) << 4);
     else
-      return r * kRowBytes + ((c ^ ((r & 3) << 2)) << 4);   // 32 or 16 chunks; tr16 reads take 4 k-rows x 64 B
+      return r * 128 + ((c ^ ((r >> 1 & 3) | (r >> 2 & 4))) << 4);
   }
 };
 
@@ -1113,11 +1428,11 @@ struct STile {
 // for an MN-contiguous operand and a pair of slices for a K-contiguous one.
 // EDGE: the operand ends inside the tile, along M / N or along K. Its loads go through a buffer descriptor whose base follows K
 // as a scalar; a lane whose 16 bytes do not exist holds an offset beyond the descriptor's range, for which the load writes zeros
-// to LDS and touches no memory. The offsets of rows beyond M / N are so from the start; those of k beyond the end become so
-// with the first unit that holds any (mask()).
-template <int ES, bool KC, int WAVES, int ROWS, int NS, bool EDGE>
+// to LDS and touches no memory. The offsets of rows beyond M / N are so from the start; those of k beyond the end are chosen
+// with every load (offset()).
+template <int ES, bool KC, int WAVES, int ROWS, int NS, int SIDE, bool EDGE>
 struct SLoader {
-  using T = STile<ES, KC, ROWS, NS>;
+  using T = STile<ES, KC, ROWS, NS, SIDE>;
   static constexpr unsigned kRange = 0xC0000000u, kOutside = 0xE0000000u;  // (the host checks that offsets stay below kRange)
   static constexpr int kUnitBytes = KC ? 2 * T::kBytes : T::kBytes;
   static constexpr int kBlocks = kUnitBytes / 1024 / WAVES;  // KiB blocks per wave and unit
@@ -1125,7 +1440,8 @@ struct SLoader {
   const char *tile_base;
   size_t k_step;           // bytes from one unit to the next
   unsigned off[kBlocks];   // global byte offsets of this lane
-  unsigned lds[kBlocks];   // LDS byte offsets (inside the operand's region, stage 0) of the blocks
+  unsigned lds;            // LDS byte offset (inside the operand's region, stage 0) of block 0
+  static constexpr unsigned kBlockStep = KC ? T::kGroup : 1024;  // ... and from one block to the next
   unsigned k_lane;         // EDGE: where along K the lane's 16 bytes of block 0 lie in a unit - KC: bytes, MC: k rows
   unsigned k_total;        // EDGE: bytes / k rows of K
 
@@ -1134,6 +1450,7 @@ struct SLoader {
     // vector add and a v_readfirstlane per load, and lds[] lives in scalar registers.
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
     tile_base = base + (mn0 >> 6) * s1 * ES;
+    lds = wave * kBlocks * kBlockStep;
     if constexpr (EDGE) {  // spelled out as scalars, like the step below: a descriptor in vector registers costs a loop over the lanes per load
       const uintptr_t at = (uintptr_t)tile_base;
       tile_base = (const char *)(((uintptr_t)(unsigned)__builtin_amdgcn_readfirstlane((int)(at >> 32)) << 32) | (unsigned)__builtin_amdgcn_readfirstlane((int)at));
@@ -1143,9 +1460,8 @@ struct SLoader {
       const int b = wave * kBlocks + i;
       if constexpr (KC) {  // block = 8 rows x (64 bytes of the even slice, then 64 bytes of the odd one)
         const int half = lane >> 5, row = 8 * b + ((lane & 31) >> 2), pos = lane & 3;
-        const int c = pos ^ ((row >> 2) & 3);
+        const int c = pos ^ T::turn(row);
         off[i] = (unsigned)(((size_t)(row >> 6) * s1 + (size_t)(row & 63) * s0) * ES + half * 64 + c * 16);
-        lds[i] = b * T::kGroup;
         if constexpr (EDGE) {
           static_assert(kBlocks % 2 == 0, "c of block i is that of block 0 with its second bit turned for odd i");
           if (i == 0) k_lane = half * 64 + c * 16;
@@ -1156,7 +1472,6 @@ struct SLoader {
         const int kr = kRowsPerBlock * b + lane / kLanesPerRow, pos = lane % kLanesPerRow;
         const int mn = ((T::chunk(kr, pos) - kr * T::kRowBytes) >> 4) * (16 / ES);  // the chunk stored at position `pos`
         off[i] = (unsigned)(((size_t)(mn >> 6) * s1 + (size_t)(mn & 63) + (size_t)kr * sk) * ES);
-        lds[i] = b * 1024;
         if constexpr (EDGE) {
           if (i == 0) k_lane = kr;
           if (mn0 + mn >= mn_dim) off[i] = kOutside;
@@ -1170,36 +1485,33 @@ struct SLoader {
     k_step = ((size_t)(unsigned)__builtin_amdgcn_readfirstlane((int)(step >> 32)) << 32) | (unsigned)__builtin_amdgcn_readfirstlane((int)step);
   }
 
-  // EDGE: the first unit that K ends in (or ends before), and the offsets from `unit` on, one after another from that one.
+  // EDGE: how much of K (bytes / k rows) is left from the start of `unit` on, and the offset of the lane's 16 bytes of block i of a
+  // unit of which so much exists. (Chosen for every load: a branch for the last units, in a loop whose sums are all of the accumulation
+  // registers, has the compiler move a block of sums about behind a product that is still under way.)
   static constexpr unsigned kUnitK = KC ? 2 * kRingSlice : kRingSlice / ES;
-  __device__ __forceinline__ unsigned first_masked() const { return k_total / kUnitK; }
-  __device__ __forceinline__ void mask(unsigned unit) {
-#pragma unroll
-    for (int i = 0; i < kBlocks; ++i) {
-      const unsigned at = unit * kUnitK + (KC ? k_lane ^ (unsigned)(i & 1) * 32u : k_lane + (unsigned)i * (1024 / T::kRowBytes));
-      off[i] = at < k_total ? off[i] : kOutside;
-    }
+  __device__ __forceinline__ unsigned left_of(unsigned unit) const { return k_total > unit * kUnitK ? k_total - unit * kUnitK : 0; }
+  __device__ __forceinline__ unsigned offset(unsigned left, int i) const {
+    if constexpr (!EDGE) return off[i];
+    if constexpr (KC) return (k_lane ^ (unsigned)(i & 1) * 32u) < left ? off[i] : kOutside;
+    const unsigned rows_above = (unsigned)i * (1024 / T::kRowBytes);
+    return k_lane < (left > rows_above ? left - rows_above : 0) ? off[i] : kOutside;
   }
 
   // Requests block `i` of `unit`; it lands in stage `stage` (the even one of the pair for KC) of `region`.
-  __device__ __forceinline__ void issue_one(char *region, int stage, size_t unit, int i) const {
+  __device__ __forceinline__ void issue_one(char *region, int stage, size_t unit, unsigned left, int i) const {
     const char *g = tile_base + unit * k_step;
     // The lane's offset through a copy the compiler cannot follow: it otherwise widens every offset to 64 bits ahead
     // of the loop (two registers each) and adds the scalar base with a 64-bit vector add per load; this way the load
     // takes the scalar base and the 32-bit offset as they are.
-    unsigned o = off[i];
+    unsigned o = offset(left, i);
     asm volatile("" : "+v"(o));
     if constexpr (EDGE)
       __builtin_amdgcn_raw_ptr_buffer_load_lds(__builtin_amdgcn_make_buffer_rsrc((void *)g, 0, (int)kRange, 0x00027000),
-                                               (__attribute__((address_space(3))) void *)(region + stage * T::kStageStep + lds[i]), 16, (int)o, 0, 0, 0);
+                                               (__attribute__((address_space(3))) void *)(region + stage * T::kStageStep + lds + i * kBlockStep), 16, (int)o, 0, 0, 0);
     else
       __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void *)(g + o),
-                                       (__attribute__((address_space(3))) void *)(region + stage * T::kStageStep + lds[i]),
+                                       (__attribute__((address_space(3))) void *)(region + stage * T::kStageStep + lds + i * kBlockStep),
                                        16, 0, 0);
-  }
-  __device__ __forceinline__ void issue(char *region, int stage, size_t unit) const {
-#pragma unroll
-    for (int i = 0; i < kBlocks; ++i) issue_one(region, stage, unit, i);
   }
 };
 
@@ -1231,6 +1543,12 @@ __device__ __forceinline__ v4i lds_read_b128(unsigned addr) {
   return r;
 }
 template <int OFF>
+__device__ __forceinline__ v2i lds_read_b64(unsigned addr) {
+  v2i r;
+  asm volatile("ds_read_b64 %0, %1 offset:%2" : "=v"(r) : "v"(addr), "n"(OFF) : "memory");
+  return r;
+}
+template <int OFF>
 __device__ __forceinline__ v2i lds_read_tr8(unsigned addr) {
   v2i r;
   asm volatile("ds_read_b64_tr_b8 %0, %1 offset:%2" : "=v"(r) : "v"(addr), "n"(OFF) : "memory");
@@ -1243,49 +1561,53 @@ __device__ __forceinline__ v2i lds_read_tr16(unsigned addr) {
   return r;
 }
 
-// The fragments of one operand for one wave: NFRAG blocks of 32 rows, read from a stage in pieces of one
-// LDS instruction each. Offsets inside the stage are per lane and computed once; what changes from k-step to
-// k-step and from fragment to fragment is, wherever the swizzle allows, an immediate offset.
-template <int ES, bool KC, int FRB, int KB, int ROWS, int NS, int NFRAG>
+// The fragments of one operand for one wave: NFRAG blocks of SIDE rows with the 64 bytes of K of a stage, read in pieces of
+// one LDS instruction each. Lane l holds row l % SIDE; its FRB bytes of K are the (l / SIDE)-th of the stage. Offsets inside the
+// stage are per lane and computed once; what changes from fragment to fragment is, wherever the swizzle allows, an immediate
+// offset, else an exclusive or.
+// EXACT: two pieces of eight bytes, one for each of two products of 32 bytes of K. Lane groups 0 to 3 hold the first, third, second and
+// fourth eight bytes of the 32: the products are then added up in the order of the bounds-checked kernels, which take a 16-byte
+// fragment's low halves first, so that a call's sums are the same on both.
+template <int ES, bool KC, int FRB, int ROWS, int NS, int SIDE, bool EXACT>
 struct FragReader {
-  using T = STile<ES, KC, ROWS, NS>;
-  using Piece = typename std::conditional<KC, v4i, v2i>::type;
+  using T = STile<ES, KC, ROWS, NS, SIDE>;
   static constexpr int RB = T::kRowBytes;
-  static constexpr int kPieceBytes = KC ? 16 : 8;
+  static constexpr int kPieceBytes = KC && !EXACT ? 16 : 8;
+  using Piece = typename std::conditional<kPieceBytes == 16, v4i, v2i>::type;
   static constexpr int kPieces = FRB / kPieceBytes;  // LDS instructions per fragment
-  static constexpr int kSteps = kRingSlice / KB;
-  static constexpr int kBases = KC ? kSteps * kPieces : NFRAG;
+  static constexpr int kBases = KC ? kPieces : 1;
+  static constexpr int kTurn = SIDE * ES;            // fragment f: its columns' chunks are those of fragment 0 with f * kTurn turned
+  static_assert(FRB * (64 / SIDE) == kRingSlice, "a fragment takes the whole stage");
+  static_assert(!EXACT || (ES == 1 && SIDE == 16));
   unsigned base[kBases];
 
   __device__ void init(int row0) {
-    const int lane = threadIdx.x & 63, h = lane >> 5;
+    const int lane = threadIdx.x & 63, g = lane / SIDE;
+    [[maybe_unused]] const int eighth = (g & 1) * 2 + (g >> 1);  // EXACT: which eight bytes of 32
     if constexpr (KC) {
 #pragma unroll
-      for (int ks = 0; ks < kSteps; ++ks)
-#pragma unroll
-        for (int pc = 0; pc < kPieces; ++pc)
-          base[ks * kPieces + pc] = (unsigned)T::chunk(row0 + (lane & 31), ((ks * KB + h * FRB) >> 4) + pc);
-    } else if constexpr (ES == 1) {
-      const int g16 = (lane >> 4) & 1, j = lane & 15;
-#pragma unroll
-      for (int f = 0; f < NFRAG; ++f)
-        base[f] = (unsigned)(T::chunk(h * FRB + (j >> 1), ((row0 + 32 * f) >> 4) + g16) + (j & 1) * 8);
+      for (int pc = 0; pc < kPieces; ++pc)
+        base[pc] = EXACT ? (unsigned)(T::chunk(row0 + lane % SIDE, 2 * pc + (eighth >> 1)) + (eighth & 1) * 8) : (unsigned)T::chunk(row0 + lane % SIDE, ((g * FRB) >> 4) + pc);
     } else {
-      const int g16 = (lane >> 4) & 1, j = lane & 15;
-#pragma unroll
-      for (int f = 0; f < NFRAG; ++f)
-        base[f] = (unsigned)(T::chunk(h * 8 + (j >> 2), ((row0 + 32 * f) >> 3) + g16 * 2 + ((j & 3) >> 1)) + (j & 1) * 8);
+      // 16 lanes read 8 k-rows x 16 bytes (16-bit: 4 k-rows x 16 elements), lane j receives column j
+      const int g16 = SIDE == 32 ? (lane >> 4) & 1 : 0, j = lane & 15;
+      if constexpr (ES == 1)
+        base[0] = (unsigned)(T::chunk((EXACT ? eighth * 8 : g * FRB) + (j >> 1), (row0 >> 4) + g16) + (j & 1) * 8);
+      else
+        base[0] = (unsigned)(T::chunk(g * (FRB / 2) + (j >> 2), (row0 >> 3) + g16 * 2 + ((j & 3) >> 1)) + (j & 1) * 8);
     }
   }
-  // Piece PC of fragment F for k-step KS of the stage at LDS address `stage`.
-  template <int F, int KS, int PC>
+  // Piece PC of fragment F of the stage at LDS address `stage`.
+  template <int F, int PC>
   __device__ __forceinline__ Piece read(unsigned stage) const {
-    if constexpr (KC)
-      return lds_read_b128<F * 4 * T::kGroup>(stage + base[KS * kPieces + PC]);  // 32 rows = four groups of 8
+    if constexpr (KC && EXACT)
+      return lds_read_b64<F * (SIDE / 8) * T::kGroup>(stage + base[PC]);
+    else if constexpr (KC)
+      return lds_read_b128<F * (SIDE / 8) * T::kGroup>(stage + base[PC]);
     else if constexpr (ES == 1)
-      return lds_read_tr8<KS * KB * RB + PC * 8 * RB>(stage + base[F]);
+      return lds_read_tr8<PC * (EXACT ? 32 : 8) * RB>(stage + (base[0] ^ (unsigned)(F * kTurn)));
     else
-      return lds_read_tr16<KS * (KB / 2) * RB + PC * 4 * RB>(stage + base[F]);
+      return lds_read_tr16<PC * 4 * RB>(stage + (base[0] ^ (unsigned)(F * kTurn)));
   }
 };
 
@@ -1327,75 +1649,68 @@ constexpr int ceil_div(int a, int b) { return (a + b - 1) / b; }
 // more vector work than the matrix cores take for the products; here six for eight (256 columns) or four for four (128).
 // E4M3 2048 x 8192 x 2048: 77 us there,
 // 62 here (1.1 PFLOP/s, what the f16 kernel reaches).
-template <int TA, int TB, bool A_KC, bool B_KC, int BN, bool EDGE = false, int EXTRA = 0, bool CQUADS = false, bool SCAN = false, bool EXACT = false>
-__global__ void __launch_bounds__(512) gemm_mfma_ring_kernel(MfmaArgs p) {
-  using KA = Kind<TA>;
-  using M = typename std::conditional<EXACT, MmaF8Exact<TA, TB>, Mma<TA, TB>>::type;
+template <int TA, int TB, bool A_KC, bool B_KC, int BN, bool EDGE = false, bool STEPS = false, bool SCAN = false, bool EXACT = false>
+__global__ void __launch_bounds__(kRingWaves * 64) gemm_mfma_ring_kernel(MfmaArgs p) {
+  using M = RingMma<TA, TB, EXACT>;
   using Frag = typename M::Frag;
-  using Acc = typename KA::Acc;
+  using Acc = typename M::Acc;
   using AccElem = decltype(Acc{}.x);
-  constexpr int SB = kRingSlice, STAGES = ring_stages(BN);
-  static_assert(STAGES % 2 == 0, "pair loads fill two neighbouring stages");
-  constexpr int ES = KA::ES, KB = EXACT ? 32 : KA::KB, FRB = KB / 2;
-  // Eight waves: 2 x 4 blocks of 128 x 64 on a 256 x 256 tile, 4 x 2 blocks of 64 x 64 on a 256 x 128 one.
-  constexpr int BM = 256, WAVES = 8, WAVES_N = BN == 256 ? 4 : 2, WAVES_M = WAVES / WAVES_N;
-  constexpr int WM = BM / WAVES_M, WN = BN / WAVES_N, MI = WM / 32, NI = WN / 32;
-  constexpr int kEpilogueBatch = 2;              // blocks whose old C values are requested together
-  constexpr int kSteps = SB / KB;
-  constexpr int kMfmas = MI * NI;
-  constexpr int kSlots = kSteps * kMfmas;        // MFMA slots per slice
-  constexpr int kPre = (kSteps - 1) * kMfmas;    // slots before the slice's barrier
-  // Four stages per operand. A slice's fragments are read from LDS while the k-step before them is
-  // multiplied; with one k-step per slice (64 bytes of K per MFMA) that is the slice before, and the
-  // stage of the slice being multiplied is free from its barrier on. So loads run kExtra = 1 slice
-  // further ahead there: every-slice loads fill the issuing slice's own stage with slice s+4, pair loads
-  // go out on odd slices for slices s+3 and s+4. Otherwise: slice s+3, and pairs on even slices for
-  // s+2 and s+3. (Six stages for a K-contiguous operand fit the 160 KiB of LDS next to an MN-contiguous
-  // partner, and measured slower.)
-  constexpr int NSA = STAGES, NSB = STAGES;
-  constexpr int kExtra = kSteps == 1 ? 1 : 0;
-  constexpr int kEachAhead = STAGES - 1 + kExtra, kPairAhead = STAGES - 2 + kExtra;
-  constexpr int kPairU = kPairAhead & 1;             // parity of the slices that issue pair loads
-  constexpr int kPairsPrologue = (kPairU + kPairAhead) / 2;
-  using LA = SLoader<ES, A_KC, WAVES, BM, NSA, EDGE>;
-  using LB = SLoader<ES, B_KC, WAVES, BN, NSB, EDGE>;
-  using TileA = STile<ES, A_KC, BM, NSA>;
-  using TileB = STile<ES, B_KC, BN, NSB>;
-  // Load `it` of a slice's kLoads goes out behind MFMA slot it * kSlots / kLoads, pair loads first.
-  constexpr int kPairA = A_KC ? LA::kBlocks : 0, kPairB = B_KC ? LB::kBlocks : 0;
-  constexpr int kEachA = A_KC ? 0 : LA::kBlocks, kEachB = B_KC ? 0 : LB::kBlocks;
-  constexpr int kEach = kEachA + kEachB, kPairs = kPairA + kPairB;
-  constexpr int kLoadsOfU[2] = {(kPairU == 0 ? kPairs : 0) + kEach, (kPairU == 1 ? kPairs : 0) + kEach};
-  // SCAN: one more load in every even slice, the first thing that slice requests (behind its first MFMA, in front
-  // of its pair loads): older than every load of its slice, so it has landed whenever the slice's own loads are
-  // waited for. It counts as younger wherever a whole slice counted below is an even one, and in front of the
-  // barrier of its own slice when that barrier is not in the slice's first k-step.
-  constexpr int kScanSlots = 4, kScanSlot = WAVES * 1024;
-  static_assert(!SCAN || (std::is_same<AccElem, float>::value && !EDGE && EXTRA == 0 && !CQUADS), "a plain floating-point product on whole tiles");
-  static_assert(kPairAhead <= 3, "the rows requested in slice 2q are read back in slices 2q + 3 and 2q + 4");
-  constexpr int kPreOfU[2] = {ceil_div(kPre * kLoadsOfU[0], kSlots), ceil_div(kPre * kLoadsOfU[1], kSlots)};
-  constexpr auto younger = [](int u, const int (&loads)[2], int each, int pair_ahead, bool scan, int pre_slots) {
-    int n = u == 0 ? 0 : each;
-    // the whole slices counted: t - pair_ahead + u + d for d = 1 .. pair_ahead - 1 - u, t (of parity u) being this slice
-    for (int d = 1; d <= pair_ahead - 1 - u; ++d) {
-      n += loads[(u + d) % 2];
-      if (scan && (pair_ahead + d) % 2 == 0) n += 1;
-    }
-    if (scan && u == 0 && pre_slots > 0) n += 1;  // this slice's own, requested in its first k-step
-    return n;
-  };
-  constexpr int kInFlightOfU[2] = {younger(0, kLoadsOfU, kEach, kPairAhead, SCAN, kPre) + kPreOfU[0],
-                                   younger(1, kLoadsOfU, kEach, kPairAhead, SCAN, kPre) + kPreOfU[1]};
-  static_assert(STAGES != 4 || SCAN || (kInFlightOfU[0] == (kExtra ? 2 * kEach + kPairs : kEach) + kPreOfU[0] &&
-                                        kInFlightOfU[1] == (kExtra ? 2 * kEach : kEach) + kPreOfU[1]),
-                "the four-stage counts, as derived by hand above");
-  static_assert(kInFlightOfU[0] < 64 && kInFlightOfU[1] < 64, "vmcnt is a 6-bit counter");
-
-  using RA = FragReader<ES, A_KC, FRB, KB, BM, NSA, MI>;
-  using RB = FragReader<ES, B_KC, FRB, KB, BN, NSB, NI>;
+  constexpr int SB = kRingSlice, NSA = ring_stages_a(A_KC, B_KC, BN, SCAN), NSB = ring_stages_b(A_KC, B_KC, BN, SCAN);
+  constexpr int ES = Kind<TA>::ES, S = M::kSide, FRB = M::kFrag;
+  constexpr int BM = 256, WAVES = kRingWaves, WAVES_N = 2, WAVES_M = WAVES / WAVES_N;
+  constexpr int WM = BM / WAVES_M, WN = BN / WAVES_N, MI = WM / S, NI = WN / S;
+  // A step is a slice: the products of the wave's blocks, once, or EXACT with each half of the fragments' bytes.
+  constexpr int kProducts = MI * NI, kSlots = (EXACT ? 2 : 1) * kProducts;
+  using LA = SLoader<ES, A_KC, WAVES, BM, NSA, S, EDGE>;
+  using LB = SLoader<ES, B_KC, WAVES, BN, NSB, S, EDGE>;
+  using TileA = STile<ES, A_KC, BM, NSA, S>;
+  using TileB = STile<ES, B_KC, BN, NSB, S>;
+  using RA = FragReader<ES, A_KC, FRB, BM, NSA, S, EXACT>;
+  using RB = FragReader<ES, B_KC, FRB, BN, NSB, S, EXACT>;
   constexpr int PA = RA::kPieces, PB = RB::kPieces;
-  constexpr int kReads = MI * PA + NI * PB;      // LDS instructions per k-step
-  constexpr int kReadSlots = kMfmas / 2;         // ... issued behind the first half of its MFMAs, the rest is time to land (all of them behind the first of four MFMAs on the narrow tile: 73.5-74.0 against 72.7-73.0 us)
+  constexpr int kReadsB = NI * PB, kReads = kReadsB + MI * PA;  // LDS instructions per step
+  constexpr int kReadSlots = kProducts * 3 / 4;                 // ... behind the first of its products, the rest is time to land
+  // Item r of n that are spread over m slots goes out in slot r * m / n.
+  constexpr auto first_in_slot = [](int q, int n, int m) { return q >= m ? n : (q * n + m - 1) / m; };
+  // ... and a load, so as not to meet a read, half of the way on to the next one's.
+  constexpr auto first_load = [](int q, int n, int m) { return q >= m ? n : q * 2 * n <= m ? 0 : (2 * q * n - m + 2 * m - 1) / (2 * m); };
+  // The loads of step s, in this order (U: parity of s):
+  //   an operand with K contiguous and four stages: behind the barrier of an odd slice the pair s + 3, s + 4, whose stages it frees;
+  //   with six stages: in odd steps the first blocks of the pair s + 5, s + 6, in even steps the rest of the pair s + 4, s + 5 -
+  //   half each, or, next to an operand of four stages, all of them in even steps;
+  //   an operand read across K: slice s + 4.
+  // What counts is that they are evenly spread: a load keeps the compute unit's address path for 16 cycles, four waves request at
+  // the same time, and a wave that has to wait for the path does not issue products either (bf16 8192^3 with K contiguous, epilogue
+  // left out: 64 loads within 512 / 768 / 1024 cycles of a step of 1024 761 / 738 / 728 us, in two steps SPREAD_US).
+  constexpr auto blocks_of = [](int u, bool kc, int ns, int blocks, bool beside_four) {
+    if (!kc) return 0;
+    if (ns == 4) return u == 1 ? blocks : 0;
+    return beside_four ? (u == 0 ? blocks : 0) : blocks / 2;
+  };
+  constexpr bool kBesideFour = A_KC && B_KC && (NSA == 4) != (NSB == 4);
+  constexpr int kPairA[2] = {blocks_of(0, A_KC, NSA, LA::kBlocks, kBesideFour), blocks_of(1, A_KC, NSA, LA::kBlocks, kBesideFour)};
+  constexpr int kPairB[2] = {blocks_of(0, B_KC, NSB, LB::kBlocks, kBesideFour), blocks_of(1, B_KC, NSB, LB::kBlocks, kBesideFour)};
+  constexpr int kEachA = A_KC ? 0 : LA::kBlocks, kEachB = B_KC ? 0 : LB::kBlocks, kEach = kEachA + kEachB;
+  constexpr int kLoadsOfU[2] = {kPairA[0] + kPairB[0] + kEach, kPairA[1] + kPairB[1] + kEach};
+  static_assert(!kBesideFour || NSA == 4, "loads of four-stage operands come first");
+  constexpr int kScanSlots = 4, kScanSlot = WAVES * 1024;
+  static_assert(!SCAN || (std::is_same<AccElem, float>::value && !EDGE && !STEPS), "a plain floating-point product on whole tiles");
+  // Loads that may be in flight at the barrier of slice s (of parity U), where slice s + 1 has to have landed: what has been requested
+  // behind the last load that brings any of it. SCAN: one more load in front of each step's.
+  constexpr auto in_flight = [=](int u) {
+    constexpr int sc = SCAN ? 1 : 0, n[2] = {kLoadsOfU[0] + sc, kLoadsOfU[1] + sc};
+    constexpr bool four = (A_KC && NSA == 4) || (B_KC && NSB == 4), six = (A_KC && NSA == 6) || (B_KC && NSB == 6);
+    constexpr int c4 = (A_KC && NSA == 4 ? LA::kBlocks : 0) + (B_KC && NSB == 4 ? LB::kBlocks : 0);
+    int most = 63;
+    const auto at_most = [&](int x) { most = x < most ? x : most; };
+    if (four) at_most(kLoadsOfU[1] - c4 + n[0] + (u == 0 ? n[1] : 0));  // step s - 2, or s - 3, then what followed
+    if (six && u == 1) at_most(kEach + n[1] + n[0]);                    // step s - 3
+    if (kEach) at_most(n[u] + n[u ^ 1]);                                // step s - 3, whose last loads these are
+    if (SCAN) at_most(kLoadsOfU[u ^ 1] + n[u] + n[u ^ 1]);              // the rows requested in step s - 3 are read in step s
+    return most;
+  };
+  constexpr int kInFlightOfU[2] = {in_flight(0), in_flight(1)};
+  static_assert(kInFlightOfU[1] + kLoadsOfU[1] < 64, "vmcnt is a 6-bit counter");
 
   extern __shared__ __attribute__((aligned(16))) char smem[];
   char *region_a = smem, *region_b = smem + TileA::kRegion;
@@ -1407,7 +1722,7 @@ __global__ void __launch_bounds__(512) gemm_mfma_ring_kernel(MfmaArgs p) {
   const unsigned tiles = p.tiles_m * p.tiles_n, split = blockIdx.x / tiles;
   tile_of_block<false>(blockIdx.x % tiles, p, tm, tn);
   const size_t m0 = (size_t)tm * BM, n0 = (size_t)tn * BN;
-  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;  // the wave index as a scalar: nothing derived from it occupies a vector register across the main loop
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);  // as a scalar: nothing derived from it occupies a vector register across the main loop
   const int wm = (wave / WAVES_N) * WM, wn = (wave % WAVES_N) * WN;
 
   LA la;
@@ -1425,36 +1740,34 @@ __global__ void __launch_bounds__(512) gemm_mfma_ring_kernel(MfmaArgs p) {
 #pragma unroll
     for (int j = 0; j < NI; ++j)
 #pragma unroll
-      for (int r = 0; r < 16; ++r) acc[i][j][r] = 0;
+      for (int r = 0; r < (int)(sizeof(Acc) / 4); ++r) acc[i][j][r] = 0;
 
   // K is a whole number of slice pairs (EDGE: what is missing is zeros). Units beyond the end are requested as the last unit
   // again: in range, and the stage they land in is never read, which keeps the load counts static.
   // (32-bit counters - the host refuses a K of 2^31 slices or more: a 64-bit "less than" of two scalars is a vector
   // compare and two vector registers)
   const unsigned slices = EDGE ? (unsigned)((p.k * ES + 2 * SB - 1) / (2 * SB)) * 2 : (unsigned)(p.k * ES / SB), pairs = slices / 2;
-  [[maybe_unused]] const unsigned mask_a = EDGE ? la.first_masked() : 0, mask_b = EDGE ? lb.first_masked() : 0;
 
-  // SCAN: the tile's old C, 1 KiB per wave and two slices (the host has checked that K has the slices for it and
+  // SCAN: the tile's old C, 1 KiB per wave and slice (the host has checked that K has the slices for it and
   // that C is row-major with 16-byte aligned rows).
   unsigned long long scan_bad = 0;   // lanes that have seen a NaN or an infinity
-  v2i scan_pend = {0, 0};            // the 8 bytes read back during the k-step before
+  v4i scan_pend = {0, 0, 0, 0};      // the 16 bytes read back during the step before
   char *const scan_region = smem + TileA::kRegion + TileB::kRegion + wave * 1024;
   const unsigned scan_addr = addr_b + TileB::kRegion + wave * 1024;
   // (row of this wave's first load, and the bytes from one load's rows to the next: scalars, 64 x rsc0 fits 32 bits)
   constexpr unsigned kScanRowsPerLoad = BN == 256 ? 1 : 2, kScanLoadsPerWave = BM / (WAVES * kScanRowsPerLoad);
   // C in panels of 64 x 64 contiguous values (rsc0 == 64): 1 KiB is four rows of a panel; the tile's panels row by
-  // row, 16 such pieces each, piece 8 q + w is wave w's load q.
+  // row, 16 such pieces each, piece WAVES * q + w is wave w's load q.
   const bool scan_panels = p.rsc0 == 64 && p.rsc1 != 64 * 64;
   const char *const scan_rows = scan_panels ? reinterpret_cast<const char *>(p.c) + ((m0 >> 6) * p.rsc1 + (n0 >> 6) * p.csc1) * 4
                                             : reinterpret_cast<const char *>(p.c) + ((m0 + (size_t)wave * kScanRowsPerLoad) * p.rsc0 + n0) * 4;
   const unsigned scan_step = (unsigned)p.rsc0 * (WAVES * kScanRowsPerLoad * 4u);
-  [[maybe_unused]] auto scan_issue = [&](size_t s) {  // s even: load s / 2 of this wave (the last one again beyond the tile)
-    const unsigned q = (unsigned)(s >> 1) < kScanLoadsPerWave ? (unsigned)(s >> 1) : kScanLoadsPerWave - 1;  // uniform
-    const char *rows = scan_rows + (size_t)q * scan_step;
-    if (scan_panels) {
-      const unsigned piece = q * WAVES + wave, panel = piece >> 4, pi = panel / (BN / 64), pj = panel % (BN / 64);
-      rows = scan_rows + ((size_t)pi * p.rsc1 + (size_t)pj * p.csc1) * 4 + (piece & 15u) * 1024u;
-    }
+  [[maybe_unused]] auto scan_issue = [&](unsigned s) {  // load s of this wave (the last one again beyond the tile)
+    const unsigned q = s < kScanLoadsPerWave ? s : kScanLoadsPerWave - 1;  // uniform
+    // (no branch, see SLoader::offset)
+    const unsigned piece = q * WAVES + wave, panel = piece >> 4, pi = panel / (BN / 64), pj = panel % (BN / 64);
+    const size_t in_panels = ((size_t)pi * p.rsc1 + (size_t)pj * p.csc1) * 4 + (piece & 15u) * 1024u;
+    const char *rows = scan_rows + (scan_panels ? in_panels : (size_t)q * scan_step);
     // The lane's own part of the address is computed anew for every load, from a lane index the compiler cannot
     // follow: held across the loop it would be a register that the loop does not have.
     unsigned l = __builtin_amdgcn_mbcnt_hi(~0u, __builtin_amdgcn_mbcnt_lo(~0u, 0u));
@@ -1465,59 +1778,48 @@ __global__ void __launch_bounds__(512) gemm_mfma_ring_kernel(MfmaArgs p) {
     else
       mine = (l & 31u) * 16u + ((unsigned)((int)(l << 26) >> 31) & (scan_panels ? 512u : (unsigned)p.rsc0 * 4u));  // lanes 32-63: the row below (panels: the next 512 bytes)
     __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void *)(rows + mine),
-                                     (__attribute__((address_space(3))) void *)(scan_region + (unsigned)((s >> 1) % kScanSlots) * kScanSlot), 16, 0, 0);
+                                     (__attribute__((address_space(3))) void *)(scan_region + s % kScanSlots * kScanSlot), 16, 0, 0);
   };
-  [[maybe_unused]] auto scan_read = [&](unsigned slot, unsigned half) {  // 512 of this wave's 1024 bytes in `slot`; the value counts from the next lgkmcnt(0) on
+  [[maybe_unused]] auto scan_read = [&](unsigned slot) {  // this wave's 1024 bytes in `slot`; the value counts from the next lgkmcnt(0) on
     unsigned l = __builtin_amdgcn_mbcnt_hi(~0u, __builtin_amdgcn_mbcnt_lo(~0u, 0u));
     asm volatile("" : "+v"(l));
-    const unsigned addr = scan_addr + slot * kScanSlot + half * 512 + l * 8;
-    asm volatile("ds_read_b64 %0, %1" : "=v"(scan_pend) : "v"(addr) : "memory");
+    const unsigned addr = scan_addr + slot * kScanSlot + l * 16;
+    asm volatile("ds_read_b128 %0, %1" : "=v"(scan_pend) : "v"(addr) : "memory");
   };
-  [[maybe_unused]] auto scan_check = [&]() {  // behind an lgkmcnt(0): NaN or infinity, either sign, in either dword
+  [[maybe_unused]] auto scan_check = [&]() {  // behind an lgkmcnt(0): NaN or infinity, either sign, in any dword
     asm volatile("" : "+v"(scan_pend));
-    unsigned long long x, y;
-    asm volatile("v_cmp_class_f32_e64 %0, %1, %2" : "=s"(x) : "v"(scan_pend.x), "s"(0x207));
-    asm volatile("v_cmp_class_f32_e64 %0, %1, %2" : "=s"(y) : "v"(scan_pend.y), "s"(0x207));
-    scan_bad |= x | y;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      unsigned long long x;
+      const int word = scan_pend[e];
+      asm volatile("v_cmp_class_f32_e64 %0, %1, %2" : "=s"(x) : "v"(word), "s"(0x207));
+      scan_bad |= x;
+    }
   };
 
-  if constexpr (A_KC) {
+  // What the steps before the first would have requested, in their order, so that the counts of the main loop hold from its start.
+  // (Units beyond the end are requested as the last one again; so are they in the main loop.)
+  const auto request_a = [&](int unit, int first, int last) __attribute__((always_inline)) {
+    const unsigned u = (unsigned)unit < (A_KC ? pairs : slices) ? (unsigned)unit : (A_KC ? pairs : slices) - 1;
 #pragma unroll
-    for (int i = 0; i < kPairsPrologue; ++i) {
-      const unsigned unit = (unsigned)i < pairs ? (unsigned)i : pairs - 1;
-      if constexpr (EDGE) {
-        if (unit >= mask_a) la.mask(unit);
-      }
-      la.issue(region_a, 2 * i, unit);
-    }
-  } else {
+    for (int i = first; i < last; ++i) la.issue_one(region_a, (A_KC ? 2 : 1) * unit, u, EDGE ? la.left_of(u) : 0, i);
+  };
+  const auto request_b = [&](int unit, int first, int last) __attribute__((always_inline)) {
+    const unsigned u = (unsigned)unit < (B_KC ? pairs : slices) ? (unsigned)unit : (B_KC ? pairs : slices) - 1;
 #pragma unroll
-    for (int i = 0; i < kEachAhead; ++i) {
-      const unsigned unit = (unsigned)i < slices ? (unsigned)i : slices - 1;
-      if constexpr (EDGE) {
-        if (unit >= mask_a) la.mask(unit);
-      }
-      la.issue(region_a, i, unit);
-    }
-  }
-  if constexpr (B_KC) {
+    for (int i = first; i < last; ++i) lb.issue_one(region_b, (B_KC ? 2 : 1) * unit, u, EDGE ? lb.left_of(u) : 0, i);
+  };
 #pragma unroll
-    for (int i = 0; i < kPairsPrologue; ++i) {
-      const unsigned unit = (unsigned)i < pairs ? (unsigned)i : pairs - 1;
-      if constexpr (EDGE) {
-        if (unit >= mask_b) lb.mask(unit);
-      }
-      lb.issue(region_b, 2 * i, unit);
-    }
-  } else {
-#pragma unroll
-    for (int i = 0; i < kEachAhead; ++i) {
-      const unsigned unit = (unsigned)i < slices ? (unsigned)i : slices - 1;
-      if constexpr (EDGE) {
-        if (unit >= mask_b) lb.mask(unit);
-      }
-      lb.issue(region_b, i, unit);
-    }
+  for (int step = -5; step < 0; ++step) {
+    const int u = step & 1;
+    if (A_KC && NSA == 4 && u == 1 && step + 3 >= 0) request_a((step + 3) / 2, 0, LA::kBlocks);
+    if (B_KC && NSB == 4 && u == 1 && step + 3 >= 0) request_b((step + 3) / 2, 0, LB::kBlocks);
+    if (A_KC && NSA == 6 && u == 1) request_a((step + 5) / 2, 0, kPairA[1]);
+    if (A_KC && NSA == 6 && u == 0) request_a((step + 4) / 2, kPairA[1], LA::kBlocks);
+    if (B_KC && NSB == 6 && u == 1) request_b((step + 5) / 2, 0, kPairB[1]);
+    if (B_KC && NSB == 6 && u == 0) request_b((step + 4) / 2, kPairB[1], LB::kBlocks);
+    if (!A_KC && step + 4 >= 0) request_a(step + 4, 0, LA::kBlocks);
+    if (!B_KC && step + 4 >= 0) request_b(step + 4, 0, LB::kBlocks);
   }
   if constexpr (SCAN) {  // the slots start as zeros: the first slices read slots that no load has filled yet
 #pragma unroll
@@ -1526,33 +1828,22 @@ __global__ void __launch_bounds__(512) gemm_mfma_ring_kernel(MfmaArgs p) {
       for (int quarter = 0; quarter < 4; ++quarter)
         *reinterpret_cast<float *>(scan_region + slot * kScanSlot + quarter * 256 + (threadIdx.x & 63) * 4) = 0.0f;
   }
-  wait_loads_upto<0>();
-  __syncthreads();
+  wait_loads_upto<(SCAN ? 0 : kInFlightOfU[1] + kLoadsOfU[1])>();  // slice 0
+  asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+  __builtin_amdgcn_s_barrier();
 
   typename RA::Piece pa[2][MI][PA];
   typename RB::Piece pb[2][NI][PB];
-
-  // Read item R of a k-step: fragment by fragment, A and B alternating, so that
-  // what the next k-step's first MFMAs need is requested first.
-  auto read_item = [&](auto rc, auto ksc, int buf, unsigned stage_a, unsigned stage_b) {
-    constexpr int R = decltype(rc)::value, KS = decltype(ksc)::value;
-    constexpr int kPair = PA + PB, kBoth = (MI < NI ? MI : NI) * kPair;
-    if constexpr (R < kBoth) {
-      constexpr int F = R / kPair, W = R % kPair;
-      if constexpr (W < PA)
-        pa[buf][F][W] = ra.template read<F, KS, W>(stage_a);
-      else
-        pb[buf][F][W - PA] = rb.template read<F, KS, W - PA>(stage_b);
-    } else if constexpr (MI > NI) {
-      constexpr int X = R - kBoth, F = NI + X / PA, W = X % PA;
-      pa[buf][F][W] = ra.template read<F, KS, W>(stage_a);
-    } else {
-      constexpr int X = R - kBoth, F = MI + X / PB, W = X % PB;
-      pb[buf][F][W] = rb.template read<F, KS, W>(stage_b);
-    }
+  // LDS read R of a step, into the registers of buffer `buf`: B's fragments, then A's in the order of their use.
+  const auto read_item = [&](auto rc, auto bufc, unsigned stage_a, unsigned stage_b) __attribute__((always_inline)) {
+    constexpr int R = decltype(rc)::value, BUF = decltype(bufc)::value;
+    if constexpr (R < kReadsB)
+      pb[BUF][R / PB][R % PB] = rb.template read<R / PB, R % PB>(stage_b);
+    else
+      pa[BUF][(R - kReadsB) / PA][(R - kReadsB) % PA] = ra.template read<(R - kReadsB) / PA, (R - kReadsB) % PA>(stage_a);
   };
   // All reads in flight have landed; from here on the compiler may use buffer `buf`.
-  auto landed = [&](int buf) {
+  const auto landed = [&](int buf) __attribute__((always_inline)) {
     asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
 #pragma unroll
     for (int i = 0; i < MI; ++i)
@@ -1565,218 +1856,148 @@ __global__ void __launch_bounds__(512) gemm_mfma_ring_kernel(MfmaArgs p) {
   };
 
   [&]<int... Rs>(std::integer_sequence<int, Rs...>) __attribute__((always_inline)) {
-    (read_item(std::integral_constant<int, Rs>{}, std::integral_constant<int, 0>{}, 0, addr_a, addr_b), ...);
+    (read_item(std::integral_constant<int, Rs>{}, std::integral_constant<int, 0>{}, addr_a, addr_b), ...);
   }(std::make_integer_sequence<int, kReads>{});
 
-  // Two slices per trip: the parity of the slice decides which loads it issues, and (for the
-  // operand kinds with one k-step per slice) which fragment buffer a k-step uses.
-  for (unsigned s0 = 0; s0 < slices; s0 += 2) {
+  // EXACT: the operands as they are multiplied. A's fragments are widened a row of blocks ahead, B's half a step ahead.
+  [[maybe_unused]] v8h wide_a[2], wide_b[EXACT ? 2 : 1][NI];
+  if constexpr (EXACT) {
+    landed(0);
+    wide_a[0] = M::widen_a(join_pieces<Frag>(pa[0][0]), 0);
+#pragma unroll
+    for (int j = 0; j < NI; ++j) wide_b[0][j] = M::widen_b(join_pieces<Frag>(pb[0][j]), 0);
+  }
+
+  // Two slices per trip: the parity of the slice decides which loads follow its barrier and which registers hold its fragments.
+  [[maybe_unused]] unsigned six = 0;  // s0 % 6
+  unsigned s0 = 0;
+  do {  // (K is not empty)
+    [[maybe_unused]] const unsigned six_next = six == 4 ? 0 : six + 2;
     [&]<int... Us>(std::integer_sequence<int, Us...>) __attribute__((always_inline)) {
       (
           [&](auto uc) __attribute__((always_inline)) {
             constexpr int U = decltype(uc)::value;
             constexpr int kLoads = kLoadsOfU[U];
             const unsigned s = s0 + U;
-            const unsigned fill_slice = s + kEachAhead < slices ? s + kEachAhead : slices - 1;  // every-slice operands
-            const unsigned fill_pair = (s + kPairAhead) / 2 < pairs ? (s + kPairAhead) / 2 : pairs - 1;  // pair operands (s of parity kPairU)
-            const unsigned s32 = s;
-            const int cur_a = (int)(s32 % NSA), nxt_a = (int)((s32 + 1) % NSA), cur_b = (int)(s32 % NSB), nxt_b = (int)((s32 + 1) % NSB);
-            const int fill_a = (int)((s32 + (A_KC ? kPairAhead : kEachAhead)) % NSA), fill_b = (int)((s32 + (B_KC ? kPairAhead : kEachAhead)) % NSB);
-            [&]<int... KSs>(std::integer_sequence<int, KSs...>) __attribute__((always_inline)) {
+            unsigned unit_a, unit_b, next_a, next_b;
+            [[maybe_unused]] unsigned left_a = 0, left_b = 0;  // of K, from these units on (EDGE)
+            int fill_a, fill_b;
+            [[maybe_unused]] unsigned lds_a, lds_b;
+            [[maybe_unused]] const char *from_a, *from_b;
+            // The reads below are of the next slice: its data must have landed for every wave. Own reads first: the stage refilled
+            // behind the barrier is the one that everybody has read.
+            wait_loads_upto<kInFlightOfU[U]>();
+            landed(U);
+            __builtin_amdgcn_s_barrier();
+            __builtin_amdgcn_sched_barrier(0);
+            [&]<int... Qs>(std::integer_sequence<int, Qs...>) __attribute__((always_inline)) {
               (
-                  [&](auto ksc) __attribute__((always_inline)) {
-                    constexpr int KS = decltype(ksc)::value;
-                    constexpr bool kLast = KS == kSteps - 1;
-                    constexpr int KSN = kLast ? 0 : KS + 1;  // k-step whose fragments are read during this one
-                    constexpr int cur = (U * kSteps + KS) & 1, nx = cur ^ 1;
-                    if constexpr (kLast) {
-                      // The reads below cross into the next slice: its data must have landed for every wave.
-                      // Own reads first, so that nobody's read of the stage refilled next is still in flight.
-                      wait_loads_upto<kInFlightOfU[U]>();
-                      landed(cur);
-                      __builtin_amdgcn_s_barrier();
-                    } else {
-                      landed(cur);
-                    }
-                    Frag fa[MI], fb[NI];
-#pragma unroll
-                    for (int i = 0; i < MI; ++i) fa[i] = join_pieces<Frag>(pa[cur][i]);
-#pragma unroll
-                    for (int j = 0; j < NI; ++j) fb[j] = join_pieces<Frag>(pb[cur][j]);
-                    decltype(prep_a<M>(fa[0])) wa[MI];  // as the multiply wants them
-                    decltype(prep_b<M>(fb[0])) wb[NI];
-                    if constexpr (EXACT) {
-                      wa[0] = prep_a<M>(fa[0]);
-#pragma unroll
-                      for (int j = 0; j < NI; ++j) wb[j] = prep_b<M>(fb[j]);
-                    } else {
-#pragma unroll
-                      for (int i = 0; i < MI; ++i) wa[i] = fa[i];
-#pragma unroll
-                      for (int j = 0; j < NI; ++j) wb[j] = fb[j];
-                    }
-                    const unsigned sa = addr_a + (kLast ? nxt_a : cur_a) * TileA::kStageStep;
-                    const unsigned sb = addr_b + (kLast ? nxt_b : cur_b) * TileB::kStageStep;
+                  [&](auto qc) __attribute__((always_inline)) {
+                    constexpr int Q = decltype(qc)::value, X = Q / kProducts, i = Q % kProducts / NI, j = Q % NI;  // X: half of the fragments' bytes (EXACT)
+                    const auto fragment_a = [&]() __attribute__((always_inline)) { if constexpr (EXACT) return wide_a[i & 1]; else return join_pieces<Frag>(pa[U][i]); };
+                    const auto fragment_b = [&]() __attribute__((always_inline)) { if constexpr (EXACT) return wide_b[X][j]; else return join_pieces<Frag>(pb[U][j]); };
+                    // this slot's load, if it has one
+                    constexpr int L = first_load(Q, kLoads, kSlots), kLoadsHere = first_load(Q + 1, kLoads, kSlots) - L;
+                    constexpr bool kHasLoad = kLoadsHere > 0 && !EDGE && Q > 0;  // with the product (what it needs is worked out behind the first)
+                    // load l is block block_of(l) of A's unit or (not of_a(l)) of B's; of six stages, odd steps load the first blocks, even ones the rest
+                    constexpr auto of_a = [](int l) { return l < kPairA[U] || (l >= kPairA[U] + kPairB[U] && l - kPairA[U] - kPairB[U] < kEachA); };
+                    constexpr auto block_of = [](int l) {
+                      constexpr int six_a = A_KC && NSA == 6 && U == 0 ? kPairA[1] : 0, six_b = B_KC && NSB == 6 && U == 0 ? kPairB[1] : 0;
+                      if (l < kPairA[U]) return l + six_a;
+                      if (l < kPairA[U] + kPairB[U]) return l - kPairA[U] + six_b;
+                      const int each = l - kPairA[U] - kPairB[U];
+                      return each < kEachA ? each : each - kEachA;
+                    };
+                    constexpr bool kOfA = of_a(L);
+                    constexpr int kBlock = kHasLoad ? block_of(L) : 0;
+                    constexpr bool kInA = ring_sum_in_a<MI, NI, Acc>(i, j);
+                    if constexpr (!kHasLoad)
+                      M::template run<kInA>(fragment_a(), fragment_b(), acc[i][j]);
+                    else if constexpr (kOfA)
+                      M::template run<kInA, (kBlock * LA::kBlockStep)>(fragment_a(), fragment_b(), acc[i][j], lds_a, from_a, la.off[kBlock]);
+                    else
+                      M::template run<kInA, (kBlock * LB::kBlockStep)>(fragment_a(), fragment_b(), acc[i][j], lds_b, from_b, lb.off[kBlock]);
+                    // The MFMA first, what belongs to its slot in its shadow. Left to itself the compiler moves a slot's address
+                    // arithmetic, reads and loads in front of the MFMA - and behind a barrier, which the waves leave together,
+                    // instructions in front of the first MFMA are a gap in every SIMD's matrix core at once.
                     __builtin_amdgcn_sched_barrier(0);
-                    [&]<int... Qs>(std::integer_sequence<int, Qs...>) __attribute__((always_inline)) {
-                      (
-                          [&](auto qc) __attribute__((always_inline)) {
-                            constexpr int Q = decltype(qc)::value, kSlot = KS * kMfmas + Q;
-                            constexpr int i = Q / NI, j = Q % NI;
-                            acc[i][j] = M::run(wa[i], wb[j], acc[i][j]);
-                            // The MFMA first, what belongs to its slot in its shadow. Left to itself the compiler moves a slot's address
-                            // arithmetic, reads and loads in front of the MFMA - and behind a barrier, which the waves leave together,
-                            // instructions in front of the first MFMA are a gap in every SIMD's matrix core at once (measured, same job,
-                            // alternating libraries: int8 8192^3 -1.5 %, fp8 with column-major A -3 %, bf16 config 3 -2.3 %; for the
-                            // extra instructions of SCAN the difference between +43 and +14 us).
-                            __builtin_amdgcn_sched_barrier(0);
-                            if constexpr (EXACT && j == 0 && i + 1 < MI) wa[i + 1] = prep_a<M>(fa[i + 1]);
-                            if constexpr (EDGE && kSlot == 0) {  // what this slice requests may reach the end of K
-                              if constexpr (!A_KC || U == kPairU) {
-                                if ((A_KC ? fill_pair : fill_slice) >= mask_a) la.mask(A_KC ? fill_pair : fill_slice);
-                              }
-                              if constexpr (!B_KC || U == kPairU) {
-                                if ((B_KC ? fill_pair : fill_slice) >= mask_b) lb.mask(B_KC ? fill_pair : fill_slice);
-                              }
-                            }
-                            if constexpr (SCAN && U == 0 && kSlot == 0) scan_issue(s);
-                            if constexpr (SCAN && kSlot == 1) scan_check();  // what the last slot of the k-step before has read, behind this k-step's lgkmcnt(0)
-                            // Behind the barrier of slice 2q + 3 the rows requested in slice 2q have landed: half of them is
-                            // read back in that slice, half in the next (the first slices find zeros).
-                            if constexpr (SCAN && kSlot == kSlots - 1) scan_read(((s32 >> 1) + kScanSlots - (U == 1 ? 1 : 2)) % kScanSlots, U == 1 ? 0 : 1);
-                            // this slot's share of the next k-step's reads
-                            [&]<int... Rs>(std::integer_sequence<int, Rs...>) __attribute__((always_inline)) {
-                              (
-                                  [&](auto rc) __attribute__((always_inline)) {
-                                    constexpr int R = decltype(rc)::value;
-                                    if constexpr (R * kReadSlots / kReads == Q)
-                                      read_item(rc, std::integral_constant<int, KSN>{}, nx, sa, sb);
-                                  }(std::integral_constant<int, Rs>{}),
-                                  ...);
-                            }(std::make_integer_sequence<int, kReads>{});
-                            // and this slot's share of the slice's loads
-                            [&]<int... Ls>(std::integer_sequence<int, Ls...>) __attribute__((always_inline)) {
-                              (
-                                  [&](auto lc) __attribute__((always_inline)) {
-                                    constexpr int L = decltype(lc)::value;
-                                    if constexpr (L * kSlots / kLoads == kSlot) {
-                                      constexpr int kPairsNow = U == kPairU ? kPairs : 0;
-                                      if constexpr (L < kPairsNow) {
-                                        if constexpr (L < kPairA)
-                                          la.issue_one(region_a, fill_a, fill_pair, L);
-                                        else
-                                          lb.issue_one(region_b, fill_b, fill_pair, L - kPairA);
-                                      } else if constexpr (L - kPairsNow < kEachA) {
-                                        la.issue_one(region_a, fill_a, fill_slice, L - kPairsNow);
-                                      } else {
-                                        lb.issue_one(region_b, fill_b, fill_slice, L - kPairsNow - kEachA);
-                                      }
-                                    }
-                                  }(std::integral_constant<int, Ls>{}),
-                                  ...);
-                            }(std::make_integer_sequence<int, kLoads>{});
-                            __builtin_amdgcn_sched_barrier(0);
-                          }(std::integral_constant<int, Qs>{}),
-                          ...);
-                    }(std::make_integer_sequence<int, kMfmas>{});
-                  }(std::integral_constant<int, KSs>{}),
+                    if constexpr (Q == 0) {
+                      // The stage of the next slice, the unit to load and the stage it goes to, of an operand with `stages` stages.
+                      const auto next_stage = [&](int stages) { return stages == 6 ? (U == 0 ? six + 1 : six_next) : (s + 1) % 4; };
+                      const auto unit = [&](bool kc, int stages) {
+                        const unsigned x = kc ? (stages == 6 ? s0 + 4 + 2 * U : s + 3) / 2 : s + 4, most = (kc ? pairs : slices) - 1;
+                        return x < most ? x : most;
+                      };
+                      const auto fill_stage = [&](bool kc, int stages) { return stages == 6 ? (U == 1 ? six : six == 0 ? 4 : six - 2) : (s + (kc ? 3 : 4)) % 4; };
+                      unit_a = unit(A_KC, NSA), unit_b = unit(B_KC, NSB);
+                      if constexpr (EDGE) left_a = la.left_of(unit_a), left_b = lb.left_of(unit_b);
+                      fill_a = (int)fill_stage(A_KC, NSA), fill_b = (int)fill_stage(B_KC, NSB);
+                      next_a = addr_a + next_stage(NSA) * TileA::kStageStep, next_b = addr_b + next_stage(NSB) * TileB::kStageStep;
+                      lds_a = addr_a + fill_a * TileA::kStageStep + la.lds, lds_b = addr_b + fill_b * TileB::kStageStep + lb.lds;
+                      from_a = la.tile_base + (size_t)unit_a * la.k_step;
+                      from_b = lb.tile_base + (size_t)unit_b * lb.k_step;
+                    }
+                    if constexpr (EXACT) {
+                      static_assert(MI % 2 == 0);
+                      if constexpr (X == 1 && Q == kProducts) landed(U ^ 1);
+                      if constexpr (j == 0) {
+                        if constexpr (i + 1 < MI) wide_a[(i + 1) & 1] = M::widen_a(join_pieces<Frag>(pa[U][i + 1]), X);
+                        else wide_a[0] = M::widen_a(join_pieces<Frag>(pa[X ? U ^ 1 : U][0]), X ^ 1);
+                      }
+                      if constexpr (j == NI / 2 && i < NI) wide_b[X ^ 1][i] = M::widen_b(join_pieces<Frag>(pb[X ? U ^ 1 : U][i]), X ^ 1);
+                    }
+                    if constexpr (SCAN && Q == 0) scan_issue(s);
+                    if constexpr (SCAN && Q == 1) scan_check();  // what the last read of the step before has brought, behind this step's wait
+                    // this slot's share of the next step's reads
+                    [&]<int... Rs>(std::integer_sequence<int, Rs...>) __attribute__((always_inline)) {
+                      (read_item(std::integral_constant<int, first_in_slot(Q, kReads, kReadSlots) + Rs>{}, std::integral_constant<int, U ^ 1>{}, next_a, next_b), ...);
+                    }(std::make_integer_sequence<int, first_in_slot(Q + 1, kReads, kReadSlots) - first_in_slot(Q, kReads, kReadSlots)>{});
+                    if constexpr (SCAN && Q == kReadSlots) scan_read((s + 1) % kScanSlots);  // the rows of three slices before (the first slices find zeros)
+#pragma unroll
+                    for (int l = L + (kHasLoad ? 1 : 0); l < L + kLoadsHere; ++l) {
+                      if (of_a(l))
+                        la.issue_one(region_a, fill_a, unit_a, left_a, block_of(l));
+                      else
+                        lb.issue_one(region_b, fill_b, unit_b, left_b, block_of(l));
+                    }
+                    __builtin_amdgcn_sched_barrier(0);
+                  }(std::integral_constant<int, Qs>{}),
                   ...);
-            }(std::make_integer_sequence<int, kSteps>{});
+            }(std::make_integer_sequence<int, kSlots>{});
           }(std::integral_constant<int, Us>{}),
           ...);
     }(std::make_integer_sequence<int, 2>{});
-  }
-  asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");
+    // The sums' registers are not to be read before the last product has written them, and the compiler, to which these are no matrix
+    // instructions, may copy one as soon as the loop is left: the time the product takes anyway.
+    asm volatile("s_nop %0" ::"n"(S == 32 ? 15 : 3));
+    six = six_next;
+    s0 += 2;
+  } while (s0 < slices);
+  __builtin_amdgcn_s_waitcnt(0x0070);  // vmcnt(0) lgkmcnt(0), as the compiler understands it: it takes the loads to LDS above for pending with every read of LDS below
+  landed(0);  // the last step's reads, of a slice that does not exist: their registers are theirs up to here
+  asm volatile("s_nop 15\n\ts_nop 15" ::: "memory");  // the last products' results (the compiler does not see that these are matrix instructions)
+  [&]<int... Bs>(std::integer_sequence<int, Bs...>) __attribute__((always_inline)) {
+    ((acc[Bs / NI][Bs % NI] = fetched<ring_sum_in_a<MI, NI, Acc>(Bs / NI, Bs % NI)>(acc[Bs / NI][Bs % NI])), ...);
+  }(std::make_integer_sequence<int, MI * NI>{});
   if constexpr (SCAN) {
-    // The last rows requested have not been read back or in part only, and the last 8 bytes read have not been
-    // tested: all slots once more (a row tested twice changes nothing).
+    // The last rows requested have not been read back: all slots once more (a row tested twice changes nothing).
     scan_check();
 #pragma unroll
-    for (int slot = 0; slot < kScanSlots; ++slot)
-#pragma unroll
-      for (int half = 0; half < 2; ++half) {
-        scan_read(slot, half);
-        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-        scan_check();
-      }
+    for (int slot = 0; slot < kScanSlots; ++slot) {
+      scan_read(slot);
+      asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+      scan_check();
+    }
   }
 
   if (p.splits > 1) {  // a share of K: the raw sums go to this split's M x N plane
-    AccElem *plane = reinterpret_cast<AccElem *>(p.partial) + (size_t)split * p.m * p.n;
-#pragma unroll
-    for (int j = 0; j < NI; ++j) {
-      const size_t col = n0 + wn + j * 32 + (lane & 31);
-      if (EDGE && col >= p.n) continue;
-#pragma unroll
-      for (int i = 0; i < MI; ++i)
-#pragma unroll
-        for (int r = 0; r < 16; ++r) {
-          const size_t row = m0 + wm + i * 32 + (r >> 2) * 8 + (lane >> 5) * 4 + (r & 3);
-          if (!EDGE || row < p.m) plane[row * p.n + col] = acc[i][j][r];
-        }
-    }
+    write_wave_plane<MI, NI, EDGE>(p, acc, m0 + wm, n0 + wn, split);
     return;
   }
-  if constexpr (CQUADS) {
-    // A lane holds four consecutive rows of one column, and with blocks of four columns a row of a block is 16
-    // bytes: stored as they are, a wave's stores are 16-byte runs 64 bytes apart (8192^3: 100 us more than a
-    // row-major C). The four lanes of a quad hold the four columns of those rows, so the 4 x 4 values are exchanged
-    // inside the quad - lane q ends up with row q's four columns - and every lane moves 16 bytes per instruction: a
-    // quad covers 64 contiguous bytes, lanes 0-31 eight neighbouring blocks.
-    static_assert(std::is_same<AccElem, int>::value && !EDGE && EXTRA == 0, "int32 C, whole tiles, no fused steps");
-    int *c = reinterpret_cast<int *>(p.c);
-    const bool init = p.beta.i == 0;
-    const int qd = lane & 3;
-    const size_t cmask = (size_t(1) << p.ccs) - 1, rmask = (size_t(1) << p.crs) - 1;
-#pragma unroll
-    for (int j = 0; j < NI; ++j) {
-      const size_t col4 = n0 + wn + j * 32 + (lane & 28);   // the quad's first column, a multiple of four
-      const size_t col_off = (col4 >> p.ccs) * p.csc1 + (col4 & cmask);
-#pragma unroll
-      for (int i0 = 0; i0 < MI; i0 += kEpilogueBatch) {
-        v4i *out[kEpilogueBatch][4];
-        v4i old[kEpilogueBatch][4];
-#pragma unroll
-        for (int i = 0; i < kEpilogueBatch; ++i)
-#pragma unroll
-          for (int g = 0; g < 4; ++g) {
-            const size_t row = m0 + wm + (i0 + i) * 32 + g * 8 + (lane >> 5) * 4 + qd;
-            out[i][g] = reinterpret_cast<v4i *>(c + (row >> p.crs) * p.rsc1 + (row & rmask) * p.rsc0 + col_off);
-          }
-        if (!init) {
-#pragma unroll
-          for (int i = 0; i < kEpilogueBatch; ++i)
-#pragma unroll
-            for (int g = 0; g < 4; ++g) old[i][g] = *out[i][g];
-        }
-#pragma unroll
-        for (int i = 0; i < kEpilogueBatch; ++i)
-#pragma unroll
-          for (int g = 0; g < 4; ++g) {
-            const Acc &t = acc[i0 + i][j];
-            v4i r;
-#define SKL_ROW_OF_QUAD(CC, CTRL)                                                                                    \
-  {                                                                                                                   \
-    const int b0 = __builtin_amdgcn_update_dpp(0, t[4 * g + 0], CTRL, 0xF, 0xF, true), b1 = __builtin_amdgcn_update_dpp(0, t[4 * g + 1], CTRL, 0xF, 0xF, true); \
-    const int b2 = __builtin_amdgcn_update_dpp(0, t[4 * g + 2], CTRL, 0xF, 0xF, true), b3 = __builtin_amdgcn_update_dpp(0, t[4 * g + 3], CTRL, 0xF, 0xF, true); \
-    r[CC] = qd == 0 ? b0 : qd == 1 ? b1 : qd == 2 ? b2 : b3;                                                          \
-  }
-            SKL_ROW_OF_QUAD(0, 0x00)   // quad_perm: every lane reads the quad's lane 0 - column 0 of the four rows
-            SKL_ROW_OF_QUAD(1, 0x55)
-            SKL_ROW_OF_QUAD(2, 0xAA)
-            SKL_ROW_OF_QUAD(3, 0xFF)
-#undef SKL_ROW_OF_QUAD
-            v4i v;
-#pragma unroll
-            for (int e = 0; e < 4; ++e) v[e] = init ? skl_initialise(r[e], (const int *)nullptr, p.alpha, p.beta) : skl_combine(r[e], old[i][g][e], p.alpha, p.beta);
-            __builtin_nontemporal_store(v, out[i][g]);
-          }
-      }
-    }
-    return;
-  }
+  constexpr int kStageBytes = S * wave_rows_pitch<WN>() * 4;
+  static_assert(WAVES * kStageBytes <= TileA::kRegion + TileB::kRegion, "the waves' rows take the place of the operand stages");
   if constexpr (SCAN) {
-    // What the eight waves have found, put together: each wave's word where its first slot began (its own reads of
+    // What the waves have found, put together: each wave's word where its first slot began (its own reads of
     // the slots are over), a barrier, and everybody reads all eight.
     unsigned *const found = reinterpret_cast<unsigned *>(smem + TileA::kRegion + TileB::kRegion);
     found[wave * 256] = scan_bad != 0;
@@ -1786,14 +2007,10 @@ __global__ void __launch_bounds__(512) gemm_mfma_ring_kernel(MfmaArgs p) {
     for (int w = 0; w < WAVES; ++w) any |= found[w * 256];
     MfmaArgs q = p;
     if (any == 0) q.beta.fz.skip_c_read = 1;  // 0 * c is a zero everywhere in this tile
-    write_wave_tile<MI, NI, EDGE, EXTRA>(q, acc, m0 + wm, n0 + wn);
-  } else if constexpr (EXTRA == kStagedSteps) {
-    constexpr int kStageBytes = 32 * staged_pitch<NI>() * 4;
-    static_assert(WAVES * kStageBytes <= TileA::kRegion + TileB::kRegion, "the waves' rows take the place of the operand stages");
-    __syncthreads();  // every wave's reads of the stages and loads into them are over
-    write_wave_tile_staged<MI, NI, EDGE>(p, acc, m0 + wm, n0 + wn, smem + wave * kStageBytes);
+    write_wave_rows<MI, NI, EDGE, STEPS>(q, acc, m0 + wm, n0 + wn, smem + wave * kStageBytes);
   } else {
-    write_wave_tile<MI, NI, EDGE, EXTRA>(p, acc, m0 + wm, n0 + wn);
+    __syncthreads();  // every wave's reads of the stages and loads into them are over
+    write_wave_rows<MI, NI, EDGE, STEPS>(p, acc, m0 + wm, n0 + wn, smem + wave * kStageBytes);
   }
 }
 
@@ -1926,22 +2143,14 @@ inline bool c_in_row_quads(const MfmaArgs &p) {
          (((uintptr_t)p.c | (p.rsc0 * 4) | (p.rsc1 * 4) | (p.csc1 * 4)) & 15) == 0;
 }
 
-template <int TA, int TB, bool A_KC, bool B_KC, int BN, bool EDGE = false, int EXTRA = 0, bool CQUADS = false, bool SCAN = false, bool EXACT = false>
+template <int TA, int TB, bool A_KC, bool B_KC, int BN, bool EDGE = false, bool STEPS = false, bool SCAN = false, bool EXACT = false>
 int launch_ring(const MfmaArgs &args) {
-  if constexpr (EXTRA == 0 && !CQUADS && !SCAN && kRingCarriesExtraSteps<TA, TB>) {
-    using Steps = FusedSteps<decltype(typename Kind<TA>::Acc{}.x), 2>;
-    if ((args.rq.act || args.rq.q) && !(!EDGE && !EXACT && Steps::dword_copy(args.rq)))
-      return launch_ring<TA, TB, A_KC, B_KC, BN, EDGE, kStagedSteps, false, false, EXACT>(args);
-  }
-  if constexpr (EXTRA == 0 && kRingCarriesExtraSteps<TA, TB> && !EDGE && !EXACT) {
-    if (args.rq.q) return args.rq.q_only ? launch_ring<TA, TB, A_KC, B_KC, BN, EDGE, 2>(args) : launch_ring<TA, TB, A_KC, B_KC, BN, EDGE, 3>(args);
-  }
-  if constexpr (TA == SKL_DT_I8 && TB == SKL_DT_I8 && A_KC && B_KC && !EDGE && EXTRA == 0 && !CQUADS) {  // what copies of blocked operands look like
-    if (c_in_row_quads(args)) return launch_ring<TA, TB, A_KC, B_KC, BN, EDGE, 0, true>(args);
+  if constexpr (!STEPS && !SCAN && kRingCarriesExtraSteps<TA, TB>) {
+    if (args.rq.act || args.rq.q) return launch_ring<TA, TB, A_KC, B_KC, BN, EDGE, true, false, EXACT>(args);
   }
   constexpr int ES = Kind<TA>::ES;
   using AccElem = decltype(typename Kind<TA>::Acc{}.x);
-  if constexpr (std::is_same<AccElem, float>::value && !EDGE && EXTRA == 0 && !CQUADS && !SCAN && !EXACT) {
+  if constexpr (std::is_same<AccElem, float>::value && !EDGE && !STEPS && !SCAN && !EXACT) {
     // beta == 0 evaluated as the reference's loops do (0 * c: a NaN or an infinity in C stays a NaN): the old C is
     // looked through while the tile is multiplied, 8 KiB of it per two slices - needs 64 slices on the wide tile, 32
     // on the narrow one, a tile to itself (no shared K) and a row-major C.
@@ -1955,10 +2164,11 @@ int launch_ring(const MfmaArgs &args) {
     const bool panels = args.csc0 == 1 && args.rsc0 == 64 && args.crs == 6 && args.ccs == 6 && args.rsc1 != 64 * 64 &&
                         (((uintptr_t)args.c | (args.rsc1 * 4) | (args.csc1 * 4)) & 15) == 0;
     if (args.beta.f == 0.0f && args.beta.fz.skip_c_read == 0 && !shared_k && (row_major || panels) && scan_slices >= (BN == 256 ? 64 : 32))
-      return launch_ring<TA, TB, A_KC, B_KC, BN, EDGE, EXTRA, CQUADS, true>(args);
+      return launch_ring<TA, TB, A_KC, B_KC, BN, EDGE, false, true>(args);
   }
-  constexpr int lds = ring_stages(BN) * (256 + BN) * kRingSlice + (SCAN ? 4 * 8 * 1024 : 0);
-  auto kernel = gemm_mfma_ring_kernel<TA, TB, A_KC, B_KC, BN, EDGE, EXTRA, CQUADS, SCAN, EXACT>;
+  constexpr int lds = (ring_stages_a(A_KC, B_KC, BN, SCAN) * 256 + ring_stages_b(A_KC, B_KC, BN, SCAN) * BN) * kRingSlice + (SCAN ? 4 * kRingWaves * 1024 : 0);
+  static_assert(lds <= 160 * 1024);
+  auto kernel = gemm_mfma_ring_kernel<TA, TB, A_KC, B_KC, BN, EDGE, STEPS, SCAN, EXACT>;
   static std::atomic<bool> configured{false};  // per instantiation; racing threads set the same value
   if (!configured.load(std::memory_order_acquire)) {
     int rc = skl_check_hip(hipFuncSetAttribute(reinterpret_cast<const void *>(kernel),
@@ -1990,7 +2200,7 @@ int launch_ring(const MfmaArgs &args) {
     skl_hip_record_error(-2, "gemm_mfma: grid too large");
     return -2;
   }
-  kernel<<<(unsigned)grid, 512, lds, skl_current_stream()>>>(p);
+  kernel<<<(unsigned)grid, kRingWaves * 64, lds, skl_current_stream()>>>(p);
   int rc = skl_check_launch("gemm_mfma_ring");
   if (rc != 0 || p.splits == 1) return rc;
   return launch_split_reduce<AccElem>(p, "gemm_split_reduce");
@@ -2155,8 +2365,8 @@ int launch_whole_tiles(const MfmaArgs &p) {
   constexpr int ES = Kind<TA>::ES;
   constexpr size_t kRing128FromTiles = 96;
   using AccElem = decltype(typename Kind<TA>::Acc{}.x);
-  const auto wide = [](const MfmaArgs &q) { return launch_ring<TA, TB, A_KC, B_KC, 256, false, 0, false, false, EXACT>(q); };
-  const auto narrow = [](const MfmaArgs &q) { return launch_ring<TA, TB, A_KC, B_KC, 128, false, 0, false, false, EXACT>(q); };
+  const auto wide = [](const MfmaArgs &q) { return launch_ring<TA, TB, A_KC, B_KC, 256, false, false, false, EXACT>(q); };
+  const auto narrow = [](const MfmaArgs &q) { return launch_ring<TA, TB, A_KC, B_KC, 128, false, false, false, EXACT>(q); };
   if (p.m % 256 != 0 || p.n % 128 != 0 || (p.k * ES) % 128 != 0 || p.a_loose || p.b_loose) return kNotWholeTiles;
   const size_t tiles_m = p.m / 256, slices = p.k * ES / kRingSlice;
   const size_t tiles = p.n % 256 == 0 ? tiles_m * (p.n / 256) : 0, tiles128 = tiles_m * (p.n / 128);
@@ -2167,7 +2377,7 @@ int launch_whole_tiles(const MfmaArgs &p) {
   const bool long_k = slices % 4 == 0 && slices / 2 >= kRingMinSlicesPerSplit;
   const bool extra = p.rq.act || p.rq.q;
   if (extra && !kRingCarriesExtraSteps<TA, TB>) return kNotWholeTiles;
-  const bool staged = extra && !(!EXACT && FusedSteps<AccElem, 2>::dword_copy(p.rq));
+  const bool staged = extra && !(!EXACT && dword_copy<AccElem>(p.rq));
   if ((staged || EXACT) &&
       !ring_pays<AccElem, EXACT, A_KC, B_KC, TA == SKL_DT_F8E4M3 || TA == SKL_DT_F8E5M2>(
           p, staged, tiles >= 200 ? tiles : tiles128, p.k * ES, long_k, tiles >= 200 ? rounds_filled(tiles, tail_round) : rounds_filled(tiles128)))
