@@ -93,8 +93,8 @@ extern "C" int skl_hip_gemm_mfma_padded_plan(const skl_gemm_canon *g, size_t *mp
   // place, is the faster one for merely ragged sizes (bf16 2000 x 5000 x 3000 with SiLU 127 against 139 us, E4M3
   // 1027 x 8190 x 4096 into E4M3 87 against 114), the padded copies behind its own copies (int8 3001 x 4099 x 5003
   // with ReLU into int8 172 against 124 us). Nor for whole tiles: the one operand that breaks the 16-byte rule is copied
-  // and the streaming kernel reads the other where it lies, with the epilogue without LDS rows and the trailing round of
-  // narrow tiles where those apply (padded copies take 1.25 times as long with a copy in dwords, 1.16 with other steps:
+  // and the streaming kernel reads the other where it lies, with the trailing round of
+  // narrow tiles where that applies (padded copies take 1.25 times as long with a copy in dwords, 1.16 with other steps:
   // medians of 42 and of 133 random layers). Only where both are copied, and padding N to 256 columns gives a chip full
   // of the larger tiles, are padded copies as good or better (0.93, 14 layers).
   const bool fused = g->rq.act || g->rq.q, wide_enough = (g->m + 255) / 256 * ((g->n + 255) / 256) >= 200;

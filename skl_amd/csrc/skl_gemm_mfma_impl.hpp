@@ -263,6 +263,12 @@ struct RingMma<SKL_DT_I8, SKL_DT_I8, false> {
   using Acc = v4i;
   SKL_RING_MMA("i32_16x16x64_i8", "", v4i)
 };
+struct RingMmaI8Large {  // 32 x 32 blocks, a fragment's halves one behind the other; see ring_few_issue_slots
+  using Frag = v8i;
+  static constexpr int kSide = 32, kFrag = 32;
+  using Acc = v16i;
+  SKL_RING_MMA("i32_32x32x32_i8", "", v4i)
+};
 template <>
 struct RingMma<SKL_DT_BF16, SKL_DT_BF16, false> {
   using Frag = v4i;
@@ -484,7 +490,7 @@ __device__ __forceinline__ auto read_frag(const char *tile, int row0, int kb) {
 }
 
 // ---------------------------------------------------------------------------
-// The epilogue of both kernels: one wave writes its MI x NI blocks of 32 x 32, lane l of a block holding column
+// The epilogue of the bounds-checked kernels: one wave writes its MI x NI blocks of 32 x 32, lane l of a block holding column
 // l % 32 and rows 8 * (r / 4) + 4 * (l / 32) + r % 4 in register r, as C = beta*C + alpha*acc followed by the fused
 // steps. C is written once and not read again: non-temporal stores keep it out of the operands' caches.
 //
@@ -625,18 +631,14 @@ __device__ __forceinline__ void write_wave_tile(const MfmaArgs &p, const Acc (&a
 }
 
 // ---------------------------------------------------------------------------
-// The streaming kernel's epilogue for fused calls with any activation and any 8-bit copy. Such steps - a GELU is some
+// The bounds-checked kernels' epilogue for fused calls with any activation and any 8-bit copy. Such steps - a GELU is some
 // fifty instructions - cannot be written out for each of a lane's 128 accumulators (spilled registers, code beyond the
 // instruction cache), and accumulators cannot be indexed by a loop counter. So a wave puts 32 rows of its tile at a time
-// into LDS, the operands' ring being over, and loops over them: a lane takes four neighbouring columns of a row, the
+// into LDS, the operands' stages being over, and loops over them: a lane takes four neighbouring columns of a row, the
 // same columns every time, so their biases, scales and offsets are fetched once, and C and the copy go out 16 and 4
 // bytes per lane where the layout has them side by side. Every element goes through the same operations in the same
 // order as in the other epilogues. `stage`: this wave's 32 x (32 NI + 8) elements; eight elements of padding put the
 // two halves of a wave's writes, four rows apart, into different banks.
-// Such calls ran on the bounds-checked 128 x 128 kernels: bf16 2048 x 8192 x 4096 with SiLU 188 -> 137 us, int8 4096^3
-// with ReLU 105 -> 72, E4M3 2048 x 8192 x 4096 with GELU into E4M3 125 -> 99 (110 while every lane multiplied out the
-// addresses of its rows); what is left of the last over the same call with ReLU, 37 us, is mostly the erfc of 16.8 million
-// elements. ring_pays says where the line lies.
 // alpha, beta and the old C are applied as a strip of 32 rows goes into LDS, and the old values of the next strip are
 // requested ahead of this one's stores: a load inside the loop waits for the stores of the pass before, every pass
 // (see write_wave_tile; C read, us, loads in the loop / ahead: E5M2 1024 x 14080 x 6272 with ReLU into int8 102 / 91, E4M3
@@ -811,15 +813,17 @@ __device__ __forceinline__ void write_wave_tile_staged(const MfmaArgs &p, const 
 // ---------------------------------------------------------------------------
 template <int COLS>
 constexpr int wave_rows_pitch() { return COLS + 4; }
-template <int MI, int NI, bool CHECK, bool STEPS, typename Acc>
+template <int MI, int NI, int ES, bool CHECK, bool STEPS, typename Acc>
 __device__ __forceinline__ void write_wave_rows(const MfmaArgs &p, const Acc (&acc)[MI][NI], size_t row0, size_t col0, char *stage_bytes) {
   using T = decltype(Acc{}.x);
   typedef T V4 __attribute__((ext_vector_type(4)));
   typedef T Run4 __attribute__((ext_vector_type(4), aligned(4)));
   constexpr int S = sizeof(Acc) == 64 ? 32 : 16, G = S == 32 ? 4 : 1, COLS = NI * S, P = wave_rows_pitch<COLS>();
-  // A pass: 8 rows by 32 columns, whole lines; by columns: S rows by 256 / S columns. A batch: four passes, side by side first.
-  constexpr int kPasses = S * COLS / 256, kBatch = 4, kSide = COLS / 32, kColsDown = 256 / S;
-  static_assert(kPasses % kBatch == 0 && kBatch % kSide == 0);
+  // A pass: 256 elements, as many whole rows as that is; by columns: S rows by 256 / S columns. A chunk: up to eight passes (four, with
+  // steps); the old values of one are under way (of two, int8 4096 x 8192 x 2048 took 3 us more, of four 13).
+  constexpr int kPasses = S * COLS / 256, kMost = STEPS ? 4 : 8, kChunk = kPasses < kMost ? kPasses : kMost, kDown = 256 / COLS, kColsDown = 256 / S;
+  constexpr int kChunks = MI * kPasses / kChunk;
+  static_assert(kPasses % kChunk == 0);
   const int lane = (int)__builtin_amdgcn_mbcnt_hi(~0u, __builtin_amdgcn_mbcnt_lo(~0u, 0u));  // (not from threadIdx, see write_wave_tile)
   T *const stage = reinterpret_cast<T *>(stage_bytes);
   T *const c = reinterpret_cast<T *>(p.c);
@@ -828,9 +832,32 @@ __device__ __forceinline__ void write_wave_rows(const MfmaArgs &p, const Acc (&a
   const auto col_at = [&](size_t col) { return (col >> p.ccs) * p.csc1 + (col & cmask) * p.csc0; };
   const T *const bias = reinterpret_cast<const T *>(p.bias);
   const skl_fp8::Ofp8Format f8(p.rq.q_fmt);
-  // A single round of tiles ends all at once, and its stores go faster through the caches; with more rounds the operands of the next
-  // one need the room (bf16, us, kept / past the caches: 4096^3 97.5 / 100.2, 8192^3 743 / 721).
-  const bool kept = p.tiles_m * p.tiles_n <= 256;
+  // Stores go faster through the caches (us, through / past them: bf16 4096^3 97.5 / 100.2, 4096 x 8192 x 512 50 / 60, 8192^2 x 1024
+  // 141 / 153; E4M3 8192^2 x 2048 143 / 149), until with several rounds of tiles C and the operands of the next round are more than the
+  // 256 MiB behind them (bf16 4096 x 8192^2 373 / 369, 8192^3 743 / 721, 8192 x 16384 x 2048 452 / 435; E4M3 8192 x 16384 x 1024
+  // 217 / 192): the line is where both took the same, 8192^2 with 4 KiB of K (bf16 229.5 / 231, E4M3 232.2 / 232.7). With several rounds
+  // of a C that is read the stores are in its way (int8 4096 x 8192 x 2048 128 / 114, one round 4096^2 x 1024 35.1 / 36.2).
+  const bool one_round = p.tiles_m * p.tiles_n <= 256, fits = (p.m + p.n) * p.k * ES + p.m * p.n * 4 < (size_t(320) << 20);
+
+  // Row of blocks i's sums to LDS (accumulators cannot be indexed: a branch for each).
+  const auto put = [&](unsigned i) __attribute__((always_inline)) {
+    T *const to = stage + lane % S * P + lane / S * 4;
+    [&]<int... Is>(std::integer_sequence<int, Is...>) __attribute__((always_inline)) {
+      (
+          [&](auto ic) __attribute__((always_inline)) {
+            constexpr int I = decltype(ic)::value;
+            if (i == I) {
+#pragma unroll
+              for (int j = 0; j < NI; ++j) {
+                const Acc sums = j < NI / 2 ? fetched<ring_sum_in_a<MI, NI, Acc>(I, 0)>(acc[I][j]) : fetched<ring_sum_in_a<MI, NI, Acc>(I, NI - 1)>(acc[I][j]);
+#pragma unroll
+                for (int g = 0; g < G; ++g) *reinterpret_cast<V4 *>(to + j * S + g * 8) = V4{sums[4 * g], sums[4 * g + 1], sums[4 * g + 2], sums[4 * g + 3]};
+              }
+            }
+          }(std::integral_constant<int, Is>{}),
+          ...);
+    }(std::make_integer_sequence<int, MI>{});
+  };
 
   // RUN: four columns lie side by side in C. Otherwise, `down`, a lane's four elements are four rows of a column: side by side in a C by
   // columns, and in any other C as good as four columns. UPDATE: C is read (not only where a zero's sign asks for it). FUSED: there are
@@ -838,40 +865,46 @@ __device__ __forceinline__ void write_wave_rows(const MfmaArgs &p, const Acc (&a
   const auto write = [&](auto run, auto update, auto fused) __attribute__((always_inline)) {
     constexpr bool RUN = decltype(run)::value, UPDATE = decltype(update)::value, FUSED = decltype(fused)::value;
     // the lane's first row and column in a pass, from those of the pass
-    const int r_lane = RUN ? lane / 8 : lane % (S / 4) * 4, c_lane = RUN ? lane % 8 * 4 : lane / (S / 4);
-    // C's place of the lane's elements in a pass: that of the pass, a scalar, and this (passes begin at multiples of 8 rows and 16 or
-    // more columns, blocks of C are powers of two)
-    T *const c_lane_at = c + row_at(r_lane) + col_at(c_lane);
+    const int r_lane = RUN ? lane / (COLS / 4) : lane % (S / 4) * 4, c_lane = RUN ? lane % (COLS / 4) * 4 : lane / (S / 4);
+    // Where in C the lane's elements of pass y of a row of blocks are: that of the row of blocks, a scalar, and this (passes begin at
+    // multiples of their rows and columns, rows of blocks at multiples of theirs, and blocks of C are powers of two)
+    T *const c_lane_at = c + row_at(r_lane) + col_at(col0) + col_at(c_lane);
+    size_t step[kChunk];  // from a chunk's first pass to its others
+#pragma unroll
+    for (int t = 0; t < kChunk; ++t) step[t] = RUN ? row_at(t * kDown) : col_at(t * kColsDown);
     const auto cols_in = [&](size_t col) -> int {  // of four columns from `col` on
       if constexpr (!CHECK) return 4;
       return col >= p.n ? 0 : p.n - col < 4 ? (int)(p.n - col) : 4;
     };
     const auto column_at = [&](size_t k) { return !CHECK || k < p.n ? k : 0; };
-    T bias_of[RUN ? kSide : 1][4];
-    float scale_of[RUN ? kSide : 1][4];
+    T bias_of[4];
+    float scale_of[4];
     if constexpr (RUN && FUSED) {
 #pragma unroll
-      for (int t = 0; t < kSide; ++t)
-#pragma unroll
-        for (int e = 0; e < 4; ++e) {
-          const size_t k = column_at(col0 + t * 32 + c_lane + e);
-          bias_of[t][e] = bias ? bias[k] : T(0);
-          scale_of[t][e] = STEPS && p.rq.q ? p.rq.q_scale[p.rq.q_per_column ? k : 0] : 0.0f;
-        }
-      __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0): in the loop they would be waited for with every batch, and its stores with them
+      for (int e = 0; e < 4; ++e) {
+        const size_t k = column_at(col0 + c_lane + e);
+        bias_of[e] = bias ? bias[k] : T(0);
+        scale_of[e] = STEPS && p.rq.q ? p.rq.q_scale[p.rq.q_per_column ? k : 0] : 0.0f;
+      }
+      __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0): in the loop they would be waited for with every chunk, and its stores with them
     }
     const bool q_run = STEPS && RUN && p.rq.csq == 1 && (p.rq.rsq & 3) == 0 && ((uintptr_t)p.rq.q & 3) == 0;
     T running = skl_lowest<T>();
 
-    // Pass x of a row of blocks that begins at row `top`: its first row and column.
-    const auto first_row = [&](size_t top, unsigned x) { return top + (RUN ? x / kSide * 8 : 0); };
-    const auto first_col = [&](unsigned x) { return col0 + (RUN ? x % kSide * 32 : x * kColsDown); };
-    const auto request = [&](size_t top, unsigned x, V4 (&old)[kBatch]) __attribute__((always_inline)) {
+    // Chunk x: its first row and column, and, from those on, the lane's first row and column of its pass t.
+    constexpr unsigned kOfRow = kPasses / kChunk;  // chunks of a row of blocks
+    const auto top_of = [&](unsigned x) { return row0 + (RUN ? x * (kChunk * kDown) : x / kOfRow * S); };
+    const auto left_of = [&](unsigned x) { return RUN ? size_t(0) : (size_t)(x % kOfRow * (kChunk * kColsDown)); };
+    const auto row_of = [&](size_t top, int t) { return top + (RUN ? t * kDown : 0) + r_lane; };
+    const auto col_of = [&](size_t left, int t) { return col0 + left + (RUN ? 0 : t * kColsDown) + c_lane; };
+    const auto request = [&](unsigned x, V4 (&old)[kChunk]) __attribute__((always_inline)) {
+      const size_t top = top_of(x), left = left_of(x);
+      const T *const at = c_lane_at + row_at(top) + col_at(left);
 #pragma unroll
-      for (int t = 0; t < kBatch; ++t) {
-        const size_t row = first_row(top, x + t) + r_lane, k = first_col(x + t) + c_lane;
+      for (int t = 0; t < kChunk; ++t) {
+        const size_t row = row_of(top, t), k = col_of(left, t);
         if constexpr (RUN && !CHECK) {
-          old[t] = *reinterpret_cast<const Run4 *>(c_lane_at + row_at(first_row(top, x + t)) + col_at(first_col(x + t)));
+          old[t] = *reinterpret_cast<const Run4 *>(at + step[t]);
         } else if constexpr (RUN) {  // (rows and columns that do not exist: some that do)
           old[t] = *reinterpret_cast<const Run4 *>(c + row_at(row < p.m ? row : p.m - 1) + col_at(k + 4 > p.n ? p.n - 4 : k));
         } else {
@@ -889,163 +922,192 @@ __device__ __forceinline__ void write_wave_rows(const MfmaArgs &p, const Acc (&a
       return o;
     };
 
-    V4 next[kBatch];
-    if constexpr (UPDATE) request(row0, 0, next);
-#pragma clang loop unroll(disable)
-    for (unsigned i = 0; i < (unsigned)MI; ++i) {
-      // this row of blocks' sums (accumulators cannot be indexed: a branch for each)
-      T *const to = stage + lane % S * P + lane / S * 4;
-      [&]<int... Is>(std::integer_sequence<int, Is...>) __attribute__((always_inline)) {
-        (
-            [&](auto ic) __attribute__((always_inline)) {
-              constexpr int I = decltype(ic)::value;
-              if (i == I) {
+    // `next`: the old values of chunk x, then those of the next.
+    const auto chunk = [&](unsigned x, V4 (&next)[kChunk]) __attribute__((always_inline)) {
+      const size_t top = top_of(x), left = left_of(x);
+      const unsigned in_row = x % kOfRow;
+      const T *const stage_x = stage + (RUN ? (in_row * (kChunk * kDown) + r_lane) * P + c_lane : r_lane * P + in_row * (kChunk * kColsDown) + c_lane);
+      V4 v[kChunk];
 #pragma unroll
-                for (int j = 0; j < NI; ++j) {
-                  const Acc sums = j < NI / 2 ? fetched<ring_sum_in_a<MI, NI, Acc>(I, 0)>(acc[I][j]) : fetched<ring_sum_in_a<MI, NI, Acc>(I, NI - 1)>(acc[I][j]);
+      for (int t = 0; t < kChunk; ++t) {
+        if constexpr (RUN) {
+          v[t] = *reinterpret_cast<const V4 *>(stage_x + t * kDown * P);
+        } else {
 #pragma unroll
-                  for (int g = 0; g < G; ++g) *reinterpret_cast<V4 *>(to + j * S + g * 8) = V4{sums[4 * g], sums[4 * g + 1], sums[4 * g + 2], sums[4 * g + 3]};
-                }
-              }
-            }(std::integral_constant<int, Is>{}),
-            ...);
-      }(std::make_integer_sequence<int, MI>{});
-      // the wave's own LDS accesses complete in order; the compiler must not move them across each other
+          for (int e = 0; e < 4; ++e) v[t][e] = stage_x[e * P + t * kColsDown];
+        }
+      }
+      // The wave's own LDS accesses complete in order; the compiler must not move them across each other. The next row of blocks goes to
+      // LDS under what follows.
       __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
       __builtin_amdgcn_wave_barrier();
-      const size_t top = row0 + i * S;
-#pragma clang loop unroll(disable)
-      for (unsigned x = 0; x < (unsigned)kPasses; x += kBatch) {
-        V4 v[kBatch];
+      if (in_row == kOfRow - 1) put(x / kOfRow + 1);
+      __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+      __builtin_amdgcn_wave_barrier();
+      if constexpr (UPDATE) {
 #pragma unroll
-        for (int t = 0; t < kBatch; ++t) {
-          const unsigned y = x + t;
-          if constexpr (RUN) {
-            v[t] = *reinterpret_cast<const V4 *>(stage + (y / kSide * 8 + r_lane) * P + y % kSide * 32 + c_lane);
-          } else {
+        for (int t = 0; t < kChunk; ++t) {
+          const V4 old = moved(col_of(left, t), next[t]);
 #pragma unroll
-            for (int e = 0; e < 4; ++e) v[t][e] = stage[(r_lane + e) * P + y * kColsDown + c_lane];
-          }
+          for (int e = 0; e < 4; ++e) v[t][e] = skl_combine(v[t][e], old[e], p.alpha, p.beta);
         }
-        if constexpr (UPDATE) {
+        __builtin_amdgcn_sched_barrier(0);  // the values to come take these registers
+        request(x + 1 < (unsigned)kChunks ? x + 1 : x, next);  // (beyond the end: some, not used)
+      } else {
+        bool need = false;
 #pragma unroll
-          for (int t = 0; t < kBatch; ++t) {
-            const V4 old = moved(first_col(x + t) + c_lane, next[t]);
+        for (int t = 0; t < kChunk; ++t)
 #pragma unroll
-            for (int e = 0; e < 4; ++e) v[t][e] = skl_combine(v[t][e], old[e], p.alpha, p.beta);
+          for (int e = 0; e < 4; ++e) need |= skl_initialise_needs_c(v[t][e], p.alpha, p.beta);
+        if (!std::is_same<T, int>::value && __builtin_amdgcn_ballot_w64(need) != 0) {  // the old values decide the sign of some zeros
+          V4 signs[kChunk];
+          request(x, signs);
+#pragma unroll
+          for (int t = 0; t < kChunk; ++t) {
+            const V4 o = moved(col_of(left, t), signs[t]);
+#pragma unroll
+            for (int e = 0; e < 4; ++e) v[t][e] = skl_initialise_with(v[t][e], o[e], p.alpha, p.beta);
           }
-          __builtin_amdgcn_sched_barrier(0);  // the next batch's take these registers
-          const bool more = x + kBatch < (unsigned)kPasses, end = !more && i + 1 == (unsigned)MI;  // (the end: once more, not used)
-          request(more || end ? top : top + S, more ? x + kBatch : end ? x : 0, next);
         } else {
-          bool need = false;
 #pragma unroll
-          for (int t = 0; t < kBatch; ++t)
+          for (int t = 0; t < kChunk; ++t)
 #pragma unroll
-            for (int e = 0; e < 4; ++e) need |= skl_initialise_needs_c(v[t][e], p.alpha, p.beta);
-          if (!std::is_same<T, int>::value && __builtin_amdgcn_ballot_w64(need) != 0) {  // the old values decide the sign of some zeros
-            V4 signs[kBatch];
-            request(top, x, signs);
+            for (int e = 0; e < 4; ++e) v[t][e] = skl_initialise_plain(v[t][e], p.alpha, p.beta);
+        }
+      }
+      if constexpr (FUSED) {
+        if (bias) {
 #pragma unroll
-            for (int t = 0; t < kBatch; ++t) {
-              const V4 o = moved(first_col(x + t) + c_lane, signs[t]);
+          for (int t = 0; t < kChunk; ++t) {
+            const T by_column = RUN ? T(0) : bias[column_at(col_of(left, t))];
 #pragma unroll
-              for (int e = 0; e < 4; ++e) v[t][e] = skl_initialise_with(v[t][e], o[e], p.alpha, p.beta);
-            }
-          } else {
-#pragma unroll
-            for (int t = 0; t < kBatch; ++t)
-#pragma unroll
-              for (int e = 0; e < 4; ++e) v[t][e] = skl_initialise_plain(v[t][e], p.alpha, p.beta);
+            for (int e = 0; e < 4; ++e) v[t][e] = skl_add_bias(v[t][e], RUN ? bias_of[e] : by_column);
           }
         }
-        if constexpr (FUSED) {
-          if (bias) {
+        if constexpr (STEPS) {  // (the choice outside of the elements: chains of instructions then run side by side)
+          const auto activate = [&](auto act) __attribute__((always_inline)) {
 #pragma unroll
-            for (int t = 0; t < kBatch; ++t) {
-              const T by_column = RUN ? T(0) : bias[column_at(first_col(x + t) + c_lane)];
+            for (int t = 0; t < kChunk; ++t)
 #pragma unroll
-              for (int e = 0; e < 4; ++e) v[t][e] = skl_add_bias(v[t][e], RUN ? bias_of[t % kSide][e] : by_column);
-            }
-          }
-          if constexpr (STEPS) {  // (the choice outside of the elements: a batch's chains of instructions then run side by side)
-            const auto activate = [&](auto act) __attribute__((always_inline)) {
-#pragma unroll
-              for (int t = 0; t < kBatch; ++t)
-#pragma unroll
-                for (int e = 0; e < 4; ++e) v[t][e] = skl_activate(v[t][e], decltype(act)::value);
-            };
-            if (p.rq.act == 1) activate(std::integral_constant<int, 1>{});
-            if constexpr (!std::is_same<T, int>::value) {
-              if (p.rq.act == 2) activate(std::integral_constant<int, 2>{});
-              if (p.rq.act >= 3) activate(std::integral_constant<int, 3>{});
-            }
-          }
-          if (p.max) {
-#pragma unroll
-            for (int t = 0; t < kBatch; ++t) {
-              const size_t row = first_row(top, x + t) + r_lane, k = first_col(x + t) + c_lane;
-#pragma unroll
-              for (int e = 0; e < 4; ++e)
-                if ((!CHECK || (row + (RUN ? 0 : e) < p.m && k + (RUN ? e : 0) < p.n)) && v[t][e] > running) running = v[t][e];
-            }
+              for (int e = 0; e < 4; ++e) v[t][e] = skl_activate(v[t][e], decltype(act)::value);
+          };
+          if (p.rq.act == 1) activate(std::integral_constant<int, 1>{});
+          if constexpr (!std::is_same<T, int>::value) {
+            if (p.rq.act == 2) activate(std::integral_constant<int, 2>{});
+            if (p.rq.act >= 3) activate(std::integral_constant<int, 3>{});
           }
         }
-        if (!STEPS || !p.rq.q_only) {
+        if (p.max) {
 #pragma unroll
-          for (int t = 0; t < kBatch; ++t) {
-            const size_t row = first_row(top, x + t) + r_lane, k = first_col(x + t) + c_lane;
+          for (int t = 0; t < kChunk; ++t) {
+            const size_t row = row_of(top, t), k = col_of(left, t);
+#pragma unroll
+            for (int e = 0; e < 4; ++e)
+              if ((!CHECK || (row + (RUN ? 0 : e) < p.m && k + (RUN ? e : 0) < p.n)) && v[t][e] > running) running = v[t][e];
+          }
+        }
+      }
+      T *const at = c_lane_at + row_at(top) + col_at(left);
+      if (!STEPS || !p.rq.q_only) {
+        const auto store = [&](auto kept_c) __attribute__((always_inline)) {
+#pragma unroll
+          for (int t = 0; t < kChunk; ++t) {
+            const size_t row = row_of(top, t), k = col_of(left, t);
+            T *const to = at + step[t];
             if constexpr (RUN) {
               if (!CHECK || (row < p.m && cols_in(k) == 4)) {
-                Run4 *const at = reinterpret_cast<Run4 *>(c_lane_at + row_at(first_row(top, x + t)) + col_at(first_col(x + t)));
-                if (kept) *at = v[t];
-                else __builtin_nontemporal_store((Run4)v[t], at);
+                if constexpr (decltype(kept_c)::value) *reinterpret_cast<Run4 *>(to) = v[t];
+                else __builtin_nontemporal_store((Run4)v[t], reinterpret_cast<Run4 *>(to));
               } else if (row < p.m) {
 #pragma unroll
                 for (int e = 0; e < 3; ++e)
                   if (k + e < p.n) c[row_at(row) + col_at(k + e)] = v[t][e];
               }
             } else {
-              T *const at = c + row_at(row) + col_at(k);
               if (p.rsc0 == 1 && (!CHECK || (row + 4 <= p.m && k < p.n))) {
-                *reinterpret_cast<Run4 *>(at) = v[t];
+                *reinterpret_cast<Run4 *>(to) = v[t];
               } else {
 #pragma unroll
                 for (int e = 0; e < 4; ++e)
-                  if (!CHECK || (row + e < p.m && k < p.n)) at[e * p.rsc0] = v[t][e];
+                  if (!CHECK || (row + e < p.m && k < p.n)) to[e * p.rsc0] = v[t][e];
               }
             }
           }
-        }
-        if constexpr (STEPS) {
-          if (p.rq.q) {
+        };
+        if (!RUN || one_round || (!UPDATE && fits)) store(std::true_type{});
+        else store(std::false_type{});
+      }
+      if constexpr (STEPS) {
+        if (p.rq.q) {
+          // The copy's four bytes of each pass. OCP fp8: where no value of the chunk leaves the format's finite range the instruction's
+          // codes are the rule's, two values at a time.
+          float w[kChunk][4];
+          unsigned packed[kChunk];
 #pragma unroll
-            for (int t = 0; t < kBatch; ++t) {
-              const size_t row = first_row(top, x + t) + r_lane, k = first_col(x + t) + c_lane;
-              const float by_column = RUN ? 0.0f : p.rq.q_scale[p.rq.q_per_column ? column_at(k) : 0];
-              unsigned packed = 0;
+          for (int t = 0; t < kChunk; ++t) {
+            const float by_column = RUN ? 0.0f : p.rq.q_scale[p.rq.q_per_column ? column_at(col_of(left, t)) : 0];
+#pragma unroll
+            for (int e = 0; e < 4; ++e) w[t][e] = (float)v[t][e], w[t][e] = p.rq.q_fmt == 0 ? w[t][e] : __fmul_rn(w[t][e], RUN ? scale_of[e] : by_column);
+          }
+          if (p.rq.q_fmt == 0) {
+#pragma unroll
+            for (int t = 0; t < kChunk; ++t) {
+              const float by_column = RUN ? 0.0f : p.rq.q_scale[p.rq.q_per_column ? column_at(col_of(left, t)) : 0];
+              packed[t] = 0;
+#pragma unroll
+              for (int e = 0; e < 4; ++e)
+                packed[t] |= ((unsigned)skl_requantise_int(w[t][e], RUN ? scale_of[e] : by_column, p.rq.q_zero) & 0xFFu) << (8 * e);
+            }
+          } else {
+            unsigned largest = 0;
+#pragma unroll
+            for (int t = 0; t < kChunk; ++t)
 #pragma unroll
               for (int e = 0; e < 4; ++e) {
-                const float scale = RUN ? scale_of[t % kSide][e] : by_column;
-                const unsigned byte = p.rq.q_fmt == 0 ? (unsigned)skl_requantise_int((float)v[t][e], scale, p.rq.q_zero) & 0xFFu
-                                                      : skl_fp8::encode_ofp8_hw(__fmul_rn((float)v[t][e], scale), f8) & 0xFFu;
-                packed |= byte << (8 * e);
+                const unsigned bits = __float_as_uint(w[t][e]) & 0x7FFFFFFFu;
+                largest = bits > largest ? bits : largest;
               }
-              int8_t *const q = reinterpret_cast<int8_t *>(p.rq.q) + row * p.rq.rsq + k * p.rq.csq;
-              if (q_run && (!CHECK || (row < p.m && cols_in(k) == 4))) {
-                *reinterpret_cast<unsigned *>(q) = packed;
-              } else {
+            const float limit = f8.e5m2 ? 57344.0f : 448.0f;
+            if (__builtin_amdgcn_ballot_w64(largest > __float_as_uint(limit)) != 0) {
 #pragma unroll
-                for (int e = 0; e < 4; ++e)
-                  if (!CHECK || (row + (RUN ? 0 : e) < p.m && k + (RUN ? e : 0) < p.n)) q[e * (RUN ? p.rq.csq : p.rq.rsq)] = (int8_t)(packed >> (8 * e));
+              for (int t = 0; t < kChunk; ++t) {
+                packed[t] = 0;
+#pragma unroll
+                for (int e = 0; e < 4; ++e) packed[t] |= (skl_fp8::encode_ofp8_hw(w[t][e], f8) & 0xFFu) << (8 * e);
               }
+            } else if (f8.e5m2) {
+#pragma unroll
+              for (int t = 0; t < kChunk; ++t)
+                packed[t] = (unsigned)__builtin_amdgcn_cvt_pk_bf8_f32(w[t][2], w[t][3], __builtin_amdgcn_cvt_pk_bf8_f32(w[t][0], w[t][1], 0, false), true);
+            } else {
+#pragma unroll
+              for (int t = 0; t < kChunk; ++t)
+                packed[t] = (unsigned)__builtin_amdgcn_cvt_pk_fp8_f32(w[t][2], w[t][3], __builtin_amdgcn_cvt_pk_fp8_f32(w[t][0], w[t][1], 0, false), true);
+            }
+          }
+#pragma unroll
+          for (int t = 0; t < kChunk; ++t) {
+            const size_t row = row_of(top, t), k = col_of(left, t);
+            int8_t *const q = reinterpret_cast<int8_t *>(p.rq.q) + row * p.rq.rsq + k * p.rq.csq;
+            if (q_run && (!CHECK || (row < p.m && cols_in(k) == 4))) {
+              *reinterpret_cast<unsigned *>(q) = packed[t];
+            } else {
+#pragma unroll
+              for (int e = 0; e < 4; ++e)
+                if (!CHECK || (row + (RUN ? 0 : e) < p.m && k + (RUN ? e : 0) < p.n)) q[e * (RUN ? p.rq.csq : p.rq.rsq)] = (int8_t)(packed[t] >> (8 * e));
             }
           }
         }
       }
-      __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-      __builtin_amdgcn_wave_barrier();
-    }
+    };
+
+    put(0);
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    V4 next[kChunk];
+    if constexpr (UPDATE) request(0, next);
+#pragma clang loop unroll(disable)
+    for (unsigned x = 0; x < (unsigned)kChunks; ++x) chunk(x, next);
     if (FUSED && p.max) {
       const T best = skl_wave_max(running);
       if (lane == 0 && best > skl_lowest<T>()) skl_atomic_max(reinterpret_cast<T *>(p.max), best);
@@ -1375,23 +1437,33 @@ __global__ void __launch_bounds__(WAVES_M *WAVES_N * 64, (BM == 64 ? 2 : 4)) gem
 // ===========================================================================
 // Streaming kernel for whole tiles (256 x 256 or 256 x 128): global -> LDS
 // without passing through registers (global_load_lds_dwordx4), K in slices of
-// 64 bytes held in a ring of four LDS stages. Each wave-level load deposits
+// 64 bytes held in a ring of four or six LDS stages. Each wave-level load deposits
 // 64 x 16 bytes as one contiguous KiB of LDS, so tiles are stored without
 // padding and bank conflicts are avoided by an XOR swizzle of the 16-byte
 // chunk index instead; the swizzle is applied on the global side (which chunk
-// a lane fetches) and again by the fragment reads. Eight waves, two per SIMD.
+// a lane fetches) and again by the fragment reads. Four waves, one per SIMD, a
+// quarter of the tile each, so that every byte in LDS is read by two waves
+// (eight waves of a quarter of the columns read a half more; bf16 with K
+// contiguous, us, eight waves of 32 x 32 products / this: 8192^3 843 / 721,
+// 4096^3 115 / 97.5).
 //
 // An MN-contiguous operand (k-rows of ROWS elements) is loaded a slice at a
 // time: a load covers whole k-rows, i.e. whole 128-byte lines. A K-contiguous
 // operand is different: a 64-byte slice is HALF a line of each row, and loads
 // made of half lines run at less than half the rate of loads made of whole
 // ones. So its loads cover 8 rows x 128 bytes - two slices at once - and the
-// four stages of such an operand are interleaved in LDS at 512-byte granularity
+// stages of such an operand are interleaved in LDS at 512-byte granularity
 // (8 rows x 64 bytes of stage 0, then of stage 1, ...), which puts the two
 // halves of such a load next to each other: one KiB, as the load writes it.
 // ===========================================================================
 constexpr int kRingSlice = 64;   // bytes of K per stage
-constexpr int kRingWaves = 4;
+// Waves: four, each a quarter of the tile, so that as little as possible is read twice. 8-bit operands both read across K into a 256 x
+// 128 tile are the exception: reads of eight bytes per lane and an address for each leave four waves of 16 x 16 products short of issue
+// slots. There fp8 takes eight waves, two to a SIMD, and int8 products of 32 x 32, half as many (us, with four waves and 16 x 16 / so;
+// 1024 x 4096^2, half the compute units: E4M3 27.2 / 24.9, int8 29.6 / 26.9; 2048 x 4096^2, all of them: 33.7 / 34.4 and 35.1 / 36.7).
+constexpr bool ring_few_issue_slots(int es, bool a_kc, bool b_kc, int bn) { return es == 1 && !a_kc && !b_kc && bn == 128; }
+template <int TA, bool A_KC, bool B_KC, int BN, bool EXACT>
+constexpr int kRingWaves = TA != SKL_DT_I8 && !EXACT && ring_few_issue_slots(Kind<TA>::ES, A_KC, B_KC, BN) ? 8 : 4;
 // Stages of an operand's ring: four, or six of an operand with K contiguous where 160 KiB of LDS hold them (see the kernel's loads).
 constexpr int ring_stages_a(bool a_kc, bool b_kc, int bn, bool scan) { return !a_kc || (bn == 256 && (b_kc || scan)) ? 4 : 6; }
 constexpr int ring_stages_b(bool, bool b_kc, int bn, bool scan) { return !b_kc || (bn == 256 && scan) ? 4 : 6; }
@@ -1520,16 +1592,16 @@ struct SLoader {
 //   * Fragment reads are inline assembly. The compiler cannot tell an LDS read
 //     from the LDS writes of outstanding global->LDS loads apart and makes every
 //     ds_read_tr wait for ALL loads in flight (vmcnt(0)), and it waits for reads
-//     it has only just issued (lgkmcnt(0) in front of every k-step) - either
-//     one exposes a memory latency per k-step. Here the kernel does its own
-//     counting: one lgkmcnt(0) at the top of a k-step, when the only reads in
-//     flight are the ones issued during the previous k-step; one vmcnt(n) per
+//     it has only just issued (lgkmcnt(0) in front of every step) - either
+//     one exposes a memory latency per step. Here the kernel does its own
+//     counting: one lgkmcnt(0) at the top of a step, when the only reads in
+//     flight are the ones issued during the previous step; one vmcnt(n) per
 //     slice in front of the barrier.
 //   * Reads and loads are dealt out one at a time behind the MFMAs instead of
 //     going out in bursts: a wave issues in order, and a burst that finds the
 //     LDS or the load path busy is a stretch in which it issues no MFMA. The
-//     reads sit behind the first half of a k-step's MFMAs, which leaves the
-//     second half for them to land.
+//     reads sit behind the first three quarters of a step's MFMAs, which leaves
+//     the last quarter for them to land.
 // ---------------------------------------------------------------------------
 template <int N>
 __device__ __forceinline__ void wait_loads_upto() {
@@ -1624,43 +1696,44 @@ __device__ __forceinline__ Frag join_pieces(const Piece (&pc)[N]) {
   }
 }
 
+template <int X>
+__device__ __forceinline__ v4i half_of(v8i f) { return v4i{f[4 * X], f[4 * X + 1], f[4 * X + 2], f[4 * X + 3]}; }
+
 constexpr int ceil_div(int a, int b) { return (a + b - 1) / b; }
 
 // EDGE: problems that are not whole tiles, or whole pairs of slices along K: the loads take nothing from beyond the operands
 // (SLoader), and the epilogue touches no row or column beyond p.m / p.n.
-// CQUADS: an int32 C in small blocks with contiguous rows (the 4 x 4 blocks of src/gemm/packed-gemm.md:270-298, up to
-// 16 columns), no fused steps - see the epilogue.
 // SCAN (floating-point row-major C, beta == 0 evaluated like the reference's loops, whole tiles, K of at least 64
 // slices on the wide tile and 32 on the narrow one): whether 0 * c is a zero for every old c of the tile - i.e. no NaN,
-// no infinity - is found out while the tile is multiplied. Every even slice each wave requests 1 KiB of the tile's
-// old C (a row of the wide tile, two rows of the narrow one; wave w takes every eighth) into one of four slots of LDS
-// behind the operand stages; three and four slices later it reads them back, 8 bytes per lane and slice (its own
+// no infinity - is found out while the tile is multiplied. Every slice each wave requests 1 KiB of the tile's
+// old C (a row of the wide tile, two rows of the narrow one; wave w takes every fourth, or eighth) into one of four slots of LDS
+// behind the operand stages; three slices later it reads them back, 16 bytes per lane (its own
 // loads, its own counter: no barrier), and tests the exponents. After the loop the waves put their findings together.
 // A tile without such a value is then written as an initialised one (the sign of exact zeros is still taken from the
-// old c, see write_wave_tile); a tile with one takes the path that reads all of C. Either way the bits are those of
+// old c, see write_wave_rows); a tile with one takes the path that reads all of C. Either way the bits are those of
 // 0 * c + alpha * acc.
 // (Measured on fp8 8192^3, old C in memory: a first version - every wave its own block, lane addresses for any
 // layout of C, 64-bit block arithmetic per load - cost 62-70 us of 415 whether it loaded 4 bytes per lane every slice
 // or 16 every other one, 25-43 us of that with the rows already in cache: the instructions between two MFMAs, not the
 // loads. Hence contiguous rows, whose address is a scalar product and a shift of the lane index.)
-// EXACT: OCP fp8 operands multiplied exactly (MmaF8Exact). The bytes travel and are read like int8's; a fragment is
-// widened behind the MFMAs in front of its first use, B's NI and A's first at the top of the k-step. A wave widens
+// EXACT: OCP fp8 operands multiplied exactly (MmaF8Exact). The bytes travel like int8's; a fragment is widened behind the
+// products in front of its first use, for each half of its bytes anew, A's a row of blocks ahead, B's half a step. A wave widens
 // MI + NI fragments for MI x NI products - on the 128 x 128 kernels, with 64 x 32 per wave, three for two, which is
-// more vector work than the matrix cores take for the products; here six for eight (256 columns) or four for four (128).
-// E4M3 2048 x 8192 x 2048: 77 us there,
-// 62 here (1.1 PFLOP/s, what the f16 kernel reaches).
+// more vector work than the matrix cores take for the products; here sixteen for 64 (256 columns) or twelve for 32 (128).
+// E4M3 2048 x 8192 x 2048: 77 us there, 62 with eight waves of 32 x 32 products here; with a bias, into E4M3, 73 so and now 59.
 template <int TA, int TB, bool A_KC, bool B_KC, int BN, bool EDGE = false, bool STEPS = false, bool SCAN = false, bool EXACT = false>
-__global__ void __launch_bounds__(kRingWaves * 64) gemm_mfma_ring_kernel(MfmaArgs p) {
-  using M = RingMma<TA, TB, EXACT>;
+__global__ void __launch_bounds__((kRingWaves<TA, A_KC, B_KC, BN, EXACT> * 64)) gemm_mfma_ring_kernel(MfmaArgs p) {
+  constexpr bool kLarge = TA == SKL_DT_I8 && ring_few_issue_slots(1, A_KC, B_KC, BN);
+  using M = typename std::conditional<kLarge, RingMmaI8Large, RingMma<TA, TB, EXACT>>::type;
   using Frag = typename M::Frag;
   using Acc = typename M::Acc;
   using AccElem = decltype(Acc{}.x);
   constexpr int SB = kRingSlice, NSA = ring_stages_a(A_KC, B_KC, BN, SCAN), NSB = ring_stages_b(A_KC, B_KC, BN, SCAN);
   constexpr int ES = Kind<TA>::ES, S = M::kSide, FRB = M::kFrag;
-  constexpr int BM = 256, WAVES = kRingWaves, WAVES_N = 2, WAVES_M = WAVES / WAVES_N;
+  constexpr int BM = 256, WAVES = kRingWaves<TA, A_KC, B_KC, BN, EXACT>, WAVES_N = 2, WAVES_M = WAVES / WAVES_N;
   constexpr int WM = BM / WAVES_M, WN = BN / WAVES_N, MI = WM / S, NI = WN / S;
   // A step is a slice: the products of the wave's blocks, once, or EXACT with each half of the fragments' bytes.
-  constexpr int kProducts = MI * NI, kSlots = (EXACT ? 2 : 1) * kProducts;
+  constexpr int kProducts = MI * NI, kSlots = (EXACT || kLarge ? 2 : 1) * kProducts;
   using LA = SLoader<ES, A_KC, WAVES, BM, NSA, S, EDGE>;
   using LB = SLoader<ES, B_KC, WAVES, BN, NSB, S, EDGE>;
   using TileA = STile<ES, A_KC, BM, NSA, S>;
@@ -1669,7 +1742,7 @@ __global__ void __launch_bounds__(kRingWaves * 64) gemm_mfma_ring_kernel(MfmaArg
   using RB = FragReader<ES, B_KC, FRB, BN, NSB, S, EXACT>;
   constexpr int PA = RA::kPieces, PB = RB::kPieces;
   constexpr int kReadsB = NI * PB, kReads = kReadsB + MI * PA;  // LDS instructions per step
-  constexpr int kReadSlots = kProducts * 3 / 4;                 // ... behind the first of its products, the rest is time to land
+  constexpr int kReadSlots = (EXACT ? kProducts : kSlots) * 3 / 4;  // ... behind the first of its products, the rest is time to land
   // Item r of n that are spread over m slots goes out in slot r * m / n.
   constexpr auto first_in_slot = [](int q, int n, int m) { return q >= m ? n : (q * n + m - 1) / m; };
   // ... and a load, so as not to meet a read, half of the way on to the next one's.
@@ -1681,7 +1754,7 @@ __global__ void __launch_bounds__(kRingWaves * 64) gemm_mfma_ring_kernel(MfmaArg
   //   an operand read across K: slice s + 4.
   // What counts is that they are evenly spread: a load keeps the compute unit's address path for 16 cycles, four waves request at
   // the same time, and a wave that has to wait for the path does not issue products either (bf16 8192^3 with K contiguous, epilogue
-  // left out: 64 loads within 512 / 768 / 1024 cycles of a step of 1024 761 / 738 / 728 us, in two steps SPREAD_US).
+  // left out: 64 loads within 512 / 768 / 1024 cycles of a step of 1024 761 / 738 / 728 us; in two steps another 1.6 per cent less).
   constexpr auto blocks_of = [](int u, bool kc, int ns, int blocks, bool beside_four) {
     if (!kc) return 0;
     if (ns == 4) return u == 1 ? blocks : 0;
@@ -1894,8 +1967,8 @@ __global__ void __launch_bounds__(kRingWaves * 64) gemm_mfma_ring_kernel(MfmaArg
               (
                   [&](auto qc) __attribute__((always_inline)) {
                     constexpr int Q = decltype(qc)::value, X = Q / kProducts, i = Q % kProducts / NI, j = Q % NI;  // X: half of the fragments' bytes (EXACT)
-                    const auto fragment_a = [&]() __attribute__((always_inline)) { if constexpr (EXACT) return wide_a[i & 1]; else return join_pieces<Frag>(pa[U][i]); };
-                    const auto fragment_b = [&]() __attribute__((always_inline)) { if constexpr (EXACT) return wide_b[X][j]; else return join_pieces<Frag>(pb[U][j]); };
+                    const auto fragment_a = [&]() __attribute__((always_inline)) { if constexpr (EXACT) return wide_a[i & 1]; else if constexpr (kLarge) return half_of<X>(join_pieces<Frag>(pa[U][i])); else return join_pieces<Frag>(pa[U][i]); };
+                    const auto fragment_b = [&]() __attribute__((always_inline)) { if constexpr (EXACT) return wide_b[X][j]; else if constexpr (kLarge) return half_of<X>(join_pieces<Frag>(pb[U][j])); else return join_pieces<Frag>(pb[U][j]); };
                     // this slot's load, if it has one
                     constexpr int L = first_load(Q, kLoads, kSlots), kLoadsHere = first_load(Q + 1, kLoads, kSlots) - L;
                     constexpr bool kHasLoad = kLoadsHere > 0 && !EDGE && Q > 0;  // with the product (what it needs is worked out behind the first)
@@ -1998,7 +2071,7 @@ __global__ void __launch_bounds__(kRingWaves * 64) gemm_mfma_ring_kernel(MfmaArg
   static_assert(WAVES * kStageBytes <= TileA::kRegion + TileB::kRegion, "the waves' rows take the place of the operand stages");
   if constexpr (SCAN) {
     // What the waves have found, put together: each wave's word where its first slot began (its own reads of
-    // the slots are over), a barrier, and everybody reads all eight.
+    // the slots are over), a barrier, and everybody reads all of them.
     unsigned *const found = reinterpret_cast<unsigned *>(smem + TileA::kRegion + TileB::kRegion);
     found[wave * 256] = scan_bad != 0;
     __syncthreads();
@@ -2007,10 +2080,10 @@ __global__ void __launch_bounds__(kRingWaves * 64) gemm_mfma_ring_kernel(MfmaArg
     for (int w = 0; w < WAVES; ++w) any |= found[w * 256];
     MfmaArgs q = p;
     if (any == 0) q.beta.fz.skip_c_read = 1;  // 0 * c is a zero everywhere in this tile
-    write_wave_rows<MI, NI, EDGE, STEPS>(q, acc, m0 + wm, n0 + wn, smem + wave * kStageBytes);
+    write_wave_rows<MI, NI, ES, EDGE, STEPS>(q, acc, m0 + wm, n0 + wn, smem + wave * kStageBytes);
   } else {
     __syncthreads();  // every wave's reads of the stages and loads into them are over
-    write_wave_rows<MI, NI, EDGE, STEPS>(p, acc, m0 + wm, n0 + wn, smem + wave * kStageBytes);
+    write_wave_rows<MI, NI, ES, EDGE, STEPS>(p, acc, m0 + wm, n0 + wn, smem + wave * kStageBytes);
   }
 }
 
@@ -2129,15 +2202,12 @@ struct SequenceGuard {
 
 constexpr size_t kRingMinSlicesPerSplit = 64;  // below 8 KiB of K per row the pass over the planes costs what the split saves
 
-// The streaming kernels for whole tiles also exist with the activation (none or ReLU) and requantisation steps written
-// out per accumulator, for a copy that can be written as dwords (a quantised layer's 8-bit output at a quarter of C's
-// bytes: int8 behind an int32 C, fp8 behind an fp32 C); every other call with those steps takes the epilogue that loops
-// over rows in LDS (kStagedSteps).
+// The streaming kernels also exist with the activation and requantisation steps (STEPS).
 template <int TA, int TB>
 constexpr bool kRingCarriesExtraSteps = TA == TB;   // every kind but the mixed fp8 pairings, which have no fused entry point
 
-// An int32 C the streaming kernel writes 16 bytes per lane: blocks of 4 to 16 columns with contiguous rows, a
-// multiple of four rows per block, everything on 16-byte boundaries, no fused steps.
+// An int32 C in blocks of 4 to 16 columns (the 4 x 4 blocks of src/gemm/packed-gemm.md:270-298) that the streaming kernel writes 16
+// bytes per lane like a row-major one: contiguous rows, a multiple of four per block, on 16-byte boundaries, no fused steps.
 inline bool c_in_row_quads(const MfmaArgs &p) {
   return !p.bias && !p.max && !p.rq.act && !p.rq.q && p.csc0 == 1 && p.ccs >= 2 && p.ccs <= 4 && p.crs >= 2 &&
          (((uintptr_t)p.c | (p.rsc0 * 4) | (p.rsc1 * 4) | (p.csc1 * 4)) & 15) == 0;
@@ -2152,7 +2222,7 @@ int launch_ring(const MfmaArgs &args) {
   using AccElem = decltype(typename Kind<TA>::Acc{}.x);
   if constexpr (std::is_same<AccElem, float>::value && !EDGE && !STEPS && !SCAN && !EXACT) {
     // beta == 0 evaluated as the reference's loops do (0 * c: a NaN or an infinity in C stays a NaN): the old C is
-    // looked through while the tile is multiplied, 8 KiB of it per two slices - needs 64 slices on the wide tile, 32
+    // looked through while the tile is multiplied, a KiB of it per wave and slice - needs 64 slices on the wide tile, 32
     // on the narrow one, a tile to itself (no shared K) and a row-major C.
     const size_t scan_slices = args.k * ES / kRingSlice, scan_tiles = (args.m / 256) * (args.n / BN);
     const bool shared_k = scan_tiles <= 128 && scan_slices % 4 == 0 && scan_slices / 2 >= kRingMinSlicesPerSplit;
@@ -2166,7 +2236,8 @@ int launch_ring(const MfmaArgs &args) {
     if (args.beta.f == 0.0f && args.beta.fz.skip_c_read == 0 && !shared_k && (row_major || panels) && scan_slices >= (BN == 256 ? 64 : 32))
       return launch_ring<TA, TB, A_KC, B_KC, BN, EDGE, false, true>(args);
   }
-  constexpr int lds = (ring_stages_a(A_KC, B_KC, BN, SCAN) * 256 + ring_stages_b(A_KC, B_KC, BN, SCAN) * BN) * kRingSlice + (SCAN ? 4 * kRingWaves * 1024 : 0);
+  constexpr int kWaves = kRingWaves<TA, A_KC, B_KC, BN, EXACT>;
+  constexpr int lds = (ring_stages_a(A_KC, B_KC, BN, SCAN) * 256 + ring_stages_b(A_KC, B_KC, BN, SCAN) * BN) * kRingSlice + (SCAN ? 4 * kWaves * 1024 : 0);
   static_assert(lds <= 160 * 1024);
   auto kernel = gemm_mfma_ring_kernel<TA, TB, A_KC, B_KC, BN, EDGE, STEPS, SCAN, EXACT>;
   static std::atomic<bool> configured{false};  // per instantiation; racing threads set the same value
@@ -2200,7 +2271,7 @@ int launch_ring(const MfmaArgs &args) {
     skl_hip_record_error(-2, "gemm_mfma: grid too large");
     return -2;
   }
-  kernel<<<(unsigned)grid, kRingWaves * 64, lds, skl_current_stream()>>>(p);
+  kernel<<<(unsigned)grid, kWaves * 64, lds, skl_current_stream()>>>(p);
   int rc = skl_check_launch("gemm_mfma_ring");
   if (rc != 0 || p.splits == 1) return rc;
   return launch_split_reduce<AccElem>(p, "gemm_split_reduce");

@@ -1,0 +1,46 @@
+"""How the streaming kernel starts and ends a tile: K of one to five pairs of slices (as many as it requests ahead, fewer, more),
+both tile widths, and C as its rows in LDS are handed out - row-major on and off 16-byte boundaries, by columns, read and not,
+with every step behind the product. int8, so that all of it is exact and compared bit for bit with the product in int64; the
+values behind alpha = 0x01010101 use all 32 bits."""
+import numpy as np
+import pytest
+
+import support
+from gpu_support import run_fused_gemm
+from support import GemmCase
+from test_oracle_gemm import fused_expectation
+
+pytestmark = pytest.mark.gpu
+
+SIZES = ((2048, 1536), (4096, 3328))  # 96 tiles of 256 x 128, 208 of 256 x 256
+
+
+@pytest.mark.parametrize("a_kc,b_kc", ((True, True), (True, False), (False, False), (False, True)))
+@pytest.mark.parametrize("m,n", SIZES)
+def test_streamed_tiles_from_short_to_longer_k(gpu, m, n, a_kc, b_kc):
+    rng = np.random.default_rng(m + 2 * a_kc + b_kc)
+    for i, k in enumerate((128, 256, 384, 512, 640)):
+        by_columns, pad, beta = i % 4 == 2, (0, 3, 5, 4, 1)[i], (0, -77, 1, 0, 3)[i]
+        rsc, csc = (1, m + pad) if by_columns else (n + pad, 1)
+        case = GemmCase("i8", None, (1, 0x01010101, -3, 7, 2)[i], beta, m0=1, n0=1, k0=1, m1=m, n1=n, k1=k, rsa0=0, csa0=0,
+                        rsa1=k if a_kc else 1, csa1=1 if a_kc else m, rsb0=0, csb0=0, rsb1=1 if b_kc else n, csb1=k if b_kc else 1,
+                        rsc0=0, csc0=0, rsc1=rsc, csc1=csc)
+        a, b, c = case.make_inputs(k + n)
+        c[:] = rng.integers(-2 ** 31, 2 ** 31, size=c.size)
+        x, y = a.reshape(m, k) if a_kc else a.reshape(k, m).T, b.reshape(n, k).T if b_kc else b.reshape(k, n)
+        rows = support.blocked_offsets(case.m1, case.n1, case.m0, case.n0, case.rsc0, case.csc0, case.rsc1, case.csc1)
+        sums = (x.astype(np.float64) @ y.astype(np.float64)).astype(np.int64).reshape(rows.shape)
+        plain = c.copy()
+        plain[rows] = (case.alpha * sums + beta * c[rows].astype(np.int64)).astype(np.int32)
+        bias = rng.integers(-1 << 12, 1 << 12, n).astype(np.int32) if i % 2 else None
+        start = np.array([-1 << 30], np.int32) if i >= 3 else None
+        act, rq = int(i == 3 or i == 2), None
+        if i >= 2:
+            rsq, csq = (1, m + 3) if i == 4 else (n + 4 * (i == 3), 1)
+            rq = dict(q=np.full((m - 1) * rsq + (n - 1) * csq + 1, 0x55, np.int8), rsq=rsq, csq=csq, per_column=bool(i % 2),
+                      scale=(rng.uniform(0.25, 2.0, n if i % 2 else 1) * 100.0 / 2.0 ** 31).astype(np.float32), zero=i, only=False, format=0)
+        out = run_fused_gemm(gpu, "rc", case, a, b, c, bias, start, "device", activation=act, requant=rq)
+        want = fused_expectation(case, plain, bias, start, activation=act, requant=rq)
+        assert np.array_equal(out[0], want[0]), (k, vars(case))
+        assert start is None or out[1][0] == want[1][0], k
+        assert rq is None or np.array_equal(out[2], want[2]), k
