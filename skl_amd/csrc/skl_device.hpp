@@ -135,27 +135,69 @@ __device__ __forceinline__ int skl_activate(int v, int act) {
   const int floor = act == 1 ? 0 : (int)0x80000000;  // uniform: one max per element
   return v < floor ? floor : v;
 }
+// f of 2^n 2^f = 2^(p C), C = c1 + c2, for n the whole number next to p C: at most a half, and exact to the last fused product.
+__device__ __forceinline__ float skl_exponent(float p, float c1, float c2, float n) {
+  return __builtin_fmaf(p, c2, __builtin_fmaf(p, c1, -n));
+}
 // SiLU, x * logistic(x). ref/sigmoid/sigmoid_f32.c:10-28 evaluates 1 / (1 + exp(-x)) * x in double and rounds once;
 // here in fp32, arranged so that nothing cancels and nothing leaves the normal range before the last product:
 // below -17, 1 + e^x is 1 to beyond fp32 and the value is x e^x; below -80, where e^x is a denormal and would
 // carry only a few bits, e^(x + 64) is multiplied in first and e^-64 last. Within a few ulp of the reference's
 // value (its own vector kernels are tested to 52 ulp, test/sigmoid/sigmoid_f32_zve32f.c).
+// From -17 on the exponential and the quotient are written out, without what expf and a division do for ranges that do not occur
+// (ns per value and wave, one wave per SIMD: 85.9, now 67.1; largest error in ulp 2.1 for both).
 __device__ __forceinline__ float skl_silu(float x) {
   if (x < -17.0f) {
     const bool deep = x < -80.0f;
     const float r = x * expf(deep ? x + 64.0f : x);
     return deep ? r * 1.6038108905486378e-28f : r;  // e^-64
   }
-  return x / (1.0f + expf(-x));
+  constexpr float c1 = -1.44269504088896341f, c2 = (float)(-1.44269504088896340736 - (double)c1);  // -log2 e
+  const float y = x < 100.0f ? x : 100.0f, n = __builtin_rintf(y * c1);  // (a NaN comes back with the quotient)
+  const float d = 1.0f + __builtin_ldexpf(__builtin_amdgcn_exp2f(skl_exponent(y, c1, c2, n)), (int)n);
+  float r = __builtin_amdgcn_rcpf(d);
+  r = __builtin_fmaf(__builtin_fmaf(-d, r, 1.0f), r, r);
+  float q = x * r;
+  q = __builtin_fmaf(__builtin_fmaf(-d, q, x), r, q);
+  return __builtin_amdgcn_div_fixupf(q, d, x);
 }
 // GELU, x Phi(x), in the reference's arrangement (ref/gelu/gelu_f32.c:12-22): an offset from the ReLU,
 // fma(-|x| / 2, erfc(|x| / sqrt 2), relu(x)) - nothing cancels on either side of zero. The reference evaluates erfc
 // and the fma in double; here fp32 (its own vector kernels are tested to 4 to 62 ulp by range,
 // test/gelu/skl_gelu_f32_zve32f.c).
+// erfc(t / sqrt 2) = exp(-t^2 / 2) g(t), t^2 with what its rounding leaves out, g a polynomial in (t - 3) / (t + 3) = 2 t / (t + 3) - 1;
+// below 0.55 erfc is 1 - t q(t^2) instead, whose leading 1 is exact. Both polynomials are least-squares fits of scipy's erfcx and erfc
+// reweighted towards the smallest largest relative error (Lawson's iteration): 1.5e-1 and 6e-4 units of 2^-24. Beyond 20 erfc is zero
+// in fp32. No branch, so that the chains of several values run side by side, and half of erfcf's instructions (ns per value and wave,
+// one wave per SIMD: erfcf of a rounded |x| / sqrt 2 117.3, now 76.2; largest error in ulp for x in [-14, -12], [-12, -8], [-8, -4],
+// [-4, -2], [-2, -1], [-1, -0.5], [-0.5, 0.5], above: 199, 177, 64, 17, 6.8, 3.1, 2.9, 1.5, now 17, 8.7, 8.6, 5.2, 3.8, 3.0, 1.6, 1.6).
 __device__ __forceinline__ float skl_gelu(float x) {
-  const float h = -0.5f * __builtin_fabsf(x);
-  const float e = erfcf(-1.41421356237309504880f * h);
-  return __builtin_fmaf(h, e, x > 0.0f ? x : -0.0f);
+  const float size = __builtin_fabsf(x), t = size < 20.0f ? size : 20.0f, p = t * t;
+  const float d = t + 3.0f, r = __builtin_amdgcn_rcpf(d);
+  float s = t * r;
+  s = __builtin_fmaf(__builtin_fmaf(-s, d, t), r, s);
+  const float y = __builtin_fmaf(s, 2.0f, -1.0f);
+  float g = 1.063238014e-04f;
+  g = __builtin_fmaf(g, y, 2.300272754e-04f);
+  g = __builtin_fmaf(g, y, -6.780256517e-04f);
+  g = __builtin_fmaf(g, y, -1.966576325e-03f);
+  g = __builtin_fmaf(g, y, 5.808774848e-03f);
+  g = __builtin_fmaf(g, y, 1.226388477e-02f);
+  g = __builtin_fmaf(g, y, -9.242652357e-02f);
+  g = __builtin_fmaf(g, y, 2.464500815e-01f);
+  g = __builtin_fmaf(g, y, -4.128052294e-01f);
+  g = __builtin_fmaf(g, y, 2.430278957e-01f);
+  constexpr float c1 = -0.72134752044448170f, c2 = (float)(-0.72134752044448170368 - (double)c1);  // -log2 e / 2
+  const float rest = __builtin_fmaf(t, t, -p), n = __builtin_rintf(p * c1);
+  const float f = __builtin_fmaf(rest, c1, skl_exponent(p, c1, c2, n));
+  float e = __builtin_ldexpf(__builtin_amdgcn_exp2f(f) * g, (int)n);
+  float q = 2.154276735e-04f;
+  q = __builtin_fmaf(q, p, -2.369920956e-03f);
+  q = __builtin_fmaf(q, p, 1.994646899e-02f);
+  q = __builtin_fmaf(q, p, -1.329807192e-01f);
+  q = __builtin_fmaf(q, p, 7.978845835e-01f);
+  e = t < 0.55f ? __builtin_fmaf(-t, q, 1.0f) : e;
+  return __builtin_fmaf(-0.5f * size, e, x > 0.0f ? x : -0.0f);
 }
 // 0 none, 1 ReLU, 2 SiLU, 3 GELU (floating point only).
 __device__ __forceinline__ float skl_activate(float v, int act) {
