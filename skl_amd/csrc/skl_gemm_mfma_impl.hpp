@@ -1461,12 +1461,15 @@ constexpr int kRingSlice = 64;   // bytes of K per stage
 // 128 tile are the exception: reads of eight bytes per lane and an address for each leave four waves of 16 x 16 products short of issue
 // slots. There fp8 takes eight waves, two to a SIMD, and int8 products of 32 x 32, half as many (us, with four waves and 16 x 16 / so;
 // 1024 x 4096^2, half the compute units: E4M3 27.2 / 24.9, int8 29.6 / 26.9; 2048 x 4096^2, all of them: 33.7 / 34.4 and 35.1 / 36.7).
+// And the 16-bit kinds' 256 x 128 tiles, whose starts and ends two waves to a SIMD cover better (bf16, four / eight waves: K contiguous
+// 1024 x 5632 x 896 17.7 / 16.2, 3328 x 1280 x 1152 19.8 / 18.1, 2048 x 4096^2 57.6 / 57.6; read across K 19.6 / 17.7, 22.2 / 20.1, 60.7 /
+// 61.8; of 8-bit operands full rounds lose what small problems gain: E4M3 4096 x 8192 x 1024 69 / 77, 3328 x 1280 x 1152 14.3 / 13.0).
 constexpr bool ring_few_issue_slots(int es, bool a_kc, bool b_kc, int bn) { return es == 1 && !a_kc && !b_kc && bn == 128; }
 template <int TA, bool A_KC, bool B_KC, int BN, bool EXACT>
-constexpr int kRingWaves = TA != SKL_DT_I8 && !EXACT && ring_few_issue_slots(Kind<TA>::ES, A_KC, B_KC, BN) ? 8 : 4;
+constexpr int kRingWaves = (BN == 128 && Kind<TA>::ES == 2) || (TA != SKL_DT_I8 && !EXACT && ring_few_issue_slots(Kind<TA>::ES, A_KC, B_KC, BN)) ? 8 : 4;
 // Stages of an operand's ring: four, or six of an operand with K contiguous where 160 KiB of LDS hold them (see the kernel's loads).
-constexpr int ring_stages_a(bool a_kc, bool b_kc, int bn, bool scan) { return !a_kc || (bn == 256 && (b_kc || scan)) ? 4 : 6; }
-constexpr int ring_stages_b(bool, bool b_kc, int bn, bool scan) { return !b_kc || (bn == 256 && scan) ? 4 : 6; }
+constexpr int ring_stages_a(bool a_kc, bool b_kc, int bn, bool scan) { return !a_kc || scan || (bn == 256 && b_kc) ? 4 : 6; }
+constexpr int ring_stages_b(bool, bool b_kc, int, bool scan) { return !b_kc || scan ? 4 : 6; }
 template <int ES, bool KC, int ROWS, int NS, int SIDE>
 struct STile {
   static constexpr int kStages = NS;
@@ -2385,46 +2388,52 @@ inline unsigned rounds_filled(size_t tiles, bool tail = false) {
   return (unsigned)(tiles * 200 / (256 * half_rounds));
 }
 
-// Whether the streaming kernel beats the bounds-checked ones on whole tiles where it has a handicap: the epilogue over
-// LDS rows (`staged`: an activation or a copy), which nothing overlaps while the bounds-checked kernels have several
-// workgroups on a compute unit, or the products of a short fp8 K, which are not long enough to outweigh a tile's start and
-// end. What decides is how full its last round is, how much K there is to gain on, and whether C is read, which it
-// requests earlier than the others do.
-// Its time over theirs, medians of some 1900 random problems of more than one round, by K in bytes and `filled`
-// (50-60 / 60-70 / 70-80 / 80-90 / 90-100 per cent); "-": no such problem was drawn:
-//   16 bits, SiLU or GELU, C read   below 1024  1.08 1.13 1.10 1.06 1.02   from 1024  1.12 1.08 1.07 0.91 0.95   from 2048  1.04 1.05 0.98 0.91 0.91   from 4096  0.99 0.97 0.90 0.90 0.80
-//                         not read  below 1024  1.22 1.20 1.29 1.03 1.07   from 1024    -  1.25 1.14 1.07 1.08   from 2048  1.16 1.06 1.12 0.92 1.01   from 4096  1.03 1.04 0.96 0.92 0.86
-//   16 bits, none or ReLU, C read   below 1024  0.73 1.00 0.95 0.94 0.89   from 1024  0.95 0.98 0.97 0.80 0.81   from 2048  1.01 0.91 0.90 0.87 0.79   from 4096  0.91 0.94 0.85 0.86 0.80
-//                         not read  below 1024  1.16 1.08 1.07 1.06 0.95   from 1024  1.05 1.15 0.93 0.91   -    from 2048  1.08 1.07 0.82   -  0.89   from 4096  0.97 0.88 0.96 0.82 0.81
-//   short fp8, SiLU or GELU, C read below 1024  1.19 1.22 1.17 1.07 1.02   from 1024  1.12 1.06 1.09 0.99 0.93
-//                         not read  below 1024  1.43 1.33 1.22 1.07 1.04   from 1024  1.31 1.21 1.13 1.03 0.96
-//   short fp8, none or ReLU, C read below 1024  1.01 1.01 0.92 0.90 0.91   from 1024  1.03 1.03 0.93 0.93 0.92
-//                         not read  below 1024  1.25 1.11 1.11 1.06 1.01   from 1024  1.09 1.15 1.07 0.97 0.90   with an fp8 copy 0.97 to 1.02 from 512 on
-//   short fp8, no steps, C read     up to 1024  0.90 0.92 0.87 0.85 0.85   beyond     0.99 0.92 0.89 0.84 0.80
-//                         not read  up to 256   1.11 1.13 1.14 1.08 1.08   up to 1024 1.10 1.06 1.05 0.96 0.95   beyond 1.04 0.99 1.00 0.90 0.84
-//   int8                            C read 0.60 to 0.91, not read 0.67 to 0.99, at any K
-// A single round, full or nearly: 0.7 to 0.95 for all of them, short fp8 without steps 1.06 up to K = 256. With a K of 8 KiB
-// and more also 129 to 199 tiles, 0.82, and 65 to 128, which share K, 0.78; exactly 64 are 128 bounds-checked tiles, which
-// share it four ways: 1.12 to 1.24. (At 96 tiles of a shorter K f16 1024 x 3072 x 1024 with ReLU takes 23.3 us against 22.1.)
+// Whether the streaming kernel beats the bounds-checked ones on whole tiles: those have several workgroups on a compute unit, whose
+// starts and ends overlap with others' products, it has one. What decides is how full its last round is, how much K there is to gain
+// on, and whether C is read, which it requests earlier than the others do; an activation of some thirty or forty instructions (SiLU,
+// GELU) is covered by nothing there. Its time over theirs, geometric means over random problems, by K in bytes; more than one round, by
+// `filled` (50-60 / 60-70 / 70-80 / 80-90 / 90-100 per cent); "-": fewer than three were drawn:
+//   16 bits, plain        from 1024  1.19 1.19 1.14 1.03 1.00   from 2048  1.00 1.02 0.93 0.91 0.91   from 4096  0.94 0.92 0.80 0.85  -
+//     C read              from 1024  1.01 1.01 0.95 0.92 0.91   from 2048  0.99 0.94 0.93 0.88 0.82
+//     ReLU or a copy      from 1024  1.02 1.01 0.97 0.91 0.87   from 2048  0.98 0.95 0.89 0.87  -
+//     SiLU or GELU        from 1024  1.38 1.25 1.28 1.18 1.12   from 2048  1.18 1.13 1.10 1.04  -     from 4096  1.06 1.03 0.97 0.89 0.87   from 8192  0.95 0.94 0.84 - -
+//   fp8, plain            from 2305  1.04 1.05 0.95  -    -     from 4096  0.95 0.96  -    -    -
+//   short fp8, plain      from  512  1.45 1.39 1.25 1.21 1.18   from 1024  1.32 1.24 1.09 1.10 1.00   from 2048  1.23  -   -    -    -
+//     C read              from  512  1.12 1.06 1.00 1.02 0.97   from 1024  1.16 1.14 1.04 0.99 0.93
+//     ReLU or a copy      from  512  1.19 1.16 1.11 1.04 0.97   from 1024  1.17 1.12 1.09 0.99 0.88   from 2048   -   1.15  -  0.92  -
+//     SiLU or GELU        from  512  1.45 1.47  -   1.19 1.21   from 1024  1.36 1.31 1.37 1.14 1.02
+//   int8, plain           from  512  1.16 1.14 1.16 1.10 1.09   from 1024  1.08 1.08 0.98 1.01 0.98   from 2048  0.94 0.99 0.94 0.85  -
+//     C read              0.69 to 0.85 at any K
+//     ReLU or a copy      from  512  1.22 1.16 1.14 1.08 1.11   from 1024  1.11 1.12 1.07 1.00 0.93   from 2048  1.00  -   1.01  -   0.95
+// A single round of 200 to 256 tiles: short fp8 plain 1.07 below 2048, with SiLU or GELU 1.15 below 1024, all others less than one.
+// 129 to 199 tiles: SiLU or GELU 0.83 from 4096 (fp8 0.89), short fp8 with C read, ReLU or a copy 0.92. 96 to 128 tiles, half of the
+// chip: plain 16 bits 1.37 from 1024, 1.23 from 2048, fp8 1.20 from 2305, int8 1.27, 1.21 and 1.14 from 512, 1024 and 2048. With a K of 8 KiB
+// and more also 65 to 128 tiles with steps, which share K, 0.78; exactly 64 are 128 bounds-checked tiles, which
+// share it four ways: 1.12 to 1.24.
 template <typename AccElem, bool EXACT, bool A_KC, bool B_KC, bool FP8>
-bool ring_pays(const MfmaArgs &p, bool staged, size_t tiles, size_t k_bytes, bool long_k, unsigned filled) {
+bool ring_pays(const MfmaArgs &p, size_t tiles, size_t k_bytes, bool long_k, unsigned filled) {
   constexpr bool kInt = std::is_same<AccElem, int>::value;
   constexpr bool kSlowOthers = FP8 && !EXACT && !(A_KC && B_KC);  // transposed fragments of 32 bytes: they take two to four times as long
   constexpr unsigned kNever = 101;
   const bool reads_c = kInt ? p.beta.i != 0 : !(p.beta.fz.skip_c_read && p.beta.f == 0.0f);
-  if (tiles < 200) return staged && long_k && (tiles > 64 || kSlowOthers);
-  if (tiles <= 256) return staged || reads_c || k_bytes > 256;
-  if (!staged) return reads_c || filled >= (k_bytes > 1024 ? 60 : k_bytes > 256 ? 80 : kNever);
-  if (kInt || kSlowOthers) return true;
-  if (!p.rq.q_only && p.csc0 != 1) return true;  // C written by columns: the others take three to four times as long
-  if (p.rq.act >= 2) {
-    if (reads_c) return filled >= (k_bytes >= 4096 ? 0 : k_bytes >= 2048 ? 70 : k_bytes >= 1024 ? 80 : kNever);
-    return filled >= (k_bytes >= 4096 ? 70 : k_bytes >= 2048 ? 80 : EXACT && k_bytes >= 1024 ? 90 : kNever);
+  const bool steps = p.rq.act || p.rq.q, many_steps = p.rq.act >= 2;
+  const bool in_rows = p.csc0 == 1 && (p.ccs >= 6 || p.csc1 == (size_t(1) << p.ccs));  // a C that is not: the others take three to four times as long
+  if (tiles < 200) {
+    if (long_k) return tiles > 64 || !steps || kSlowOthers;
+    if (EXACT) return tiles > 128 && (reads_c || (steps && !many_steps));
+    if (steps && !dword_copy<AccElem>(p.rq)) return many_steps && tiles > 128 && k_bytes >= 4096;
+    return steps || tiles > 128 || reads_c || k_bytes >= 4096 || kSlowOthers || !in_rows;
   }
-  if (reads_c) return !EXACT || filled >= 70;
-  if (EXACT && p.rq.q && p.rq.q_fmt != 0) return k_bytes >= 512 || filled >= 70;
-  if (EXACT) return filled >= (k_bytes >= 1024 ? 80 : kNever);
-  return filled >= (k_bytes >= 4096 ? 0 : k_bytes >= 1024 ? 70u : 90u);
+  if (tiles <= 256) return !EXACT || reads_c || k_bytes >= (many_steps ? 1024 : steps ? 0 : 2048);
+  if (kSlowOthers || (!in_rows && (!EXACT || steps) && !p.rq.q_only)) return true;
+  if (many_steps) {
+    if (reads_c) return filled >= (k_bytes >= 4096 ? 0 : k_bytes >= 2048 ? 70 : k_bytes >= 1024 ? 80 : kNever);
+    return filled >= (k_bytes >= 8192 ? 0 : k_bytes >= 4096 ? 70 : k_bytes >= 2048 ? 80 : EXACT && k_bytes >= 1024 ? 90 : kNever);
+  }
+  if (EXACT) return filled >= (reads_c ? 80 : steps ? k_bytes >= 1024 ? 80 : 90 : k_bytes >= 2048 ? 80 : k_bytes >= 1024 ? 90 : kNever);
+  if (reads_c) return true;
+  if (kInt) return steps || filled >= (k_bytes >= 2048 ? 0 : k_bytes >= 1024 ? 70 : kNever);
+  return filled >= (k_bytes >= 2048 || steps ? 0 : 80);
 }
 
 // The streaming kernel takes problems that its tiles divide evenly: 256 x 256 tiles when those can fill the 256 compute
@@ -2448,10 +2457,8 @@ int launch_whole_tiles(const MfmaArgs &p) {
   const bool long_k = slices % 4 == 0 && slices / 2 >= kRingMinSlicesPerSplit;
   const bool extra = p.rq.act || p.rq.q;
   if (extra && !kRingCarriesExtraSteps<TA, TB>) return kNotWholeTiles;
-  const bool staged = extra && !(!EXACT && dword_copy<AccElem>(p.rq));
-  if ((staged || EXACT) &&
-      !ring_pays<AccElem, EXACT, A_KC, B_KC, TA == SKL_DT_F8E4M3 || TA == SKL_DT_F8E5M2>(
-          p, staged, tiles >= 200 ? tiles : tiles128, p.k * ES, long_k, tiles >= 200 ? rounds_filled(tiles, tail_round) : rounds_filled(tiles128)))
+  if (!ring_pays<AccElem, EXACT, A_KC, B_KC, TA == SKL_DT_F8E4M3 || TA == SKL_DT_F8E5M2>(
+          p, tiles >= 200 ? tiles : tiles128, p.k * ES, long_k, tiles >= 200 ? rounds_filled(tiles, tail_round) : rounds_filled(tiles128)))
     return kNotWholeTiles;
   if (tiles >= 200) {
     if (!tail_round) return wide(p);
@@ -2475,27 +2482,43 @@ int launch_whole_tiles(const MfmaArgs &p) {
 }
 
 // The streaming kernel on problems that are not whole tiles (EDGE): the tile's columns, or 0 where the bounds-checked kernels
-// are as good. Those have 512 tiles of 128 x 128 on the chip at a time and waste little of a last round; a round of 256 x 256
-// tiles takes as long as about 745 of theirs, from 4 KiB of K on (below, starts and ends of the larger tiles show: bf16
-// 6016 x 6848 x 896 with SiLU 176 against 153 us). The 256 x 128 tiles gain nothing on full rounds; a single round of them
-// does, over 353 tiles and more that are one long round there too, where C is read, which they request earlier, or where
-// operands read across K are long. Bounds-checked / streaming, us: bf16 3000 x 5000 x 7000 267 / 207, int8 2176 x 2816 x 512
-// reading C 33.8 / 19.9, bf16 2880 x 2176 x 5425 with A by columns 98 / 71; over 367 random problems the rule takes 22, at
-// 0.82 of the bounds-checked kernels' time, the worst 1.10.
+// are as good. Those have 512 tiles of 128 x 128 on the chip at a time and waste little of a last round, so what counts is how much
+// of the larger tiles' rounds the 128 x 128 ones that exist would fill (per cent), then K, and as in ring_pays whether C is read
+// and what is behind the product. Streaming over bounds-checked, geometric means over 4829 random problems, 256 columns from the line on
+// to ten per cent beyond it: int8 reading C 0.77 to 0.83, else 0.79 to 0.93; other kinds 0.90 to 0.98, from 8 KiB of K 0.81, with SiLU or GELU
+// 0.94 and 0.90; below the line 1.00 to 1.35. 128 columns 0.82 to 0.95. The problems that the rule moves take 0.73 (int8 reading C) to
+// 0.95 (16 bits reading C, 128 columns) of the time.
+// Floating point only beyond 256 tiles of 128 x 128: fewer share K, and sums of several parts are the more exact ones.
 template <int TA, int TB, bool A_KC, bool B_KC>
 int ragged_tile_cols(const MfmaArgs &p) {
   constexpr size_t ES = Kind<TA>::ES, limit = 0xB0000000u;
   if (p.a_loose || p.b_loose || ((p.rq.act || p.rq.q) && !kRingCarriesExtraSteps<TA, TB>)) return 0;
+  if (p.m % 256 == 0 && p.n % 128 == 0 && p.k * ES % 128 == 0) return 0;  // whole tiles: launch_whole_tiles has decided
   // 16 bytes along K that K ends in would need zeros behind it; the offsets inside a tile stay in the descriptor's range
   if (p.k * ES % 16 != 0 && (A_KC || B_KC)) return 0;
   if ((3 * p.a_s1 + (A_KC ? 63 * p.a_s0 : 64 * p.a_sk)) * ES >= limit || (3 * p.b_s1 + (B_KC ? 63 * p.b_s0 : 64 * p.b_sk)) * ES >= limit) return 0;
   const size_t tiles_m = (p.m + 255) / 256, wide = tiles_m * ((p.n + 255) / 256), narrow = tiles_m * ((p.n + 127) / 128);
   const size_t small = (size_t)skl_div_up(p.m, 128) * skl_div_up(p.n, 128), k_bytes = p.k * ES;
-  if (k_bytes >= 4096 && small >= (wide + 255) / 256 * 745) return 256;
-  const bool reads_c = std::is_same<decltype(typename Kind<TA>::Acc{}.x), int>::value ? p.beta.i != 0 : !(p.beta.fz.skip_c_read && p.beta.f == 0.0f);
-  const bool plain = !p.rq.act && !p.rq.q;
-  if (plain && narrow <= 256 && small >= 353 && (reads_c || (k_bytes >= 8192 && !(A_KC && B_KC)))) return 128;
-  return 0;
+  constexpr bool kInt = std::is_same<decltype(typename Kind<TA>::Acc{}.x), int>::value;
+  constexpr unsigned kNever = 101;
+  const bool reads_c = kInt ? p.beta.i != 0 : !(p.beta.fz.skip_c_read && p.beta.f == 0.0f);
+  const unsigned of_wide = (unsigned)(small * 100 / ((wide + 255) / 256 * 1024)), of_narrow = (unsigned)(small * 100 / ((narrow + 255) / 256 * 512));
+  const auto by_k = [&](unsigned from_512, unsigned from_1k, unsigned from_2k, unsigned from_4k, unsigned from_8k) {
+    return k_bytes >= 8192 ? from_8k : k_bytes >= 4096 ? from_4k : k_bytes >= 2048 ? from_2k : k_bytes >= 1024 ? from_1k : k_bytes >= 512 ? from_512 : kNever;
+  };
+  if (!kInt && small <= 256) return 0;
+  unsigned from_wide, from_narrow;
+  if (kInt) {
+    from_wide = reads_c ? by_k(65, 65, 55, 55, 55) : by_k(kNever, kNever, 80, 55, 55);
+    from_narrow = reads_c ? by_k(55, 55, 55, 55, 55) : by_k(kNever, kNever, kNever, 55, 55);
+  } else if (p.rq.act >= 2) {
+    from_wide = by_k(kNever, kNever, kNever, 70, 52);
+    from_narrow = by_k(kNever, kNever, kNever, kNever, 55);
+  } else {
+    from_wide = by_k(kNever, reads_c ? 80 : kNever, 70, 60, 52);
+    from_narrow = by_k(kNever, kNever, kNever, 70, 52);
+  }
+  return of_wide >= from_wide ? 256 : of_narrow >= from_narrow ? 128 : 0;
 }
 template <int TA, int TB, bool A_KC, bool B_KC>
 int launch_ragged(const MfmaArgs &p, int tile_cols) {

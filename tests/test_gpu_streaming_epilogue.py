@@ -1,7 +1,7 @@
 """How the streaming kernel starts and ends a tile: K of one to five pairs of slices (as many as it requests ahead, fewer, more),
-both tile widths, and C as its rows in LDS are handed out - row-major on and off 16-byte boundaries, by columns, read and not,
-with every step behind the product. int8, so that all of it is exact and compared bit for bit with the product in int64; the
-values behind alpha = 0x01010101 use all 32 bits."""
+both tile widths, whole tiles and ragged ones at the lines where the dispatch takes them, and C as its rows in LDS are handed out -
+row-major on and off 16-byte boundaries, by columns, read and not, with every step behind the product. int8, so that all of it is
+exact and compared bit for bit with the product in int64; the values behind alpha = 0x01010101 use all 32 bits."""
 import numpy as np
 import pytest
 
@@ -12,22 +12,32 @@ from test_oracle_gemm import fused_expectation
 
 pytestmark = pytest.mark.gpu
 
-SIZES = ((2048, 1536), (4096, 3328))  # 96 tiles of 256 x 128, 208 of 256 x 256
+SHORT = (128, 256, 384, 512, 640)
+# 136 tiles of 256 x 128, 208 of 256 x 256; 180 and 208 ragged ones (360 and 832 of 128 x 128, 70 and 81 per cent of a round), and a
+# little below and above the line for 256 x 128 ones where C is read (280 and 306 of 512)
+SIZES = ((4352, 1024, SHORT), (4096, 3328, SHORT), (2300, 2500, (528, 1040, 2064, 4112, 656)), (4001, 3300, (528, 2064, 1072, 1040, 4112)),
+         (2500, 1790, (528, 2064, 528, 4112, 656)), (2300, 2070, (528, 2064, 656, 4112, 1040)))
+
+
+def matrix(x, rows, run, ld):
+    return np.lib.stride_tricks.as_strided(x, (rows, run), (ld * x.itemsize, x.itemsize))
 
 
 @pytest.mark.parametrize("a_kc,b_kc", ((True, True), (True, False), (False, False), (False, True)))
-@pytest.mark.parametrize("m,n", SIZES)
-def test_streamed_tiles_from_short_to_longer_k(gpu, m, n, a_kc, b_kc):
+@pytest.mark.parametrize("m,n,ks", SIZES)
+def test_streamed_tiles_from_short_to_longer_k(gpu, m, n, ks, a_kc, b_kc):
     rng = np.random.default_rng(m + 2 * a_kc + b_kc)
-    for i, k in enumerate((128, 256, 384, 512, 640)):
+    for i, k in enumerate(ks):
         by_columns, pad, beta = i % 4 == 2, (0, 3, 5, 4, 1)[i], (0, -77, 1, 0, 3)[i]
+        lda, ldb = k if a_kc else -(-m // 16) * 16, k if b_kc else -(-n // 16) * 16
         rsc, csc = (1, m + pad) if by_columns else (n + pad, 1)
         case = GemmCase("i8", None, (1, 0x01010101, -3, 7, 2)[i], beta, m0=1, n0=1, k0=1, m1=m, n1=n, k1=k, rsa0=0, csa0=0,
-                        rsa1=k if a_kc else 1, csa1=1 if a_kc else m, rsb0=0, csb0=0, rsb1=1 if b_kc else n, csb1=k if b_kc else 1,
+                        rsa1=lda if a_kc else 1, csa1=1 if a_kc else lda, rsb0=0, csb0=0, rsb1=1 if b_kc else ldb, csb1=ldb if b_kc else 1,
                         rsc0=0, csc0=0, rsc1=rsc, csc1=csc)
         a, b, c = case.make_inputs(k + n)
         c[:] = rng.integers(-2 ** 31, 2 ** 31, size=c.size)
-        x, y = a.reshape(m, k) if a_kc else a.reshape(k, m).T, b.reshape(n, k).T if b_kc else b.reshape(k, n)
+        x = matrix(a, m, k, lda) if a_kc else matrix(a, k, m, lda).T
+        y = matrix(b, n, k, ldb).T if b_kc else matrix(b, k, n, ldb)
         rows = support.blocked_offsets(case.m1, case.n1, case.m0, case.n0, case.rsc0, case.csc0, case.rsc1, case.csc1)
         sums = (x.astype(np.float64) @ y.astype(np.float64)).astype(np.int64).reshape(rows.shape)
         plain = c.copy()
