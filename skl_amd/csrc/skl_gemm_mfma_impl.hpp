@@ -1461,15 +1461,15 @@ constexpr int kRingSlice = 64;   // bytes of K per stage
 // 128 tile are the exception: reads of eight bytes per lane and an address for each leave four waves of 16 x 16 products short of issue
 // slots. There fp8 takes eight waves, two to a SIMD, and int8 products of 32 x 32, half as many (us, with four waves and 16 x 16 / so;
 // 1024 x 4096^2, half the compute units: E4M3 27.2 / 24.9, int8 29.6 / 26.9; 2048 x 4096^2, all of them: 33.7 / 34.4 and 35.1 / 36.7).
-// And the 16-bit kinds' 256 x 128 tiles, whose starts and ends two waves to a SIMD cover better (bf16, four / eight waves: K contiguous
-// 1024 x 5632 x 896 17.7 / 16.2, 3328 x 1280 x 1152 19.8 / 18.1, 2048 x 4096^2 57.6 / 57.6; read across K 19.6 / 17.7, 22.2 / 20.1, 60.7 /
-// 61.8; of 8-bit operands full rounds lose what small problems gain: E4M3 4096 x 8192 x 1024 69 / 77, 3328 x 1280 x 1152 14.3 / 13.0).
+// And the 16-bit kinds' ragged 256 x 128 tiles, whose starts, ends and chosen offsets two waves to a SIMD cover better (f16 2944 x 2048 x
+// 8125 read across K 121 / 109). Not whole ones: small problems gain what full rounds lose (bf16, four / eight waves: 1024 x 5632 x
+// 896 17.7 / 16.2, 3328 x 1280 x 1152 19.8 / 18.1, but 2048 x 4096^2 reading C 62.3 / 65.5; E4M3 4096 x 8192 x 1024 69 / 77).
 constexpr bool ring_few_issue_slots(int es, bool a_kc, bool b_kc, int bn) { return es == 1 && !a_kc && !b_kc && bn == 128; }
-template <int TA, bool A_KC, bool B_KC, int BN, bool EXACT>
-constexpr int kRingWaves = (BN == 128 && Kind<TA>::ES == 2) || (TA != SKL_DT_I8 && !EXACT && ring_few_issue_slots(Kind<TA>::ES, A_KC, B_KC, BN)) ? 8 : 4;
+template <int TA, bool A_KC, bool B_KC, int BN, bool EDGE, bool EXACT>
+constexpr int kRingWaves = (BN == 128 && EDGE && Kind<TA>::ES == 2) || (TA != SKL_DT_I8 && !EXACT && ring_few_issue_slots(Kind<TA>::ES, A_KC, B_KC, BN)) ? 8 : 4;
 // Stages of an operand's ring: four, or six of an operand with K contiguous where 160 KiB of LDS hold them (see the kernel's loads).
-constexpr int ring_stages_a(bool a_kc, bool b_kc, int bn, bool scan) { return !a_kc || scan || (bn == 256 && b_kc) ? 4 : 6; }
-constexpr int ring_stages_b(bool, bool b_kc, int, bool scan) { return !b_kc || scan ? 4 : 6; }
+constexpr int ring_stages_a(bool a_kc, bool b_kc, int bn, bool scan) { return !a_kc || (bn == 256 && (b_kc || scan)) ? 4 : 6; }
+constexpr int ring_stages_b(bool, bool b_kc, int bn, bool scan) { return !b_kc || (bn == 256 && scan) ? 4 : 6; }
 template <int ES, bool KC, int ROWS, int NS, int SIDE>
 struct STile {
   static constexpr int kStages = NS;
@@ -1725,7 +1725,7 @@ constexpr int ceil_div(int a, int b) { return (a + b - 1) / b; }
 // more vector work than the matrix cores take for the products; here sixteen for 64 (256 columns) or twelve for 32 (128).
 // E4M3 2048 x 8192 x 2048: 77 us there, 62 with eight waves of 32 x 32 products here; with a bias, into E4M3, 73 so and now 59.
 template <int TA, int TB, bool A_KC, bool B_KC, int BN, bool EDGE = false, bool STEPS = false, bool SCAN = false, bool EXACT = false>
-__global__ void __launch_bounds__((kRingWaves<TA, A_KC, B_KC, BN, EXACT> * 64)) gemm_mfma_ring_kernel(MfmaArgs p) {
+__global__ void __launch_bounds__((kRingWaves<TA, A_KC, B_KC, BN, EDGE, EXACT> * 64)) gemm_mfma_ring_kernel(MfmaArgs p) {
   constexpr bool kLarge = TA == SKL_DT_I8 && ring_few_issue_slots(1, A_KC, B_KC, BN);
   using M = typename std::conditional<kLarge, RingMmaI8Large, RingMma<TA, TB, EXACT>>::type;
   using Frag = typename M::Frag;
@@ -1733,7 +1733,7 @@ __global__ void __launch_bounds__((kRingWaves<TA, A_KC, B_KC, BN, EXACT> * 64)) 
   using AccElem = decltype(Acc{}.x);
   constexpr int SB = kRingSlice, NSA = ring_stages_a(A_KC, B_KC, BN, SCAN), NSB = ring_stages_b(A_KC, B_KC, BN, SCAN);
   constexpr int ES = Kind<TA>::ES, S = M::kSide, FRB = M::kFrag;
-  constexpr int BM = 256, WAVES = kRingWaves<TA, A_KC, B_KC, BN, EXACT>, WAVES_N = 2, WAVES_M = WAVES / WAVES_N;
+  constexpr int BM = 256, WAVES = kRingWaves<TA, A_KC, B_KC, BN, EDGE, EXACT>, WAVES_N = 2, WAVES_M = WAVES / WAVES_N;
   constexpr int WM = BM / WAVES_M, WN = BN / WAVES_N, MI = WM / S, NI = WN / S;
   // A step is a slice: the products of the wave's blocks, once, or EXACT with each half of the fragments' bytes.
   constexpr int kProducts = MI * NI, kSlots = (EXACT || kLarge ? 2 : 1) * kProducts;
@@ -2239,7 +2239,7 @@ int launch_ring(const MfmaArgs &args) {
     if (args.beta.f == 0.0f && args.beta.fz.skip_c_read == 0 && !shared_k && (row_major || panels) && scan_slices >= (BN == 256 ? 64 : 32))
       return launch_ring<TA, TB, A_KC, B_KC, BN, EDGE, false, true>(args);
   }
-  constexpr int kWaves = kRingWaves<TA, A_KC, B_KC, BN, EXACT>;
+  constexpr int kWaves = kRingWaves<TA, A_KC, B_KC, BN, EDGE, EXACT>;
   constexpr int lds = (ring_stages_a(A_KC, B_KC, BN, SCAN) * 256 + ring_stages_b(A_KC, B_KC, BN, SCAN) * BN) * kRingSlice + (SCAN ? 4 * kWaves * 1024 : 0);
   static_assert(lds <= 160 * 1024);
   auto kernel = gemm_mfma_ring_kernel<TA, TB, A_KC, B_KC, BN, EDGE, STEPS, SCAN, EXACT>;
@@ -2404,7 +2404,8 @@ inline unsigned rounds_filled(size_t tiles, bool tail = false) {
 //     SiLU or GELU        from  512  1.45 1.47  -   1.19 1.21   from 1024  1.36 1.31 1.37 1.14 1.02
 //   int8, plain           from  512  1.16 1.14 1.16 1.10 1.09   from 1024  1.08 1.08 0.98 1.01 0.98   from 2048  0.94 0.99 0.94 0.85  -
 //     C read              0.69 to 0.85 at any K
-//     ReLU or a copy      from  512  1.22 1.16 1.14 1.08 1.11   from 1024  1.11 1.12 1.07 1.00 0.93   from 2048  1.00  -   1.01  -   0.95
+//     ReLU or a copy      from  512  1.22 1.16 1.14 1.08 1.11   from 1024  1.11 1.12 1.07 1.00 0.93   from 2048  1.00  -   1.01  -   0.95 (a copy in dwords; ReLU into C
+//                         the other way, 6656 x 4864 x 640 40 against 46 us: the streaming kernel keeps both)
 // A single round of 200 to 256 tiles: short fp8 plain 1.07 below 2048, with SiLU or GELU 1.15 below 1024, all others less than one.
 // 129 to 199 tiles: SiLU or GELU 0.83 from 4096 (fp8 0.89), short fp8 with C read, ReLU or a copy 0.92. 96 to 128 tiles, half of the
 // chip: plain 16 bits 1.37 from 1024, 1.23 from 2048, fp8 1.20 from 2305, int8 1.27, 1.21 and 1.14 from 512, 1024 and 2048. With a K of 8 KiB
