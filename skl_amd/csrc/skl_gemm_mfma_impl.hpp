@@ -227,7 +227,7 @@ constexpr size_t kF8ExactMaxK = 2304;
 // vector registers (IN_A false): where all accumulation registers are taken the compiler copies a block out and back around a
 // product, which it does not know to be under way.
 // run() with a load: also 16 bytes per lane from g + off to LDS at `lds` + AT (a load to LDS takes its place there from M0, which is
-// to be written an instruction ahead).
+// to be written an instruction ahead; the compiler takes no clobber of M0, so every other load of such a kernel is load_to_lds).
 #define SKL_RING_PRODUCT(IN_, INSN, MODS) asm volatile("v_mfma_" INSN " %0, %1, %2, %0" MODS : "+" IN_(c) : "v"(b), "v"(a))
 #define SKL_RING_PRODUCT_LOAD(IN_, INSN, MODS)                                                                       \
   asm volatile("s_add_u32 m0, %3, %6\n\tv_mfma_" INSN " %0, %1, %2, %0" MODS "\n\tglobal_load_lds_dwordx4 %4, %5"   \
@@ -1499,6 +1499,12 @@ struct STile {
   }
 };
 
+// 16 bytes per lane from g + off to LDS at `lds`, where the wave's KiB begins. (In assembly, like the loads that go out with a product
+// (RingMma): those write M0 without the compiler's knowing, so no load beside them may be one for which it keeps M0.)
+__device__ __forceinline__ void load_to_lds(unsigned lds, const char *g, unsigned off) {
+  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(lds), "v"(off), "s"(g) : "memory");
+}
+
 // Global -> LDS loads of one operand, this wave's share. `unit` below is a slice
 // for an MN-contiguous operand and a pair of slices for a K-contiguous one.
 // EDGE: the operand ends inside the tile, along M / N or along K. Its loads go through a buffer descriptor whose base follows K
@@ -1526,10 +1532,10 @@ struct SLoader {
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
     tile_base = base + (mn0 >> 6) * s1 * ES;
     lds = wave * kBlocks * kBlockStep;
-    if constexpr (EDGE) {  // spelled out as scalars, like the step below: a descriptor in vector registers costs a loop over the lanes per load
-      const uintptr_t at = (uintptr_t)tile_base;
-      tile_base = (const char *)(((uintptr_t)(unsigned)__builtin_amdgcn_readfirstlane((int)(at >> 32)) << 32) | (unsigned)__builtin_amdgcn_readfirstlane((int)at));
-    }
+    // spelled out as scalars, like the step below: the loads take their base as one (EDGE: a descriptor in vector registers costs a
+    // loop over the lanes per load)
+    const uintptr_t at = (uintptr_t)tile_base;
+    tile_base = (const char *)(((uintptr_t)(unsigned)__builtin_amdgcn_readfirstlane((int)(at >> 32)) << 32) | (unsigned)__builtin_amdgcn_readfirstlane((int)at));
 #pragma unroll
     for (int i = 0; i < kBlocks; ++i) {
       const int b = wave * kBlocks + i;
@@ -1575,18 +1581,16 @@ struct SLoader {
   // Requests block `i` of `unit`; it lands in stage `stage` (the even one of the pair for KC) of `region`.
   __device__ __forceinline__ void issue_one(char *region, int stage, size_t unit, unsigned left, int i) const {
     const char *g = tile_base + unit * k_step;
-    // The lane's offset through a copy the compiler cannot follow: it otherwise widens every offset to 64 bits ahead
-    // of the loop (two registers each) and adds the scalar base with a 64-bit vector add per load; this way the load
-    // takes the scalar base and the 32-bit offset as they are.
-    unsigned o = offset(left, i);
-    asm volatile("" : "+v"(o));
-    if constexpr (EDGE)
+    if constexpr (EDGE) {
+      // The lane's offset through a copy the compiler cannot follow: it otherwise widens every offset to 64 bits ahead
+      // of the loop, two registers each.
+      unsigned o = offset(left, i);
+      asm volatile("" : "+v"(o));
       __builtin_amdgcn_raw_ptr_buffer_load_lds(__builtin_amdgcn_make_buffer_rsrc((void *)g, 0, (int)kRange, 0x00027000),
                                                (__attribute__((address_space(3))) void *)(region + stage * T::kStageStep + lds + i * kBlockStep), 16, (int)o, 0, 0, 0);
-    else
-      __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void *)(g + o),
-                                       (__attribute__((address_space(3))) void *)(region + stage * T::kStageStep + lds + i * kBlockStep),
-                                       16, 0, 0);
+    } else {
+      load_to_lds((unsigned)(size_t)LDS_PTR(char, region) + stage * T::kStageStep + lds + i * kBlockStep, g, off[i]);
+    }
   }
 };
 
@@ -1853,8 +1857,7 @@ __global__ void __launch_bounds__((kRingWaves<TA, A_KC, B_KC, BN, EDGE, EXACT> *
       mine = l * 16u;                                                                // 64 lanes x 16 bytes: one row of 256 columns
     else
       mine = (l & 31u) * 16u + ((unsigned)((int)(l << 26) >> 31) & (scan_panels ? 512u : (unsigned)p.rsc0 * 4u));  // lanes 32-63: the row below (panels: the next 512 bytes)
-    __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void *)(rows + mine),
-                                     (__attribute__((address_space(3))) void *)(scan_region + s % kScanSlots * kScanSlot), 16, 0, 0);
+    load_to_lds(scan_addr + s % kScanSlots * kScanSlot, rows, mine);
   };
   [[maybe_unused]] auto scan_read = [&](unsigned slot) {  // this wave's 1024 bytes in `slot`; the value counts from the next lgkmcnt(0) on
     unsigned l = __builtin_amdgcn_mbcnt_hi(~0u, __builtin_amdgcn_mbcnt_lo(~0u, 0u));
