@@ -1841,13 +1841,13 @@ __global__ void __launch_bounds__((kRingWaves<TA, A_KC, B_KC, BN, EDGE, EXACT> *
   const bool scan_panels = p.rsc0 == 64 && p.rsc1 != 64 * 64;
   const char *const scan_rows = scan_panels ? reinterpret_cast<const char *>(p.c) + ((m0 >> 6) * p.rsc1 + (n0 >> 6) * p.csc1) * 4
                                             : reinterpret_cast<const char *>(p.c) + ((m0 + (size_t)wave * kScanRowsPerLoad) * p.rsc0 + n0) * 4;
-  const unsigned scan_step = (unsigned)p.rsc0 * (WAVES * kScanRowsPerLoad * 4u);
+  // (each layout's own steps, the other's are zero: a choice inside the loop would be a branch, see SLoader::offset)
+  const unsigned scan_step = scan_panels ? 0u : (unsigned)p.rsc0 * (WAVES * kScanRowsPerLoad * 4u), scan_piece = scan_panels ? 1024u : 0u;
+  const size_t scan_panel_row = scan_panels ? p.rsc1 * 4 : 0, scan_panel_col = scan_panels ? p.csc1 * 4 : 0;
   [[maybe_unused]] auto scan_issue = [&](unsigned s) {  // load s of this wave (the last one again beyond the tile)
     const unsigned q = s < kScanLoadsPerWave ? s : kScanLoadsPerWave - 1;  // uniform
-    // (no branch, see SLoader::offset)
     const unsigned piece = q * WAVES + wave, panel = piece >> 4, pi = panel / (BN / 64), pj = panel % (BN / 64);
-    const size_t in_panels = ((size_t)pi * p.rsc1 + (size_t)pj * p.csc1) * 4 + (piece & 15u) * 1024u;
-    const char *rows = scan_rows + (scan_panels ? in_panels : (size_t)q * scan_step);
+    const char *rows = scan_rows + (pi * scan_panel_row + pj * scan_panel_col + (piece & 15u) * scan_piece + (size_t)q * scan_step);
     // The lane's own part of the address is computed anew for every load, from a lane index the compiler cannot
     // follow: held across the loop it would be a register that the loop does not have.
     unsigned l = __builtin_amdgcn_mbcnt_hi(~0u, __builtin_amdgcn_mbcnt_lo(~0u, 0u));
@@ -2046,9 +2046,10 @@ __global__ void __launch_bounds__((kRingWaves<TA, A_KC, B_KC, BN, EDGE, EXACT> *
           }(std::integral_constant<int, Us>{}),
           ...);
     }(std::make_integer_sequence<int, 2>{});
-    // The sums' registers are not to be read before the last product has written them, and the compiler, to which these are no matrix
-    // instructions, may copy one as soon as the loop is left: the time the product takes anyway.
-    asm volatile("s_nop %0" ::"n"(S == 32 ? 15 : 3));
+    // The sums' registers are not to be touched before the last product has written them, and the compiler, to which these are no matrix
+    // instructions, may copy one as soon as the loop is left: the product's passes (16 x 16: 4, fp8 32 x 32: 16) and four states.
+    asm volatile("s_nop %0" ::"n"(S == 32 ? 15 : 7));
+    if constexpr (S == 32) asm volatile("s_nop 3");
     six = six_next;
     s0 += 2;
   } while (s0 < slices);

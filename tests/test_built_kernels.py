@@ -94,6 +94,22 @@ def test_operands_of_a_product_are_written_two_states_ahead(kernels):
                     assert not registers(operands(instruction)[0] if operands(instruction) else "") & read, (name, instruction, code[at])
 
 
+def test_the_loop_is_not_left_with_a_product_under_way(kernels):
+    """From the last product of a loop to its end: what the compiler puts behind the loop may read any sum."""
+    loops = 0
+    for name, code in kernels.items():
+        marks = list(products(code))
+        for (at, passes), following in zip(marks, [m[0] for m in marks[1:]] + [len(code)]):
+            waited = 0
+            for instruction in code[at + 1:following]:
+                if instruction.startswith("s_cbranch"):
+                    loops += 1
+                    assert waited >= latency(passes), (name, code[at], waited)
+                    break
+                waited += states(instruction)
+    assert loops >= len(kernels)
+
+
 def test_every_load_to_lds_has_its_m0_written_in_front_of_it(kernels):
     """Where loads are part of assembly, which writes M0 unseen, no M0 is held from one load to another."""
     seen = 0
