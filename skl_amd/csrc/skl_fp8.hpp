@@ -62,7 +62,7 @@ __device__ __forceinline__ unsigned encode_ofp8(unsigned bits, bool sat) {
 struct Ofp8Format {
   bool e5m2;
   unsigned max, overflow_sign, overflow_code;
-  __host__ __device__ explicit Ofp8Format(int fmt) {
+  __host__ __device__ __forceinline__ explicit Ofp8Format(int fmt) {
     const bool sat = fmt == 2 || fmt == 4;
     e5m2 = fmt >= 3;
     max = e5m2 ? 0x7Bu : 0x7Eu;

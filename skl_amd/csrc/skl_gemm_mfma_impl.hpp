@@ -821,7 +821,7 @@ __device__ __forceinline__ void write_wave_rows(const MfmaArgs &p, const Acc (&a
   constexpr int S = sizeof(Acc) == 64 ? 32 : 16, G = S == 32 ? 4 : 1, COLS = NI * S, P = wave_rows_pitch<COLS>();
   // A pass: 256 elements, as many whole rows as that is; by columns: S rows by 256 / S columns. A chunk: up to eight passes (four, with
   // steps); the old values of one are under way (of two, int8 4096 x 8192 x 2048 took 3 us more, of four 13).
-  constexpr int kPasses = S * COLS / 256, kMost = STEPS ? 4 : 8, kChunk = kPasses < kMost ? kPasses : kMost, kDown = 256 / COLS, kColsDown = 256 / S;
+  constexpr int kPasses = S * COLS / 256, kMost = STEPS || (S == 32 && COLS == 64) ? 4 : 8, kChunk = kPasses < kMost ? kPasses : kMost, kDown = 256 / COLS, kColsDown = 256 / S;
   constexpr int kChunks = MI * kPasses / kChunk;
   static_assert(kPasses % kChunk == 0);
   const int lane = (int)__builtin_amdgcn_mbcnt_hi(~0u, __builtin_amdgcn_mbcnt_lo(~0u, 0u));  // (not from threadIdx, see write_wave_tile)

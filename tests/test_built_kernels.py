@@ -39,6 +39,20 @@ def kernels(code_objects):
     return out
 
 
+def test_no_streaming_kernel_touches_scratch_memory(code_objects):
+    """A scratch access behind the stores of C waits for all of them."""
+    seen, bad = 0, []
+    for obj in code_objects:
+        notes = subprocess.run([os.path.join(LLVM, "llvm-readelf"), "--notes", obj], check=True, capture_output=True, text=True).stdout
+        for kernel in re.split(r"\n  - \.agpr_count", notes)[1:]:
+            value = lambda key: re.search(rf"\.{key}:\s+(\S+)", kernel).group(1)
+            if STREAMING in value("name"):
+                seen += 1
+                if int(value("private_segment_fixed_size")) or int(value("vgpr_spill_count")):
+                    bad.append(value("name"))
+    assert seen > 100 and not bad, bad
+
+
 def registers(operand):
     """The vector and accumulation registers of an operand, as (file, number)."""
     one = re.fullmatch(r"([va])(\d+)", operand)
