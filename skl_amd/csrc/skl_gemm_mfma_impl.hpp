@@ -832,12 +832,15 @@ __device__ __forceinline__ void write_wave_rows(const MfmaArgs &p, const Acc (&a
   const auto col_at = [&](size_t col) { return (col >> p.ccs) * p.csc1 + (col & cmask) * p.csc0; };
   const T *const bias = reinterpret_cast<const T *>(p.bias);
   const skl_fp8::Ofp8Format f8(p.rq.q_fmt);
-  // Stores go faster through the caches (us, through / past them: bf16 4096^3 97.5 / 100.2, 4096 x 8192 x 512 50 / 60, 8192^2 x 1024
-  // 141 / 153; E4M3 8192^2 x 2048 143 / 149), until with several rounds of tiles C and the operands of the next round are more than the
-  // 256 MiB behind them (bf16 4096 x 8192^2 373 / 369, 8192^3 743 / 721, 8192 x 16384 x 2048 452 / 435; E4M3 8192 x 16384 x 1024
-  // 217 / 192): the line is where both took the same, 8192^2 with 4 KiB of K (bf16 229.5 / 231, E4M3 232.2 / 232.7). With several rounds
-  // of a C that is read the stores are in its way (int8 4096 x 8192 x 2048 128 / 114, one round 4096^2 x 1024 35.1 / 36.2).
-  const bool one_round = p.tiles_m * p.tiles_n <= 256, fits = (p.m + p.n) * p.k * ES + p.m * p.n * 4 < (size_t(320) << 20);
+  // Which way the stores go. Through the caches they are the faster ones (us, through / past: 4096 x 8192 x 512 bf16 48.4 / 59.1, int8 of
+  // 8192^2 x 2048 134 / 147, E4M3 212 / 227, one round of 64 MiB, 2048 x 8192 x 512, 27.0 / 30.6), as long as the 256 MiB behind them
+  // hold all that is written (8192 x 8448 x 2048 bf16 253 / 235, int8 149 / 142; 8192 x 12288 x 512 148 / 130) with what the next round reads
+  // (the same at 8192^2 and 4 KiB of K). Little is better past them: it would still lie in the L2s, which are written back when the kernel
+  // ends (4352 x 1024 x 512 int8 9.6 / 8.5, bf16 12.8 / 11.3; 2048 x 4096 x 512 16.5 / 15.1). A C that is read meets its stores there
+  // when there are several rounds (8192^2 x 512 bf16 178 / 154), not in one (2048 x 8192 x 512 39 / 42).
+  const bool one_round = p.tiles_m * p.tiles_n <= 256;
+  const size_t written = p.m * p.n * ((p.rq.q_only ? 0 : 4) + (p.rq.q ? 1 : 0));
+  const bool fits = written > (size_t(48) << 20) && written <= (size_t(256) << 20) && (p.m + p.n) * p.k * ES + written < (size_t(320) << 20);
 
   // Row of blocks i's sums to LDS (accumulators cannot be indexed: a branch for each).
   const auto put = [&](unsigned i) __attribute__((always_inline)) {
@@ -1009,14 +1012,18 @@ __device__ __forceinline__ void write_wave_rows(const MfmaArgs &p, const Acc (&a
       }
       T *const at = c_lane_at + row_at(top) + col_at(left);
       if (!STEPS || !p.rq.q_only) {
+        // (the two ways with an empty instruction of each one's own around them: the compiler takes the stores for the same and makes
+        // one of them otherwise)
         const auto store = [&](auto kept_c) __attribute__((always_inline)) {
+          constexpr bool KEPT = decltype(kept_c)::value;
+          if constexpr (RUN) asm volatile("; %0" ::"n"(KEPT));
 #pragma unroll
           for (int t = 0; t < kChunk; ++t) {
             const size_t row = row_of(top, t), k = col_of(left, t);
             T *const to = at + step[t];
             if constexpr (RUN) {
               if (!CHECK || (row < p.m && cols_in(k) == 4)) {
-                if constexpr (decltype(kept_c)::value) *reinterpret_cast<Run4 *>(to) = v[t];
+                if constexpr (KEPT) *reinterpret_cast<Run4 *>(to) = v[t];
                 else __builtin_nontemporal_store((Run4)v[t], reinterpret_cast<Run4 *>(to));
               } else if (row < p.m) {
 #pragma unroll
@@ -1033,8 +1040,9 @@ __device__ __forceinline__ void write_wave_rows(const MfmaArgs &p, const Acc (&a
               }
             }
           }
+          if constexpr (RUN) asm volatile("; %0" ::"n"(KEPT));
         };
-        if (!RUN || one_round || (!UPDATE && fits)) store(std::true_type{});
+        if (!RUN || (UPDATE ? one_round : fits)) store(std::true_type{});
         else store(std::false_type{});
       }
       if constexpr (STEPS) {

@@ -137,3 +137,11 @@ def test_every_load_to_lds_has_its_m0_written_in_front_of_it(kernels):
             writes = [x for x in code[max(at - 2, 0):at] if re.match(r"s_\S+ m0,", x)]
             assert len(writes) == 1 and re.match(r"s_\S+ m0,", code[at - 2]), (name, code[at - 3:at + 1])
     assert seen
+
+
+def test_both_ways_of_the_stores_are_there(kernels):
+    """Stores of C through the caches and past them differ in one bit, and the compiler makes one of two branches that differ in it alone."""
+    for name, code in kernels.items():
+        past = sum(x.startswith("global_store_dwordx4") and x.endswith(" nt") for x in code)
+        through = sum(x.startswith("global_store_dwordx4") and not x.endswith(" nt") for x in code)
+        assert past and through, (name, past, through)
