@@ -93,7 +93,7 @@ __device__ __forceinline__ Acc fetched(Acc acc) {
 // A row-major copy on 4-byte boundaries with no activation beyond ReLU, in the format that goes with C's type (int8 behind an int32
 // C, OCP fp8 behind a floating-point one): steps of a few instructions per element.
 template <typename T>
-bool dword_copy(const skl_requant &r) {
+__host__ __device__ inline bool dword_copy(const skl_requant &r) {
   return r.q && r.act <= 1 && (r.q_fmt != 0) == !std::is_same<T, int>::value && r.csq == 1 && (r.rsq & 3) == 0 && ((uintptr_t)r.q & 3) == 0;
 }
 
@@ -797,6 +797,13 @@ __device__ __forceinline__ void write_wave_tile_staged(const MfmaArgs &p, const 
 }
 
 // ---------------------------------------------------------------------------
+// 16 bytes per lane of sums to LDS from the accumulation (IN_A) or vector registers that hold them: the compiler copies them first.
+template <bool IN_A, int AT, typename V4>
+__device__ __forceinline__ void lds_write_b128(unsigned to, V4 four) {
+  if constexpr (IN_A) asm volatile("ds_write_b128 %0, %1 offset:%2" ::"v"(to), "a"(four), "n"(AT) : "memory");
+  else asm volatile("ds_write_b128 %0, %1 offset:%2" ::"v"(to), "v"(four), "n"(AT) : "memory");
+}
+
 // The streaming kernel's epilogue: one wave writes its MI x NI blocks, of which a lane holds four consecutive columns of a row at a
 // time (acc[i][j][4 g + e]: row S i + lane % S, column S j + 8 g + 4 (lane / S) + e). The operands' ring being over, the rows of one row
 // of blocks at a time go to LDS as they are, and a loop takes them from there in the order that C wants: a wave's rows of 128 (64)
@@ -844,17 +851,24 @@ __device__ __forceinline__ void write_wave_rows(const MfmaArgs &p, const Acc (&a
 
   // Row of blocks i's sums to LDS (accumulators cannot be indexed: a branch for each).
   const auto put = [&](unsigned i) __attribute__((always_inline)) {
-    T *const to = stage + lane % S * P + lane / S * 4;
+    [[maybe_unused]] const unsigned to = (unsigned)(size_t)LDS_PTR(char, stage_bytes) + (lane % S * P + lane / S * 4) * (unsigned)sizeof(T);
     [&]<int... Is>(std::integer_sequence<int, Is...>) __attribute__((always_inline)) {
       (
           [&](auto ic) __attribute__((always_inline)) {
             constexpr int I = decltype(ic)::value;
             if (i == I) {
+              if constexpr (G == 1) {
+                [&]<int... Js>(std::integer_sequence<int, Js...>) __attribute__((always_inline)) {
+                  (lds_write_b128<ring_sum_in_a<MI, NI, Acc>(I, Js), Js * S * (int)sizeof(T)>(to, acc[I][Js]), ...);
+                }(std::make_integer_sequence<int, NI>{});
+              } else {
 #pragma unroll
-              for (int j = 0; j < NI; ++j) {
-                const Acc sums = j < NI / 2 ? fetched<ring_sum_in_a<MI, NI, Acc>(I, 0)>(acc[I][j]) : fetched<ring_sum_in_a<MI, NI, Acc>(I, NI - 1)>(acc[I][j]);
+                for (int j = 0; j < NI; ++j) {
+                  const Acc sums = j < NI / 2 ? fetched<ring_sum_in_a<MI, NI, Acc>(I, 0)>(acc[I][j]) : fetched<ring_sum_in_a<MI, NI, Acc>(I, NI - 1)>(acc[I][j]);
 #pragma unroll
-                for (int g = 0; g < G; ++g) *reinterpret_cast<V4 *>(to + j * S + g * 8) = V4{sums[4 * g], sums[4 * g + 1], sums[4 * g + 2], sums[4 * g + 3]};
+                  for (int g = 0; g < G; ++g)
+                    *reinterpret_cast<V4 *>(stage + lane % S * P + lane / S * 4 + j * S + g * 8) = V4{sums[4 * g], sums[4 * g + 1], sums[4 * g + 2], sums[4 * g + 3]};
+                }
               }
             }
           }(std::integral_constant<int, Is>{}),
@@ -865,8 +879,8 @@ __device__ __forceinline__ void write_wave_rows(const MfmaArgs &p, const Acc (&a
   // RUN: four columns lie side by side in C. Otherwise, `down`, a lane's four elements are four rows of a column: side by side in a C by
   // columns, and in any other C as good as four columns. UPDATE: C is read (not only where a zero's sign asks for it). FUSED: there are
   // steps behind the alpha/beta step.
-  const auto write = [&](auto run, auto update, auto fused) __attribute__((always_inline)) {
-    constexpr bool RUN = decltype(run)::value, UPDATE = decltype(update)::value, FUSED = decltype(fused)::value;
+  const auto write = [&](auto run, auto update, auto fused, auto ones) __attribute__((always_inline)) {
+    constexpr bool RUN = decltype(run)::value, UPDATE = decltype(update)::value, FUSED = decltype(fused)::value, ONES = decltype(ones)::value;
     // the lane's first row and column in a pass, from those of the pass
     const int r_lane = RUN ? lane / (COLS / 4) : lane % (S / 4) * 4, c_lane = RUN ? lane % (COLS / 4) * 4 : lane / (S / 4);
     // Where in C the lane's elements of pass y of a row of blocks are: that of the row of blocks, a scalar, and this (passes begin at
@@ -891,6 +905,7 @@ __device__ __forceinline__ void write_wave_rows(const MfmaArgs &p, const Acc (&a
       }
       __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0): in the loop they would be waited for with every chunk, and its stores with them
     }
+    int8_t *const q_lane_at = p.rq.q + (row0 + r_lane) * p.rq.rsq + (col0 + c_lane) * p.rq.csq;  // as c_lane_at: the rest are scalars
     const bool q_run = STEPS && RUN && p.rq.csq == 1 && (p.rq.rsq & 3) == 0 && ((uintptr_t)p.rq.q & 3) == 0;
     T running = skl_lowest<T>();
 
@@ -952,11 +967,14 @@ __device__ __forceinline__ void write_wave_rows(const MfmaArgs &p, const Acc (&a
         for (int t = 0; t < kChunk; ++t) {
           const V4 old = moved(col_of(left, t), next[t]);
 #pragma unroll
-          for (int e = 0; e < 4; ++e) v[t][e] = skl_combine(v[t][e], old[e], p.alpha, p.beta);
+          for (int e = 0; e < 4; ++e) {
+            if constexpr (ONES) v[t][e] = skl_add_bias(v[t][e], old[e]);
+            else v[t][e] = skl_combine(v[t][e], old[e], p.alpha, p.beta);
+          }
         }
         __builtin_amdgcn_sched_barrier(0);  // the values to come take these registers
         request(x + 1 < (unsigned)kChunks ? x + 1 : x, next);  // (beyond the end: some, not used)
-      } else {
+      } else if constexpr (!ONES) {
         bool need = false;
 #pragma unroll
         for (int t = 0; t < kChunk; ++t)
@@ -1096,7 +1114,7 @@ __device__ __forceinline__ void write_wave_rows(const MfmaArgs &p, const Acc (&a
 #pragma unroll
           for (int t = 0; t < kChunk; ++t) {
             const size_t row = row_of(top, t), k = col_of(left, t);
-            int8_t *const q = reinterpret_cast<int8_t *>(p.rq.q) + row * p.rq.rsq + k * p.rq.csq;
+            int8_t *const q = q_lane_at + (RUN ? (top - row0 + t * kDown) * p.rq.rsq : (top - row0) * p.rq.rsq + (left + t * kColsDown) * p.rq.csq);
             if (q_run && (!CHECK || (row < p.m && cols_in(k) == 4))) {
               *reinterpret_cast<unsigned *>(q) = packed[t];
             } else {
@@ -1121,20 +1139,114 @@ __device__ __forceinline__ void write_wave_rows(const MfmaArgs &p, const Acc (&a
       if (lane == 0 && best > skl_lowest<T>()) skl_atomic_max(reinterpret_cast<T *>(p.max), best);
     }
   };
+  // int8 copies in dwords of whole numbers with no activation but ReLU, of a C that is not read: the loop with nothing but their steps.
+  // (The general loop decides at every turn what there is to be done, and its branches cost such a copy more than its arithmetic: us, the
+  // general loop / this, each with eight waves: 7424 x 7040 x 512 with ReLU 76 / 71, 4352 x 1024 x 128 9.4 / 8.6.)
+  const auto write_int8 = [&]() __attribute__((always_inline)) {
+    const int r_lane = lane / (COLS / 4), c_lane = lane % (COLS / 4) * 4;
+    const auto column_at = [&](size_t k) { return !CHECK || k < p.n ? k : 0; };
+    T *const c_at = c + row_at(r_lane) + row_at(row0) + col_at(col0) + col_at(c_lane);
+    int8_t *const q_at = reinterpret_cast<int8_t *>(p.rq.q) + (row0 + r_lane) * p.rq.rsq + col0 + c_lane;
+    T bias_of[4];
+    float scale_of[4];
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      const size_t k = column_at(col0 + c_lane + e);
+      bias_of[e] = bias ? bias[k] : T(0);
+      scale_of[e] = p.rq.q_scale[p.rq.q_per_column ? k : 0];
+    }
+    __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0), as above
+    const T floor = p.rq.act == 1 ? T(0) : skl_lowest<T>();
+    const bool there = !CHECK || col0 + c_lane + 4 <= p.n;
+    constexpr unsigned kOfRow = kPasses / kChunk;
+    put(0);
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+#pragma clang loop unroll(disable)
+    for (unsigned x = 0; x < (unsigned)kChunks; ++x) {
+      const size_t top = x * (kChunk * kDown);
+      const T *const stage_x = stage + (x % kOfRow * (kChunk * kDown) + r_lane) * P + c_lane;
+      V4 v[kChunk];
+#pragma unroll
+      for (int t = 0; t < kChunk; ++t) v[t] = *reinterpret_cast<const V4 *>(stage_x + t * kDown * P);
+      __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+      __builtin_amdgcn_wave_barrier();
+      if (x % kOfRow == kOfRow - 1) put(x / kOfRow + 1);
+      __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+      __builtin_amdgcn_wave_barrier();
+      if (p.alpha.i != 1) {
+#pragma unroll
+        for (int t = 0; t < kChunk; ++t)
+#pragma unroll
+          for (int e = 0; e < 4; ++e) v[t][e] = skl_initialise_plain(v[t][e], p.alpha, p.beta);
+      }
+#pragma unroll
+      for (int t = 0; t < kChunk; ++t)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          const T w = skl_add_bias(v[t][e], bias_of[e]);
+          v[t][e] = w < floor ? floor : w;
+        }
+      const auto store = [&](auto kept_c) __attribute__((always_inline)) {
+        constexpr bool KEPT = decltype(kept_c)::value;
+        asm volatile("; %0" ::"n"(KEPT));
+#pragma unroll
+        for (int t = 0; t < kChunk; ++t) {
+          Run4 *const to = reinterpret_cast<Run4 *>(c_at + row_at(top) + row_at(t * kDown));
+          if (there && (!CHECK || row0 + top + t * kDown + r_lane < p.m)) {
+            if constexpr (KEPT) *to = v[t];
+            else __builtin_nontemporal_store((Run4)v[t], to);
+          }
+        }
+        asm volatile("; %0" ::"n"(KEPT));
+      };
+      if (!p.rq.q_only) {
+        if (fits) store(std::true_type{});
+        else store(std::false_type{});
+      }
+#pragma unroll
+      for (int t = 0; t < kChunk; ++t) {
+        unsigned packed = 0;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) packed |= ((unsigned)skl_requantise_int((float)v[t][e], scale_of[e], p.rq.q_zero) & 0xFFu) << (8 * e);
+        if (there && (!CHECK || row0 + top + t * kDown + r_lane < p.m)) *reinterpret_cast<unsigned *>(q_at + (top + t * kDown) * p.rq.rsq) = packed;
+      }
+    }
+  };
   // any row-major C, blocks of four columns and more (a lane at the edge reads its old values from the last four columns)
   const bool run = p.csc0 == 1 && p.ccs >= 2 && (!CHECK || (p.n >= 4 && (p.n % 4 == 0 || p.csc1 == (size_t(1) << p.ccs))));
   const bool update = !skl_beta_is_zero<T>(p.beta);
-  if (run && (STEPS || p.bias || p.max)) {
-    if (update) write(std::true_type{}, std::true_type{}, std::true_type{});
-    else write(std::true_type{}, std::false_type{}, std::true_type{});
-  } else if (run) {
-    if constexpr (!STEPS) {
-      if (update) write(std::true_type{}, std::true_type{}, std::false_type{});
-      else write(std::true_type{}, std::false_type{}, std::false_type{});
+  constexpr std::true_type yes;
+  constexpr std::false_type no;
+  if (!run) {
+    if (update) write(no, yes, yes, no);
+    else write(no, no, yes, no);
+    return;
+  }
+  const auto write_run = [&](auto fused, auto ones) __attribute__((always_inline)) {
+    if (update) write(yes, yes, fused, ones);
+    else write(yes, no, fused, ones);
+  };
+  const auto write_scaled = [&](auto fused) __attribute__((always_inline)) {
+    if constexpr (std::is_same<T, int>::value && !(CHECK && STEPS)) {  // multiplications of whole numbers take four times as long as anything else here
+      if (p.alpha.i == 1 && (p.beta.i == 0 || p.beta.i == 1)) {
+        write_run(fused, yes);
+        return;
+      }
     }
+    write_run(fused, no);
+  };
+  if constexpr (STEPS) {
+    if constexpr (std::is_same<T, int>::value) {
+      if (!update && !p.max && dword_copy<T>(p.rq) && (!CHECK || p.n % 4 == 0)) {
+        write_int8();
+        return;
+      }
+    }
+    write_scaled(yes);
   } else {
-    if (update) write(std::false_type{}, std::true_type{}, std::true_type{});
-    else write(std::false_type{}, std::false_type{}, std::true_type{});
+    if (p.bias || p.max) write_scaled(yes);
+    else write_scaled(no);
   }
 }
 

@@ -54,3 +54,27 @@ def test_streamed_tiles_from_short_to_longer_k(gpu, m, n, ks, a_kc, b_kc):
         assert np.array_equal(out[0], want[0]), (k, vars(case))
         assert start is None or out[1][0] == want[1][0], k
         assert rq is None or np.array_equal(out[2], want[2]), k
+
+
+@pytest.mark.parametrize("m,n,k", ((4096, 3328, 256), (4352, 1024, 384), (2300, 2500, 4112), (4001, 3300, 2064), (2304, 3584, 128)))
+def test_int8_copies_in_dwords(gpu, m, n, k):
+    """The loop of its own that such copies have where C is not read: whole tiles of both widths and ragged ones (rows and columns that
+    end inside a tile, in a chunk and in a lane's dword's neighbour), with C and without, scalars of one and others, ReLU and none, one
+    scale and one per column, with a bias and without, rows of the copy farther apart than they are long."""
+    rng = np.random.default_rng(m + n)
+    for i in range(4):
+        alpha, act, only, per_column, pad = (1, 0x01010101, 1, -3)[i], i & 1, i >= 2, i in (1, 2), (0, 4, 8, 12)[i]
+        case = GemmCase("i8", None, alpha, 0, m0=1, n0=1, k0=1, m1=m, n1=n, k1=k, rsa0=0, csa0=0, rsa1=k, csa1=1, rsb0=0, csb0=0, rsb1=1, csb1=k,
+                        rsc0=0, csc0=0, rsc1=n + pad // 4, csc1=1)
+        a, b, c = case.make_inputs(k + n + i)
+        sums = (matrix(a, m, k, k).astype(np.float64) @ matrix(b, n, k, k).T.astype(np.float64)).astype(np.int64)
+        rows = support.blocked_offsets(case.m1, case.n1, case.m0, case.n0, case.rsc0, case.csc0, case.rsc1, case.csc1)
+        plain = c.copy()
+        plain[rows] = (alpha * sums.reshape(rows.shape)).astype(np.int32)
+        bias = rng.integers(-1 << 12, 1 << 12, n).astype(np.int32) if i != 3 else None
+        spread = 2.0 ** 31 if abs(alpha) > 3 else 40.0 * 5461.0 * np.sqrt(k)
+        rq = dict(q=np.full((m - 1) * (n + pad) + n, 0x55, np.int8), rsq=n + pad, csq=1, per_column=per_column,
+                  scale=(rng.uniform(0.25, 2.0, n if per_column else 1) * 4000.0 / spread).astype(np.float32), zero=(0, -128, 127, 5)[i], only=only, format=0)
+        out = run_fused_gemm(gpu, "rc", case, a, b, c, bias, None, "device", activation=act, requant=rq)
+        want = fused_expectation(case, plain, bias, None, activation=act, requant=rq)
+        assert np.array_equal(out[0], c if only else want[0]) and np.array_equal(out[2], want[2]), (i, vars(case))
