@@ -820,15 +820,16 @@ __device__ __forceinline__ void lds_write_b128(unsigned to, V4 four) {
 // ---------------------------------------------------------------------------
 template <int COLS>
 constexpr int wave_rows_pitch() { return COLS + 4; }
-template <int MI, int NI, int ES, bool CHECK, bool STEPS, typename Acc>
+template <int MI, int NI, int ES, int MOST, bool CHECK, bool STEPS, typename Acc>
 __device__ __forceinline__ void write_wave_rows(const MfmaArgs &p, const Acc (&acc)[MI][NI], size_t row0, size_t col0, char *stage_bytes) {
   using T = decltype(Acc{}.x);
   typedef T V4 __attribute__((ext_vector_type(4)));
   typedef T Run4 __attribute__((ext_vector_type(4), aligned(4)));
   constexpr int S = sizeof(Acc) == 64 ? 32 : 16, G = S == 32 ? 4 : 1, COLS = NI * S, P = wave_rows_pitch<COLS>();
-  // A pass: 256 elements, as many whole rows as that is; by columns: S rows by 256 / S columns. A chunk: up to eight passes (four, with
-  // steps); the old values of one are under way (of two, int8 4096 x 8192 x 2048 took 3 us more, of four 13).
-  constexpr int kPasses = S * COLS / 256, kMost = STEPS || (S == 32 && COLS == 64) ? 4 : 8, kChunk = kPasses < kMost ? kPasses : kMost, kDown = 256 / COLS, kColsDown = 256 / S;
+  // A pass: 256 elements, as many whole rows as that is; by columns: S rows by 256 / S columns. A chunk: up to MOST passes. Under way are the
+  // old values of one chunk of eight passes, or of two of four where eight waves write (4096 x 8192 x 512, us, one / two: bf16 81 / 74,
+  // int8 73 / 62; four waves with two or four of eight: int8 4096 x 8192 x 2048 3 and 13 us more than with one).
+  constexpr int kPasses = S * COLS / 256, kMost = MOST, kChunk = kPasses < kMost ? kPasses : kMost, kDown = 256 / COLS, kColsDown = 256 / S;
   constexpr int kChunks = MI * kPasses / kChunk;
   static_assert(kPasses % kChunk == 0);
   const int lane = (int)__builtin_amdgcn_mbcnt_hi(~0u, __builtin_amdgcn_mbcnt_lo(~0u, 0u));  // (not from threadIdx, see write_wave_tile)
@@ -879,7 +880,7 @@ __device__ __forceinline__ void write_wave_rows(const MfmaArgs &p, const Acc (&a
   // RUN: four columns lie side by side in C. Otherwise, `down`, a lane's four elements are four rows of a column: side by side in a C by
   // columns, and in any other C as good as four columns. UPDATE: C is read (not only where a zero's sign asks for it). FUSED: there are
   // steps behind the alpha/beta step.
-  const auto write = [&](auto run, auto update, auto fused, auto ones) __attribute__((always_inline)) {
+  const auto write = [&](auto run, auto update, auto fused, auto ones, auto through) __attribute__((always_inline)) {
     constexpr bool RUN = decltype(run)::value, UPDATE = decltype(update)::value, FUSED = decltype(fused)::value, ONES = decltype(ones)::value;
     // the lane's first row and column in a pass, from those of the pass
     const int r_lane = RUN ? lane / (COLS / 4) : lane % (S / 4) * 4, c_lane = RUN ? lane % (COLS / 4) * 4 : lane / (S / 4);
@@ -911,6 +912,8 @@ __device__ __forceinline__ void write_wave_rows(const MfmaArgs &p, const Acc (&a
 
     // Chunk x: its first row and column, and, from those on, the lane's first row and column of its pass t.
     constexpr unsigned kOfRow = kPasses / kChunk;  // chunks of a row of blocks
+    constexpr int kAhead = UPDATE && !STEPS && !CHECK && MOST == 4 ? 2 : 1;  // chunks whose old values are under way
+    static_assert(kChunks % kAhead == 0);
     const auto top_of = [&](unsigned x) { return row0 + (RUN ? x * (kChunk * kDown) : x / kOfRow * S); };
     const auto left_of = [&](unsigned x) { return RUN ? size_t(0) : (size_t)(x % kOfRow * (kChunk * kColsDown)); };
     const auto row_of = [&](size_t top, int t) { return top + (RUN ? t * kDown : 0) + r_lane; };
@@ -940,7 +943,7 @@ __device__ __forceinline__ void write_wave_rows(const MfmaArgs &p, const Acc (&a
       return o;
     };
 
-    // `next`: the old values of chunk x, then those of the next.
+    // `next`: the old values of chunk x, then those of the next but kAhead - 1.
     const auto chunk = [&](unsigned x, V4 (&next)[kChunk]) __attribute__((always_inline)) {
       const size_t top = top_of(x), left = left_of(x);
       const unsigned in_row = x % kOfRow;
@@ -973,7 +976,7 @@ __device__ __forceinline__ void write_wave_rows(const MfmaArgs &p, const Acc (&a
           }
         }
         __builtin_amdgcn_sched_barrier(0);  // the values to come take these registers
-        request(x + 1 < (unsigned)kChunks ? x + 1 : x, next);  // (beyond the end: some, not used)
+        request(x + kAhead < (unsigned)kChunks ? x + kAhead : x, next);  // (beyond the end: some, not used)
       } else if constexpr (!ONES) {
         bool need = false;
 #pragma unroll
@@ -1060,7 +1063,9 @@ __device__ __forceinline__ void write_wave_rows(const MfmaArgs &p, const Acc (&a
           }
           if constexpr (RUN) asm volatile("; %0" ::"n"(KEPT));
         };
-        if (!RUN || (UPDATE ? one_round : fits)) store(std::true_type{});
+        if constexpr (!RUN) store(std::true_type{});
+        else if constexpr (UPDATE) store(through);  // (no branch: what waits for old values would wait for the stores that might have been left out)
+        else if (fits) store(std::true_type{});
         else store(std::false_type{});
       }
       if constexpr (STEPS) {
@@ -1130,10 +1135,19 @@ __device__ __forceinline__ void write_wave_rows(const MfmaArgs &p, const Acc (&a
     put(0);
     __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
     __builtin_amdgcn_wave_barrier();
-    V4 next[kChunk];
-    if constexpr (UPDATE) request(0, next);
+    V4 next[kAhead][kChunk];
+    if constexpr (UPDATE) {
+#pragma unroll
+      for (int a = 0; a < kAhead; ++a) request(a, next[a]);
+    }
+    if constexpr (kAhead > 1) {  // written out: a loop waits for what its first turn would have to wait for, which has fewer stores in front
+      [&]<int... Xs>(std::integer_sequence<int, Xs...>) __attribute__((always_inline)) {
+        (chunk(Xs, next[Xs % kAhead]), ...);
+      }(std::make_integer_sequence<int, kChunks>{});
+    } else {
 #pragma clang loop unroll(disable)
-    for (unsigned x = 0; x < (unsigned)kChunks; ++x) chunk(x, next);
+      for (unsigned x = 0; x < (unsigned)kChunks; ++x) chunk(x, next[0]);
+    }
     if (FUSED && p.max) {
       const T best = skl_wave_max(running);
       if (lane == 0 && best > skl_lowest<T>()) skl_atomic_max(reinterpret_cast<T *>(p.max), best);
@@ -1219,13 +1233,14 @@ __device__ __forceinline__ void write_wave_rows(const MfmaArgs &p, const Acc (&a
   constexpr std::true_type yes;
   constexpr std::false_type no;
   if (!run) {
-    if (update) write(no, yes, yes, no);
-    else write(no, no, yes, no);
+    if (update) write(no, yes, yes, no, yes);
+    else write(no, no, yes, no, yes);
     return;
   }
   const auto write_run = [&](auto fused, auto ones) __attribute__((always_inline)) {
-    if (update) write(yes, yes, fused, ones);
-    else write(yes, no, fused, ones);
+    if (!update) write(yes, no, fused, ones, yes);
+    else if (one_round) write(yes, yes, fused, ones, yes);
+    else write(yes, yes, fused, ones, no);
   };
   const auto write_scaled = [&](auto fused) __attribute__((always_inline)) {
     if constexpr (std::is_same<T, int>::value && !(CHECK && STEPS)) {  // multiplications of whole numbers take four times as long as anything else here
@@ -1577,16 +1592,31 @@ __global__ void __launch_bounds__(WAVES_M *WAVES_N * 64, (BM == 64 ? 2 : 4)) gem
 // halves of such a load next to each other: one KiB, as the load writes it.
 // ===========================================================================
 constexpr int kRingSlice = 64;   // bytes of K per stage
-// Waves: four, each a quarter of the tile, so that as little as possible is read twice. 8-bit operands both read across K into a 256 x
-// 128 tile are the exception: reads of eight bytes per lane and an address for each leave four waves of 16 x 16 products short of issue
-// slots. There fp8 takes eight waves, two to a SIMD, and int8 products of 32 x 32, half as many (us, with four waves and 16 x 16 / so;
-// 1024 x 4096^2, half the compute units: E4M3 27.2 / 24.9, int8 29.6 / 26.9; 2048 x 4096^2, all of them: 33.7 / 34.4 and 35.1 / 36.7).
-// And the 16-bit kinds' ragged 256 x 128 tiles, whose starts, ends and chosen offsets two waves to a SIMD cover better (f16 2944 x 2048 x
-// 8125 read across K 121 / 109). Not whole ones: small problems gain what full rounds lose (bf16, four / eight waves: 1024 x 5632 x
-// 896 17.7 / 16.2, 3328 x 1280 x 1152 19.8 / 18.1, but 2048 x 4096^2 reading C 62.3 / 65.5; E4M3 4096 x 8192 x 1024 69 / 77).
+// Waves. Four, one per SIMD, each a quarter of the tile, so that as little as possible is read twice: the fastest main loop. Eight, two
+// per SIMD, where what is around the loop counts: one wave's start, old C, steps and stores lie under the other's. Eight over four waves,
+// geometric means over 600 random problems, by K in bytes from 512 / 1024 / 2048 / 4096 / 8192:
+//                            256 x 256 tiles                          256 x 128 tiles
+//   ragged, 16 bits, plain   0.79 0.90 0.91 0.89 0.89                 0.82 0.87 0.90 0.91 0.97
+//           int8, plain       -   0.93 0.93  -    -                   0.87 0.93 0.94  -   0.94    fp8, beyond the exact K  0.94 0.96 0.98
+//           with steps       0.77 to 0.87 (int8 0.81 to 0.87)         0.78 to 0.93 (int8 0.83 to 0.96, fp8 0.88 to 0.96)
+//   whole, with steps        16 bits 0.80 0.83 0.89 0.93 0.92         0.82 0.84 0.88 0.93 0.96
+//                            exact fp8 0.86 0.90 0.82, int8 0.89 to 0.96   0.81 0.87 0.85, int8 0.90 0.94 0.96 1.01 1.04, fp8 0.85 0.91 0.94
+//          exact fp8, plain  0.96 0.95                                0.89 0.92 0.94    fp8 beyond it, plain or C read, 0.96 to 0.99
+//          16 bits, C read   1.02 1.02 1.00 0.98 1.03                 0.92 0.93 0.98 0.98 0.99     plain  -   0.94 0.94 0.96 0.99
+//          int8, C read       -   1.02 1.00  -    -                    -   0.97 0.98 1.00 1.02     plain 0.93 0.99 1.02 0.99
+// fp8 beyond the exact K keeps four on 256 x 256 tiles: fragments of 32 x 32 products leave eight no registers. So do the calls whose old C
+// is looked through (SCAN): its slots would not fit beside the stages.
 constexpr bool ring_few_issue_slots(int es, bool a_kc, bool b_kc, int bn) { return es == 1 && !a_kc && !b_kc && bn == 128; }
-template <int TA, bool A_KC, bool B_KC, int BN, bool EDGE, bool EXACT>
-constexpr int kRingWaves = (BN == 128 && EDGE && Kind<TA>::ES == 2) || (TA != SKL_DT_I8 && !EXACT && ring_few_issue_slots(Kind<TA>::ES, A_KC, B_KC, BN)) ? 8 : 4;
+template <int TA, bool A_KC, bool B_KC, int BN, bool EDGE, bool STEPS, bool SCAN, bool EXACT>
+constexpr int ring_waves() {  // 0: ring_waves_by_size
+  constexpr bool fp8 = TA == SKL_DT_F8E4M3 || TA == SKL_DT_F8E5M2;
+  if (fp8 && !EXACT && BN == 256) return 4;
+  if (SCAN) return fp8 && ring_few_issue_slots(1, A_KC, B_KC, BN) ? 8 : 4;
+  return fp8 || EDGE || STEPS ? 8 : 0;
+}
+// Of them side by side: two; eight of 256 x 256 tiles four where that holds fewer widened fragments (EXACT; the other way 34 registers
+// are spilled) and where C is read (us, two / four: int8 8192^2 x 1024 162 / 149, 4096 x 8192 x 2048 103 / 102, bf16 the same).
+constexpr int ring_waves_n(int waves, int bn, bool edge, bool steps, bool exact) { return waves == 8 && bn == 256 && (exact || !(edge || steps)) ? 4 : 2; }
 // Stages of an operand's ring: four, or six of an operand with K contiguous where 160 KiB of LDS hold them (see the kernel's loads).
 constexpr int ring_stages_a(bool a_kc, bool b_kc, int bn, bool scan) { return !a_kc || (bn == 256 && (b_kc || scan)) ? 4 : 6; }
 constexpr int ring_stages_b(bool, bool b_kc, int bn, bool scan) { return !b_kc || (bn == 256 && scan) ? 4 : 6; }
@@ -1848,8 +1878,8 @@ constexpr int ceil_div(int a, int b) { return (a + b - 1) / b; }
 // MI + NI fragments for MI x NI products - on the 128 x 128 kernels, with 64 x 32 per wave, three for two, which is
 // more vector work than the matrix cores take for the products; here sixteen for 64 (256 columns) or twelve for 32 (128).
 // E4M3 2048 x 8192 x 2048: 77 us there, 62 with eight waves of 32 x 32 products here; with a bias, into E4M3, 73 so and now 59.
-template <int TA, int TB, bool A_KC, bool B_KC, int BN, bool EDGE = false, bool STEPS = false, bool SCAN = false, bool EXACT = false>
-__global__ void __launch_bounds__((kRingWaves<TA, A_KC, B_KC, BN, EDGE, EXACT> * 64)) gemm_mfma_ring_kernel(MfmaArgs p) {
+template <int TA, int TB, bool A_KC, bool B_KC, int BN, bool EDGE, bool STEPS, bool SCAN, bool EXACT, int WAVES>
+__global__ void __launch_bounds__((WAVES * 64)) gemm_mfma_ring_kernel(MfmaArgs p) {
   constexpr bool kLarge = TA == SKL_DT_I8 && ring_few_issue_slots(1, A_KC, B_KC, BN);
   using M = typename std::conditional<kLarge, RingMmaI8Large, RingMma<TA, TB, EXACT>>::type;
   using Frag = typename M::Frag;
@@ -1857,7 +1887,7 @@ __global__ void __launch_bounds__((kRingWaves<TA, A_KC, B_KC, BN, EDGE, EXACT> *
   using AccElem = decltype(Acc{}.x);
   constexpr int SB = kRingSlice, NSA = ring_stages_a(A_KC, B_KC, BN, SCAN), NSB = ring_stages_b(A_KC, B_KC, BN, SCAN);
   constexpr int ES = Kind<TA>::ES, S = M::kSide, FRB = M::kFrag;
-  constexpr int BM = 256, WAVES = kRingWaves<TA, A_KC, B_KC, BN, EDGE, EXACT>, WAVES_N = 2, WAVES_M = WAVES / WAVES_N;
+  constexpr int BM = 256, WAVES_N = ring_waves_n(WAVES, BN, EDGE, STEPS, EXACT), WAVES_M = WAVES / WAVES_N;
   constexpr int WM = BM / WAVES_M, WN = BN / WAVES_N, MI = WM / S, NI = WN / S;
   // A step is a slice: the products of the wave's blocks, once, or EXACT with each half of the fragments' bytes.
   constexpr int kProducts = MI * NI, kSlots = (EXACT || kLarge ? 2 : 1) * kProducts;
@@ -2195,6 +2225,7 @@ __global__ void __launch_bounds__((kRingWaves<TA, A_KC, B_KC, BN, EDGE, EXACT> *
     return;
   }
   constexpr int kStageBytes = S * wave_rows_pitch<WN>() * 4;
+  constexpr int kPassesAtOnce = WAVES == 8 && BN == 256 && STEPS && (EXACT || EDGE) ? 2 : WAVES == 8 || STEPS ? 4 : 8;  // (more are spilled registers)
   static_assert(WAVES * kStageBytes <= TileA::kRegion + TileB::kRegion, "the waves' rows take the place of the operand stages");
   if constexpr (SCAN) {
     // What the waves have found, put together: each wave's word where its first slot began (its own reads of
@@ -2207,10 +2238,10 @@ __global__ void __launch_bounds__((kRingWaves<TA, A_KC, B_KC, BN, EDGE, EXACT> *
     for (int w = 0; w < WAVES; ++w) any |= found[w * 256];
     MfmaArgs q = p;
     if (any == 0) q.beta.fz.skip_c_read = 1;  // 0 * c is a zero everywhere in this tile
-    write_wave_rows<MI, NI, ES, EDGE, STEPS>(q, acc, m0 + wm, n0 + wn, smem + wave * kStageBytes);
+    write_wave_rows<MI, NI, ES, kPassesAtOnce, EDGE, STEPS>(q, acc, m0 + wm, n0 + wn, smem + wave * kStageBytes);
   } else {
     __syncthreads();  // every wave's reads of the stages and loads into them are over
-    write_wave_rows<MI, NI, ES, EDGE, STEPS>(p, acc, m0 + wm, n0 + wn, smem + wave * kStageBytes);
+    write_wave_rows<MI, NI, ES, kPassesAtOnce, EDGE, STEPS>(p, acc, m0 + wm, n0 + wn, smem + wave * kStageBytes);
   }
 }
 
@@ -2340,14 +2371,30 @@ inline bool c_in_row_quads(const MfmaArgs &p) {
          (((uintptr_t)p.c | (p.rsc0 * 4) | (p.rsc1 * 4) | (p.csc1 * 4)) & 15) == 0;
 }
 
-template <int TA, int TB, bool A_KC, bool B_KC, int BN, bool EDGE = false, bool STEPS = false, bool SCAN = false, bool EXACT = false>
+// The waves of plain products on whole tiles, int8 or 16 bits (see ring_waves): 256 x 256 tiles take eight only for C that is read over
+// two rounds, or more with a short K (us, four / eight: 4096 x 8192 x 512 int8 73 / 62, bf16 84 / 74, x 2048 104 / 97, 148 / 144; 8192^2 x 1024 int8
+// 162 / 156, but x 2048 198 / 204; one round, 4096^2 x 512, 29 / 33); 256 x 128 tiles below the K from which the main loop is what counts - except
+// int8 read across K on both sides, whose 32 x 32 products are four waves' (2048 x 4096^2 36.2 / 37.9 us).
+template <typename AccElem, bool A_KC, bool B_KC, int BN>
+int ring_waves_by_size(const MfmaArgs &p) {
+  constexpr bool kInt = std::is_same<AccElem, int>::value;
+  const bool reads_c = kInt ? p.beta.i != 0 : !(p.beta.fz.skip_c_read && p.beta.f == 0.0f);
+  if (BN == 256) {
+    const size_t tiles = (p.m / 256) * (p.n / 256);
+    return reads_c && tiles > 256 && (tiles <= 512 || p.k * (kInt ? 1 : 2) < 2048) ? 8 : 4;
+  }
+  if (kInt) return !A_KC && !B_KC ? 4 : p.k < (reads_c ? 4096 : 2048) ? 8 : 4;
+  return p.k * 2 < 8192 ? 8 : 4;
+}
+
+template <int TA, int TB, bool A_KC, bool B_KC, int BN, bool EDGE = false, bool STEPS = false, bool SCAN = false, bool EXACT = false, int WAVES = 0>
 int launch_ring(const MfmaArgs &args) {
   if constexpr (!STEPS && !SCAN && kRingCarriesExtraSteps<TA, TB>) {
     if (args.rq.act || args.rq.q) return launch_ring<TA, TB, A_KC, B_KC, BN, EDGE, true, false, EXACT>(args);
   }
   constexpr int ES = Kind<TA>::ES;
   using AccElem = decltype(typename Kind<TA>::Acc{}.x);
-  if constexpr (std::is_same<AccElem, float>::value && !EDGE && !STEPS && !SCAN && !EXACT) {
+  if constexpr (std::is_same<AccElem, float>::value && !EDGE && !STEPS && !SCAN && !EXACT && WAVES == 0) {
     // beta == 0 evaluated as the reference's loops do (0 * c: a NaN or an infinity in C stays a NaN): the old C is
     // looked through while the tile is multiplied, a KiB of it per wave and slice - needs 64 slices on the wide tile, 32
     // on the narrow one, a tile to itself (no shared K) and a row-major C.
@@ -2363,10 +2410,15 @@ int launch_ring(const MfmaArgs &args) {
     if (args.beta.f == 0.0f && args.beta.fz.skip_c_read == 0 && !shared_k && (row_major || panels) && scan_slices >= (BN == 256 ? 64 : 32))
       return launch_ring<TA, TB, A_KC, B_KC, BN, EDGE, false, true>(args);
   }
-  constexpr int kWaves = kRingWaves<TA, A_KC, B_KC, BN, EDGE, EXACT>;
-  constexpr int lds = (ring_stages_a(A_KC, B_KC, BN, SCAN) * 256 + ring_stages_b(A_KC, B_KC, BN, SCAN) * BN) * kRingSlice + (SCAN ? 4 * kWaves * 1024 : 0);
+  if constexpr (WAVES == 0) {
+    constexpr int waves = ring_waves<TA, A_KC, B_KC, BN, EDGE, STEPS, SCAN, EXACT>();
+    if constexpr (waves != 0) return launch_ring<TA, TB, A_KC, B_KC, BN, EDGE, STEPS, SCAN, EXACT, waves>(args);
+    else if (ring_waves_by_size<AccElem, A_KC, B_KC, BN>(args) == 8) return launch_ring<TA, TB, A_KC, B_KC, BN, EDGE, STEPS, SCAN, EXACT, 8>(args);
+    else return launch_ring<TA, TB, A_KC, B_KC, BN, EDGE, STEPS, SCAN, EXACT, 4>(args);
+  } else {
+  constexpr int lds = (ring_stages_a(A_KC, B_KC, BN, SCAN) * 256 + ring_stages_b(A_KC, B_KC, BN, SCAN) * BN) * kRingSlice + (SCAN ? 4 * WAVES * 1024 : 0);
   static_assert(lds <= 160 * 1024);
-  auto kernel = gemm_mfma_ring_kernel<TA, TB, A_KC, B_KC, BN, EDGE, STEPS, SCAN, EXACT>;
+  auto kernel = gemm_mfma_ring_kernel<TA, TB, A_KC, B_KC, BN, EDGE, STEPS, SCAN, EXACT, WAVES>;
   static std::atomic<bool> configured{false};  // per instantiation; racing threads set the same value
   if (!configured.load(std::memory_order_acquire)) {
     int rc = skl_check_hip(hipFuncSetAttribute(reinterpret_cast<const void *>(kernel),
@@ -2398,10 +2450,11 @@ int launch_ring(const MfmaArgs &args) {
     skl_hip_record_error(-2, "gemm_mfma: grid too large");
     return -2;
   }
-  kernel<<<(unsigned)grid, kWaves * 64, lds, skl_current_stream()>>>(p);
+  kernel<<<(unsigned)grid, WAVES * 64, lds, skl_current_stream()>>>(p);
   int rc = skl_check_launch("gemm_mfma_ring");
   if (rc != 0 || p.splits == 1) return rc;
   return launch_split_reduce<AccElem>(p, "gemm_split_reduce");
+  }
 }
 
 constexpr size_t kMinBytesPerSplit = 512, kSplitFromBytes = 4096, kSplitEarlyTiles = 96, kSplitPlaneLimit = size_t(64) << 20;
