@@ -16,12 +16,39 @@ namespace {
 bool aligned_a(const skl_gemm_canon *g, size_t es) { return operand_ok(g->a, es, g->a_s1, g->a_s0, g->a_sk, g->m, g->k); }
 bool aligned_b(const skl_gemm_canon *g, size_t es) { return operand_ok(g->b, es, g->b_s1, g->b_s0, g->b_sk, g->n, g->k); }
 
-// Whole tiles enough for the streaming kernel, wherever the operands lie. (The rule of launch_whole_tiles for calls without
-// activation or copy and beyond the short fp8 K; its callers decide about those themselves.)
-bool tiles_to_stream(const skl_gemm_canon *g, size_t es) {
+MfmaArgs args_of(const skl_gemm_canon *g) {
+  MfmaArgs p;
+  p.a = (const char *)g->a;
+  p.b = (const char *)g->b;
+  p.c = (char *)g->c;
+  p.m = g->m, p.n = g->n, p.k = g->k;
+  p.a_s1 = g->a_s1, p.a_s0 = g->a_s0, p.a_sk = g->a_sk;
+  p.b_s1 = g->b_s1, p.b_s0 = g->b_s0, p.b_sk = g->b_sk;
+  p.rsc0 = g->rsc0, p.csc0 = g->csc0, p.rsc1 = g->rsc1, p.csc1 = g->csc1;
+  p.crs = g->c_row_shift, p.ccs = g->c_col_shift;
+  p.alpha = g->alpha, p.beta = g->beta;
+  p.bias = (const char *)g->bias, p.max = (char *)g->max;
+  p.rq = g->rq;
+  p.tiles_m = p.tiles_n = 0;
+  p.splits = 1, p.slices_per_split = 0, p.partial = nullptr;
+  return p;
+}
+
+// The kind, with operands that are copied - what has no unit stride or is off the 16-byte rule - as their copies: K contiguous.
+RingKind ring_kind_of(const skl_gemm_canon *g, size_t es) {
+  const bool fp8 = g->ta == SKL_DT_F8E4M3 || g->ta == SKL_DT_F8E5M2;
+  return {g->ta == SKL_DT_I8, fp8 && g->k <= kF8ExactMaxK, fp8, g->a_sk == 1 || !aligned_a(g, es), g->b_sk == 1 || !aligned_b(g, es), g->ta == g->tb, es};
+}
+
+// Whole tiles enough for the streaming kernel, wherever the operands lie ...
+bool tiles_enough(const skl_gemm_canon *g, size_t es) {
   if (g->m % 256 != 0 || (g->k * es) % 128 != 0) return false;
   const size_t tiles_m = g->m / 256;
   return (g->n % 256 == 0 && tiles_m * (g->n / 256) >= 200) || (g->n % 128 == 0 && tiles_m * (g->n / 128) >= 96);
+}
+// ... and whether it takes them (by launch_whole_tiles' own rule), what is off the 16-byte rule being copied.
+bool tiles_to_stream(const skl_gemm_canon *g, size_t es) {
+  return tiles_enough(g, es) && whole_tiles(args_of(g), ring_kind_of(g, es)).cols != 0;
 }
 
 }  // namespace
@@ -65,17 +92,24 @@ extern "C" int skl_hip_gemm_mfma_in_place_pays(const skl_gemm_canon *g) {
   return rounds_filled(wide >= 200 ? wide : tiles_m * ((g->n + 127) / 128)) < 60;
 }
 
+// Which of the matrix-core kernels takes the problem as it lies: 0 none, 1 the bounds-checked tiles, 256 / 128 the streaming kernel's
+// tiles of so many columns, with 1000 more where they are ragged.
+extern "C" int skl_hip_gemm_mfma_route(const skl_gemm_canon *g) {
+  if (!skl_hip_gemm_mfma_supported(g)) return 0;
+  const size_t es = (g->ta == SKL_DT_BF16 || g->ta == SKL_DT_F16) ? 2 : 1;
+  if (!aligned_a(g, es) || !aligned_b(g, es)) return 1;
+  const RingKind kind = ring_kind_of(g, es);
+  const MfmaArgs p = args_of(g);
+  if (const int cols = whole_tiles(p, kind).cols) return cols;
+  const int cols = kind.exact ? 0 : ragged_tile_cols(p, kind);
+  return cols ? 1000 + cols : 1;
+}
+
 // Would the streaming kernel take this int8 problem as it lies and write its C 16 bytes per lane (C in blocks of 4
 // to 16 columns with contiguous rows)? Then a blocked C costs no more than a row-major one.
 extern "C" int skl_hip_gemm_mfma_streams_c_quads(const skl_gemm_canon *g) {
   if (g->ta != SKL_DT_I8 || g->tb != SKL_DT_I8 || g->a_sk != 1 || g->b_sk != 1 || !streams_in_place(g, 1)) return 0;
-  MfmaArgs p;
-  p.c = (char *)g->c;
-  p.rsc0 = g->rsc0, p.csc0 = g->csc0, p.rsc1 = g->rsc1, p.csc1 = g->csc1;
-  p.crs = g->c_row_shift, p.ccs = g->c_col_shift;
-  p.bias = (const char *)g->bias, p.max = (char *)g->max;
-  p.rq = g->rq;
-  return c_in_row_quads(p);
+  return c_in_row_quads(args_of(g));
 }
 
 // A problem the streaming kernel does not take as it lies in memory - ragged M, N or K, operands off the 16-byte
@@ -88,7 +122,7 @@ extern "C" int skl_hip_gemm_mfma_padded_plan(const skl_gemm_canon *g, size_t *mp
   const bool fp8a = g->ta >= SKL_DT_F8E4M3, fp8b = g->tb >= SKL_DT_F8E4M3;
   if (!(g->ta == g->tb || (fp8a && fp8b)) || ((uintptr_t)g->c & 3) != 0) return 0;
   const size_t es = (g->ta == SKL_DT_BF16 || g->ta == SKL_DT_F16) ? 2 : 1;
-  if (streams_in_place(g, es)) return 0;
+  if (skl_hip_gemm_mfma_supported(g) && aligned_a(g, es) && aligned_b(g, es) && tiles_enough(g, es)) return 0;
   // With an activation or an 8-bit copy only where the operands would be copied anyway: the bounds-checked kernel, in
   // place, is the faster one for merely ragged sizes (bf16 2000 x 5000 x 3000 with SiLU 127 against 139 us, E4M3
   // 1027 x 8190 x 4096 into E4M3 87 against 114), the padded copies behind its own copies (int8 3001 x 4099 x 5003
@@ -109,13 +143,17 @@ extern "C" int skl_hip_gemm_mfma_padded_plan(const skl_gemm_canon *g, size_t *mp
   const size_t tiles_m = (g->m + 255) / 256;
   int tile_cols = 0;
   if (wide_enough) tile_cols = 256;
-  else if (tiles_m * ((g->n + 127) / 128) >= (fused ? 200 : 96)) tile_cols = 128;  // the rules of launch_whole_tiles
+  else if (tiles_m * ((g->n + 127) / 128) >= (fused ? 200 : 96)) tile_cols = 128;
   if (!tile_cols) return 0;
+  // Without steps by launch_whole_tiles' rule, the copies being whole tiles with K contiguous: below its lines the bounds-checked
+  // kernels are the faster ones on copies of their own as well.
+  const size_t tiles = tiles_m * ((g->n + tile_cols - 1) / tile_cols);
+  if (!fused && !ring_pays(args_of(g), {g->ta == SKL_DT_I8, false, fp8a, true, true, g->ta == g->tb, es}, tiles, false, rounds_filled(tiles))) return 0;
   // The epilogue of a fused call overlaps nothing, so its last round has to be fairly full (over the bounds-checked kernel
   // behind its own copies: 0.86 from 70 per cent on, 1.02 and up to 1.6 below; medians of 130 random layers) - unless that
   // kernel would read an fp8 operand across K where it lies (0.35 to 0.6), or for int8 of some K (0.8 to 0.95).
   const bool across_k = fp8a && ((a_ok && g->a_sk != 1) || (b_ok && g->b_sk != 1));
-  if (fused && !across_k && !(g->ta == SKL_DT_I8 && g->k >= 1024) && rounds_filled(tiles_m * ((g->n + tile_cols - 1) / tile_cols)) < 70) return 0;
+  if (fused && !across_k && !(g->ta == SKL_DT_I8 && g->k >= 1024) && rounds_filled(tiles) < 70) return 0;
   *mp = tiles_m * 256;
   *np = (g->n + tile_cols - 1) / tile_cols * tile_cols;
   *kp = (g->k * es + 127) / 128 * 128 / es;
@@ -134,20 +172,7 @@ extern "C" int skl_hip_launch_gemm_mfma_padded(const skl_gemm_canon *g, int tile
     skl_hip_record_error(-2, "gemm_mfma_padded: not a padded problem");
     return -2;
   }
-  MfmaArgs p;
-  p.a = (const char *)g->a;
-  p.b = (const char *)g->b;
-  p.c = (char *)g->c;
-  p.m = g->m, p.n = g->n, p.k = g->k;
-  p.a_s1 = g->a_s1, p.a_s0 = g->a_s0, p.a_sk = g->a_sk;
-  p.b_s1 = g->b_s1, p.b_s0 = g->b_s0, p.b_sk = g->b_sk;
-  p.rsc0 = g->rsc0, p.csc0 = g->csc0, p.rsc1 = g->rsc1, p.csc1 = g->csc1;
-  p.crs = g->c_row_shift, p.ccs = g->c_col_shift;
-  p.alpha = g->alpha, p.beta = g->beta;
-  p.bias = (const char *)g->bias, p.max = (char *)g->max;
-  p.rq = g->rq;
-  p.tiles_m = p.tiles_n = 0;
-  p.splits = 1, p.slices_per_split = 0, p.partial = nullptr;
+  MfmaArgs p = args_of(g);
   switch (g->ta * 8 + g->tb) {
     case SKL_DT_I8 * 8 + SKL_DT_I8: return skl_mfma_launch_padded_i8(p, tile_cols);
     case SKL_DT_BF16 * 8 + SKL_DT_BF16: return skl_mfma_launch_padded_bf16(p, tile_cols);
@@ -226,20 +251,7 @@ extern "C" int skl_hip_launch_gemm_mfma(const skl_gemm_canon *g) {
     skl_hip_record_error(-2, "gemm_mfma: unsupported problem");
     return -2;
   }
-  MfmaArgs p;
-  p.a = (const char *)g->a;
-  p.b = (const char *)g->b;
-  p.c = (char *)g->c;
-  p.m = g->m, p.n = g->n, p.k = g->k;
-  p.a_s1 = g->a_s1, p.a_s0 = g->a_s0, p.a_sk = g->a_sk;
-  p.b_s1 = g->b_s1, p.b_s0 = g->b_s0, p.b_sk = g->b_sk;
-  p.rsc0 = g->rsc0, p.csc0 = g->csc0, p.rsc1 = g->rsc1, p.csc1 = g->csc1;
-  p.crs = g->c_row_shift, p.ccs = g->c_col_shift;
-  p.alpha = g->alpha, p.beta = g->beta;
-  p.bias = (const char *)g->bias, p.max = (char *)g->max;
-  p.rq = g->rq;
-  p.tiles_m = p.tiles_n = 0;
-  p.splits = 1, p.slices_per_split = 0, p.partial = nullptr;
+  MfmaArgs p = args_of(g);
   const size_t es = (g->ta == SKL_DT_BF16 || g->ta == SKL_DT_F16) ? 2 : 1;
   p.a_loose = !aligned_a(g, es), p.b_loose = !aligned_b(g, es);
   switch (g->ta * 8 + g->tb) {

@@ -2558,6 +2558,65 @@ int launch_one(const MfmaArgs &args) {
   return launch_split_reduce<AccElem>(p, "gemm_split_reduce");
 }
 
+// What the lines below depend on besides the problem: C's type, whether fp8 is multiplied exactly, which operands have K contiguous,
+// whether the fp8 instructions multiply (FP8), whether the kind has kernels with steps.
+struct RingKind {
+  bool is_int, exact, fp8, a_kc, b_kc, carries_steps;
+  size_t es;
+};
+inline bool reads_old_c(const MfmaArgs &p, bool is_int) { return is_int ? p.beta.i != 0 : !(p.beta.fz.skip_c_read && p.beta.f == 0.0f); }
+
+// Whether the streaming kernel beats the bounds-checked ones on whole tiles: those have several workgroups on a compute unit, whose
+// starts and ends overlap with others' products, it has one. What decides is how full its last round is, how much K there is to gain
+// on, and whether C is read, which it requests earlier than the others do; an activation of some thirty or forty instructions (SiLU,
+// GELU) is covered by less there. Its time over theirs, geometric means over 720 random problems, by K in bytes; more than one round, by
+// `filled` (50-60 / 60-70 / 70-80 / 80-90 / 90-100 per cent); "-": none drawn:
+//   16 bits, plain        from  512  1.17  -   1.01 1.07 1.07   from 1024  1.16 1.11 0.89 0.99 0.94   from 2048   -   1.00 0.84 0.85 0.91   from 4096  -   0.93 -  0.83 0.80
+//     C read              from  512  1.04 1.13 1.02  -   0.95   from 1024   -   0.95  -   0.95 0.93   from 2048   -    -   0.88 0.87 0.79
+//     ReLU                from  512   -   0.94  -   0.94 0.82   from 1024   -    -   0.81 0.89 0.89   from 2048  0.93  -   0.90  -   0.86
+//     a copy              0.67 to 0.90 at any K
+//     SiLU or GELU        from  512  1.03 1.04 0.96 0.94 0.95   from 1024  1.13 1.05 1.00 1.03 0.90   from 2048   -   0.89 0.91 0.92 0.83   from 4096  0.97 - 0.89 0.74 -
+//   fp8, plain            from 2305  0.99  -   1.07 0.96  -     from 4096  0.92  -   0.86 0.78 0.85
+//     C read, ReLU, a copy  from 2305  0.89 0.96 0.92  -  0.84  from 4096  0.96 0.89 0.87 0.83 0.78
+//     SiLU or GELU        from 2305   -   1.12  -   0.95 0.85   from 4096  1.13 0.93 1.07 0.99  -     from 8192  0.90 0.87 0.83 0.74 -
+//   short fp8, plain      from  512  1.27 1.28 1.11 0.99 0.99   from 1024  1.18  -   1.05 0.93 1.01
+//     C read              from  512  1.07 1.02 0.92 1.00 0.99   from 1024  1.09 1.05 0.93 0.92 0.94
+//     ReLU                from  512  1.07  -    -   0.99 0.92   from 1024   -   1.08  -   0.92 0.84
+//     a copy              from  512  1.07  -    -   0.83 0.78   from 1024  1.00 0.94 0.83 0.84 0.83
+//     SiLU or GELU        from  512  1.14  -   1.09 0.99 0.93   from 1024   -   1.06 1.02 0.93 0.98   from 2048   -   1.14  -    -    -
+//   int8, plain           from  512  1.12  -   1.13  -   1.07   from 1024  1.17 1.12 0.92 1.13 1.08   from 2048  0.98 0.98 0.83  -   0.76
+//     C read              0.67 to 0.84 at any K
+//     ReLU                from  512   -    -   1.00  -   1.01   from 1024   -   1.01  -   1.14 0.96   from 2048   -   0.84  -    -    -
+//     a copy              from  512   -    -    -   0.94 0.89   from 1024  0.97 0.87 0.90 0.91 0.93   from 2048   -   0.96 0.89 0.85  -
+// A single round of 200 to 256 tiles: 16 bits plain 1.07 below 1024, short fp8 1.01, all others 0.65 to 0.97. 129 to 199 tiles: 0.64 to 0.98,
+// everything. 96 to 128 tiles, half of the chip: plain 1.09 (16 bits), 1.06 (fp8), 1.33 (short fp8) and 1.06 to 1.10 (int8) below 4096, from there on
+// 0.78 to 0.81, C read 0.76 to 0.93, a copy 0.72 to 0.90, short fp8 with SiLU or GELU 1.07. With a K of 8 KiB and more also 65 to 128 tiles with steps,
+// which share K, 0.78; exactly 64 are 128 bounds-checked tiles, which share it four ways: 1.12 to 1.24.
+inline bool ring_pays(const MfmaArgs &p, const RingKind &kind, size_t tiles, bool long_k, unsigned filled) {
+  const bool slow_others = kind.fp8 && !kind.exact && !(kind.a_kc && kind.b_kc);  // transposed fragments of 32 bytes: they take two to four times as long
+  constexpr unsigned kNever = 101;
+  const size_t k_bytes = p.k * kind.es;
+  const bool reads_c = reads_old_c(p, kind.is_int), steps = p.rq.act || p.rq.q, many_steps = p.rq.act >= 2;
+  const bool dwords = kind.is_int ? dword_copy<int>(p.rq) : dword_copy<float>(p.rq);
+  const bool in_rows = p.csc0 == 1 && (p.ccs >= 6 || p.csc1 == (size_t(1) << p.ccs));  // a C that is not: the others take three to four times as long
+  if (tiles < 200) {
+    if (long_k) return tiles > 64 || !steps || slow_others;
+    if (tiles > 128) return true;
+    if (kind.exact) return dwords;
+    if (steps) return dwords;
+    return reads_c || k_bytes >= 4096 || slow_others || !in_rows;
+  }
+  if (tiles <= 256) return reads_c || steps || kind.is_int || k_bytes >= 1024;
+  if (slow_others || (!in_rows && (!kind.exact || steps) && !p.rq.q_only)) return true;
+  if (many_steps) {
+    if (reads_c) return filled >= (k_bytes >= 4096 ? 0 : k_bytes >= 2048 ? 70 : k_bytes >= 1024 ? 80 : kNever);
+    return filled >= (k_bytes >= 8192 ? 0 : k_bytes >= 4096 || (k_bytes >= 2048 && kind.es == 2) ? 60 : 80);
+  }
+  if (kind.exact) return filled >= (reads_c || p.rq.q ? 70 : 80);
+  if (kind.is_int) return reads_c || p.rq.q || filled >= (k_bytes >= 2048 ? 0 : k_bytes >= 1024 ? steps ? 90 : 70 : kNever);
+  return steps || filled >= (k_bytes >= 2048 ? 0 : k_bytes >= 1024 ? reads_c ? 60 : 70 : reads_c ? 80 : kNever);
+}
+
 // How well `tiles` workgroups, one at a time on each of the 256 compute units, fill the rounds they take, in per cent.
 // `tail`: the last round runs as 256 x 128 tiles, half as long.
 inline unsigned rounds_filled(size_t tiles, bool tail = false) {
@@ -2565,98 +2624,59 @@ inline unsigned rounds_filled(size_t tiles, bool tail = false) {
   return (unsigned)(tiles * 200 / (256 * half_rounds));
 }
 
-// Whether the streaming kernel beats the bounds-checked ones on whole tiles: those have several workgroups on a compute unit, whose
-// starts and ends overlap with others' products, it has one. What decides is how full its last round is, how much K there is to gain
-// on, and whether C is read, which it requests earlier than the others do; an activation of some thirty or forty instructions (SiLU,
-// GELU) is covered by nothing there. Its time over theirs, geometric means over random problems, by K in bytes; more than one round, by
-// `filled` (50-60 / 60-70 / 70-80 / 80-90 / 90-100 per cent); "-": fewer than three were drawn:
-//   16 bits, plain        from 1024  1.19 1.19 1.14 1.03 1.00   from 2048  1.00 1.02 0.93 0.91 0.91   from 4096  0.94 0.92 0.80 0.85  -
-//     C read              from 1024  1.01 1.01 0.95 0.92 0.91   from 2048  0.99 0.94 0.93 0.88 0.82
-//     ReLU or a copy      from 1024  1.02 1.01 0.97 0.91 0.87   from 2048  0.98 0.95 0.89 0.87  -
-//     SiLU or GELU        from 1024  1.38 1.25 1.28 1.18 1.12   from 2048  1.18 1.13 1.10 1.04  -     from 4096  1.06 1.03 0.97 0.89 0.87   from 8192  0.95 0.94 0.84 - -
-//   fp8, plain            from 2305  1.04 1.05 0.95  -    -     from 4096  0.95 0.96  -    -    -
-//   short fp8, plain      from  512  1.45 1.39 1.25 1.21 1.18   from 1024  1.32 1.24 1.09 1.10 1.00   from 2048  1.23  -   -    -    -
-//     C read              from  512  1.12 1.06 1.00 1.02 0.97   from 1024  1.16 1.14 1.04 0.99 0.93
-//     ReLU or a copy      from  512  1.19 1.16 1.11 1.04 0.97   from 1024  1.17 1.12 1.09 0.99 0.88   from 2048   -   1.15  -  0.92  -
-//     SiLU or GELU        from  512  1.45 1.47  -   1.19 1.21   from 1024  1.36 1.31 1.37 1.14 1.02
-//   int8, plain           from  512  1.16 1.14 1.16 1.10 1.09   from 1024  1.08 1.08 0.98 1.01 0.98   from 2048  0.94 0.99 0.94 0.85  -
-//     C read              0.69 to 0.85 at any K
-//     ReLU or a copy      from  512  1.22 1.16 1.14 1.08 1.11   from 1024  1.11 1.12 1.07 1.00 0.93   from 2048  1.00  -   1.01  -   0.95 (a copy in dwords; ReLU into C
-//                         the other way, 6656 x 4864 x 640 40 against 46 us: the streaming kernel keeps both)
-// A single round of 200 to 256 tiles: short fp8 plain 1.07 below 2048, with SiLU or GELU 1.15 below 1024, all others less than one.
-// 129 to 199 tiles: SiLU or GELU 0.83 from 4096 (fp8 0.89), short fp8 with C read, ReLU or a copy 0.92. 96 to 128 tiles, half of the
-// chip: plain 16 bits 1.37 from 1024, 1.23 from 2048, fp8 1.20 from 2305, int8 1.27, 1.21 and 1.14 from 512, 1024 and 2048. With a K of 8 KiB
-// and more also 65 to 128 tiles with steps, which share K, 0.78; exactly 64 are 128 bounds-checked tiles, which
-// share it four ways: 1.12 to 1.24.
-template <typename AccElem, bool EXACT, bool A_KC, bool B_KC, bool FP8>
-bool ring_pays(const MfmaArgs &p, size_t tiles, size_t k_bytes, bool long_k, unsigned filled) {
-  constexpr bool kInt = std::is_same<AccElem, int>::value;
-  constexpr bool kSlowOthers = FP8 && !EXACT && !(A_KC && B_KC);  // transposed fragments of 32 bytes: they take two to four times as long
-  constexpr unsigned kNever = 101;
-  const bool reads_c = kInt ? p.beta.i != 0 : !(p.beta.fz.skip_c_read && p.beta.f == 0.0f);
-  const bool steps = p.rq.act || p.rq.q, many_steps = p.rq.act >= 2;
-  const bool in_rows = p.csc0 == 1 && (p.ccs >= 6 || p.csc1 == (size_t(1) << p.ccs));  // a C that is not: the others take three to four times as long
-  if (tiles < 200) {
-    if (long_k) return tiles > 64 || !steps || kSlowOthers;
-    if (EXACT) return tiles > 128 && (reads_c || (steps && !many_steps));
-    if (steps && !dword_copy<AccElem>(p.rq)) return many_steps && tiles > 128 && k_bytes >= 4096;
-    return steps || tiles > 128 || reads_c || k_bytes >= 4096 || kSlowOthers || !in_rows;
-  }
-  if (tiles <= 256) return !EXACT || reads_c || k_bytes >= (many_steps ? 1024 : steps ? 0 : 2048);
-  if (kSlowOthers || (!in_rows && (!EXACT || steps) && !p.rq.q_only)) return true;
-  if (many_steps) {
-    if (reads_c) return filled >= (k_bytes >= 4096 ? 0 : k_bytes >= 2048 ? 70 : k_bytes >= 1024 ? 80 : kNever);
-    return filled >= (k_bytes >= 8192 ? 0 : k_bytes >= 4096 ? 70 : k_bytes >= 2048 ? 80 : EXACT && k_bytes >= 1024 ? 90 : kNever);
-  }
-  if (EXACT) return filled >= (reads_c ? 80 : steps ? k_bytes >= 1024 ? 80 : 90 : k_bytes >= 2048 ? 80 : k_bytes >= 1024 ? 90 : kNever);
-  if (reads_c) return true;
-  if (kInt) return steps || filled >= (k_bytes >= 2048 ? 0 : k_bytes >= 1024 ? 70 : kNever);
-  return filled >= (k_bytes >= 2048 || steps ? 0 : 80);
-}
-
-// The streaming kernel takes problems that its tiles divide evenly: 256 x 256 tiles when those can fill the 256 compute
-// units, 256 x 128 tiles for the sizes below that, from 96 tiles on, or from 64 when K is long enough to be shared between
-// two workgroups per tile. Returns kNotWholeTiles for the others, and where the bounds-checked kernels are faster.
-constexpr int kNotWholeTiles = 0x7FFFFFFF;
-template <int TA, int TB, bool A_KC, bool B_KC, bool EXACT>
-int launch_whole_tiles(const MfmaArgs &p) {
-  constexpr int ES = Kind<TA>::ES;
-  constexpr size_t kRing128FromTiles = 96;
-  using AccElem = decltype(typename Kind<TA>::Acc{}.x);
-  const auto wide = [](const MfmaArgs &q) { return launch_ring<TA, TB, A_KC, B_KC, 256, false, false, false, EXACT>(q); };
-  const auto narrow = [](const MfmaArgs &q) { return launch_ring<TA, TB, A_KC, B_KC, 128, false, false, false, EXACT>(q); };
-  if (p.m % 256 != 0 || p.n % 128 != 0 || (p.k * ES) % 128 != 0 || p.a_loose || p.b_loose) return kNotWholeTiles;
-  const size_t tiles_m = p.m / 256, slices = p.k * ES / kRingSlice;
+// How the streaming kernel takes a problem that its tiles divide evenly (operands on the 16-byte rule): 256 x 256 tiles when those can
+// fill the 256 compute units, 256 x 128 tiles for the sizes below that, from 96 tiles on, or from 64 when K is long enough to be shared
+// between two workgroups per tile. No columns: the tiles don't divide it, or the bounds-checked kernels are faster.
+struct WholeTiles {
+  int cols;
+  size_t tail_tiles;  // 256 x 256 tiles of a last round that runs as 256 x 128 ones
+};
+inline WholeTiles whole_tiles(const MfmaArgs &p, const RingKind &kind) {
+  if (p.m % 256 != 0 || p.n % 128 != 0 || (p.k * kind.es) % 128 != 0) return {0, 0};
+  if ((p.rq.act || p.rq.q) && !kind.carries_steps) return {0, 0};
+  const size_t tiles_m = p.m / 256, slices = p.k * kind.es / kRingSlice;
   const size_t tiles = p.n % 256 == 0 ? tiles_m * (p.n / 256) : 0, tiles128 = tiles_m * (p.n / 128);
   // A last round of 256 x 256 tiles that would fill at most half of the 256 compute units is run as 256 x 128 tiles
   // instead (a second launch on the trailing columns): twice the workgroups at half the length.
   const size_t rest = tiles % 256;
-  const bool tail_round = rest != 0 && rest <= 128 && rest % tiles_m == 0;
+  const bool wide = tiles >= 200, tail_round = rest != 0 && rest <= 128 && rest % tiles_m == 0;
   const bool long_k = slices % 4 == 0 && slices / 2 >= kRingMinSlicesPerSplit;
-  const bool extra = p.rq.act || p.rq.q;
-  if (extra && !kRingCarriesExtraSteps<TA, TB>) return kNotWholeTiles;
-  if (!ring_pays<AccElem, EXACT, A_KC, B_KC, TA == SKL_DT_F8E4M3 || TA == SKL_DT_F8E5M2>(
-          p, tiles >= 200 ? tiles : tiles128, p.k * ES, long_k, tiles >= 200 ? rounds_filled(tiles, tail_round) : rounds_filled(tiles128)))
-    return kNotWholeTiles;
-  if (tiles >= 200) {
-    if (!tail_round) return wide(p);
-    const size_t tail_cols = rest / tiles_m * 256, head_cols = p.n - tail_cols;
-    MfmaArgs head = p, tail = p;
-    head.n = head_cols;
-    tail.n = tail_cols;
-    tail.b = p.b + (head_cols / 64) * p.b_s1 * ES;
-    tail.c = p.c + (head_cols >> p.ccs) * p.csc1 * sizeof(float);  // whole blocks; C elements are 4 bytes for every kind
-    if (p.bias) tail.bias = p.bias + head_cols * sizeof(float);
-    if (p.rq.q) tail.rq.q = p.rq.q + head_cols * p.rq.csq;
-    if (p.rq.q && p.rq.q_per_column) tail.rq.q_scale = p.rq.q_scale + head_cols;
-    // The tail may be tiles few enough to share K (launch_ring): what it needs for that is there before the head has written
-    // its columns of C, which no other kernel could then start from.
-    if (tiles_m * (tail_cols / 128) <= 128 && long_k && !skl_workspace((size_t)2 * p.m * tail_cols * 4)) return -4;
-    const int rc = wide(head);
-    return rc != 0 ? rc : narrow(tail);
-  }
-  if (tiles128 >= kRing128FromTiles || (tiles128 >= 64 && long_k)) return narrow(p);
-  return kNotWholeTiles;
+  if (!wide && tiles128 < 96 && !(tiles128 >= 64 && long_k)) return {0, 0};
+  if (!ring_pays(p, kind, wide ? tiles : tiles128, long_k, wide ? rounds_filled(tiles, tail_round) : rounds_filled(tiles128))) return {0, 0};
+  return {wide ? 256 : 128, wide && tail_round ? rest : 0};
+}
+
+template <int TA, int TB, bool A_KC, bool B_KC, bool EXACT>
+constexpr RingKind ring_kind() {
+  constexpr bool fp8 = TA == SKL_DT_F8E4M3 || TA == SKL_DT_F8E5M2;
+  return {TA == SKL_DT_I8, EXACT, fp8, A_KC, B_KC, kRingCarriesExtraSteps<TA, TB>, (size_t)Kind<TA>::ES};
+}
+constexpr int kNotWholeTiles = 0x7FFFFFFF;
+template <int TA, int TB, bool A_KC, bool B_KC, bool EXACT>
+int launch_whole_tiles(const MfmaArgs &p) {
+  constexpr int ES = Kind<TA>::ES;
+  const auto wide = [](const MfmaArgs &q) { return launch_ring<TA, TB, A_KC, B_KC, 256, false, false, false, EXACT>(q); };
+  const auto narrow = [](const MfmaArgs &q) { return launch_ring<TA, TB, A_KC, B_KC, 128, false, false, false, EXACT>(q); };
+  if (p.a_loose || p.b_loose) return kNotWholeTiles;
+  const WholeTiles how = whole_tiles(p, ring_kind<TA, TB, A_KC, B_KC, EXACT>());
+  if (how.cols == 0) return kNotWholeTiles;
+  if (how.cols == 128) return narrow(p);
+  if (how.tail_tiles == 0) return wide(p);
+  const size_t tiles_m = p.m / 256, tail_cols = how.tail_tiles / tiles_m * 256, head_cols = p.n - tail_cols, slices = p.k * ES / kRingSlice;
+  MfmaArgs head = p, tail = p;
+  head.n = head_cols;
+  tail.n = tail_cols;
+  tail.b = p.b + (head_cols / 64) * p.b_s1 * ES;
+  tail.c = p.c + (head_cols >> p.ccs) * p.csc1 * sizeof(float);  // whole blocks; C elements are 4 bytes for every kind
+  if (p.bias) tail.bias = p.bias + head_cols * sizeof(float);
+  if (p.rq.q) tail.rq.q = p.rq.q + head_cols * p.rq.csq;
+  if (p.rq.q && p.rq.q_per_column) tail.rq.q_scale = p.rq.q_scale + head_cols;
+  // The tail may be tiles few enough to share K (launch_ring): what it needs for that is there before the head has written
+  // its columns of C, which no other kernel could then start from.
+  const bool long_k = slices % 4 == 0 && slices / 2 >= kRingMinSlicesPerSplit;
+  if (tiles_m * (tail_cols / 128) <= 128 && long_k && !skl_workspace((size_t)2 * p.m * tail_cols * 4)) return -4;
+  const int rc = wide(head);
+  return rc != 0 ? rc : narrow(tail);
 }
 
 // The streaming kernel on problems that are not whole tiles (EDGE): the tile's columns, or 0 where the bounds-checked kernels
@@ -2667,26 +2687,25 @@ int launch_whole_tiles(const MfmaArgs &p) {
 // 0.94 and 0.90; below the line 1.00 to 1.35. 128 columns 0.82 to 0.95. The problems that the rule moves take 0.73 (int8 reading C) to
 // 0.95 (16 bits reading C, 128 columns) of the time.
 // Floating point only beyond 256 tiles of 128 x 128: fewer share K, and sums of several parts are the more exact ones.
-template <int TA, int TB, bool A_KC, bool B_KC>
-int ragged_tile_cols(const MfmaArgs &p) {
-  constexpr size_t ES = Kind<TA>::ES, limit = 0xB0000000u;
-  if (p.a_loose || p.b_loose || ((p.rq.act || p.rq.q) && !kRingCarriesExtraSteps<TA, TB>)) return 0;
-  if (p.m % 256 == 0 && p.n % 128 == 0 && p.k * ES % 128 == 0) return 0;  // whole tiles: launch_whole_tiles has decided
+inline int ragged_tile_cols(const MfmaArgs &p, const RingKind &kind) {
+  constexpr size_t limit = 0xB0000000u;
+  const size_t es = kind.es;
+  if (p.a_loose || p.b_loose || ((p.rq.act || p.rq.q) && !kind.carries_steps)) return 0;
+  if (p.m % 256 == 0 && p.n % 128 == 0 && p.k * es % 128 == 0) return 0;  // whole tiles: launch_whole_tiles has decided
   // 16 bytes along K that K ends in would need zeros behind it; the offsets inside a tile stay in the descriptor's range
-  if (p.k * ES % 16 != 0 && (A_KC || B_KC)) return 0;
-  if ((3 * p.a_s1 + (A_KC ? 63 * p.a_s0 : 64 * p.a_sk)) * ES >= limit || (3 * p.b_s1 + (B_KC ? 63 * p.b_s0 : 64 * p.b_sk)) * ES >= limit) return 0;
+  if (p.k * es % 16 != 0 && (kind.a_kc || kind.b_kc)) return 0;
+  if ((3 * p.a_s1 + (kind.a_kc ? 63 * p.a_s0 : 64 * p.a_sk)) * es >= limit || (3 * p.b_s1 + (kind.b_kc ? 63 * p.b_s0 : 64 * p.b_sk)) * es >= limit) return 0;
   const size_t tiles_m = (p.m + 255) / 256, wide = tiles_m * ((p.n + 255) / 256), narrow = tiles_m * ((p.n + 127) / 128);
-  const size_t small = (size_t)skl_div_up(p.m, 128) * skl_div_up(p.n, 128), k_bytes = p.k * ES;
-  constexpr bool kInt = std::is_same<decltype(typename Kind<TA>::Acc{}.x), int>::value;
+  const size_t small = (size_t)skl_div_up(p.m, 128) * skl_div_up(p.n, 128), k_bytes = p.k * es;
   constexpr unsigned kNever = 101;
-  const bool reads_c = kInt ? p.beta.i != 0 : !(p.beta.fz.skip_c_read && p.beta.f == 0.0f);
+  const bool reads_c = reads_old_c(p, kind.is_int);
   const unsigned of_wide = (unsigned)(small * 100 / ((wide + 255) / 256 * 1024)), of_narrow = (unsigned)(small * 100 / ((narrow + 255) / 256 * 512));
   const auto by_k = [&](unsigned from_512, unsigned from_1k, unsigned from_2k, unsigned from_4k, unsigned from_8k) {
     return k_bytes >= 8192 ? from_8k : k_bytes >= 4096 ? from_4k : k_bytes >= 2048 ? from_2k : k_bytes >= 1024 ? from_1k : k_bytes >= 512 ? from_512 : kNever;
   };
-  if (!kInt && small <= 256) return 0;
+  if (!kind.is_int && small <= 256) return 0;
   unsigned from_wide, from_narrow;
-  if (kInt) {
+  if (kind.is_int) {
     from_wide = reads_c ? by_k(65, 65, 55, 55, 55) : by_k(kNever, kNever, 80, 55, 55);
     from_narrow = reads_c ? by_k(55, 55, 55, 55, 55) : by_k(kNever, kNever, kNever, 55, 55);
   } else if (p.rq.act >= 2) {
@@ -2694,7 +2713,7 @@ int ragged_tile_cols(const MfmaArgs &p) {
     from_narrow = by_k(kNever, kNever, kNever, kNever, 55);
   } else {
     from_wide = by_k(kNever, reads_c ? 80 : kNever, 70, 60, 52);
-    from_narrow = by_k(kNever, kNever, kNever, 70, 52);
+    from_narrow = by_k(kNever, kNever, reads_c ? 70 : kNever, 70, 52);
   }
   return of_wide >= from_wide ? 256 : of_narrow >= from_narrow ? 128 : 0;
 }
@@ -2740,7 +2759,7 @@ int launch_tile(const MfmaArgs &p) {
   }
   const int rc = launch_whole_tiles<TA, TB, A_KC, B_KC, false>(p);
   if (rc != kNotWholeTiles) return rc;
-  if (const int cols = ragged_tile_cols<TA, TB, A_KC, B_KC>(p)) return launch_ragged<TA, TB, A_KC, B_KC>(p, cols);
+  if (const int cols = ragged_tile_cols(p, ring_kind<TA, TB, A_KC, B_KC, false>())) return launch_ragged<TA, TB, A_KC, B_KC>(p, cols);
   if (small_tiles<ES, TA == SKL_DT_I8, A_KC, B_KC>(p))
     return launch_one<TA, TB, A_KC, B_KC, 64, 64, 2, 2>(p);
   return launch_one<TA, TB, A_KC, B_KC, 128, 128, 2, 4>(p);

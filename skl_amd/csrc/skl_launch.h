@@ -114,6 +114,8 @@ int skl_hip_launch_gemm_tiled(const skl_gemm_canon *g);
 int skl_hip_gemm_mfma_supported(const skl_gemm_canon *g);
 /* ... and whether that beats copies padded to whole tiles. */
 int skl_hip_gemm_mfma_in_place_pays(const skl_gemm_canon *g);
+/* Which of its kernels takes the problem as it lies (skl_gemm_mfma.hip), for tests and reports. */
+int skl_hip_gemm_mfma_route(const skl_gemm_canon *g);
 int skl_hip_launch_gemm_mfma(const skl_gemm_canon *g);
 
 /* The streaming kernel on copies of A and B padded to whole tiles (see skl_gemm_mfma.hip): the plan returns the tile

@@ -154,3 +154,52 @@ def test_where_k_contiguous_decode_batches_leave_the_streaming_kernel():
         assert not streams_k_contiguous(*case), case
     # columns that start inside lines take half as long again
     assert streams_k_contiguous(I8, 16, 256, 14336) and not streams_k_contiguous(I8, 16, 256, 14336, pitch=14352)
+
+
+RAGGED = 1000
+
+
+def route(kind, m, n, k, a_rows=True, b_rows=True, pad=0, beta=0, act=0, q=None, kind_b=None, lda=None):
+    """The matrix-core kernel that takes a problem as it lies: 0 none, 1 the bounds-checked tiles, else the columns of the streaming
+    kernel's tiles, RAGGED more where those are ragged. `pad` elements between rows; `q` the format of a row-major 8-bit copy."""
+    g = Canon(ta=kind, tb=kind if kind_b is None else kind_b, m=m, n=n, k=k, a=1 << 20, b=1 << 20, c=1 << 20, c_row_shift=6, c_col_shift=6)
+    lda, ldb = lda or (k if a_rows else m) + pad, (n if b_rows else k) + pad
+    g.a_s0, g.a_sk = (lda, 1) if a_rows else (1, lda)
+    g.b_s0, g.b_sk = (1, ldb) if b_rows else (ldb, 1)
+    g.a_s1, g.b_s1 = 64 * g.a_s0, 64 * g.b_s0
+    g.rsc0, g.csc0, g.rsc1, g.csc1 = n, 1, 64 * n, 64
+    g.rq.act = act
+    if q is not None:
+        g.rq.q, g.rq.rsq, g.rq.csq, g.rq.q_scale, g.rq.q_fmt = 1 << 20, (n + 3) // 4 * 4, 1, 1 << 20, q
+    scalar = ct.c_int32 if kind == I8 else ct.c_float
+    scalar.from_buffer(g, Canon.beta.offset).value = beta
+    if kind != I8:
+        ct.c_uint32.from_buffer(g, Canon.beta.offset + 4).value = 1  # C is not read where beta is zero
+    fn = ct.CDLL(skl_amd.library_path()).skl_hip_gemm_mfma_route
+    fn.argtypes = [ct.POINTER(Canon)]
+    return fn(ct.byref(g))
+
+
+def test_whole_tiles_go_where_they_were_measured_to_be_faster():
+    """A copy of whole numbers, a C that is read, SiLU: the streaming kernel; short plain products on half of the chip: not."""
+    for kind, k in ((I8, 1024), (BF16, 512), (F16, 1024), (E4M3, 1024)):
+        assert route(kind, 4096, 1024, k) == 1 and route(kind, 4096, 1024, 8192 if kind != E4M3 else 16384) == 128   # 128 tiles of 256 x 128
+        assert route(kind, 4352, 1024, k) == 128 and route(kind, 4352, 1024, k, beta=1) == 128                       # 136
+        assert route(kind, 4096, 3328, k, act=1, q=0 if kind == I8 else 2) == 256                                    # 208 of 256 x 256
+    assert route(I8, 4096, 1024, 1024, beta=1) == 128 and route(BF16, 4096, 1024, 512, beta=1) == 128
+    assert route(I8, 7424, 7168, 512, act=1, q=0) == 256 and route(I8, 7424, 7168, 512, act=1) == 1                  # 812: a copy, ReLU into C
+    assert route(I8, 8192, 8192, 1024) == 256 and route(I8, 7424, 7168, 512) == 1
+    assert route(E4M3, 8192, 12032, 640) == 256 and route(E4M3, 4352, 4608, 640) == 1                                # 1504 and 306 of 256 x 256
+
+
+@pytest.mark.parametrize("kind", (I8, BF16, F16, E4M3))
+def test_whole_tiles_off_the_16_byte_rule_are_copied_only_to_stream(kind):
+    """128 tiles of 256 x 128 with a short K run on the bounds-checked tiles, in place, whatever the leading dimension; with a C that is
+    read, or more tiles, the copy of the operand lets the streaming kernel run. The padded plan follows the same lines."""
+    k = 512 if kind in (BF16, F16) else 1024
+    assert route(kind, 4096, 1024, k) == 1 and route(kind, 4096, 1024, k, lda=k + 1) == 1
+    assert route(kind, 4352, 1024, k) == 128 and route(kind, 4352, 1024, k, lda=k + 1) == 0
+    if kind != E4M3:
+        assert route(kind, 4096, 1024, k, beta=1, lda=k + 1) == 0
+    if kind == I8:
+        assert plan(kind, 4090, 1020, k, lda=k + 1, ldb=1021) == 0 and plan(kind, 4346, 1020, k, lda=k + 1, ldb=1021) == 128

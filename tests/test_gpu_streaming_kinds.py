@@ -1,15 +1,18 @@
 """Streaming kernels that no other test names one by one: ragged 256 x 128 tiles of every kind and layout, fp8 beyond the exact K on
-256 x 128 tiles read across K, eight waves under a C that is read over several rounds."""
+256 x 128 tiles read across K, eight waves under a C that is read over several rounds. Each test asks the dispatch first which kernel
+the problem takes, so that a line that moves fails here instead of leaving a kernel without its test."""
 import numpy as np
 import pytest
 
 import support
 from gpu_support import run_gemm
+from test_dispatch_rules import BF16, E4M3, E5M2, F16, I8, RAGGED, route
 from test_gpu_gemm import _dense_case
 from test_gpu_gemm_in_place import ragged_large
 
 pytestmark = pytest.mark.gpu
 
+KINDS = {"i8": I8, "bf16": BF16, "f16": F16, "f8e4m3": E4M3, "f8e5m2": E5M2}
 LAYOUTS = ((True, True), (True, False), (False, True), (False, False))
 # one round of 256 x 128 tiles, the last ones 16 rows and columns wide; K in whole pairs of slices and eight or sixteen bytes, ending in
 # an odd slice, and - where no operand has K contiguous - anywhere
@@ -23,6 +26,8 @@ RAGGED_K = [("i8", 528, 1, False), ("i8", 577, 1, False), ("i8", 4112, 0, True),
 def test_ragged_tiles_of_128_columns(gpu, ta, k, beta, relu, a_rows, b_rows):
     if k % 8 and (a_rows or not b_rows):
         pytest.skip("16 bytes along K that end inside: the bounds-checked kernels")
+    pad = 32 // support.ETYPES[ta].dtype.itemsize
+    assert route(KINDS[ta], 2320, 2832, k, a_rows, b_rows, pad=pad, beta=beta, act=int(relu)) == RAGGED + 128
     ragged_large(gpu, ta, 2320, 2832, k, a_rows, b_rows, beta, relu)
 
 
@@ -53,6 +58,7 @@ def against_fp64(gpu, ta, tb, m, n, k, a_kc, b_kc, alpha, beta, reference_mode=F
 @pytest.mark.parametrize("beta,reference_mode", ((0.5, False), (0.0, False), (0.0, True)))
 def test_fp8_beyond_the_exact_k_read_across_k(gpu, ta, tb, beta, reference_mode):
     """256 x 128 tiles, K of 2432 elements: C read, not read, and looked through while the tile is multiplied."""
+    assert route(KINDS[ta], 2048, 1664, 2432, False, True, kind_b=KINDS[tb or ta], beta=beta) == 128
     against_fp64(gpu, ta, tb, 2048, 1664, 2432, False, False, 1.5, beta, reference_mode)
 
 
@@ -63,4 +69,5 @@ def test_c_read_over_two_rounds_of_tiles(gpu, ta, a_rows, b_rows):
     exact on both."""
     k = {"i8": 128, "bf16": 512, "f8e4m3": 256}[ta]
     for m, n in ((4352, 5632), (2048, 8704)):
+        assert route(KINDS[ta], m, n, k, a_rows, b_rows, beta=1) == 256
         against_fp64(gpu, ta, None, m, n, k, a_rows, not b_rows, 3 if ta == "i8" else 1.5, -2 if ta == "i8" else 0.5)
