@@ -148,7 +148,7 @@ extern "C" int skl_hip_gemm_mfma_padded_plan(const skl_gemm_canon *g, size_t *mp
   // Without steps by launch_whole_tiles' rule, the copies being whole tiles with K contiguous: below its lines the bounds-checked
   // kernels are the faster ones on copies of their own as well.
   const size_t tiles = tiles_m * ((g->n + tile_cols - 1) / tile_cols);
-  if (!fused && !ring_pays(args_of(g), {g->ta == SKL_DT_I8, false, fp8a, true, true, g->ta == g->tb, es}, tiles, false, rounds_filled(tiles))) return 0;
+  if (!fused && !ring_pays(args_of(g), {g->ta == SKL_DT_I8, false, fp8a, true, true, g->ta == g->tb, es}, wide_enough, tiles, false, rounds_filled(tiles))) return 0;
   // The epilogue of a fused call overlaps nothing, so its last round has to be fairly full (over the bounds-checked kernel
   // behind its own copies: 0.86 from 70 per cent on, 1.02 and up to 1.6 below; medians of 130 random layers) - unless that
   // kernel would read an fp8 operand across K where it lies (0.35 to 0.6), or for int8 of some K (0.8 to 0.95).

@@ -632,7 +632,7 @@ __device__ __forceinline__ void write_wave_tile(const MfmaArgs &p, const Acc (&a
 
 // ---------------------------------------------------------------------------
 // The bounds-checked kernels' epilogue for fused calls with any activation and any 8-bit copy. Such steps - a GELU is some
-// fifty instructions - cannot be written out for each of a lane's 128 accumulators (spilled registers, code beyond the
+// forty instructions - cannot be written out for each of a lane's 128 accumulators (spilled registers, code beyond the
 // instruction cache), and accumulators cannot be indexed by a loop counter. So a wave puts 32 rows of its tile at a time
 // into LDS, the operands' stages being over, and loops over them: a lane takes four neighbouring columns of a row, the
 // same columns every time, so their biases, scales and offsets are fetched once, and C and the copy go out 16 and 4
@@ -807,7 +807,7 @@ __device__ __forceinline__ void lds_write_b128(unsigned to, V4 four) {
 // The streaming kernel's epilogue: one wave writes its MI x NI blocks, of which a lane holds four consecutive columns of a row at a
 // time (acc[i][j][4 g + e]: row S i + lane % S, column S j + 8 g + 4 (lane / S) + e). The operands' ring being over, the rows of one row
 // of blocks at a time go to LDS as they are, and a loop takes them from there in the order that C wants: a wave's rows of 128 (64)
-// columns in whole lines, 16 bytes per lane. A loop, because what is behind it - a GELU is some fifty instructions - cannot be written
+// columns in whole lines, 16 bytes per lane. A loop, because what is behind it - a GELU is some forty instructions - cannot be written
 // out for each of a lane's 256 sums: eight copies of the loop, one behind every row of blocks, are 250 KB of code and were three times
 // as slow (E4M3 2048 x 8192 x 2048 with GELU into E4M3, all of it 137 us). And whole lines, because the sums as they lie make pieces of 64
 // bytes (32 x 32 blocks: 32 bytes), which took 17.5 us for the 64 MiB of 4096^2 (with 32 x 32 blocks 35).
@@ -1576,11 +1576,11 @@ __global__ void __launch_bounds__(WAVES_M *WAVES_N * 64, (BM == 64 ? 2 : 4)) gem
 // 64 x 16 bytes as one contiguous KiB of LDS, so tiles are stored without
 // padding and bank conflicts are avoided by an XOR swizzle of the 16-byte
 // chunk index instead; the swizzle is applied on the global side (which chunk
-// a lane fetches) and again by the fragment reads. Four waves, one per SIMD, a
-// quarter of the tile each, so that every byte in LDS is read by two waves
-// (eight waves of a quarter of the columns read a half more; bf16 with K
+// a lane fetches) and again by the fragment reads. Four waves, one per
+// SIMD, a quarter of the tile each, so that every byte in LDS is read by two
+// waves (eight waves of a quarter of the columns read a half more; bf16 with K
 // contiguous, us, eight waves of 32 x 32 products / this: 8192^3 843 / 721,
-// 4096^3 115 / 97.5).
+// 4096^3 115 / 97.5), or eight, two per SIMD (ring_waves).
 //
 // An MN-contiguous operand (k-rows of ROWS elements) is loaded a slice at a
 // time: a load covers whole k-rows, i.e. whole 128-byte lines. A K-contiguous
@@ -1612,6 +1612,7 @@ constexpr int ring_waves() {  // 0: ring_waves_by_size
   constexpr bool fp8 = TA == SKL_DT_F8E4M3 || TA == SKL_DT_F8E5M2;
   if (fp8 && !EXACT && BN == 256) return 4;
   if (SCAN) return fp8 && ring_few_issue_slots(1, A_KC, B_KC, BN) ? 8 : 4;
+  if (EXACT && BN == 256 && !EDGE && !STEPS) return 0;
   return fp8 || EDGE || STEPS ? 8 : 0;
 }
 // Of them side by side: two; eight of 256 x 256 tiles four where that holds fewer widened fragments (EXACT; the other way 34 registers
@@ -1876,8 +1877,8 @@ constexpr int ceil_div(int a, int b) { return (a + b - 1) / b; }
 // EXACT: OCP fp8 operands multiplied exactly (MmaF8Exact). The bytes travel like int8's; a fragment is widened behind the
 // products in front of its first use, for each half of its bytes anew, A's a row of blocks ahead, B's half a step. A wave widens
 // MI + NI fragments for MI x NI products - on the 128 x 128 kernels, with 64 x 32 per wave, three for two, which is
-// more vector work than the matrix cores take for the products; here sixteen for 64 (256 columns) or twelve for 32 (128).
-// E4M3 2048 x 8192 x 2048: 77 us there, 62 with eight waves of 32 x 32 products here; with a bias, into E4M3, 73 so and now 59.
+// more vector work than the matrix cores take for the products; here twelve for 32 (256 columns) or eight for 16 (128).
+// E4M3 2048 x 8192 x 2048: 77 us there, 62 with eight waves of 32 x 32 products here; with a bias, into E4M3, 73 so and now 56.
 template <int TA, int TB, bool A_KC, bool B_KC, int BN, bool EDGE, bool STEPS, bool SCAN, bool EXACT, int WAVES>
 __global__ void __launch_bounds__((WAVES * 64)) gemm_mfma_ring_kernel(MfmaArgs p) {
   constexpr bool kLarge = TA == SKL_DT_I8 && ring_few_issue_slots(1, A_KC, B_KC, BN);
@@ -2371,16 +2372,18 @@ inline bool c_in_row_quads(const MfmaArgs &p) {
          (((uintptr_t)p.c | (p.rsc0 * 4) | (p.rsc1 * 4) | (p.csc1 * 4)) & 15) == 0;
 }
 
-// The waves of plain products on whole tiles, int8 or 16 bits (see ring_waves): 256 x 256 tiles take eight only for C that is read over
+// The waves of plain products on whole tiles, int8, 16 bits or exact fp8 (see ring_waves): 256 x 256 tiles of exact fp8 take four only for C
+// that is read in one round (E4M3 4096^2 x 512 34 / 36 us, x 2048 63 / 67), those of the others eight only for C that is read over
 // two rounds, or more with a short K (us, four / eight: 4096 x 8192 x 512 int8 73 / 62, bf16 84 / 74, x 2048 104 / 97, 148 / 144; 8192^2 x 1024 int8
 // 162 / 156, but x 2048 198 / 204; one round, 4096^2 x 512, 29 / 33); 256 x 128 tiles below the K from which the main loop is what counts - except
 // int8 read across K on both sides, whose 32 x 32 products are four waves' (2048 x 4096^2 36.2 / 37.9 us).
-template <typename AccElem, bool A_KC, bool B_KC, int BN>
+template <typename AccElem, bool A_KC, bool B_KC, int BN, bool EXACT>
 int ring_waves_by_size(const MfmaArgs &p) {
   constexpr bool kInt = std::is_same<AccElem, int>::value;
   const bool reads_c = kInt ? p.beta.i != 0 : !(p.beta.fz.skip_c_read && p.beta.f == 0.0f);
   if (BN == 256) {
     const size_t tiles = (p.m / 256) * (p.n / 256);
+    if (EXACT) return reads_c && tiles <= 256 ? 4 : 8;
     return reads_c && tiles > 256 && (tiles <= 512 || p.k * (kInt ? 1 : 2) < 2048) ? 8 : 4;
   }
   if (kInt) return !A_KC && !B_KC ? 4 : p.k < (reads_c ? 4096 : 2048) ? 8 : 4;
@@ -2413,7 +2416,7 @@ int launch_ring(const MfmaArgs &args) {
   if constexpr (WAVES == 0) {
     constexpr int waves = ring_waves<TA, A_KC, B_KC, BN, EDGE, STEPS, SCAN, EXACT>();
     if constexpr (waves != 0) return launch_ring<TA, TB, A_KC, B_KC, BN, EDGE, STEPS, SCAN, EXACT, waves>(args);
-    else if (ring_waves_by_size<AccElem, A_KC, B_KC, BN>(args) == 8) return launch_ring<TA, TB, A_KC, B_KC, BN, EDGE, STEPS, SCAN, EXACT, 8>(args);
+    else if (ring_waves_by_size<AccElem, A_KC, B_KC, BN, EXACT>(args) == 8) return launch_ring<TA, TB, A_KC, B_KC, BN, EDGE, STEPS, SCAN, EXACT, 8>(args);
     else return launch_ring<TA, TB, A_KC, B_KC, BN, EDGE, STEPS, SCAN, EXACT, 4>(args);
   } else {
   constexpr int lds = (ring_stages_a(A_KC, B_KC, BN, SCAN) * 256 + ring_stages_b(A_KC, B_KC, BN, SCAN) * BN) * kRingSlice + (SCAN ? 4 * WAVES * 1024 : 0);
@@ -2568,7 +2571,7 @@ inline bool reads_old_c(const MfmaArgs &p, bool is_int) { return is_int ? p.beta
 
 // Whether the streaming kernel beats the bounds-checked ones on whole tiles: those have several workgroups on a compute unit, whose
 // starts and ends overlap with others' products, it has one. What decides is how full its last round is, how much K there is to gain
-// on, and whether C is read, which it requests earlier than the others do; an activation of some thirty or forty instructions (SiLU,
+// on, and whether C is read, which it requests earlier than the others do; an activation of some twenty or forty instructions (SiLU,
 // GELU) is covered by less there. Its time over theirs, geometric means over 720 random problems, by K in bytes; more than one round, by
 // `filled` (50-60 / 60-70 / 70-80 / 80-90 / 90-100 per cent); "-": none drawn:
 //   16 bits, plain        from  512  1.17  -   1.01 1.07 1.07   from 1024  1.16 1.11 0.89 0.99 0.94   from 2048   -   1.00 0.84 0.85 0.91   from 4096  -   0.93 -  0.83 0.80
@@ -2591,8 +2594,9 @@ inline bool reads_old_c(const MfmaArgs &p, bool is_int) { return is_int ? p.beta
 // A single round of 200 to 256 tiles: 16 bits plain 1.07 below 1024, short fp8 1.01, all others 0.65 to 0.97. 129 to 199 tiles: 0.64 to 0.98,
 // everything. 96 to 128 tiles, half of the chip: plain 1.09 (16 bits), 1.06 (fp8), 1.33 (short fp8) and 1.06 to 1.10 (int8) below 4096, from there on
 // 0.78 to 0.81, C read 0.76 to 0.93, a copy 0.72 to 0.90, short fp8 with SiLU or GELU 1.07. With a K of 8 KiB and more also 65 to 128 tiles with steps,
-// which share K, 0.78; exactly 64 are 128 bounds-checked tiles, which share it four ways: 1.12 to 1.24.
-inline bool ring_pays(const MfmaArgs &p, const RingKind &kind, size_t tiles, bool long_k, unsigned filled) {
+// which share K, 0.78; exactly 64 are 128 bounds-checked tiles, which share it four ways: 1.12 to 1.24. Several rounds of 256 x 128 tiles (N no
+// multiple of 256) below 2 KiB of K: plain 1.08 (16 bits), 1.05 to 1.15 (short fp8), 1.11 (int8), int8 with ReLU 1.09, SiLU or GELU 0.99.
+inline bool ring_pays(const MfmaArgs &p, const RingKind &kind, bool wide, size_t tiles, bool long_k, unsigned filled) {
   const bool slow_others = kind.fp8 && !kind.exact && !(kind.a_kc && kind.b_kc);  // transposed fragments of 32 bytes: they take two to four times as long
   constexpr unsigned kNever = 101;
   const size_t k_bytes = p.k * kind.es;
@@ -2608,12 +2612,13 @@ inline bool ring_pays(const MfmaArgs &p, const RingKind &kind, size_t tiles, boo
   }
   if (tiles <= 256) return reads_c || steps || kind.is_int || k_bytes >= 1024;
   if (slow_others || (!in_rows && (!kind.exact || steps) && !p.rq.q_only)) return true;
+  if (!wide && k_bytes < 2048 && !reads_c && !p.rq.q && !(steps && !kind.is_int)) return false;
   if (many_steps) {
     if (reads_c) return filled >= (k_bytes >= 4096 ? 0 : k_bytes >= 2048 ? 70 : k_bytes >= 1024 ? 80 : kNever);
-    return filled >= (k_bytes >= 8192 ? 0 : k_bytes >= 4096 || (k_bytes >= 2048 && kind.es == 2) ? 60 : 80);
+    return filled >= (k_bytes >= 8192 ? 0 : k_bytes >= 4096 || (k_bytes >= 2048 && kind.es == 2) ? 60 : wide || k_bytes >= 2048 ? 80 : 90);
   }
   if (kind.exact) return filled >= (reads_c || p.rq.q ? 70 : 80);
-  if (kind.is_int) return reads_c || p.rq.q || filled >= (k_bytes >= 2048 ? 0 : k_bytes >= 1024 ? steps ? 90 : 70 : kNever);
+  if (kind.is_int) return reads_c || steps || filled >= (k_bytes >= 2048 ? 0 : k_bytes >= 1024 ? 70 : kNever);
   return steps || filled >= (k_bytes >= 2048 ? 0 : k_bytes >= 1024 ? reads_c ? 60 : 70 : reads_c ? 80 : kNever);
 }
 
@@ -2642,7 +2647,7 @@ inline WholeTiles whole_tiles(const MfmaArgs &p, const RingKind &kind) {
   const bool wide = tiles >= 200, tail_round = rest != 0 && rest <= 128 && rest % tiles_m == 0;
   const bool long_k = slices % 4 == 0 && slices / 2 >= kRingMinSlicesPerSplit;
   if (!wide && tiles128 < 96 && !(tiles128 >= 64 && long_k)) return {0, 0};
-  if (!ring_pays(p, kind, wide ? tiles : tiles128, long_k, wide ? rounds_filled(tiles, tail_round) : rounds_filled(tiles128))) return {0, 0};
+  if (!ring_pays(p, kind, wide, wide ? tiles : tiles128, long_k, wide ? rounds_filled(tiles, tail_round) : rounds_filled(tiles128))) return {0, 0};
   return {wide ? 256 : 128, wide && tail_round ? rest : 0};
 }
 
@@ -2747,8 +2752,8 @@ int launch_tile(const MfmaArgs &p) {
   constexpr bool kFp8 = TA == SKL_DT_F8E4M3 || TA == SKL_DT_F8E5M2;
   if constexpr (kFp8) {
     // short K: exact products (see MmaF8Exact), on the streaming kernel when its tiles fill the chip and ring_pays() (us,
-    // bounds-checked 128 x 128 / streaming: 2048 x 8192 x 2048 77 / 62, with GELU into E4M3 111 / 94; 2048 x 4096 x 2048
-    // 42 / 34; on 128 tiles, 512 x 8192 x 2048, 25.4 / 26.2)
+    // bounds-checked 128 x 128 / streaming: 2048 x 8192 x 2048 77 / 56, 2048 x 4096 x 2048 42 / 33; on 128 tiles,
+    // 512 x 8192 x 2048, 25.4 / 26.2)
     if (p.k <= kF8ExactMaxK || few_off_rule<ES>(p)) {
       const int rc = launch_whole_tiles<TA, TB, A_KC, B_KC, true>(p);  // (not of operands off the 16-byte rule)
       if (rc != kNotWholeTiles) return rc;

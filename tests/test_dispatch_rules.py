@@ -187,7 +187,9 @@ def test_whole_tiles_go_where_they_were_measured_to_be_faster():
         assert route(kind, 4352, 1024, k) == 128 and route(kind, 4352, 1024, k, beta=1) == 128                       # 136
         assert route(kind, 4096, 3328, k, act=1, q=0 if kind == I8 else 2) == 256                                    # 208 of 256 x 256
     assert route(I8, 4096, 1024, 1024, beta=1) == 128 and route(BF16, 4096, 1024, 512, beta=1) == 128
-    assert route(I8, 7424, 7168, 512, act=1, q=0) == 256 and route(I8, 7424, 7168, 512, act=1) == 1                  # 812: a copy, ReLU into C
+    assert route(I8, 7424, 7168, 512, act=1, q=0) == 256 and route(I8, 7424, 7040, 512, act=1, q=0) == 128           # 812, and 1595 of 256 x 128
+    assert route(I8, 7424, 7168, 512, act=1) == 256 and route(I8, 7424, 7040, 512, act=1) == 1                       # ReLU into C
+    assert route(BF16, 7424, 7040, 512) == 1 and route(BF16, 7424, 7040, 1024) == 128                                # from 2 KiB of K on
     assert route(I8, 8192, 8192, 1024) == 256 and route(I8, 7424, 7168, 512) == 1
     assert route(E4M3, 8192, 12032, 640) == 256 and route(E4M3, 4352, 4608, 640) == 1                                # 1504 and 306 of 256 x 256
 
