@@ -2595,7 +2595,8 @@ inline bool reads_old_c(const MfmaArgs &p, bool is_int) { return is_int ? p.beta
 // everything. 96 to 128 tiles, half of the chip: plain 1.09 (16 bits), 1.06 (fp8), 1.33 (short fp8) and 1.06 to 1.10 (int8) below 4096, from there on
 // 0.78 to 0.81, C read 0.76 to 0.93, a copy 0.72 to 0.90, short fp8 with SiLU or GELU 1.07. With a K of 8 KiB and more also 65 to 128 tiles with steps,
 // which share K, 0.78; exactly 64 are 128 bounds-checked tiles, which share it four ways: 1.12 to 1.24. Several rounds of 256 x 128 tiles (N no
-// multiple of 256) below 2 KiB of K: plain 1.08 (16 bits), 1.05 to 1.15 (short fp8), 1.11 (int8), int8 with ReLU 1.09, SiLU or GELU 0.99.
+// multiple of 256) below 2 KiB of K: plain 1.08 (16 bits), 1.05 to 1.15 (short fp8), 1.11 (int8), int8 with ReLU 1.09, SiLU or GELU
+// 0.99 (80 to 90 per cent 1.02), with a copy there 0.84 to 0.94.
 inline bool ring_pays(const MfmaArgs &p, const RingKind &kind, bool wide, size_t tiles, bool long_k, unsigned filled) {
   const bool slow_others = kind.fp8 && !kind.exact && !(kind.a_kc && kind.b_kc);  // transposed fragments of 32 bytes: they take two to four times as long
   constexpr unsigned kNever = 101;
@@ -2615,7 +2616,7 @@ inline bool ring_pays(const MfmaArgs &p, const RingKind &kind, bool wide, size_t
   if (!wide && k_bytes < 2048 && !reads_c && !p.rq.q && !(steps && !kind.is_int)) return false;
   if (many_steps) {
     if (reads_c) return filled >= (k_bytes >= 4096 ? 0 : k_bytes >= 2048 ? 70 : k_bytes >= 1024 ? 80 : kNever);
-    return filled >= (k_bytes >= 8192 ? 0 : k_bytes >= 4096 || (k_bytes >= 2048 && kind.es == 2) ? 60 : wide || k_bytes >= 2048 ? 80 : 90);
+    return filled >= (k_bytes >= 8192 ? 0 : k_bytes >= 4096 || (k_bytes >= 2048 && kind.es == 2) ? 60 : wide || k_bytes >= 2048 || p.rq.q ? 80 : 90);
   }
   if (kind.exact) return filled >= (reads_c || p.rq.q ? 70 : 80);
   if (kind.is_int) return reads_c || steps || filled >= (k_bytes >= 2048 ? 0 : k_bytes >= 1024 ? 70 : kNever);

@@ -192,6 +192,8 @@ def test_whole_tiles_go_where_they_were_measured_to_be_faster():
     assert route(BF16, 7424, 7040, 512) == 1 and route(BF16, 7424, 7040, 1024) == 128                                # from 2 KiB of K on
     assert route(I8, 8192, 8192, 1024) == 256 and route(I8, 7424, 7168, 512) == 1
     assert route(E4M3, 8192, 12032, 640) == 256 and route(E4M3, 4352, 4608, 640) == 1                                # 1504 and 306 of 256 x 256
+    for kind in (BF16, F16, E4M3):                                                                                   # GELU on 651 of 256 x 128, 2.5 rounds
+        assert route(kind, 7936, 2688, 640, b_rows=False, act=3, q=2) == 128 and route(kind, 7936, 2688, 640, b_rows=False, act=3) == 1
 
 
 @pytest.mark.parametrize("kind", (I8, BF16, F16, E4M3))
