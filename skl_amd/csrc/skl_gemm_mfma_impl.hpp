@@ -842,13 +842,14 @@ __device__ __forceinline__ void write_wave_rows(const MfmaArgs &p, const Acc (&a
   const skl_fp8::Ofp8Format f8(p.rq.q_fmt);
   // Which way the stores go. Through the caches they are the faster ones (us, through / past: 4096 x 8192 x 512 bf16 48.4 / 59.1, int8 of
   // 8192^2 x 2048 134 / 147, E4M3 212 / 227, one round of 64 MiB, 2048 x 8192 x 512, 27.0 / 30.6), as long as the 256 MiB behind them
-  // hold all that is written (8192 x 8448 x 2048 bf16 253 / 235, int8 149 / 142; 8192 x 12288 x 512 148 / 130) with what the next round reads
-  // (the same at 8192^2 and 4 KiB of K). Little is better past them: it would still lie in the L2s, which are written back when the kernel
+  // hold all that is written (8192 x 8448 x 2048 bf16 253 / 235, int8 149 / 142; 8192 x 12288 x 512 148 / 130) and A and B, which are
+  // read again and again, are no more than half of that (E4M3 of 8192^2 by 4096, 6144 and 8192: 223 / 228, 310 / 312, 396 / 392; 4096 x 14336
+  // by 8192, 144 MiB: 359 / 347, int8 361 / 345). Little is better past them: it would still lie in the L2s, which are written back when the kernel
   // ends (4352 x 1024 x 512 int8 9.6 / 8.5, bf16 12.8 / 11.3; 2048 x 4096 x 512 16.5 / 15.1). A C that is read meets its stores there
   // when there are several rounds (8192^2 x 512 bf16 178 / 154), not in one (2048 x 8192 x 512 39 / 42).
   const bool one_round = p.tiles_m * p.tiles_n <= 256;
   const size_t written = p.m * p.n * ((p.rq.q_only ? 0 : 4) + (p.rq.q ? 1 : 0));
-  const bool fits = written > (size_t(48) << 20) && written <= (size_t(256) << 20) && (p.m + p.n) * p.k * ES + written < (size_t(320) << 20);
+  const bool fits = written > (size_t(48) << 20) && written <= (size_t(256) << 20) && (p.m + p.n) * p.k * ES <= (size_t(128) << 20);
 
   // Row of blocks i's sums to LDS (accumulators cannot be indexed: a branch for each).
   const auto put = [&](unsigned i) __attribute__((always_inline)) {
