@@ -220,8 +220,8 @@ constexpr size_t kF8ExactMaxK = 2304;
 
 // What the streaming kernel multiplies with: blocks of SIDE x SIDE, 64 bytes of K. The instructions take B's columns as their
 // first operand, A's rows as their second, so that a lane holds four consecutive columns of a row of C: 16 bytes of a row-major C.
-// 16 x 16 blocks take the device a seventh less energy per product than 32 x 32 ones (instructions alone on random operands, P/s for
-// 32 x 32 / 16 x 16: bf16 1.67 / 1.86, f16 1.55 / 1.75, int8 3.18 / 3.69), with the same error against 64 bits.
+// 16 x 16 blocks run no slower by themselves than 32 x 32 ones (instructions alone on random operands, P/s for 32 x 32 / 16 x 16: bf16
+// 1.75 / 1.75, f16 1.62 / 1.66, int8 3.32 / 3.49), their sums are there after half as many passes, and the error against 64 bits is the same.
 // Written in assembly for the registers' sake: a wave's operands are vector registers that LDS reads under way will write, its sums
 // accumulation registers, and left to itself the compiler moves both about. Of the 256 sums per lane of a 256 x 256 tile a few are
 // vector registers (IN_A false): where all accumulation registers are taken the compiler copies a block out and back around a
